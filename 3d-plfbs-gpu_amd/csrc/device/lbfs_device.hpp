@@ -10,9 +10,8 @@
 // the reference's flux sums are exactly
 //   sum_k e_k f_k       = (1 - tau) rho_I u_I + tau S1      (= S1, since rho_I u_I = S1)
 //   sum_k e_k e_k^T f_k = (1 - tau) rho_I (I/3 + u_I u_I^T / gamma) + tau Pi
-// so only S0, S1 and Pi are needed.  They are accumulated as unweighted
-// pair sums per lattice weight class (13 values in registers) and weighted
-// once per face.
+// so only S0, S1 and Pi are needed, summed from the pairs of opposite points and
+// weighted once per face.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -121,7 +120,7 @@ struct DevMesh {
 };
 
 struct DevParams {
-    double visc, gamma, invgam, visc3_invgam, force, cfl, ceff, ref_rho, ref_mom, tol;
+    double visc, gamma, invgam, visc3_invgam, c45, c15, force, cfl, ceff, ref_rho, ref_mom, tol;
     double rho0;  // FP32 storage: density offset (rho = rho0 + stored value)
     int time_stepping;
     int use_body_force;
@@ -228,97 +227,118 @@ __device__ __forceinline__ void ghost_grad(const DevPatch &P, const T n[3], T dm
 // Lattice evaluation (src/Solver.cpp:840-1374 restructured as moments)
 // ---------------------------------------------------------------------------
 
-// Unweighted pair sums h = feq / w.  Each axis pair (weight 1/9) feeds
-// exactly one component of each moment, so its sum S and difference D are kept
-// as they are; the four body diagonals (weight 1/72) all feed S0 and every
-// diagonal of Pi with the same sum, which is therefore accumulated once.  The
-// weights are applied once per face.
-template <typename T>
-struct PairSums {
-    T ax_s[3], ax_d[3];           // axis pairs x, y, z: S and D
-    T dg_s, dg_x, dg_y, dg_z;     // diagonals: sum S, sum e_a D
-    T dg_xy, dg_xz, dg_yz;        // diagonals: sum e_a e_b S
-};
-
-// Equilibrium of one lattice point e at state (r, u, v, w), divided by its
-// weight.  With DEV (FP32 storage) the density is a deviation r = rho - rho0
-// and the value returned is h = (feq - w rho0) / w = r (1 + X) + rho0 X,
-// X = 3 e.u + (4.5 (e.u)^2 - 1.5 u^2)/gamma, so the O(1) part rho0 never enters
-// single precision.
-template <int EX, int EY, int EZ, bool DEV, typename T>
-__device__ __forceinline__ T pop_eq(T r, T u, T v, T w, T c45, T c15, T rho0) {
-    const T eu = (T)EX * u + (T)EY * v + (T)EZ * w;
-    const T usq = u * u + v * v + w * w;
-    // X = 3 e.u + (4.5 (e.u)^2 - 1.5 u^2) / gamma, as e.u (3 + c45 e.u) - c15 u^2
-    // with c45 = 4.5 / gamma and c15 = 1.5 / gamma
-    const T X = eu * ((T)3 + c45 * eu) - c15 * usq;
-    if constexpr (DEV) return r + (r + rho0) * X;
-    else return r + r * X;
-}
-
 // e.g of one lattice direction from a gradient triple g (x, y, z) and its sum
 // s = gx + gy + gz: the four body diagonals share s.
 template <int EX, int EY, int EZ, typename T>
 __device__ __forceinline__ T dir_deriv(const T *g, T s) {
     if constexpr (EX != 0 && EY != 0 && EZ != 0) {
-        // EX, EY, EZ in {+-1}: at most one of them is -1 in kLatticePairs' order
+        // EX, EY, EZ in {+-1}: at most one of them is -1 in the pairs' order
         if constexpr (EX < 0) return s - (T)2 * g[0];
         else if constexpr (EY < 0) return s - (T)2 * g[1];
         else if constexpr (EZ < 0) return s - (T)2 * g[2];
         else return s;
     } else {
-        return (T)EX * g[0] + (T)EY * g[1] + (T)EZ * g[2];
+        // (no products with zero: the compiler may not drop them, 0 x inf is NaN)
+        return g[EX ? 0 : (EY ? 1 : 2)];
     }
 }
 
-// Lattice pair +e / -e (pair index P, order of kLatticePairs).  Point +e takes
-// the neighbour side iff e.n < 0 and point -e iff e.n > 0 (the reference's "sum
-// of signed normal components > 0" tests, src/Solver.cpp:958-1273).  The two
-// decisions per pair are precomputed on the host in FP64 (bits 2P and 2P+1 of
-// `side`): for faces containing a lattice direction, e.n is zero analytically
-// and its sign is rounding noise, so evaluating it in another precision would
-// pick the other side.  The pair enters the moments through its sum
-// S = h(+e) + h(-e) (even moments) and difference D = h(+e) - h(-e) (odd ones).
-template <int P, int EX, int EY, int EZ, bool DEV, typename T>
-__device__ __forceinline__ void lattice_pair(PairSums<T> &M, unsigned side, T dt, const T pI[4], const T gO[12],
-                                             const T sO[4], const T pN[4], const T gN[12], const T sN[4], T c45,
-                                             T c15, T rho0) {
-    const bool up = (side >> (2 * P)) & 1u;      // +e point from the neighbour side
-    const bool dn = (side >> (2 * P + 1)) & 1u;  // -e point from the neighbour side
-    T a[4], b[4];
+// e.u of a lattice direction (axis directions are +1 here).
+template <int EX, int EY, int EZ, typename T>
+__device__ __forceinline__ T dir_dot(T u, T v, T w) {
+    if constexpr (EX == 0 && EY == 0 && EZ == 0) return (T)0;
+    else if constexpr (EX != 0 && EY != 0 && EZ != 0) return (T)EX * u + (T)EY * v + (T)EZ * w;
+    else return EX ? u : (EY ? v : w);
+}
+
+// Equilibrium at state (r, u, v, w) divided by the lattice weight, for the
+// direction +-e with s3 = +-3.  With DEV (FP32 storage) the density is a deviation
+// r = rho - rho0 and the value returned is h = (feq - w rho0) / w =
+// r (1 + X) + rho0 X, X = 3 e.u + (4.5 (e.u)^2 - 1.5 u^2)/gamma, so the O(1) part
+// rho0 never enters single precision.
+template <int EX, int EY, int EZ, bool DEV, typename T>
+__device__ __forceinline__ T pop_eq(T r, T u, T v, T w, T s3, T c45, T c15, T rho0) {
+    const T eu = dir_dot<EX, EY, EZ, T>(u, v, w);
+    const T usq = u * u + v * v + w * w;
+    // X = +-3 e.u + (4.5 (e.u)^2 - 1.5 u^2) / gamma, as e.u (s3 + c45 e.u) - c15 u^2
+    // with c45 = 4.5 / gamma and c15 = 1.5 / gamma
+    const bool rest = EX == 0 && EY == 0 && EZ == 0;
+    const T X = rest ? -(c15 * usq) : eu * (s3 + c45 * eu) - c15 * usq;
+    if constexpr (DEV) return r + (r + rho0) * X;
+    else return r + r * X;
+}
+
+// Passes a value through an empty asm statement (no instruction is emitted), so
+// that what follows is not merged with another use of the same value.
+template <typename T>
+__device__ __forceinline__ T opaque(T x) {
+    asm volatile("" : "+v"(x));
+    return x;
+}
+
+// x with its sign flipped where bit k of `bits` is set.
+template <typename T>
+__device__ __forceinline__ T flip_sign(T x, unsigned bits, int k) {
+    const unsigned m = (bits << (31 - k)) & 0x80000000u;
+    if constexpr (std::is_same<T, float>::value) return __uint_as_float(__float_as_uint(x) ^ m);
+    else return __hiloint2double(__double2hiint(x) ^ (int)m, __double2loint(x));
+}
+
+// Lattice pairs +e / -e (pair index P: x, y, z, then the four body diagonals).
+// Point +e takes the neighbour side iff e.n < 0 and point -e iff e.n > 0 (the
+// reference's "sum of signed normal components > 0" tests,
+// src/Solver.cpp:958-1273).  So with d = e or -e, whichever points from the owner
+// to the neighbour, +d always comes from the owner side and -d from the neighbour
+// side, except where e.n = 0: there both come from the owner side.  The host
+// decides both in FP64: bit P of `side` is set where d = -e (e.n < 0), bit 7 + P
+// where e.n = 0.  (For faces containing a lattice direction e.n is zero
+// analytically and its sign is rounding noise, so evaluating it in another
+// precision would pick the other side.)
+//
+// One side's seven points, h[P] at +d (OUT) or -d of every pair: p is the side's
+// state at the face centre, g its gradient.
+constexpr int kPairs = 7;
+
+//
+// The owner side's pass replaces hb[P], the neighbour side's value at -d, by its own
+// where e.n = 0; a wavefront without such a face skips that by a scalar branch.
+template <int P, int EX, int EY, int EZ, bool OUT, bool DEV, typename T>
+__device__ __forceinline__ void side_point(unsigned side, T dt, const T p[4], const T g[12], const T s[4], T c45,
+                                           T c15, T rho0, T *h, T *hb) {
+    // the point that streams along +-d starts at -(+-d) dt from the face centre; +-d is e times a sign
+    const T tau = opaque(flip_sign<T>(OUT ? -dt : dt, side, P));
+    const T s3 = flip_sign<T>(OUT ? (T)3 : (T)-3, side, P);
+    T d[4];
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
-        const T po = dir_deriv<EX, EY, EZ, T>(gO + 3 * q, sO[q]);
-        const T pn = dir_deriv<EX, EY, EZ, T>(gN + 3 * q, sN[q]);
-        a[q] = up ? (pN[q] - pn * dt) : (pI[q] - po * dt);
-        b[q] = dn ? (pN[q] + pn * dt) : (pI[q] + po * dt);
+    for (int q = 0; q < 4; q++) d[q] = dir_deriv<EX, EY, EZ, T>(g + 3 * q, s[q]);
+    // one point after the other (tau and h are passed through opaque in this
+    // order): interleaved for instruction-level parallelism, which other wavefronts
+    // provide already, the points would take some 40 registers more
+    h[P] = opaque(pop_eq<EX, EY, EZ, DEV, T>(p[0] + tau * d[0], p[1] + tau * d[1], p[2] + tau * d[2],
+                                             p[3] + tau * d[3], s3, c45, c15, rho0));
+    if constexpr (OUT) {
+        const bool both = (side >> (kPairs + P)) & 1u;
+        if (__builtin_amdgcn_ballot_w64(both) != 0) {
+            const T ho = pop_eq<EX, EY, EZ, DEV, T>(p[0] - tau * d[0], p[1] - tau * d[1], p[2] - tau * d[2],
+                                                    p[3] - tau * d[3], -s3, c45, c15, rho0);
+            hb[P] = both ? ho : hb[P];
+        }
     }
-    const T fp = pop_eq<EX, EY, EZ, DEV, T>(a[0], a[1], a[2], a[3], c45, c15, rho0);
-    const T fm = pop_eq<-EX, -EY, -EZ, DEV, T>(b[0], b[1], b[2], b[3], c45, c15, rho0);
-    const T S = fp + fm, D = fp - fm;
-    if constexpr (EX == 0 || EY == 0 || EZ == 0) {
-        constexpr int ax = EX ? 0 : (EY ? 1 : 2);
-        M.ax_s[ax] = S;
-        M.ax_d[ax] = D;
-    } else if constexpr (P == 3) {
-        // the first diagonal (+1, +1, +1) starts the sums
-        static_assert(EX == 1 && EY == 1 && EZ == 1, "pair 3 is the (+1, +1, +1) diagonal");
-        M.dg_s = S;
-        M.dg_x = D;
-        M.dg_y = D;
-        M.dg_z = D;
-        M.dg_xy = S;
-        M.dg_xz = S;
-        M.dg_yz = S;
-    } else {
-        M.dg_s += S;
-        M.dg_x += (T)EX * D;
-        M.dg_y += (T)EY * D;
-        M.dg_z += (T)EZ * D;
-        M.dg_xy += (T)(EX * EY) * S;
-        M.dg_xz += (T)(EX * EZ) * S;
-        M.dg_yz += (T)(EY * EZ) * S;
-    }
+}
+
+template <bool OUT, bool DEV, typename T>
+__device__ __forceinline__ void side_points(unsigned side, T dt, const T p[4], const T g[12], T c45, T c15, T rho0,
+                                            T h[kPairs], T hb[kPairs]) {
+    T s[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) s[q] = g[3 * q] + g[3 * q + 1] + g[3 * q + 2];
+    side_point<0, 1, 0, 0, OUT, DEV, T>(side, dt, p, g, s, c45, c15, rho0, h, hb);
+    side_point<1, 0, 1, 0, OUT, DEV, T>(side, dt, p, g, s, c45, c15, rho0, h, hb);
+    side_point<2, 0, 0, 1, OUT, DEV, T>(side, dt, p, g, s, c45, c15, rho0, h, hb);
+    side_point<3, 1, 1, 1, OUT, DEV, T>(side, dt, p, g, s, c45, c15, rho0, h, hb);
+    side_point<4, 1, 1, -1, OUT, DEV, T>(side, dt, p, g, s, c45, c15, rho0, h, hb);
+    side_point<5, 1, -1, 1, OUT, DEV, T>(side, dt, p, g, s, c45, c15, rho0, h, hb);
+    side_point<6, -1, 1, 1, OUT, DEV, T>(side, dt, p, g, s, c45, c15, rho0, h, hb);
 }
 
 // Reciprocal: correctly rounded in FP64; in FP32 the hardware estimate
@@ -333,35 +353,40 @@ __device__ __forceinline__ T lattice_rcp(T x) {
 // is passed as its parts v3g / dt.  With DEV the momentum flux omits the
 // constant rho0/3 n A, whose sum over a cell's faces is a per-cell geometric
 // constant added separately.
+//
+// The two sides are evaluated one after the other, seven points each, so only one
+// side's gradient is live with the other side's seven values.  Evaluating only
+// the side each point comes from (instead of both, and a select) halves the
+// reconstruction.  The second evaluation that e.n = 0 needs is skipped by a
+// wavefront without such a face (all interior faces of a jittered mesh).
 template <bool DEV, typename T>
 __device__ __forceinline__ void lattice_flux(const T n[3], T A, T dt, T v3g, unsigned side, const T p0[4],
                                              const T pI[4], const T gO[12], const T pN[4], const T gN[12], T invgam,
-                                             T rho0, T F[4]) {
-    PairSums<T> M;
+                                             T c45, T c15, T rho0, T F[4]) {
     const T w0 = (T)(2.0 / 9.0), w1 = (T)(1.0 / 9.0), w7 = (T)(1.0 / 72.0);
-    const T c45 = (T)4.5 * invgam, c15 = (T)1.5 * invgam;
-    T sO[4], sN[4];
+    const T h0 = pop_eq<0, 0, 0, DEV, T>(p0[0], p0[1], p0[2], p0[3], (T)3, c45, c15, rho0);
+    __builtin_amdgcn_sched_barrier(0);
+    T ha[kPairs], hb[kPairs];
+    side_points<false, DEV, T>(side, dt, pN, gN, c45, c15, rho0, hb, hb);
+    side_points<true, DEV, T>(side, dt, pI, gO, c45, c15, rho0, ha, hb);
+    // pair sums S = h(+e) + h(-e) (even moments) and differences D = h(+e) - h(-e)
+    T S[kPairs], D[kPairs];
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
-        sO[q] = gO[3 * q] + gO[3 * q + 1] + gO[3 * q + 2];
-        sN[q] = gN[3 * q] + gN[3 * q + 1] + gN[3 * q + 2];
+    for (int k = 0; k < kPairs; k++) {
+        S[k] = ha[k] + hb[k];
+        D[k] = flip_sign<T>(ha[k] - hb[k], side, k);
     }
-    const T h0 = pop_eq<0, 0, 0, DEV, T>(p0[0], p0[1], p0[2], p0[3], c45, c15, rho0);
-    lattice_pair<0, 1, 0, 0, DEV, T>(M, side, dt, pI, gO, sO, pN, gN, sN, c45, c15, rho0);
-    lattice_pair<1, 0, 1, 0, DEV, T>(M, side, dt, pI, gO, sO, pN, gN, sN, c45, c15, rho0);
-    lattice_pair<2, 0, 0, 1, DEV, T>(M, side, dt, pI, gO, sO, pN, gN, sN, c45, c15, rho0);
-    lattice_pair<3, 1, 1, 1, DEV, T>(M, side, dt, pI, gO, sO, pN, gN, sN, c45, c15, rho0);
-    lattice_pair<4, 1, 1, -1, DEV, T>(M, side, dt, pI, gO, sO, pN, gN, sN, c45, c15, rho0);
-    lattice_pair<5, 1, -1, 1, DEV, T>(M, side, dt, pI, gO, sO, pN, gN, sN, c45, c15, rho0);
-    lattice_pair<6, -1, 1, 1, DEV, T>(M, side, dt, pI, gO, sO, pN, gN, sN, c45, c15, rho0);
-    // weighted moments: S0, S1 and the diagonal of Pi
-    const T dS = w7 * M.dg_s;
-    const T s0 = w0 * h0 + w1 * (M.ax_s[0] + M.ax_s[1] + M.ax_s[2]) + dS;
-    const T sx = w1 * M.ax_d[0] + w7 * M.dg_x;
-    const T sy = w1 * M.ax_d[1] + w7 * M.dg_y;
-    const T sz = w1 * M.ax_d[2] + w7 * M.dg_z;
-    const T pxx = w1 * M.ax_s[0] + dS, pyy = w1 * M.ax_s[1] + dS, pzz = w1 * M.ax_s[2] + dS;
-    const T pxy = w7 * M.dg_xy, pxz = w7 * M.dg_xz, pyz = w7 * M.dg_yz;
+    // weighted moments: S0, S1 and Pi; each axis pair feeds one component of
+    // every moment, the four diagonals all of them
+    const T a = S[3] + S[4], b = S[5] + S[6], c = S[3] - S[4], d = S[5] - S[6];
+    const T e = D[3] + D[4], f = D[5] - D[6];
+    const T dS = w7 * (a + b);
+    const T s0 = w0 * h0 + w1 * (S[0] + S[1] + S[2]) + dS;
+    const T sx = w1 * D[0] + w7 * (e + f);
+    const T sy = w1 * D[1] + w7 * (e - f);
+    const T sz = w1 * D[2] + w7 * ((D[3] - D[4]) + (D[5] + D[6]));
+    const T pxx = w1 * S[0] + dS, pyy = w1 * S[1] + dS, pzz = w1 * S[2] + dS;
+    const T pxy = w7 * (a - b), pxz = w7 * (c + d), pyz = w7 * (c - d);
     const T tau = v3g * lattice_rcp(dt);
     const T rI = DEV ? rho0 + s0 : s0;
     const T ir = lattice_rcp(rI);

@@ -147,12 +147,10 @@ __global__ __launch_bounds__(kBlock) void k_flux_border(DevMesh<S> m, DevParams 
     for (int q = 0; q < 4; q++) m.bflux[q * nbd + t] = F[q];
 }
 
-// FP32: 6 waves per SIMD (80 VGPRs, no spill) instead of the compiler's 5
-// (87 VGPRs) took the 4.1M-tet flux from 0.310 to 0.301 ms.  FP64 is left to
-// the compiler (143 VGPRs, 3 waves): forcing 4 waves spills 76 B per lane and
-// measured 0.684 ms against 0.543.
+// 6 waves per SIMD in FP32 and 4 in FP64, the most that hold without spills (77
+// and 127 VGPRs).
 template <typename S>
-constexpr int kFluxMinWaves = std::is_same<S, float>::value ? 6 : 1;
+constexpr int kFluxMinWaves = std::is_same<S, float>::value ? 6 : 4;
 
 template <typename S>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kFluxMinWaves<S>))) void k_flux_update(
@@ -650,6 +648,8 @@ int create_ctx(const plbfs_mesh_view *mesh, const plbfs_params *params, const pl
     prm.gamma = p.gamma;
     prm.invgam = 1.0 / p.gamma;
     prm.visc3_invgam = p.visc * 3 / p.gamma;
+    prm.c45 = 4.5 * prm.invgam;
+    prm.c15 = 1.5 * prm.invgam;
     prm.force = p.force;
     prm.cfl = p.cfl;
     prm.ceff = p.max_velocity * std::sqrt(1 - p.gamma + std::pow(p.gamma / std::sqrt(3) / p.max_velocity, 2));

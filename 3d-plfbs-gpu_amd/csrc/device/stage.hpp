@@ -273,60 +273,65 @@ __device__ __forceinline__ void item_flux(const DevMesh<S> &m, const DevParams &
     const S A = geo[3], dt = fmin(geo[4], (S)dtcap);
     S po[4], go[12];
     ld.side(o, po, go);
-    S pI[4], pN[4], p0[4], gN[12];
-    if (nb >= 0 || nb == -1) {
-        // interior branch: a real neighbour, or the ghost whose index equals
-        // n_cells (the reference's strict "neighbour > n_cells" test, Solver.cpp:861)
+    // both sides' states at the face centre and the neighbour side's gradient
+    S pI[4], pN[4], gN[12];
+    if (nb >= 0) {
         S pn[4];
-        if (nb >= 0) {
-            ld.side(nb, pn, gN);
-        } else {
-            const DevPatch P = m.patches[m.b_patch[0]];
-            S pp[4], gp[12], fx[4] = {0, 0, 0, 0};
-            if (P.flags & kGhostGradFromCell) ld.side(m.b_partner[0], pp, gp);
+        ld.side(nb, pn, gN);
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            pI[q] = po[q] - (geo[5] * go[3 * q] + geo[6] * go[3 * q + 1] + geo[7] * go[3 * q + 2]);
+            pN[q] = pn[q] - (geo[8] * gN[3 * q] + geo[9] * gN[3 * q + 1] + geo[10] * gN[3 * q + 2]);
+        }
+    } else {
+        const int b = -1 - nb;
+        const DevPatch P = m.patches[m.b_patch[b]];
+        S pp[4] = {0, 0, 0, 0};
+        {
+            S gp[12];
+            if (P.flags & kGhostGradFromCell) ld.side(m.b_partner[b], pp, gp);
+            ghost_grad<S>(P, n, m.b_dmag[b], po, go, gp, gN);
+        }
+        if (b == 0) {
+            // reconstructed like an interior face, from the ghost: the one whose index
+            // equals n_cells (the reference's strict "neighbour > n_cells" test,
+            // Solver.cpp:861)
+            S pn[4], fx[4] = {0, 0, 0, 0};
             if (P.flags & kGhostFixed) {
                 const V4<S> f = m.b_fix[0];
                 fx[0] = f.x; fx[1] = f.y; fx[2] = f.z; fx[3] = f.w;
             }
             ghost_state<S>(P, po, pp, fx, pn);
-            ghost_grad<S>(P, n, m.b_dmag[0], po, go, gp, gN);
-        }
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
-            pI[q] = po[q] - (geo[5] * go[3 * q] + geo[6] * go[3 * q + 1] + geo[7] * go[3 * q + 2]);
-            pN[q] = pn[q] - (geo[8] * gN[3 * q] + geo[9] * gN[3 * q + 1] + geo[10] * gN[3 * q + 2]);
-            p0[q] = (pI[q] + pN[q]) * (S)0.5;
-        }
-    } else {
-        const int b = -1 - nb;
-        const DevPatch P = m.patches[m.b_patch[b]];
-        S gp[12];
-        if (P.flags & kGhostGradFromCell) {
-            S pp[4];
-            ld.side(m.b_partner[b], pp, gp);
-        }
-        ghost_grad<S>(P, n, m.b_dmag[b], po, go, gp, gN);
-        S fv[4];
-        if (P.rho_type == 1) fv[0] = (S)P.rho;
-        else if (P.rho_type == 8) fv[0] = po[0];
-        else fv[0] = po[0] - (geo[5] * gN[0] + geo[6] * gN[1] + geo[7] * gN[2]);
-        if (P.vel_type == 1) {
-            fv[1] = (S)P.u;
-            fv[2] = (S)P.v;
-            fv[3] = (S)P.w;
-        } else if (P.vel_type == 8) {
-            fv[1] = po[1];
-            fv[2] = (S)0;
-            fv[3] = po[3];
+            for (int q = 0; q < 4; q++) {
+                pI[q] = po[q] - (geo[5] * go[3 * q] + geo[6] * go[3 * q + 1] + geo[7] * go[3 * q + 2]);
+                pN[q] = pn[q] - (geo[8] * gN[3 * q] + geo[9] * gN[3 * q + 1] + geo[10] * gN[3 * q + 2]);
+            }
         } else {
+            if (P.rho_type == 1) pI[0] = (S)P.rho;
+            else if (P.rho_type == 8) pI[0] = po[0];
+            else pI[0] = po[0] - (geo[5] * gN[0] + geo[6] * gN[1] + geo[7] * gN[2]);
+            if (P.vel_type == 1) {
+                pI[1] = (S)P.u;
+                pI[2] = (S)P.v;
+                pI[3] = (S)P.w;
+            } else if (P.vel_type == 8) {
+                pI[1] = po[1];
+                pI[2] = (S)0;
+                pI[3] = po[3];
+            } else {
 #pragma unroll
-            for (int q = 1; q < 4; q++) fv[q] = po[q] - (geo[5] * gN[3 * q] + geo[6] * gN[3 * q + 1] + geo[7] * gN[3 * q + 2]);
+                for (int q = 1; q < 4; q++)
+                    pI[q] = po[q] - (geo[5] * gN[3 * q] + geo[6] * gN[3 * q + 1] + geo[7] * gN[3 * q + 2]);
+            }
+#pragma unroll
+            for (int q = 0; q < 4; q++) pN[q] = pI[q];
         }
-#pragma unroll
-        for (int q = 0; q < 4; q++) pI[q] = pN[q] = p0[q] = fv[q];
     }
+    const S p0[4] = {(pI[0] + pN[0]) * (S)0.5, (pI[1] + pN[1]) * (S)0.5, (pI[2] + pN[2]) * (S)0.5,
+                     (pI[3] + pN[3]) * (S)0.5};
     lattice_flux<std::is_same<S, float>::value, S>(n, A, dt, (S)v3g, side, p0, pI, go, pN, gN, (S)prm.invgam,
-                                                   (S)prm.rho0, F);
+                                                   (S)prm.c45, (S)prm.c15, (S)prm.rho0, F);
 }
 
 // Residual of cell i from its faces' LDS slots, summed in the reference's face

@@ -460,8 +460,8 @@ int build_layout(const plbfs_mesh_view &m, const plbfs_params &p, const plbfs_pa
             double c = 0.0;
             for (int a = 0; a < 3; a++)
                 if (kPairs[pr][a]) c = c + kPairs[pr][a] * fn[3 * f + a];
-            if (c < 0.0) side |= 1u << (2 * pr);
-            if (c > 0.0) side |= 1u << (2 * pr + 1);
+            if (c < 0.0) side |= 1u << pr;
+            else if (!(c > 0.0)) side |= 1u << (7 + pr);
         }
         L.it_side[e] = side;
         double g[kGeoPerItem];

@@ -50,10 +50,11 @@ struct Layout {
     // face work items
     std::vector<int32_t> blk_item_off;  // [n_blocks+1]
     std::vector<int32_t> it_own, it_nbr;  // [E] new owner index; neighbour new index or -1-b
-    // [E] upwind side of the 14 moving lattice points: for pair p (directions
-    // (1,0,0),(0,1,0),(0,0,1),(1,1,1),(1,1,-1),(1,-1,1),(-1,1,1)) bit 2p is
-    // set when +e takes the neighbour side (e.n < 0), bit 2p+1 when -e does
-    // (e.n > 0); e.n summed in x,y,z order in FP64 as src/Solver.cpp:958-1273
+    // [E] which side the 14 moving lattice points take: for pair p (directions
+    // (1,0,0),(0,1,0),(0,0,1),(1,1,1),(1,1,-1),(1,-1,1),(-1,1,1)) bit p is set
+    // where e.n < 0 (+e takes the neighbour side, -e the owner's), bit 7 + p
+    // where neither e.n < 0 nor e.n > 0 (both take the owner's); e.n summed in
+    // x,y,z order in FP64 as src/Solver.cpp:958-1273
     std::vector<uint32_t> it_side;
     std::vector<double> it_geo;  // [kGeoPerItem*E], component-major
     std::vector<double> it_fc;   // [3*E] face centroid, component-major
