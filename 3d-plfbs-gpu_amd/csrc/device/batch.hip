@@ -62,11 +62,12 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) voi
     if (i >= m.N || a.done[b]) return;
     S g[12];
     lsq_grad<S>(m, i, GlobalStates<S, RecB>{st, RecB{a.B, b}}, g);
-    // the batch keeps the state apart: three gradient V4 per (cell, case) record
-    V4<S> *gi = grad + 3 * ((size_t)i * a.B + b);
+    // the batch keeps the state apart from the gradients, [cell][3][B]: the
+    // cases of a cell are contiguous in each store here and load in kb_flux
+    V4<S> *gi = grad + RecB{a.B, b}.grad(i);
     gi[0] = V4<S>{g[0], g[1], g[2], g[3]};
-    gi[1] = V4<S>{g[4], g[5], g[6], g[7]};
-    gi[2] = V4<S>{g[8], g[9], g[10], g[11]};
+    gi[a.B] = V4<S>{g[4], g[5], g[6], g[7]};
+    gi[2 * a.B] = V4<S>{g[8], g[9], g[10], g[11]};
 }
 
 // Border pass (split border): faces between two flux blocks, one thread per
@@ -80,7 +81,7 @@ void kb_flux_border(DevMesh<S> m, DevParams prm, BatchArgs a, const Ctrl *__rest
     const int64_t k = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     const int j = (int)(k / a.B), b = (int)(k - (int64_t)j * a.B);
     if (j >= m.n_border || a.done[b]) return;
-    const SideLoader<S, RecB, false> ld{st_in, grad, m.cgeo, RecB{a.B, b}, nullptr, nullptr, 0, 0, 1, 0};
+    const SideLoader<S, RecB> ld{st_in, grad, RecB{a.B, b}, nullptr, 0, 0, 1, 0};
     S F[4];
     item_flux<S>(m, prm, m.border0 + j, ld, a.v3g[b], a.dtcap[b], F);
     const size_t nbd = (size_t)m.n_border;
@@ -105,15 +106,10 @@ __global__ __launch_bounds__(kBlock) void kb_flux(DevMesh<S> m, DevParams prm, B
     const int c0 = blk * m.block_cells;
     const int ncell = min(N, c0 + m.block_cells) - c0;
     V4<S> *sRec = nullptr;
-    double4 *sCg = nullptr;
     int nst = 0;
     if (a.stage) {
-        char *base = reinterpret_cast<char *>(lds) + staged_offset<S>(m.max_items, C);
-        sRec = reinterpret_cast<V4<S> *>(base);
-        if (std::is_same<S, double>::value)
-            sCg = reinterpret_cast<double4 *>(base + (size_t)m.block_cells * C * 4 * sizeof(V4<S>));
-        stage_records<S, false>(st_in, grad, std::is_same<S, double>::value ? m.cgeo : nullptr, B, b0, C, c0, ncell, sRec,
-                         sCg);
+        sRec = reinterpret_cast<V4<S> *>(reinterpret_cast<char *>(lds) + staged_offset<S>(m.max_items, C));
+        stage_records<S>(st_in, grad, B, b0, C, c0, ncell, sRec);
         nst = ncell;
         __syncthreads();
     }
@@ -124,7 +120,7 @@ __global__ __launch_bounds__(kBlock) void kb_flux(DevMesh<S> m, DevParams prm, B
     const bool live = b < B && !a.done[b];
     if (live) {
         const double v3g = a.v3g[b], dtcap = a.dtcap[b];
-        const SideLoader<S, RecB, false> ld{st_in, grad, m.cgeo, RecB{B, b}, sRec, sCg, c0, nst, C, c};
+        const SideLoader<S, RecB> ld{st_in, grad, RecB{B, b}, sRec, c0, nst, C, c};
         for (int el = threadIdx.x / C; el < e1 - e0; el += kBlock / C) {
             S F[4];
             item_flux<S>(m, prm, e0 + el, ld, v3g, dtcap, F);

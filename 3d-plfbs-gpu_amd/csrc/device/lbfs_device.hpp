@@ -16,6 +16,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 namespace plbfs {
 
 // flags: the ghost gradient copies cell b_partner[b]'s (periodic partner, or
@@ -55,11 +57,10 @@ struct V4T<float> {
 template <typename S>
 using V4 = typename V4T<S>::type;
 
-// Gradient records gathered by the face items.  FP64: three V4 (d/dx, d/dy,
-// d/dz of rho, u, v, w), 96 B.  FP32: the cell's state followed by its three
-// gradient V4, 64 B, so that a face side is one aligned 64 B run; the
-// gradient kernel writes all four (the state it read), so its stores stay
-// contiguous.
+// Gradient records gathered by the face items of a single case.  FP64: three V4
+// (d/dx, d/dy, d/dz of rho, u, v, w), 96 B.  FP32: the cell's state followed by its
+// three gradient V4, 64 B, so that a face side is one aligned 64 B run; the
+// gradient kernel writes all four (the state it read).
 template <typename S>
 inline constexpr int kGradRec = std::is_same<S, float>::value ? 4 : 3;  // V4 per record
 template <typename S>
@@ -75,6 +76,10 @@ __device__ __forceinline__ int xcd_block(int bid, int nblk, int remap) {
     const int x = bid % kXcds, k = bid / kXcds;
     return x * q + (x < r ? x : r) + k;
 }
+
+// 16 B chunks per face item (see DevMesh::it_p).
+template <typename S>
+inline constexpr int kItemChunks = std::is_same<S, float>::value ? 3 : 5;
 
 template <typename S>
 struct DevMesh {
@@ -94,19 +99,19 @@ struct DevMesh {
     const S *st_w;
     const double *vol, *inv_vol, *cfl_area;
     const int32_t *blk_item_off;
-    // Face work items, one record each so that an item is a few wide loads
-    // from one address.  FP64 storage: it_x[e] = (owner, neighbour or -1-b,
-    // lattice side bits (see lattice_pair), 0) and it_d[2e..2e+1] = (n, A),
-    // (dt, x_face); the centroid-to-face offsets are formed on the fly from cgeo
-    // (same bits as the host's cc - fc).  FP32 storage (56 B per item):
-    // it_on[e] = (owner, neighbour or -1-b) and it_f[3e..3e+2] = (n, A),
-    // (dt, r_owner), (r_neighbour, side bits stored in the float's bits).
-    const int4 *it_x;
-    const double4 *it_d;
-    const int2 *it_on;
-    const float4 *it_f;
-    const double4 *cgeo;  // FP64 storage: per cell (cx, cy, cz, 1/V)
-    double g0x, g0y, g0z;  // centroid of the ghost of boundary face 0
+    // Face work items in groups of 64: chunk k of item e, 16 B, is it_p[((e >> 6)
+    // * kItemChunks<S> + k) * 64 + (e & 63)], so that every load of a wavefront of
+    // consecutive items is one contiguous KiB (16 B a lane at a record's stride
+    // takes the address unit two to three times as long).  An item is the area
+    // vector n A, the owner's centroid and the neighbour's centroid from the face
+    // centre, each (x, y, z); the streaming dt (FP32 here, FP64 in it_dt); and the
+    // owner and neighbour (or -1-b) as two ints.  A boundary face holds its unit
+    // normal in the neighbour's place: its ghost's centroid is only used on boundary
+    // face 0, as b0.  it_side holds the lattice side bits (see side_point).
+    const float4 *it_p;
+    const double *it_dt;
+    const uint16_t *it_side;
+    S b0[3];
     const int32_t *g_off, *g_ent;
     // [n_blocks] nonzero where a flux block holds a cell the immersed boundary
     // spreads force to; null: every block reads the body force
@@ -169,13 +174,14 @@ __device__ __forceinline__ void ghost_state(const DevPatch &P, const T po[4], co
     }
 }
 
-// Ghost gradient from the owner's state and gradient (gp: the gradient of
-// cell b_partner[b], read by type 3 and by the types whose ghost the
-// reference's update leaves unwritten).  rho_type 8 leaves the reference's
-// zero-initialised rho slot untouched, so it is zero here too.
+// Ghost gradient gg from the owner's state and gradient.  On entry gg is the
+// gradient of cell b_partner[b], which type 3 and the types whose ghost the
+// reference's update leaves unwritten keep (other patches have no partner; what gg
+// holds is not used).  rho_type 8 leaves the reference's zero-initialised rho
+// slot untouched, so it is zero here too.
 template <typename T>
 __device__ __forceinline__ void ghost_grad(const DevPatch &P, const T n[3], T dmag, const T po[4], const T go[12],
-                                           const T gp[12], T gg[12]) {
+                                           T gg[12]) {
     const int rt = P.rho_type, vt = P.vel_type;
     if (rt == 1) {
         const T q = (T)2 * ((T)P.rho - po[0]) / dmag;
@@ -190,11 +196,7 @@ __device__ __forceinline__ void ghost_grad(const DevPatch &P, const T n[3], T dm
         gg[0] = go[0];
         gg[1] = go[1];
         gg[2] = go[2];
-    } else if (rt == 3 || rt == 4 || rt == 5 || rt == 9) {
-        gg[0] = gp[0];
-        gg[1] = gp[1];
-        gg[2] = gp[2];
-    } else {
+    } else if (!(rt == 3 || rt == 4 || rt == 5 || rt == 9)) {
         gg[0] = gg[1] = gg[2] = (T)0;
     }
     if (vt == 1 || vt == 8) {
@@ -214,10 +216,7 @@ __device__ __forceinline__ void ghost_grad(const DevPatch &P, const T n[3], T dm
             gg[6 + c] = go[6 + c] * ((T)1 - n[c]);
             gg[9 + c] = go[9 + c] * ((T)1 - n[c]);
         }
-    } else if (vt == 3 || vt == 4 || vt == 5 || vt == 7 || vt == 9) {
-#pragma unroll
-        for (int q = 3; q < 12; q++) gg[q] = gp[q];
-    } else {
+    } else if (!(vt == 3 || vt == 4 || vt == 5 || vt == 7 || vt == 9)) {
 #pragma unroll
         for (int q = 3; q < 12; q++) gg[q] = (T)0;
     }
@@ -349,9 +348,8 @@ __device__ __forceinline__ T lattice_rcp(T x) {
     else return (T)1 / x;
 }
 
-// Flux through a face of area A and unit normal n (owner -> neighbour); tau
-// is passed as its parts v3g / dt.  With DEV the momentum flux omits the
-// constant rho0/3 n A, whose sum over a cell's faces is a per-cell geometric
+// Flux through a face with area vector nA (owner -> neighbour); tau is passed as
+// its parts v3g / dt.  With DEV the momentum flux omits the constant rho0/3 n A, whose sum over a cell's faces is a per-cell geometric
 // constant added separately.
 //
 // The two sides are evaluated one after the other, seven points each, so only one
@@ -360,7 +358,7 @@ __device__ __forceinline__ T lattice_rcp(T x) {
 // reconstruction.  The second evaluation that e.n = 0 needs is skipped by a
 // wavefront without such a face (all interior faces of a jittered mesh).
 template <bool DEV, typename T>
-__device__ __forceinline__ void lattice_flux(const T n[3], T A, T dt, T v3g, unsigned side, const T p0[4],
+__device__ __forceinline__ void lattice_flux(const T nA[3], T dt, T v3g, unsigned side, const T p0[4],
                                              const T pI[4], const T gO[12], const T pN[4], const T gN[12], T invgam,
                                              T c45, T c15, T rho0, T F[4]) {
     const T w0 = (T)(2.0 / 9.0), w1 = (T)(1.0 / 9.0), w7 = (T)(1.0 / 72.0);
@@ -401,10 +399,10 @@ __device__ __forceinline__ void lattice_flux(const T n[3], T A, T dt, T v3g, uns
     const T mxy = k * (ux * uy * invgam) + tau * pxy;
     const T mxz = k * (ux * uz * invgam) + tau * pxz;
     const T myz = k * (uy * uz * invgam) + tau * pyz;
-    F[0] = (sx * n[0] + sy * n[1] + sz * n[2]) * A;
-    F[1] = (mxx * n[0] + mxy * n[1] + mxz * n[2]) * A;
-    F[2] = (mxy * n[0] + myy * n[1] + myz * n[2]) * A;
-    F[3] = (mxz * n[0] + myz * n[1] + mzz * n[2]) * A;
+    F[0] = sx * nA[0] + sy * nA[1] + sz * nA[2];
+    F[1] = mxx * nA[0] + mxy * nA[1] + mxz * nA[2];
+    F[2] = mxy * nA[0] + myy * nA[1] + myz * nA[2];
+    F[3] = mxz * nA[0] + myz * nA[1] + mzz * nA[2];
 }
 
 }  // namespace plbfs

@@ -40,52 +40,58 @@ constexpr int kFinalizeThreads = 256;
 // Kernels
 // ---------------------------------------------------------------------------
 
-// Byte offset of the staged records behind the face slots in a flux block's LDS.
-
-// Face-item record loader of flux block blk; with staging, first copies the
-// block's own cell records into LDS behind the face slots (then barriers).
+// Fluxes of flux block blk's face items into their LDS slots, four arrays of
+// max_items; the caller's barrier follows.  With staging the block's own records
+// are first copied into LDS behind the slots.
 template <typename S>
-__device__ __forceinline__ SideLoader<S, Rec1> block_loader(const DevMesh<S> &m, const V4<S> *st, const V4<S> *grad,
-                                                             double *lds, int blk) {
-    SideLoader<S, Rec1> ld;
-    ld.st = st;
-    ld.grad = grad;
-    ld.cgeo = m.cgeo;
-    ld.c0 = blk * m.block_cells;
-    ld.nc = 0;
-    ld.C = 1;
-    ld.cl = 0;
-    ld.sRec = nullptr;
-    ld.sCg = nullptr;
+__device__ __forceinline__ void block_fluxes(const DevMesh<S> &m, const DevParams &prm, const V4<S> *st,
+                                             const V4<S> *grad, double *lds, int blk) {
+    const int e0 = m.blk_item_off[blk], e1 = m.blk_item_off[blk + 1];
+    const int nslot = m.max_items;
+    S *sF = reinterpret_cast<S *>(lds);
+    V4<S> *sRec = reinterpret_cast<V4<S> *>(reinterpret_cast<char *>(lds) + staged_offset<S>(m.max_items));
+    SideLoader<S, Rec1> ld{st, grad, Rec1{}, sRec, blk * m.block_cells, 0, 1, 0};
     if (m.stage) {
-        char *base = reinterpret_cast<char *>(lds) + staged_offset<S>(m.max_items);
         ld.nc = min(m.N, ld.c0 + m.block_cells) - ld.c0;
-        V4<S> *sRec = reinterpret_cast<V4<S> *>(base);
-        double4 *sCg = std::is_same<S, double>::value
-                           ? reinterpret_cast<double4 *>(base + (size_t)m.block_cells * 4 * sizeof(V4<S>))
-                           : nullptr;
-        stage_records<S>(st, grad, std::is_same<S, double>::value ? m.cgeo : nullptr, 1, 0, 1, ld.c0, ld.nc, sRec,
-                         sCg);
-        ld.sRec = sRec;
-        ld.sCg = sCg;
+        stage_records<S>(st, grad, 0, 0, 1, ld.c0, ld.nc, sRec);
         __syncthreads();
     }
-    return ld;
+    for (int e = e0 + threadIdx.x; e < e1; e += kBlock) {
+        S F[4];
+        item_flux<S>(m, prm, e, ld, prm.visc3_invgam, INFINITY, F);
+#pragma unroll
+        for (int q = 0; q < 4; q++) sF[q * nslot + (e - e0)] = F[q];
+    }
 }
 
-// Item index records (owner, neighbour, side bits, 0).
-static std::vector<int4> item_idx(const Layout &L) {
-    std::vector<int4> v((size_t)L.n_items);
-    for (size_t e = 0; e < v.size(); e++) v[e] = int4{L.it_own[e], L.it_nbr[e], (int)L.it_side[e], 0};
+// Face items in groups of 64 (see DevMesh::it_p).
+template <typename S>
+static std::vector<float4> pack_items(const Layout &L) {
+    const size_t E = (size_t)L.n_items, K = kItemChunks<S>;
+    std::vector<float4> v((E + 63) / 64 * 64 * K);
+    const double *g = L.it_geo.data();
+    for (size_t e = 0; e < E; e++) {
+        float4 *p = &v[(e >> 6) * 64 * K + (e & 63)];
+        S f[12];
+        const int third = L.it_nbr[e] < 0 ? 0 : 8;  // the normal, or the neighbour's offset
+        for (int a = 0; a < 3; a++) {
+            f[a] = (S)(g[a * E + e] * g[3 * E + e]);
+            f[3 + a] = (S)g[(5 + a) * E + e];
+            f[6 + a] = (S)g[(third + a) * E + e];
+        }
+        if (std::is_same<S, float>::value) f[9] = (S)g[4 * E + e];
+        const int32_t on[2] = {L.it_own[e], L.it_nbr[e]};
+        std::memcpy(reinterpret_cast<char *>(f) + 16 * K - sizeof on, on, sizeof on);
+        for (size_t k = 0; k < K; k++) std::memcpy(p + 64 * k, reinterpret_cast<const char *>(f) + 16 * k, 16);
+    }
     return v;
 }
 
-// Occupancy 8 waves/SIMD (<= 64 VGPRs) keeps enough gathers in flight; the
-// compiler otherwise settles at 92 VGPRs (5 waves) for the FP64 instance.
-// There the limit costs a 28 B per lane spill; 7 waves (69 VGPRs, no spill)
-// measured the same time.
+// Bound by HBM: a state read, the stencil (28 B a slot in FP64) and the record
+// written are 241 B a tet, 0.99 GB in 0.198 ms on 4.1M tets in FP64 (4.97 TB/s, where
+// a large copy reaches 4.75-5.1); 0.239 ms with each lane storing its own record.
 template <typename S>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) void k_grad(DevMesh<S> m, const Ctrl *__restrict__ ctrl,
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) void k_grad(DevMesh<S> m, const Ctrl *__restrict__ ctrl,
                                                  const V4<S> *__restrict__ st, V4<S> *__restrict__ grad) {
     if (ctrl->done) return;
     const int c0 = xcd_block(blockIdx.x, gridDim.x, m.xcd_remap) * kBlock;
@@ -94,39 +100,39 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) voi
     V4<S> si;
     const int nc = min(m.N - c0, kBlock);
     const bool live = i < m.N;
+    // the block's own states, then its records
+    constexpr int kChunks = kGradRec<S> * sizeof(V4<S>) / 16;
+    __shared__ float4 lds[kBlock * kChunks];
     if (m.grad_stage) {
         // the block's own states in LDS: most stencil neighbours are in the block
-        __shared__ V4<S> sSt[kBlock];
-        if ((int)threadIdx.x < nc) sSt[threadIdx.x] = st[i];
+        V4<S> *sSt = reinterpret_cast<V4<S> *>(lds);
+        if (live) sSt[threadIdx.x] = st[i];
         __syncthreads();
         if (live) {
             lsq_grad<S>(m, i, StagedStates<S>{st, sSt, c0, nc}, g);
             si = sSt[threadIdx.x];
         }
+        __syncthreads();
     } else if (live) {
         lsq_grad<S>(m, i, GlobalStates<S, Rec1>{st, Rec1{}}, g);
         si = st[i];
     }
-    if constexpr (kGradOff<S> == 1) {
-        // 64 B records (state + gradient): assembled in LDS, then stored by the
-        // block as one contiguous run, lane by lane
-        __shared__ V4<S> sOut[kBlock * kGradRec<S>];
-        if (live) {
-            V4<S> *o = sOut + kGradRec<S> * threadIdx.x;
-            o[0] = si;
-            o[1] = V4<S>{g[0], g[1], g[2], g[3]};
-            o[2] = V4<S>{g[4], g[5], g[6], g[7]};
-            o[3] = V4<S>{g[8], g[9], g[10], g[11]};
-        }
-        __syncthreads();
-        V4<S> *out = grad + (size_t)kGradRec<S> * c0;
-        for (int k = threadIdx.x; k < kGradRec<S> * nc; k += kBlock) out[k] = sOut[k];
-    } else {
-        if (!live) return;
-        V4<S> *gi = grad + (size_t)kGradRec<S> * i;
-        gi[0] = V4<S>{g[0], g[1], g[2], g[3]};
-        gi[1] = V4<S>{g[4], g[5], g[6], g[7]};
-        gi[2] = V4<S>{g[8], g[9], g[10], g[11]};
+    // records assembled in LDS, then stored by the block as one contiguous run:
+    // lane by lane at the records' stride a store takes the address unit two to
+    // three times as long
+    if (live) {
+        V4<S> *o = reinterpret_cast<V4<S> *>(lds) + kGradRec<S> * threadIdx.x;
+        if constexpr (kGradOff<S> == 1) o[0] = si;
+        o[kGradOff<S>] = V4<S>{g[0], g[1], g[2], g[3]};
+        o[kGradOff<S> + 1] = V4<S>{g[4], g[5], g[6], g[7]};
+        o[kGradOff<S> + 2] = V4<S>{g[8], g[9], g[10], g[11]};
+    }
+    __syncthreads();
+    float4 *out = reinterpret_cast<float4 *>(grad) + (size_t)kChunks * c0;
+#pragma unroll
+    for (int k = 0; k < kChunks; k++) {
+        const int t = threadIdx.x + k * kBlock;
+        if (t < kChunks * nc) out[t] = lds[t];
     }
 }
 
@@ -139,7 +145,7 @@ __global__ __launch_bounds__(kBlock) void k_flux_border(DevMesh<S> m, DevParams 
     if (ctrl->done) return;
     const int t = blockIdx.x * kBlock + threadIdx.x;
     if (t >= m.n_border) return;
-    const SideLoader<S, Rec1> ld{st_in, grad, m.cgeo, Rec1{}, nullptr, nullptr, 0, 0, 1, 0};
+    const SideLoader<S, Rec1> ld{st_in, grad, Rec1{}, nullptr, 0, 0, 1, 0};
     S F[4];
     item_flux<S>(m, prm, m.border0 + t, ld, prm.visc3_invgam, INFINITY, F);
     const size_t nbd = (size_t)m.n_border;
@@ -161,17 +167,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kFluxMin
     if (ctrl->done) return;
     const int N = m.N;
     const int blk = xcd_block(blockIdx.x, gridDim.x, m.xcd_remap);
-    const int e0 = m.blk_item_off[blk], e1 = m.blk_item_off[blk + 1];
     const int nslot = m.max_items;
-    S *sF = reinterpret_cast<S *>(lds);
-    const SideLoader<S, Rec1> ld = block_loader<S>(m, st_in, grad, lds, blk);
-    for (int e = e0 + threadIdx.x; e < e1; e += kBlock) {
-        S F[4];
-        item_flux<S>(m, prm, e, ld, prm.visc3_invgam, INFINITY, F);
-        const int sl = e - e0;
-#pragma unroll
-        for (int q = 0; q < 4; q++) sF[q * nslot + sl] = F[q];
-    }
+    const S *sF = reinterpret_cast<const S *>(lds);
+    block_fluxes<S>(m, prm, st_in, grad, lds, blk);
     __syncthreads();
     double sq[4] = {0, 0, 0, 0};
     int err = 0;
@@ -336,16 +334,9 @@ __global__ __launch_bounds__(kBlock) void k_residual_only(DevMesh<S> m, DevParam
     extern __shared__ double lds[];
     const int N = m.N;
     const int blk = xcd_block(blockIdx.x, gridDim.x, m.xcd_remap);
-    const int e0 = m.blk_item_off[blk], e1 = m.blk_item_off[blk + 1];
     const int nslot = m.max_items;
-    S *sF = reinterpret_cast<S *>(lds);
-    const SideLoader<S, Rec1> ld = block_loader<S>(m, st_in, grad, lds, blk);
-    for (int e = e0 + threadIdx.x; e < e1; e += kBlock) {
-        S F[4];
-        item_flux<S>(m, prm, e, ld, prm.visc3_invgam, INFINITY, F);
-#pragma unroll
-        for (int q = 0; q < 4; q++) sF[q * nslot + (e - e0)] = F[q];
-    }
+    const S *sF = reinterpret_cast<const S *>(lds);
+    block_fluxes<S>(m, prm, st_in, grad, lds, blk);
     __syncthreads();
     const int c_end = min(N, (blk + 1) * m.block_cells);
     for (int i = blk * m.block_cells + threadIdx.x; i < c_end; i += kBlock) {
@@ -519,12 +510,10 @@ int create_ctx(const plbfs_mesh_view *mesh, const plbfs_params *params, const pl
     d.n_border = (int)L.n_border;
     d.bflux = nullptr;
     d.blk_force = nullptr;
+    for (int a = 0; a < 3; a++) d.b0[a] = L.b0[a];
     d.block_cells = L.block_cells;
     d.stage = stage ? 1 : 0;
     d.grad_stage = env_flag("PLBFS_GRAD_STAGE", true) ? 1 : 0;
-    d.g0x = L.ghost0[0];
-    d.g0y = L.ghost0[1];
-    d.g0z = L.ghost0[2];
     c->cell_grid = (N + kBlock - 1) / kBlock;
     // measured on MI355X (4.09M tets): the XCD-contiguous remap is ~5% slower
     // than plain dispatch order for the flux kernel, so it is opt-in
@@ -558,27 +547,16 @@ int create_ctx(const plbfs_mesh_view *mesh, const plbfs_params *params, const pl
         (rc = upload(c, (double **)&d.vol, L.vol)) || (rc = upload(c, (double **)&d.inv_vol, L.inv_vol)) ||
         (rc = upload(c, (double **)&d.cfl_area, L.cfl_area)) ||
         (rc = upload(c, (int32_t **)&d.blk_item_off, L.blk_item_off)) ||
-        (rc = upload(c, (int4 **)&d.it_x, item_idx(L))) ||
+        (rc = upload(c, (float4 **)&d.it_p, c->f32 ? pack_items<float>(L) : pack_items<double>(L))) ||
+        (rc = upload(c, (uint16_t **)&d.it_side, std::vector<uint16_t>(L.it_side.begin(), L.it_side.end()))) ||
         (rc = upload(c, (int32_t **)&d.g_off, L.g_off)) || (rc = upload(c, (int32_t **)&d.g_ent, L.g_ent)) ||
         (rc = upload(c, (int32_t **)&d.b_patch, bpatch)) || (rc = upload(c, (int32_t **)&d.b_partner, bpartner)) ||
         (rc = upload(c, (DevPatch **)&d.patches, dp)))
         return fail(rc);
     if (!c->f32) {
-        // n, A, dt only; offsets come from the face and cell centroids
-        const size_t E = (size_t)L.n_items;
-        std::vector<double4> geo(2 * E);
-        for (size_t e = 0; e < E; e++) {
-            const double *g = L.it_geo.data();
-            geo[2 * e] = double4{g[e], g[E + e], g[2 * E + e], g[3 * E + e]};
-            geo[2 * e + 1] = double4{g[4 * E + e], L.it_fc[e], L.it_fc[E + e], L.it_fc[2 * E + e]};
-        }
-        std::vector<double> cg((size_t)4 * N);
-        for (int n = 0; n < N; n++) {
-            for (int a = 0; a < 3; a++) cg[(size_t)4 * n + a] = L.centroid[(size_t)a * N + n];
-            cg[(size_t)4 * n + 3] = L.inv_vol[n];
-        }
-        if ((rc = upload(c, (double **)&d.st_w, L.st_w)) || (rc = upload(c, (double4 **)&d.it_d, geo)) ||
-            (rc = upload(c, (double **)&d.cgeo, cg)) ||
+        if ((rc = upload(c, (double **)&d.st_w, L.st_w)) ||
+            (rc = upload(c, (double **)&d.it_dt, std::vector<double>(L.it_geo.begin() + 4 * L.n_items,
+                                                                     L.it_geo.begin() + 5 * L.n_items))) ||
             (rc = upload(c, (double **)&d.b_dmag, bdmag)))
             return fail(rc);
     } else {
@@ -588,35 +566,18 @@ int create_ctx(const plbfs_mesh_view *mesh, const plbfs_params *params, const pl
         e.N = d.N; e.G = d.G; e.n_blocks = d.n_blocks; e.max_items = d.max_items; e.E = d.E;
         e.border0 = d.border0; e.n_border = d.n_border; e.bflux = nullptr; e.blk_force = nullptr;
         e.xcd_remap = d.xcd_remap;
+        for (int a = 0; a < 3; a++) e.b0[a] = (float)L.b0[a];
         e.block_cells = d.block_cells;
         e.stage = d.stage;
         e.grad_stage = d.grad_stage;
-        e.it_d = nullptr;
-        e.cgeo = nullptr;
-        e.g0x = d.g0x; e.g0y = d.g0y; e.g0z = d.g0z;
         e.st_cnt = d.st_cnt; e.st_nbr = d.st_nbr; e.vol = d.vol; e.inv_vol = d.inv_vol; e.cfl_area = d.cfl_area;
-        e.blk_item_off = d.blk_item_off; e.it_x = nullptr; e.g_off = d.g_off;
+        e.blk_item_off = d.blk_item_off; e.it_p = d.it_p; e.it_side = d.it_side; e.it_dt = nullptr; e.g_off = d.g_off;
         e.g_ent = d.g_ent; e.b_patch = d.b_patch; e.b_partner = d.b_partner;
         e.b_fix = (const float4 *)c->b_fix;
         auto to32 = [](const std::vector<double> &v) { return std::vector<float>(v.begin(), v.end()); };
         std::vector<DevPatch> dp32 = dp;
         for (auto &q : dp32) q.rho -= p.ref_rho;
-        const size_t E = (size_t)L.n_items;
-        std::vector<float4> geo(3 * E);
-        for (size_t it = 0; it < E; it++) {
-            float g[12] = {0};
-            for (int q = 0; q < kGeoPerItem; q++) g[q] = (float)L.it_geo[(size_t)q * E + it];
-            geo[3 * it] = float4{g[0], g[1], g[2], g[3]};
-            geo[3 * it + 1] = float4{g[4], g[5], g[6], g[7]};
-            float sb;
-            const uint32_t side = L.it_side[it];
-            std::memcpy(&sb, &side, sizeof sb);
-            geo[3 * it + 2] = float4{g[8], g[9], g[10], sb};
-        }
-        std::vector<int2> on(E);
-        for (size_t it = 0; it < E; it++) on[it] = int2{L.it_own[it], L.it_nbr[it]};
-        if ((rc = upload(c, (float **)&e.st_w, to32(L.st_w))) || (rc = upload(c, (float4 **)&e.it_f, geo)) ||
-            (rc = upload(c, (int2 **)&e.it_on, on)) ||
+        if ((rc = upload(c, (float **)&e.st_w, to32(L.st_w))) ||
             (rc = upload(c, (float **)&e.b_dmag, to32(bdmag))) || (rc = upload(c, (float **)&e.corr, to32(L.corr))) ||
             (rc = upload(c, (DevPatch **)&e.patches, dp32)))
             return fail(rc);
@@ -827,9 +788,10 @@ static void launch_stages(plbfs_ctx *c, const DevMesh<S> &dm, const RunScratch &
             if (dm.n_border > 0)
                 hipLaunchKernelGGL(k_flux_border<S>, dim3((dm.n_border + kBlock - 1) / kBlock), dim3(kBlock), 0,
                                    c->stream, dm, c->prm, w.ctrl, (const V4<S> *)in, (const V4<S> *)c->grad);
-            hipLaunchKernelGGL(k_flux_update<S>, dim3(nb), dim3(kBlock), c->lds_bytes, c->stream, dm, c->prm, sa,
-                               w.ctrl, (const V4<S> *)in, (const V4<S> *)c->grad, (V4<S> *)outb,
-                               (double4 *)c->t0, (Acc<S> *)c->t1, c->dtl, c->fbody, w.partials);
+            hipLaunchKernelGGL(k_flux_update<S>, dim3(nb),
+                               dim3(kBlock), c->lds_bytes, c->stream, dm, c->prm, sa, w.ctrl, (const V4<S> *)in,
+                               (const V4<S> *)c->grad, (V4<S> *)outb, (double4 *)c->t0, (Acc<S> *)c->t1, c->dtl,
+                               c->fbody, w.partials);
         }
         std::swap(in, outb);
     }
@@ -1027,32 +989,27 @@ extern "C" int plbfs_get_residual_history(plbfs_ctx *c, double *out, int32_t max
     return PLBFS_OK;
 }
 
+template <typename S>
+static void launch_residual(plbfs_ctx *c, const DevMesh<S> &dm, double *Rd) {
+    const V4<S> *st = (const V4<S> *)c->stA;
+    V4<S> *grad = (V4<S> *)c->grad;
+    hipLaunchKernelGGL(k_grad<S>, dim3(c->cell_grid), dim3(kBlock), 0, c->stream, dm, c->ctrl, st, grad);
+    if (dm.n_border > 0)
+        hipLaunchKernelGGL(k_flux_border<S>, dim3((dm.n_border + kBlock - 1) / kBlock), dim3(kBlock), 0, c->stream,
+                           dm, c->prm, c->ctrl, st, grad);
+    hipLaunchKernelGGL(k_residual_only<S>, dim3(c->L.n_blocks),
+                       dim3(kBlock), c->lds_bytes, c->stream, dm, c->prm, st, grad, c->fbody, Rd);
+}
+
 extern "C" int plbfs_eval_residual(plbfs_ctx *c, double *grads, double *R) {
     if (!c) return plbfs_fail(PLBFS_ERR_INPUT, "null argument");
     if (int e = check_ghost_state(c)) return e;
-    const int N = c->L.N, nb = c->L.n_blocks;
+    const int N = c->L.N;
     Ctrl h{};
     HIP_TRY(hipMemcpyAsync(c->ctrl, &h, sizeof(Ctrl), hipMemcpyHostToDevice, c->stream));
     double *Rd = c->stB;  // scratch: stB is rewritten before it is read in a step
-    if (!c->f32) {
-        hipLaunchKernelGGL(k_grad<double>, dim3(c->cell_grid), dim3(kBlock), 0, c->stream, c->dm, c->ctrl,
-                           (const double4 *)c->stA, (double4 *)c->grad);
-        if (c->dm.n_border > 0)
-            hipLaunchKernelGGL(k_flux_border<double>, dim3((c->dm.n_border + kBlock - 1) / kBlock), dim3(kBlock), 0,
-                               c->stream, c->dm, c->prm, c->ctrl, (const double4 *)c->stA,
-                               (const double4 *)c->grad);
-        hipLaunchKernelGGL(k_residual_only<double>, dim3(nb), dim3(kBlock), c->lds_bytes, c->stream, c->dm, c->prm,
-                           (const double4 *)c->stA, (const double4 *)c->grad, c->fbody, Rd);
-    } else {
-        hipLaunchKernelGGL(k_grad<float>, dim3(c->cell_grid), dim3(kBlock), 0, c->stream, c->dm32, c->ctrl,
-                           (const float4 *)c->stA, (float4 *)c->grad);
-        if (c->dm32.n_border > 0)
-            hipLaunchKernelGGL(k_flux_border<float>, dim3((c->dm32.n_border + kBlock - 1) / kBlock), dim3(kBlock), 0,
-                               c->stream, c->dm32, c->prm, c->ctrl, (const float4 *)c->stA,
-                               (const float4 *)c->grad);
-        hipLaunchKernelGGL(k_residual_only<float>, dim3(nb), dim3(kBlock), c->lds_bytes, c->stream, c->dm32,
-                           c->prm, (const float4 *)c->stA, (const float4 *)c->grad, c->fbody, Rd);
-    }
+    if (!c->f32) launch_residual<double>(c, c->dm, Rd);
+    else launch_residual<float>(c, c->dm32, Rd);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(c->stream));
     if (grads) {

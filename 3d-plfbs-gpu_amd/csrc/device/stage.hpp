@@ -19,6 +19,8 @@ struct Rec1 {
 struct RecB {
     int B, b;
     __device__ __forceinline__ size_t operator()(int c) const { return (size_t)c * B + b; }
+    // first of cell c's three gradient V4, B apart ([cell][3][B])
+    __device__ __forceinline__ size_t grad(int c) const { return (size_t)c * 3 * B + b; }
 };
 
 // Per-cell RK accumulator between stages: the running sum t1 itself in FP64
@@ -145,22 +147,17 @@ __device__ __forceinline__ void unpack_side(V4<S> q, V4<S> a, V4<S> b, V4<S> d, 
     g[8] = d.x; g[9] = d.y; g[10] = d.z; g[11] = d.w;
 }
 
-// Where a face item reads a cell's state + gradient record (and, in FP64
-// storage, its centroid): cells of the block's own range [c0, c0 + nc) from
-// the copy the block staged in LDS (sRec: state, grad x3 per cell; sCg:
-// centroid + 1/V), every other cell from global memory.  With nc = 0 every
-// read goes to global memory.
-// COMB: gradient records carry the state (kGradRec<S> V4 per record, the
-// single-case FP32 layout); otherwise the state comes from `st` and the record
-// is the three gradient V4 (FP64, and the batched solver in either precision).
-template <typename S, typename R, bool COMB = (kGradOff<S> == 1)>
+// Where a face item reads a cell's state and gradient: cells of the block's own
+// range [c0, c0 + nc) from the copy the block staged in LDS (sRec: state, grad x3
+// per cell), every other cell from global memory.  With nc = 0 every read goes
+// to global memory.  The batch keeps the gradients as [cell][3][B], so that
+// consecutive cases of a cell are contiguous in each of the four loads.
+template <typename S, typename R>
 struct SideLoader {
     const V4<S> *__restrict__ st;
     const V4<S> *__restrict__ grad;
-    const double4 *__restrict__ cgeo;
     R rec;
     const V4<S> *sRec;  // staged records, cell-major then case lane: 4 * (rel * C + cl)
-    const double4 *sCg;
     int c0, nc;
     int C, cl;  // cases staged per cell and this item's case lane (1, 0 for one case)
     __device__ __forceinline__ void side(int c, S p[4], S g[12]) const {
@@ -168,42 +165,36 @@ struct SideLoader {
         if (rel < (unsigned)nc) {
             const V4<S> *q = sRec + 4 * (rel * C + cl);
             unpack_side<S>(opaque4(q[0]), opaque4(q[1]), opaque4(q[2]), opaque4(q[3]), p, g);
+        } else if constexpr (!std::is_same<R, Rec1>::value) {
+            const V4<S> *gc = grad + rec.grad(c);
+            unpack_side<S>(st[rec(c)], gc[0], gc[rec.B], gc[2 * rec.B], p, g);
+        } else if constexpr (kGradOff<S> == 1) {
+            const V4<S> *gc = grad + kGradRec<S> * (size_t)c;
+            unpack_side<S>(gc[0], gc[1], gc[2], gc[3], p, g);
         } else {
-            const size_t r = rec(c);
-            if constexpr (COMB) {
-                const V4<S> *gc = grad + kGradRec<S> * r;
-                unpack_side<S>(gc[0], gc[1], gc[2], gc[3], p, g);
-            } else {
-                const V4<S> *gc = grad + 3 * r;
-                unpack_side<S>(st[r], gc[0], gc[1], gc[2], p, g);
-            }
+            const V4<S> *gc = grad + kGradRec<S> * (size_t)c;
+            unpack_side<S>(st[c], gc[0], gc[1], gc[2], p, g);
         }
-    }
-    __device__ __forceinline__ double4 centroid(int c) const {
-        const unsigned rel = (unsigned)(c - c0);
-        if (rel < (unsigned)nc) return opaque4(sCg[rel]);
-        return cgeo[c];
     }
 };
 
 // Copies the records of cells [c0, c0 + nc) into LDS, 4 V4 per (cell, case
-// lane) for the C cases b0 .. b0 + C - 1 of a batch of B (C = B = 1 for one
-// case; lanes past the last case are left unset), and, when cgeo is given,
-// the cells' centroid records.
-template <typename S, bool COMB = (kGradOff<S> == 1)>
-__device__ __forceinline__ void stage_records(const V4<S> *__restrict__ st, const V4<S> *__restrict__ grad,
-                                              const double4 *__restrict__ cgeo, int B, int b0, int C, int c0,
-                                              int nc, V4<S> *sRec, double4 *sCg) {
+// lane) for the C cases b0 .. b0 + C - 1 of a batch of B (lanes past the last
+// case are left unset); B = 0: a single case.
+template <typename S>
+__device__ __forceinline__ void stage_records(const V4<S> *__restrict__ st, const V4<S> *__restrict__ grad, int B,
+                                              int b0, int C, int c0, int nc, V4<S> *sRec) {
     for (int k = threadIdx.x; k < nc * C * 4; k += blockDim.x) {
         const int r = k >> 2, q = k & 3;
         const int il = r / C, cl = r - il * C;
-        if (b0 + cl >= B) continue;
-        const size_t g = (size_t)(c0 + il) * B + b0 + cl;
-        if constexpr (COMB) sRec[k] = grad[kGradRec<S> * g + q];
-        else sRec[k] = q == 0 ? st[g] : grad[3 * g + q - 1];
+        if (B == 0) {
+            if constexpr (kGradOff<S> == 1) sRec[k] = grad[kGradRec<S> * (size_t)(c0 + il) + q];
+            else sRec[k] = q == 0 ? st[c0 + il] : grad[kGradRec<S> * (size_t)(c0 + il) + q - 1];
+        } else if (b0 + cl < B) {
+            const RecB rb{B, b0 + cl};
+            sRec[k] = q == 0 ? st[rb(c0 + il)] : grad[rb.grad(c0 + il) + (size_t)(q - 1) * B];
+        }
     }
-    if (cgeo)
-        for (int k = threadIdx.x; k < nc; k += blockDim.x) sCg[k] = cgeo[c0 + k];
 }
 
 // Byte offset of the staged records behind the face slots (C cases per slot)
@@ -214,14 +205,11 @@ __host__ __device__ inline size_t staged_offset(int max_items, int C = 1) {
 }
 
 // Dynamic LDS of one flux block: face slots, and with staging the block's own
-// cell records for C cases (+ centroid records in FP64 storage).
+// cell records for C cases.
 template <typename S>
 inline size_t flux_lds_bytes(int max_items, int block_cells, bool stage, int C = 1) {
     size_t b = staged_offset<S>(max_items, C);
-    if (stage) {
-        b += (size_t)block_cells * C * 4 * sizeof(V4<S>);
-        if (std::is_same<S, double>::value) b += (size_t)block_cells * sizeof(double4);
-    }
+    if (stage) b += (size_t)block_cells * C * 4 * sizeof(V4<S>);
     return b;
 }
 
@@ -233,84 +221,64 @@ inline size_t flux_lds_bytes(int max_items, int block_cells, bool stage, int C =
 template <typename S, typename LD>
 __device__ __forceinline__ void item_flux(const DevMesh<S> &m, const DevParams &prm, int64_t e, const LD &ld,
                                           double v3g, double dtcap, S F[4]) {
-    int o, nb;
-    unsigned side;
-    S geo[kGeoPerItem];  // n(3), A, dt, r_owner(3), r_neighbour(3)
+    S geo[10];  // n A, owner offset, neighbour offset or n (each x, y, z), dt
+    int2 on;
+    const float4 *ip = m.it_p + ((e >> 6) * (64 * kItemChunks<S>) + (e & 63));
+    const unsigned side = m.it_side[e];
     if constexpr (std::is_same<S, double>::value) {
-        const int4 ix = m.it_x[e];
-        o = ix.x;
-        nb = ix.y;
-        side = (unsigned)ix.z;
-        const double4 g0 = m.it_d[2 * e], g1 = m.it_d[2 * e + 1];
-        geo[0] = g0.x; geo[1] = g0.y; geo[2] = g0.z; geo[3] = g0.w;
-        geo[4] = g1.x;
-        const double fx = g1.y, fy = g1.z, fz = g1.w;
-        const double4 co = ld.centroid(o);
-        geo[5] = co.x - fx;
-        geo[6] = co.y - fy;
-        geo[7] = co.z - fz;
-        if (nb >= 0) {
-            const double4 cn = ld.centroid(nb);
-            geo[8] = cn.x - fx;
-            geo[9] = cn.y - fy;
-            geo[10] = cn.z - fz;
-        } else {
-            geo[8] = m.g0x - fx;
-            geo[9] = m.g0y - fy;
-            geo[10] = m.g0z - fz;
-        }
-    } else {
-        const int2 ix = m.it_on[e];
-        o = ix.x;
-        nb = ix.y;
-        const float4 g0 = m.it_f[3 * e], g1 = m.it_f[3 * e + 1], g2 = m.it_f[3 * e + 2];
-        geo[0] = g0.x; geo[1] = g0.y; geo[2] = g0.z; geo[3] = g0.w;
-        geo[4] = g1.x; geo[5] = g1.y; geo[6] = g1.z; geo[7] = g1.w;
-        geo[8] = g2.x; geo[9] = g2.y; geo[10] = g2.z;
-        side = __float_as_uint(g2.w);
-    }
-    const S n[3] = {geo[0], geo[1], geo[2]};
-    const S A = geo[3], dt = fmin(geo[4], (S)dtcap);
-    S po[4], go[12];
-    ld.side(o, po, go);
-    // both sides' states at the face centre and the neighbour side's gradient
-    S pI[4], pN[4], gN[12];
-    if (nb >= 0) {
-        S pn[4];
-        ld.side(nb, pn, gN);
+        double2 q[kItemChunks<S>];
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
-            pI[q] = po[q] - (geo[5] * go[3 * q] + geo[6] * go[3 * q + 1] + geo[7] * go[3 * q + 2]);
-            pN[q] = pn[q] - (geo[8] * gN[3 * q] + geo[9] * gN[3 * q + 1] + geo[10] * gN[3 * q + 2]);
-        }
+        for (int k = 0; k < kItemChunks<S>; k++) q[k] = __builtin_bit_cast(double2, ip[64 * k]);
+        geo[0] = q[0].x; geo[1] = q[0].y; geo[2] = q[1].x; geo[3] = q[1].y; geo[4] = q[2].x;
+        geo[5] = q[2].y; geo[6] = q[3].x; geo[7] = q[3].y; geo[8] = q[4].x;
+        geo[9] = m.it_dt[e];
+        on = __builtin_bit_cast(int2, q[4].y);
     } else {
+        const float4 q0 = ip[0], q1 = ip[64], q2 = ip[128];
+        geo[0] = q0.x; geo[1] = q0.y; geo[2] = q0.z; geo[3] = q0.w; geo[4] = q1.x;
+        geo[5] = q1.y; geo[6] = q1.z; geo[7] = q1.w; geo[8] = q2.x; geo[9] = q2.y;
+        on = int2{__float_as_int(q2.z), __float_as_int(q2.w)};
+    }
+    const int o = on.x, nb = on.y;
+    const S dt = fmin(geo[9], (S)dtcap);
+    // the neighbour's record; for a boundary face that of its ghost's partner cell,
+    // where it has one (and any record, not used, where it has none)
+    int j = nb;
+    if (nb < 0) {
+        j = m.b_partner[-1 - nb];
+        if (j < 0) j = o;
+    }
+    S po[4], go[12], pn[4], gN[12];
+    ld.side(o, po, go);
+    ld.side(j, pn, gN);
+    // both sides' states at the face centre, as of an interior face
+    S pI[4], pN[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        pI[q] = po[q] - (geo[3] * go[3 * q] + geo[4] * go[3 * q + 1] + geo[5] * go[3 * q + 2]);
+        pN[q] = pn[q] - (geo[6] * gN[3 * q] + geo[7] * gN[3 * q + 1] + geo[8] * gN[3 * q + 2]);
+    }
+    if (nb < 0) {
         const int b = -1 - nb;
         const DevPatch P = m.patches[m.b_patch[b]];
-        S pp[4] = {0, 0, 0, 0};
-        {
-            S gp[12];
-            if (P.flags & kGhostGradFromCell) ld.side(m.b_partner[b], pp, gp);
-            ghost_grad<S>(P, n, m.b_dmag[b], po, go, gp, gN);
-        }
+        ghost_grad<S>(P, geo + 6, m.b_dmag[b], po, go, gN);
         if (b == 0) {
             // reconstructed like an interior face, from the ghost: the one whose index
             // equals n_cells (the reference's strict "neighbour > n_cells" test,
             // Solver.cpp:861)
-            S pn[4], fx[4] = {0, 0, 0, 0};
+            S pg[4], fx[4] = {0, 0, 0, 0};
             if (P.flags & kGhostFixed) {
                 const V4<S> f = m.b_fix[0];
                 fx[0] = f.x; fx[1] = f.y; fx[2] = f.z; fx[3] = f.w;
             }
-            ghost_state<S>(P, po, pp, fx, pn);
+            ghost_state<S>(P, po, pn, fx, pg);
 #pragma unroll
-            for (int q = 0; q < 4; q++) {
-                pI[q] = po[q] - (geo[5] * go[3 * q] + geo[6] * go[3 * q + 1] + geo[7] * go[3 * q + 2]);
-                pN[q] = pn[q] - (geo[8] * gN[3 * q] + geo[9] * gN[3 * q + 1] + geo[10] * gN[3 * q + 2]);
-            }
+            for (int q = 0; q < 4; q++)
+                pN[q] = pg[q] - (m.b0[0] * gN[3 * q] + m.b0[1] * gN[3 * q + 1] + m.b0[2] * gN[3 * q + 2]);
         } else {
             if (P.rho_type == 1) pI[0] = (S)P.rho;
             else if (P.rho_type == 8) pI[0] = po[0];
-            else pI[0] = po[0] - (geo[5] * gN[0] + geo[6] * gN[1] + geo[7] * gN[2]);
+            else pI[0] = po[0] - (geo[3] * gN[0] + geo[4] * gN[1] + geo[5] * gN[2]);
             if (P.vel_type == 1) {
                 pI[1] = (S)P.u;
                 pI[2] = (S)P.v;
@@ -322,7 +290,7 @@ __device__ __forceinline__ void item_flux(const DevMesh<S> &m, const DevParams &
             } else {
 #pragma unroll
                 for (int q = 1; q < 4; q++)
-                    pI[q] = po[q] - (geo[5] * gN[3 * q] + geo[6] * gN[3 * q + 1] + geo[7] * gN[3 * q + 2]);
+                    pI[q] = po[q] - (geo[3] * gN[3 * q] + geo[4] * gN[3 * q + 1] + geo[5] * gN[3 * q + 2]);
             }
 #pragma unroll
             for (int q = 0; q < 4; q++) pN[q] = pI[q];
@@ -330,7 +298,7 @@ __device__ __forceinline__ void item_flux(const DevMesh<S> &m, const DevParams &
     }
     const S p0[4] = {(pI[0] + pN[0]) * (S)0.5, (pI[1] + pN[1]) * (S)0.5, (pI[2] + pN[2]) * (S)0.5,
                      (pI[3] + pN[3]) * (S)0.5};
-    lattice_flux<std::is_same<S, float>::value, S>(n, A, dt, (S)v3g, side, p0, pI, go, pN, gN, (S)prm.invgam,
+    lattice_flux<std::is_same<S, float>::value, S>(geo, dt, (S)v3g, side, p0, pI, go, pN, gN, (S)prm.invgam,
                                                    (S)prm.c45, (S)prm.c15, (S)prm.rho0, F);
 }
 

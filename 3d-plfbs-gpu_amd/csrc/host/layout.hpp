@@ -57,8 +57,7 @@ struct Layout {
     // x,y,z order in FP64 as src/Solver.cpp:958-1273
     std::vector<uint32_t> it_side;
     std::vector<double> it_geo;  // [kGeoPerItem*E], component-major
-    std::vector<double> it_fc;   // [3*E] face centroid, component-major
-    double ghost0[3] = {0, 0, 0};  // centroid of the ghost of boundary face 0
+    double b0[3] = {0, 0, 0};    // boundary face 0: its ghost's centroid from the face centre
     // per-cell gather list in file face order, entries (index << 2) | border << 1 | is_owner:
     // index is the block-local slot, or with the border bit the border item's index
     std::vector<int32_t> g_off;  // [N+1]
