@@ -10,13 +10,23 @@
 // scatter walk fixed per-node edge lists, so no float atomics are used and
 // results are bitwise reproducible.
 //
-// Every product runs on the matrix cores: k_gemm tiles C = op(A) op(B) into
-// 64x64 blocks of 4 wavefronts, stages 64x32 / 32x64 operand tiles in LDS as
-// bfloat16 (round to nearest even from the FP32 activations and master
-// weights), and issues v_mfma_f32_16x16x16_bf16 with FP32 accumulation.  Weight
-// gradients (reductions over all rows) are split over row ranges into FP32
-// partials that k_sum_splits adds in a fixed order.  Adam keeps FP32 master
-// weights and moments.
+// A layer is one kernel forward (k_layer_fwd) and three backward (k_node_bwd for the
+// update MLP, k_msg_bwd for the message MLP, k_dh_out for the edges' source side).  A
+// block walks over tiles of consecutive nodes with at most kTileNodes nodes and, if
+// the tile has more than one node, kTileRows in-edges; the edge rows [h_dst, h_src, f],
+// hidden activations and messages of a tile live in LDS only, so neither the E x 144
+// inputs nor the E x 64 activations and messages pass through memory.  The backward
+// pass computes the hidden activations again from the bfloat16 node states instead
+// of keeping them.
+//
+// Every product runs on the matrix cores as v_mfma_f32_16x16x16_bf16 with FP32
+// accumulation over k in steps of 16; operands are rounded to bfloat16 (nearest even)
+// from FP32 activations and master weights.  The node states are kept twice, in
+// FP32 for the residual sum and rounded once to bfloat16 as the operand that every
+// product uses.  Weights are held as register fragments by the wavefronts, each of
+// which owns 16 hidden units.  Weight gradients accumulate in registers over a
+// block's tiles; the blocks' FP32 partials are added in a fixed order.  Adam keeps
+// FP32 master weights and moments.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -43,9 +53,9 @@ constexpr int kT = 256;                 // threads per block
 typedef short bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-__device__ __forceinline__ unsigned short to_bf16(float f) {
+__host__ __device__ __forceinline__ unsigned short to_bf16(float f) {
     // round to nearest even (inputs are finite)
-    unsigned int u = __float_as_uint(f);
+    unsigned int u = __builtin_bit_cast(unsigned int, f);
     u += 0x7FFFu + ((u >> 16) & 1u);
     return (unsigned short)(u >> 16);
 }
@@ -56,180 +66,454 @@ __device__ __forceinline__ float dsilu(float a) {
     return s * (1.0f + a * (1.0f - s));
 }
 
-// C[M,N] (+)= op(A)[M,K] * op(B)[K,N] over k in [k_begin, k_end) of this
-// z-slice.  op(A)(m,k) = TA ? A[k*lda+m] : A[m*lda+k]; op(B)(k,n) = TB ?
-// B[n*ldb+k] : B[k*ldb+n].  Epilogue: + bias[n] if bias; C2 = silu(value) if C2.
-// Slice z writes to C + z * split_stride.
-constexpr int kTM = 64, kTN = 64, kTK = 32;
-constexpr int kLdsA = kTK + 8;  // row pitch (bf16) of the A tile [m][k]
-constexpr int kLdsB = kTK + 8;  // row pitch of the B tile stored transposed [n][k]
+typedef unsigned short u16;
 
-template <bool TA, bool TB>
-__global__ __launch_bounds__(kT) void k_gemm(int M, int N, int K, const float *__restrict__ A, int lda,
-                                             const float *__restrict__ B, int ldb, float *__restrict__ C, int ldc,
-                                             int k_chunk, size_t split_stride, const float *__restrict__ bias,
-                                             float *__restrict__ C2) {
-    __shared__ unsigned short sA[kTM * kLdsA];
-    __shared__ unsigned short sB[kTN * kLdsB];
-    const int m0 = blockIdx.x * kTM, n0 = blockIdx.y * kTN;
-    const int kb = blockIdx.z * k_chunk, ke = min(K, kb + k_chunk);
-    C += blockIdx.z * split_stride;
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const int wm = (wv >> 1) * 32, wn = (wv & 1) * 32;  // this wave's 32x32 sub-tile
-    f32x4 acc[2][2];
+constexpr int kTileRows = 64;   // edges or node rows of a tile
+constexpr int kTileNodes = 16;  // nodes of an edge tile
+constexpr int kPad = 8;         // bf16 elements behind every row of an LDS tile
+constexpr int kMaxParts = 512;  // blocks (weight-gradient partials) of a backward kernel: two a CU
+
+__device__ __forceinline__ bf16x4 pack4(f32x4 v) {
+    return bf16x4{(short)to_bf16(v[0]), (short)to_bf16(v[1]), (short)to_bf16(v[2]), (short)to_bf16(v[3])};
+}
+
+// Operand fragments of the 16x16x16 product D = A B, D(m, n): lane l holds
+// A(m = l % 16, k = 4 (l / 16) + q) and B(k = 4 (l / 16) + q, n = l % 16), q = 0..3, and of
+// the result D(m = 4 (l / 16) + q, n = l % 16).  With the weights as A and the rows of a
+// tile as n, a lane's four results are neighbouring columns of one row.
+struct Lane {
+    int r, g, w;  // l % 16, l / 16, wavefront
+    __device__ __forceinline__ Lane()
+        : r(threadIdx.x & 15), g((threadIdx.x & 63) >> 4), w(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) {}
+};
+
+__device__ __forceinline__ f32x4 mfma(bf16x4 a, bf16x4 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
+}
+
+// W(k, col) of a row-major weight matrix as the fragment (m = col, k)
+__device__ __forceinline__ bf16x4 wfrag(const float *W, int ld, int col, int k) {
+    return pack4(f32x4{W[k * ld + col], W[(k + 1) * ld + col], W[(k + 2) * ld + col], W[(k + 3) * ld + col]});
+}
+// ... its transpose: W(row, k) as the fragment (m = row, k)
+__device__ __forceinline__ bf16x4 wfrag_t(const float *W, int ld, int row, int k) {
+    return pack4(*reinterpret_cast<const f32x4 *>(W + row * ld + k));
+}
+__device__ __forceinline__ bf16x4 ld4(const u16 *p) { return *reinterpret_cast<const bf16x4 *>(p); }
+__device__ __forceinline__ f32x4 ldf4(const float *p) { return *reinterpret_cast<const f32x4 *>(p); }
+
+// T(row, col) of an LDS tile as the fragment (m or n = col0 + l % 16, k = row0 +
+// 4 (l / 16) + q): the transposing LDS read turns 4 rows x 16 columns per group of
+// 16 lanes, each lane naming 4 columns of one row.
+__device__ __forceinline__ bf16x4 ld4_t(const Lane &L, const u16 *t, int pitch, int row0, int col0) {
+    const u16 *p = t + (row0 + 4 * L.g + (L.r >> 2)) * pitch + col0 + 4 * (L.r & 3);
+    return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) bf16x4 *)p);
+}
+
+// Rows of MLP inputs in 16 B chunks of 8 bfloat16.
+struct ZNode {  // [a (64), b (64)]
+    const u16 *a, *b;
+    __device__ __forceinline__ uint4 operator()(int row, int c) const {
+        const u16 *p = c < kH / 8 ? a + (size_t)row * kH + 8 * c : b + (size_t)row * kH + 8 * c - kH;
+        return *reinterpret_cast<const uint4 *>(p);
+    }
+};
+struct ZInput {  // the network's FP32 input
+    const float *x;
+    __device__ __forceinline__ uint4 operator()(int row, int c) const {
+        const float *p = x + (size_t)row * kDin + 8 * c;
+        const bf16x4 v[2] = {pack4(ldf4(p)), pack4(ldf4(p + 4))};
+        return __builtin_bit_cast(uint4, v);
+    }
+};
+struct ZMsg {  // [h_dst, h_src, f] of edge `row`
+    const int *src, *dst;
+    const u16 *hb, *f;
+    __device__ __forceinline__ uint4 operator()(int row, int c) const {
+        const u16 *p;
+        if (c < kH / 8) p = hb + (size_t)dst[row] * kH + 8 * c;
+        else if (c < kH / 4) p = hb + (size_t)src[row] * kH + 8 * c - kH;
+        else p = f + (size_t)row * kDedge + 8 * c - 2 * kH;
+        return *reinterpret_cast<const uint4 *>(p);
+    }
+};
+
+// Rows row0 .. row0 + n of an MLP input into an LDS tile, zero behind them.
+template <int K, typename Z>
+__device__ __forceinline__ void load_z(const Z &z, int row0, int n, u16 *t) {
+    constexpr int kC = K / 8;
+    for (int k = threadIdx.x; k < kTileRows * kC; k += kT) {
+        const int r = k / kC, c = k - r * kC;
+        uint4 v = {0, 0, 0, 0};
+        if (r < n) v = z(row0 + r, c);
+        *reinterpret_cast<uint4 *>(t + r * (K + kPad) + 8 * c) = v;
+    }
+}
+
+// Hidden layer of row block i of a tile: W1^T z + b1 for the wavefront's 16 units.
+template <int K>
+__device__ __forceinline__ f32x4 hidden(const Lane &L, const u16 *z, int i, const bf16x4 *w1, f32x4 b1) {
+    f32x4 a = {0.f, 0.f, 0.f, 0.f};
+    const u16 *row = z + (16 * i + L.r) * (K + kPad) + 4 * L.g;
 #pragma unroll
-    for (int i = 0; i < 2; i++)
+    for (int k = 0; k < K / 16; k++) a = mfma(w1[k], ld4(row + 16 * k), a);
+    return a + b1;
+}
+
+__device__ __forceinline__ f32x4 silu4(f32x4 a) { return f32x4{silu(a[0]), silu(a[1]), silu(a[2]), silu(a[3])}; }
+
+// One layer: messages of the tile's edges, their mean per node, the update MLP and
+// the residual sum.  Thread (node slot t / 16, columns 4 (t % 16) ..) sums its node's
+// messages in edge order, over the chunks of kTileRows edges that a single node of
+// higher degree takes.  agg (training): the mean, rounded as the update uses it.
+// Bound by latency: a tile is a chain of dependent loads (node range, edge ends,
+// states) and short products.  A layer of the 221,184-cell hex mesh (1.3M edges)
+// takes 0.25 ms; gathering, two products, mean and update as kernels of their own
+// took 2.1 ms, most of it on the edge rows' way through memory.
+__global__ __launch_bounds__(kT) void k_layer_fwd(int tiles, const int *__restrict__ tile_n0,
+                                                  const int *__restrict__ in_off, ZMsg zm,
+                                                  const float *__restrict__ inv_deg, const float *__restrict__ h,
+                                                  float *__restrict__ h_out, u16 *__restrict__ hb_out,
+                                                  u16 *__restrict__ agg, const float *__restrict__ wm,
+                                                  const float *__restrict__ wu) {
+    constexpr int kZ = kKmsg + kPad, kS = kH + kPad, kU = kKupd + kPad, kM = kH + 4;
+    static_assert(kM * 4 <= kZ * 2, "the messages take the place of the edge rows");
+    __shared__ __align__(16) u16 z[kTileRows * kZ], s1[kTileRows * kS], u[kTileNodes * kU], t1[kTileNodes * kS];
+    float *msg = reinterpret_cast<float *>(z);
+    const Lane L;
+    const int j = 16 * L.w + L.r, j0 = 16 * L.w + 4 * L.g;
+    const float *m2 = wm + kKmsg * kH + kH, *v2 = wu + kKupd * kH + kH;
+    bf16x4 w1[kKmsg / 16], w2[kH / 16], u1[kKupd / 16], u2[kH / 16];
 #pragma unroll
-        for (int j = 0; j < 2; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int k0 = kb; k0 < ke; k0 += kTK) {
-        // stage A (64 x 32) and B (32 x 64, stored [n][k]); 8 elements each per thread
+    for (int k = 0; k < kKmsg / 16; k++) w1[k] = wfrag(wm, kH, j, 16 * k + 4 * L.g);
 #pragma unroll
-        for (int r = 0; r < (kTM * kTK) / kT; r++) {
-            const int idx = tid + r * kT;
-            int m, k;
-            if (TA) { m = idx % kTM; k = idx / kTM; } else { k = idx % kTK; m = idx / kTK; }
-            const int gm = m0 + m, gk = k0 + k;
-            float v = 0.f;
-            if (gm < M && gk < ke) v = TA ? A[(size_t)gk * lda + gm] : A[(size_t)gm * lda + gk];
-            sA[m * kLdsA + k] = to_bf16(v);
+    for (int k = 0; k < kKupd / 16; k++) u1[k] = wfrag(wu, kH, j, 16 * k + 4 * L.g);
+#pragma unroll
+    for (int k = 0; k < kH / 16; k++) {
+        w2[k] = wfrag(m2, kH, j, 16 * k + 4 * L.g);
+        u2[k] = wfrag(v2, kH, j, 16 * k + 4 * L.g);
+    }
+    const f32x4 mb1 = ldf4(m2 - kH + j0), mb2 = ldf4(m2 + kH * kH + j0);
+    const f32x4 ub1 = ldf4(v2 - kH + j0), ub2 = ldf4(v2 + kH * kH + j0);
+    const int slot = threadIdx.x >> 4, col = 4 * (threadIdx.x & 15);
+    for (int t = blockIdx.x; t < tiles; t += gridDim.x) {
+        const int n0 = tile_n0[t], nn = tile_n0[t + 1] - n0;
+        const int e0 = in_off[n0], e1 = in_off[n0 + nn];
+        const bool mine = slot < nn;
+        const int p0 = mine ? in_off[n0 + slot] : e1, p1 = mine ? in_off[n0 + slot + 1] : e1;
+        f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+        for (int eb = e0; eb < e1; eb += kTileRows) {
+            const int ne = min(kTileRows, e1 - eb);
+            load_z<kKmsg>(zm, eb, ne, z);
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < kTileRows / 16; i++)
+                if (16 * i < ne)
+                    *reinterpret_cast<bf16x4 *>(s1 + (16 * i + L.r) * kS + j0) =
+                        pack4(silu4(hidden<kKmsg>(L, z, i, w1, mb1)));
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < kTileRows / 16; i++)
+                if (16 * i < ne)
+                    *reinterpret_cast<f32x4 *>(msg + (16 * i + L.r) * kM + j0) = hidden<kH>(L, s1, i, w2, mb2);
+            __syncthreads();
+            for (int e = max(p0, eb); e < min(p1, eb + ne); e++) sum += ldf4(msg + (e - eb) * kM + col);
+            __syncthreads();
         }
-#pragma unroll
-        for (int r = 0; r < (kTN * kTK) / kT; r++) {
-            const int idx = tid + r * kT;
-            int n, k;
-            if (TB) { k = idx % kTK; n = idx / kTK; } else { n = idx % kTN; k = idx / kTN; }
-            const int gn = n0 + n, gk = k0 + k;
-            float v = 0.f;
-            if (gn < N && gk < ke) v = TB ? B[(size_t)gn * ldb + gk] : B[(size_t)gk * ldb + gn];
-            sB[n * kLdsB + k] = to_bf16(v);
+        if (mine) {
+            const int n = n0 + slot;
+            const bf16x4 a = pack4(sum * inv_deg[n]);
+            *reinterpret_cast<bf16x4 *>(u + slot * kU + kH + col) = a;
+            *reinterpret_cast<bf16x4 *>(u + slot * kU + col) = ld4(zm.hb + (size_t)n * kH + col);
+            if (agg) *reinterpret_cast<bf16x4 *>(agg + (size_t)n * kH + col) = a;
         }
         __syncthreads();
+        *reinterpret_cast<bf16x4 *>(t1 + L.r * kS + j0) = pack4(silu4(hidden<kKupd>(L, u, 0, u1, ub1)));
+        __syncthreads();
+        const f32x4 d = hidden<kH>(L, t1, 0, u2, ub2);
+        if (L.r < nn) {
+            const size_t at = (size_t)(n0 + L.r) * kH + j0;
+            const f32x4 hn = d + ldf4(h + at);
+            *reinterpret_cast<f32x4 *>(h_out + at) = hn;
+            *reinterpret_cast<bf16x4 *>(hb_out + at) = pack4(hn);
+        }
+    }
+}
+
+// out = W2 silu(W1 z + b1) + b2 of node rows (encoder, decoder); ob: a bfloat16 copy.
+template <int K, int O, typename Z>
+__global__ __launch_bounds__(kT) void k_node_fwd(int rows, Z zs, const float *__restrict__ w, float *__restrict__ out,
+                                                 u16 *__restrict__ ob) {
+    constexpr int kS = kH + kPad;
+    __shared__ __align__(16) u16 z[kTileRows * (K + kPad)], s1[kTileRows * kS];
+    const Lane L;
+    const int j0 = 16 * L.w + 4 * L.g;
+    const float *W2 = w + K * kH + kH;
+    // 16 outputs: the wavefronts share the row blocks instead
+    const int m0 = O == 16 ? 0 : 16 * L.w;
+    bf16x4 w1[K / 16], w2[kH / 16];
 #pragma unroll
-        for (int kk = 0; kk < kTK; kk += 16) {
-            // A fragment: row = lane % 16, k = kk + 4 * (lane / 16) + j
-            // B fragment: col = lane % 16, k = kk + 4 * (lane / 16) + j
-            bf16x4 af[2], bfr[2];
-            const int kq = kk + 4 * (lane >> 4);
+    for (int k = 0; k < K / 16; k++) w1[k] = wfrag(w, kH, 16 * L.w + L.r, 16 * k + 4 * L.g);
 #pragma unroll
-            for (int i = 0; i < 2; i++) {
-                const unsigned short *pa = &sA[(wm + i * 16 + (lane & 15)) * kLdsA + kq];
-                af[i] = bf16x4{(short)pa[0], (short)pa[1], (short)pa[2], (short)pa[3]};
-                const unsigned short *pb = &sB[(wn + i * 16 + (lane & 15)) * kLdsB + kq];
-                bfr[i] = bf16x4{(short)pb[0], (short)pb[1], (short)pb[2], (short)pb[3]};
+    for (int k = 0; k < kH / 16; k++) w2[k] = wfrag(W2, O, m0 + L.r, 16 * k + 4 * L.g);
+    const f32x4 b1 = ldf4(W2 - kH + j0), b2 = ldf4(W2 + kH * O + m0 + 4 * L.g);
+    for (int row0 = blockIdx.x * kTileRows; row0 < rows; row0 += gridDim.x * kTileRows) {
+        const int n = min(kTileRows, rows - row0);
+        load_z<K>(zs, row0, n, z);
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < kTileRows / 16; i++)
+            *reinterpret_cast<bf16x4 *>(s1 + (16 * i + L.r) * kS + j0) = pack4(silu4(hidden<K>(L, z, i, w1, b1)));
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < kTileRows / 16; i++) {
+            if (O == 16 && i != L.w) continue;
+            const f32x4 v = hidden<kH>(L, s1, i, w2, b2);
+            if (16 * i + L.r < n) {
+                const size_t at = (size_t)(row0 + 16 * i + L.r) * O + m0 + 4 * L.g;
+                *reinterpret_cast<f32x4 *>(out + at) = v;
+                if (ob) *reinterpret_cast<bf16x4 *>(ob + at) = pack4(v);
             }
+        }
+    }
+}
+
+// Backward of one MLP over tiles of kTileRows rows: z (input) and dy (gradient of the
+// output) in LDS, parameter gradients in registers until store().  NZ: 16-column
+// blocks of the input gradient that are wanted.
+template <int K, int O, int NZ>
+struct MlpBwd {
+    static constexpr int kZ = K + kPad, kS = kH + kPad, kY = O + kPad, kX = (NZ + 3) / 4;
+    struct Lds {
+        __align__(16) u16 z[kTileRows * kZ], dy[kTileRows * kY], s1[kTileRows * kS], da[kTileRows * kS];
+    };
+    Lane L;
+    bf16x4 w1[K / 16], w2t[O / 16], w1t[kX > 0 ? kX : 1][kH / 16];
+    f32x4 b1, dW1[K / 16], dW2[O / 16], db1, db2;
+
+    __device__ __forceinline__ MlpBwd(const float *w) {
+        const float *W2 = w + K * kH + kH;
+        const int j = 16 * L.w + L.r;
 #pragma unroll
-            for (int i = 0; i < 2; i++)
+        for (int k = 0; k < K / 16; k++) w1[k] = wfrag(w, kH, j, 16 * k + 4 * L.g);
 #pragma unroll
-                for (int j = 0; j < 2; j++)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(af[i], bfr[j], acc[i][j], 0, 0, 0);
+        for (int k = 0; k < O / 16; k++) w2t[k] = wfrag_t(W2, O, j, 16 * k + 4 * L.g);
+#pragma unroll
+        for (int x = 0; x < kX; x++)
+#pragma unroll
+            for (int k = 0; k < kH / 16; k++)
+                w1t[x][k] = wfrag_t(w, kH, 16 * (L.w + 4 * x) + L.r, 16 * k + 4 * L.g);
+        b1 = ldf4(W2 - kH + 16 * L.w + 4 * L.g);
+        const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int k = 0; k < K / 16; k++) dW1[k] = zero;
+#pragma unroll
+        for (int k = 0; k < O / 16; k++) dW2[k] = zero;
+        db1 = db2 = zero;
+    }
+
+    // The tile's output gradients, rounded, zero behind its n rows; a thread keeps to
+    // four columns, whose unrounded sum is the gradient of b2.
+    template <typename DY>
+    __device__ __forceinline__ void load_dy(const DY &dy, int row0, int n, u16 *t) {
+        constexpr int kC = O / 4;
+        const int c = threadIdx.x % kC;
+#pragma unroll
+        for (int i = 0; i < kTileRows * kC / kT; i++) {
+            const int r = threadIdx.x / kC + i * (kT / kC);
+            f32x4 v = {0.f, 0.f, 0.f, 0.f};
+            if (r < n) v = dy(row0 + r, 4 * c);
+            db2 += v;
+            *reinterpret_cast<bf16x4 *>(t + r * kY + 4 * c) = pack4(v);
+        }
+    }
+
+    // After load_z, load_dy and a barrier: the hidden layer again, its gradient da,
+    // and the tile's share of the parameter gradients.  Leaves da in LDS, z and dy
+    // free behind the barrier at the end.
+    __device__ __forceinline__ void tile(Lds &s) {
+        const int j0 = 16 * L.w + 4 * L.g;
+#pragma unroll 1  // (registers)
+        for (int i = 0; i < kTileRows / 16; i++) {
+            const f32x4 a = hidden<K>(L, s.z, i, w1, b1);
+            const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+            const f32x4 ds = hidden<O>(L, s.dy, i, w2t, zero);
+            const f32x4 d = {ds[0] * dsilu(a[0]), ds[1] * dsilu(a[1]), ds[2] * dsilu(a[2]), ds[3] * dsilu(a[3])};
+            db1 += d;
+            *reinterpret_cast<bf16x4 *>(s.s1 + (16 * i + L.r) * kS + j0) = pack4(silu4(a));
+            *reinterpret_cast<bf16x4 *>(s.da + (16 * i + L.r) * kS + j0) = pack4(d);
+        }
+        __syncthreads();
+#pragma unroll 1
+        for (int k = 0; k < kTileRows / 16; k++) {
+            const bf16x4 hs = ld4_t(L, s.s1, kS, 16 * k, 16 * L.w), hd = ld4_t(L, s.da, kS, 16 * k, 16 * L.w);
+#pragma unroll
+            for (int o = 0; o < O / 16; o++) dW2[o] = mfma(hs, ld4_t(L, s.dy, kY, 16 * k, 16 * o), dW2[o]);
+#pragma unroll
+            for (int c = 0; c < K / 16; c++) dW1[c] = mfma(ld4_t(L, s.z, kZ, 16 * k, 16 * c), hd, dW1[c]);
         }
         __syncthreads();
     }
-    // D fragment: col = lane % 16, row = 4 * (lane / 16) + j
+
+    // Gradient of input columns 16 (wavefront + 4 x) + 4 (l / 16) .. of row 16 i + l % 16.
+    __device__ __forceinline__ f32x4 dz(const Lds &s, int i, int x) const {
+        const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+        return hidden<kH>(L, s.da, i, w1t[x], zero);
+    }
+
+    // The block's partial gradients in the order of the parameters.
+    __device__ __forceinline__ void store(Lds &s, float *part) {
+        float *pb1 = part + K * kH, *pW2 = pb1 + kH, *pb2 = pW2 + kH * O;
 #pragma unroll
-    for (int i = 0; i < 2; i++)
+        for (int c = 0; c < K / 16; c++)
 #pragma unroll
-        for (int j = 0; j < 2; j++) {
-            const int gn = n0 + wn + j * 16 + (lane & 15);
-            if (gn >= N) continue;
-            const float bv = bias ? bias[gn] : 0.f;
+            for (int q = 0; q < 4; q++) part[(16 * c + 4 * L.g + q) * kH + 16 * L.w + L.r] = dW1[c][q];
 #pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const int gm = m0 + wm + i * 16 + 4 * (lane >> 4) + q;
-                if (gm >= M) continue;
-                const float v = acc[i][j][q] + bv;
-                C[(size_t)gm * ldc + gn] = v;
-                if (C2) C2[(size_t)gm * ldc + gn] = silu(v);
-            }
+        for (int o = 0; o < O / 16; o++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) pW2[(16 * L.w + 4 * L.g + q) * O + 16 * o + L.r] = dW2[o][q];
+#pragma unroll
+        for (int off = 8; off > 0; off >>= 1)
+#pragma unroll
+            for (int q = 0; q < 4; q++) db1[q] += __shfl_xor(db1[q], off, 64);
+        if (L.r == 0)
+#pragma unroll
+            for (int q = 0; q < 4; q++) pb1[16 * L.w + 4 * L.g + q] = db1[q];
+        constexpr int kC = O / 4;
+        static_assert(sizeof(s.s1) >= kT * sizeof(f32x4), "the sums over b2 take s1's place");
+        f32x4 *red = reinterpret_cast<f32x4 *>(s.s1);
+        __syncthreads();
+        red[threadIdx.x] = db2;
+        __syncthreads();
+        if ((int)threadIdx.x < kC) {
+            f32x4 v = red[threadIdx.x];
+            for (int t = threadIdx.x + kC; t < kT; t += kC) v += red[t];
+            *reinterpret_cast<f32x4 *>(pb2 + 4 * threadIdx.x) = v;
         }
+    }
+};
+
+struct DyNode {
+    const float *dy;
+    int ld;
+    __device__ __forceinline__ f32x4 operator()(int row, int c) const { return ldf4(dy + (size_t)row * ld + c); }
+};
+struct DyMsg {  // the mean's gradient: du[dst, 64:128] / deg
+    const int *dst;
+    const float *du, *inv_deg;
+    __device__ __forceinline__ f32x4 operator()(int row, int c) const {
+        const int d = dst[row];
+        return ldf4(du + (size_t)d * kKupd + kH + c) * inv_deg[d];
+    }
+};
+
+// Backward of an MLP on node rows: its gradient partials and, with NZ, dz [rows, 16 NZ].
+template <int K, int O, int NZ, typename Z>
+__global__ __launch_bounds__(kT, 2) void k_node_bwd(int rows, Z zs, DyNode dy, const float *__restrict__ w,
+                                                 float *__restrict__ dz, float *__restrict__ part, size_t part_ld) {
+    using B = MlpBwd<K, O, NZ>;
+    __shared__ typename B::Lds s;
+    B m(w);
+    for (int row0 = blockIdx.x * kTileRows; row0 < rows; row0 += gridDim.x * kTileRows) {
+        const int n = min(kTileRows, rows - row0);
+        load_z<K>(zs, row0, n, s.z);
+        m.load_dy(dy, row0, n, s.dy);
+        __syncthreads();
+        m.tile(s);
+#pragma unroll
+        for (int x = 0; x < B::kX; x++)
+#pragma unroll 1
+            for (int i = 0; i < kTileRows / 16; i++) {
+                const f32x4 v = m.dz(s, i, x);
+                if (16 * i + m.L.r < n)
+                    *reinterpret_cast<f32x4 *>(dz + (size_t)(row0 + 16 * i + m.L.r) * (16 * NZ) +
+                                               16 * (m.L.w + 4 * x) + 4 * m.L.g) = v;
+            }
+    }
+    m.store(s, part + blockIdx.x * part_ld);
 }
 
-// out[i] = sum_z parts[z * stride + i] in z order (deterministic split-K sum)
-__global__ __launch_bounds__(kT) void k_sum_splits(int n, int splits, size_t stride, const float *__restrict__ parts,
-                                                   float *__restrict__ out) {
-    const int i = blockIdx.x * kT + threadIdx.x;
-    if (i >= n) return;
-    float s = 0.f;
-    for (int z = 0; z < splits; z++) s += parts[z * stride + i];
-    out[i] = s;
+// Backward of the message MLP over the tiles of k_layer_fwd: its gradient partials, the
+// source half of the input gradient per edge (dzs, summed by k_dh_out), and
+//   dh[t] += du[t, 0:64] + sum_{e in in(t)} dz[e, 0:64].
+// 383k edges: 0.176 ms with two blocks a CU (what the registers allow), 0.284 with
+// one.  The kernels that this one stands for took 4 ms, 3 of them in weight
+// gradients whose few blocks each walked 4096 rows.
+__global__ __launch_bounds__(kT, 2) void k_msg_bwd(int tiles, const int *__restrict__ tile_n0,
+                                                const int *__restrict__ in_off, ZMsg zm, DyMsg dy,
+                                                const float *__restrict__ w, float *__restrict__ dh,
+                                                float *__restrict__ dzs, float *__restrict__ part, size_t part_ld) {
+    using B = MlpBwd<kKmsg, kH, 2 * kH / 16>;
+    constexpr int kM = kH + 4;
+    static_assert(kM * 4 <= B::kZ * 2, "the destination half takes the place of the edge rows");
+    __shared__ typename B::Lds s;
+    float *dzd = reinterpret_cast<float *>(s.z);
+    B m(w);
+    const int slot = threadIdx.x >> 4, col = 4 * (threadIdx.x & 15);
+    for (int t = blockIdx.x; t < tiles; t += gridDim.x) {
+        const int n0 = tile_n0[t], nn = tile_n0[t + 1] - n0;
+        const int e0 = in_off[n0], e1 = in_off[n0 + nn];
+        const bool mine = slot < nn;
+        const int p0 = mine ? in_off[n0 + slot] : e1, p1 = mine ? in_off[n0 + slot + 1] : e1;
+        const size_t at = (size_t)(n0 + slot) * kH + col;
+        f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+        if (mine) sum = ldf4(dh + at) + ldf4(dy.du + (size_t)(n0 + slot) * kKupd + col);
+        for (int eb = e0; eb < e1; eb += kTileRows) {
+            const int ne = min(kTileRows, e1 - eb);
+            load_z<kKmsg>(zm, eb, ne, s.z);
+            m.load_dy(dy, eb, ne, s.dy);
+            __syncthreads();
+            m.tile(s);
+#pragma unroll 1
+            for (int i = 0; i < kTileRows / 16; i++) {
+                const int r = 16 * i + m.L.r, c = 16 * m.L.w + 4 * m.L.g;
+                *reinterpret_cast<f32x4 *>(dzd + r * kM + c) = m.dz(s, i, 0);
+                const f32x4 v = m.dz(s, i, 1);
+                if (r < ne) *reinterpret_cast<f32x4 *>(dzs + (size_t)(eb + r) * kH + c) = v;
+            }
+            __syncthreads();
+            for (int e = max(p0, eb); e < min(p1, eb + ne); e++) sum += ldf4(dzd + (e - eb) * kM + col);
+            __syncthreads();
+        }
+        if (mine) *reinterpret_cast<f32x4 *>(dh + at) = sum;
+    }
+    m.store(s, part + blockIdx.x * part_ld);
 }
 
-// db[c] = sum over rows of d[r * ld + c] (one block per column, fixed tree order)
-__global__ __launch_bounds__(kT) void k_colsum(int rows, int ld, const float *__restrict__ d, float *__restrict__ db) {
-    __shared__ float red[kT];
-    const int c = blockIdx.x;
+//   dh[t] += sum_{e in out(t)} dzs[e]
+__global__ __launch_bounds__(kT) void k_dh_out(int N, const int *__restrict__ out_off, const int *__restrict__ out_edge,
+                                               const float *__restrict__ dzs, float *__restrict__ dh) {
+    const int64_t t = (int64_t)blockIdx.x * kT + threadIdx.x;
+    if (t >= (int64_t)N * (kH / 4)) return;
+    const int i = (int)(t / (kH / 4)), c = 4 * (int)(t - (int64_t)i * (kH / 4));
+    f32x4 s = ldf4(dh + (size_t)i * kH + c);
+    for (int q = out_off[i]; q < out_off[i + 1]; q++) s += ldf4(dzs + (size_t)out_edge[q] * kH + c);
+    *reinterpret_cast<f32x4 *>(dh + (size_t)i * kH + c) = s;
+}
+
+// g[p] = sum over the blocks' partials of parameter p, in a fixed order (four
+// interleaved sums, then their sum).  Message MLPs have parts_e partials, the
+// others parts_n.
+constexpr int kEnc = (kDin + 1) * kH + (kH + 1) * kH;
+constexpr int kMsg = (kKmsg + 1) * kH + (kH + 1) * kH;
+constexpr int kUpd = (kKupd + 1) * kH + (kH + 1) * kH;
+
+__global__ __launch_bounds__(kT) void k_sum_parts(int P, int parts_n, int parts_e, const float *__restrict__ part,
+                                                  float *__restrict__ g) {
+    __shared__ float red[4][64];
+    const int o = threadIdx.x & 63, sl = threadIdx.x >> 6;
+    const int p = blockIdx.x * 64 + o;
     float s = 0.f;
-    for (int r = threadIdx.x; r < rows; r += kT) s += d[(size_t)r * ld + c];
-    red[threadIdx.x] = s;
+    if (p < P) {
+        const int q = p - kEnc;
+        const bool msg = q >= 0 && q < kLayers * (kMsg + kUpd) && q % (kMsg + kUpd) < kMsg;
+        const int n = msg ? parts_e : parts_n;
+#pragma unroll 8
+        for (int b = sl; b < n; b += 4) s += part[(size_t)b * P + p];
+    }
+    red[sl][o] = s;
     __syncthreads();
-    for (int off = kT / 2; off > 0; off >>= 1) {
-        if ((int)threadIdx.x < off) red[threadIdx.x] += red[threadIdx.x + off];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) db[c] = red[0];
-}
-
-// z[e] = [h[dst_e], h[src_e], f_e]
-__global__ __launch_bounds__(kT) void k_gather_msg(int E, const int *__restrict__ src, const int *__restrict__ dst,
-                                                   const float *__restrict__ h, const float *__restrict__ f,
-                                                   float *__restrict__ z) {
-    const int64_t t = (int64_t)blockIdx.x * kT + threadIdx.x;
-    if (t >= (int64_t)E * kKmsg) return;
-    const int e = (int)(t / kKmsg), c = (int)(t - (int64_t)e * kKmsg);
-    float v;
-    if (c < kH) v = h[(size_t)dst[e] * kH + c];
-    else if (c < 2 * kH) v = h[(size_t)src[e] * kH + c - kH];
-    else v = f[(size_t)e * kDedge + c - 2 * kH];
-    z[t] = v;
-}
-
-// u[t] = [h[t], inv_deg[t] * sum_{e in in(t)} m[e]]
-__global__ __launch_bounds__(kT) void k_aggregate(int N, const int *__restrict__ in_off, const float *__restrict__ inv_deg,
-                                                  const float *__restrict__ h, const float *__restrict__ m,
-                                                  float *__restrict__ u) {
-    const int64_t t = (int64_t)blockIdx.x * kT + threadIdx.x;
-    if (t >= (int64_t)N * kH) return;
-    const int i = (int)(t / kH), c = (int)(t - (int64_t)i * kH);
-    float s = 0.f;
-    for (int e = in_off[i]; e < in_off[i + 1]; e++) s += m[(size_t)e * kH + c];
-    u[(size_t)i * kKupd + c] = h[t];
-    u[(size_t)i * kKupd + kH + c] = s * inv_deg[i];
-}
-
-// y[i] += x[i] (residual stream)
-__global__ __launch_bounds__(kT) void k_axpy(int64_t n, const float *__restrict__ x, float *__restrict__ y) {
-    const int64_t i = (int64_t)blockIdx.x * kT + threadIdx.x;
-    if (i < n) y[i] += x[i];
-}
-
-// d[i] *= silu'(a[i])
-__global__ __launch_bounds__(kT) void k_dsilu(int64_t n, const float *__restrict__ a, float *__restrict__ d) {
-    const int64_t i = (int64_t)blockIdx.x * kT + threadIdx.x;
-    if (i < n) d[i] *= dsilu(a[i]);
-}
-
-// Backward of aggregate + gather for one layer:
-//   dm[e]  = du[dst_e, 64:128] * inv_deg[dst_e]
-__global__ __launch_bounds__(kT) void k_dmsg(int E, const int *__restrict__ dst, const float *__restrict__ inv_deg,
-                                             const float *__restrict__ du, float *__restrict__ dm) {
-    const int64_t t = (int64_t)blockIdx.x * kT + threadIdx.x;
-    if (t >= (int64_t)E * kH) return;
-    const int e = (int)(t / kH), c = (int)(t - (int64_t)e * kH);
-    const int d = dst[e];
-    dm[t] = du[(size_t)d * kKupd + kH + c] * inv_deg[d];
-}
-
-//   dh[t] += du[t, 0:64] + sum_{e in in(t)} dz[e, 0:64] + sum_{e in out(t)} dz[e, 64:128]
-__global__ __launch_bounds__(kT) void k_dh_layer(int N, const int *__restrict__ in_off, const int *__restrict__ out_off,
-                                                 const int *__restrict__ out_edge, const float *__restrict__ du,
-                                                 const float *__restrict__ dz, float *__restrict__ dh) {
-    const int64_t t = (int64_t)blockIdx.x * kT + threadIdx.x;
-    if (t >= (int64_t)N * kH) return;
-    const int i = (int)(t / kH), c = (int)(t - (int64_t)i * kH);
-    float s = dh[t] + du[(size_t)i * kKupd + c];
-    for (int e = in_off[i]; e < in_off[i + 1]; e++) s += dz[(size_t)e * kKmsg + c];
-    for (int q = out_off[i]; q < out_off[i + 1]; q++) s += dz[(size_t)out_edge[q] * kKmsg + kH + c];
-    dh[t] = s;
+    if (sl == 0 && p < P) g[p] = (red[0][o] + red[1][o]) + (red[2][o] + red[3][o]);
 }
 
 // dy = 2 (y - t) mask / n_used; per-block partial sums of the squared error
@@ -309,31 +593,26 @@ size_t n_params_total() { return mlp_off(kMlps - 1).end; }
 
 }  // namespace
 
-// Activation caches of one MLP application: input z [rows, k], a1 and s1 [rows, 64].
-struct MlpCache {
-    float *z = nullptr, *a1 = nullptr, *s1 = nullptr;
-    int rows = 0;
-};
-
 struct plbfs_mpnn {
     int N = 0, E = 0;
     hipStream_t stream = nullptr;
     std::vector<void *> allocs;
     int *src = nullptr, *dst = nullptr, *in_off = nullptr, *out_off = nullptr, *out_edge = nullptr;
-    float *inv_deg = nullptr, *ef = nullptr;
+    float *inv_deg = nullptr;
     std::vector<int32_t> h_order;  // sorted edge -> caller edge
     size_t P = 0;
     float *w = nullptr, *g = nullptr, *m1 = nullptr, *m2 = nullptr;
     int adam_t = 0;
-    // activations
+    int tiles = 0;            // edge tiles: nodes tile_n0[t] .. tile_n0[t + 1]
+    int *tile_n0 = nullptr;
     float *x = nullptr, *y = nullptr, *tgt = nullptr, *mask = nullptr, *dy = nullptr;
-    float *h[kLayers + 1] = {};
-    MlpCache cache[kMlps];
-    float *out_tmp = nullptr;  // [max(E,N) * 64] MLP output scratch (messages, update deltas)
-    float *dbuf0 = nullptr, *dbuf1 = nullptr, *dbuf2 = nullptr;  // backward scratch
-    float *dh = nullptr;
-    float *split = nullptr;
-    size_t split_cap = 0;
+    float *h[2] = {};                // node states, ping-pong over the layers
+    u16 *hb[kLayers + 1] = {};       // ... as bfloat16, of every layer (two in turn without training)
+    u16 *agg[kLayers] = {};          // training: mean messages as bfloat16
+    u16 *fb = nullptr;               // edge inputs as bfloat16
+    float *dh = nullptr, *du = nullptr, *dzs = nullptr;  // backward scratch
+    float *part = nullptr;           // [max(parts_n, parts_e)][P] weight-gradient partials
+    int parts_n = 0, parts_e = 0;
     double *mse_part = nullptr;
     int mse_blocks = 0;
     float mse_scale = 1.f;
@@ -359,99 +638,48 @@ int upload_t(plbfs_mpnn *n, T **dst, const std::vector<T> &src) {
 
 inline dim3 grid1(int64_t n) { return dim3((unsigned)((n + kT - 1) / kT)); }
 
-// C[M,N] = op(A) op(B) (+ bias, C2 = silu) on the matrix cores.
-template <bool TA, bool TB>
-void gemm(plbfs_mpnn *n, int M, int Nn, int K, const float *A, int lda, const float *B, int ldb, float *C, int ldc,
-          const float *bias, float *C2) {
-    const dim3 grid((M + kTM - 1) / kTM, (Nn + kTN - 1) / kTN, 1);
-    hipLaunchKernelGGL((k_gemm<TA, TB>), grid, dim3(kT), 0, n->stream, M, Nn, K, A, lda, B, ldb, C, ldc, K,
-                       (size_t)0, bias, C2);
-}
+// Blocks of a kernel over `tiles` tiles: enough to fill the chip a few times, each
+// keeping its weights for several tiles where there are more.
+inline dim3 tile_grid(int tiles, int most) { return dim3((unsigned)std::max(1, std::min(tiles, most))); }
+inline int row_tiles(int rows) { return (rows + kTileRows - 1) / kTileRows; }
+constexpr int kFwdBlocks = 1024;
 
-// Weight gradient dW[K, Nn] = A^T[K, M] B[M, Nn] with the reduction over M
-// split into row ranges (deterministic fixed-order sum of the partials).
-int gemm_tn_split(plbfs_mpnn *n, int M, int Nn, int K, const float *A, int lda, const float *B, int ldb, float *C) {
-    const int chunk = 4096;
-    const int splits = std::max(1, (M + chunk - 1) / chunk);
-    const size_t stride = (size_t)K * Nn;
-    if ((size_t)splits * stride > n->split_cap) {
-        int rc = malloc_t(n, (void **)&n->split, (size_t)splits * stride * sizeof(float));
-        if (rc) return rc;
-        n->split_cap = (size_t)splits * stride;
-    }
-    // output rows = K (columns of A), reduction dimension = M (rows of A and B)
-    const dim3 grid((K + kTM - 1) / kTM, (Nn + kTN - 1) / kTN, splits);
-    hipLaunchKernelGGL((k_gemm<true, false>), grid, dim3(kT), 0, n->stream, K, Nn, M, A, lda, B, ldb, n->split, Nn,
-                       chunk, stride, (const float *)nullptr, (float *)nullptr);
-    hipLaunchKernelGGL(k_sum_splits, grid1((int64_t)stride), dim3(kT), 0, n->stream, (int)stride, splits, stride,
-                       n->split, C);
-    return PLBFS_OK;
-}
-
-// y = W2 silu(W1 z + b1) + b2 over rows rows; caches z, a1, s1.
-void mlp_fwd(plbfs_mpnn *n, int q, int rows, float *z, float *out) {
-    const MlpShape s = mlp_shape(q);
-    const MlpOff o = mlp_off(q);
-    MlpCache &c = n->cache[q];
-    c.z = z;
-    c.rows = rows;
-    gemm<false, false>(n, rows, kH, s.k, z, s.k, n->w + o.W1, kH, c.a1, kH, n->w + o.b1, c.s1);
-    gemm<false, false>(n, rows, s.o, kH, c.s1, kH, n->w + o.W2, s.o, out, s.o, n->w + o.b2, nullptr);
-}
-
-// Backward of MLP q given dy [rows, o]: writes its parameter gradients and
-// dz [rows, k] (if dz).  Scratch: dbuf0 [rows, 64].
-int mlp_bwd(plbfs_mpnn *n, int q, const float *dy, float *dz) {
-    const MlpShape s = mlp_shape(q);
-    const MlpOff o = mlp_off(q);
-    const MlpCache &c = n->cache[q];
-    const int rows = c.rows;
-    int rc;
-    if ((rc = gemm_tn_split(n, rows, s.o, kH, c.s1, kH, dy, s.o, n->g + o.W2))) return rc;
-    hipLaunchKernelGGL(k_colsum, dim3(s.o), dim3(kT), 0, n->stream, rows, s.o, dy, n->g + o.b2);
-    float *da1 = n->dbuf0;
-    gemm<false, true>(n, rows, kH, s.o, dy, s.o, n->w + o.W2, s.o, da1, kH, nullptr, nullptr);
-    hipLaunchKernelGGL(k_dsilu, grid1((int64_t)rows * kH), dim3(kT), 0, n->stream, (int64_t)rows * kH, c.a1, da1);
-    if ((rc = gemm_tn_split(n, rows, kH, s.k, c.z, s.k, da1, kH, n->g + o.W1))) return rc;
-    hipLaunchKernelGGL(k_colsum, dim3(kH), dim3(kT), 0, n->stream, rows, kH, da1, n->g + o.b1);
-    if (dz) gemm<false, true>(n, rows, s.k, kH, da1, kH, n->w + o.W1, kH, dz, s.k, nullptr, nullptr);
-    return PLBFS_OK;
-}
+ZMsg zmsg(const plbfs_mpnn *n, int layer) { return ZMsg{n->src, n->dst, n->hb[layer], n->fb}; }
 
 void forward(plbfs_mpnn *n) {
-    const int N = n->N, E = n->E;
-    mlp_fwd(n, 0, N, n->x, n->h[0]);
-    for (int l = 0; l < kLayers; l++) {
-        const int qm = 1 + 2 * l, qu = 2 + 2 * l;
-        hipLaunchKernelGGL(k_gather_msg, grid1((int64_t)E * kKmsg), dim3(kT), 0, n->stream, E, n->src, n->dst,
-                           n->h[l], n->ef, n->cache[qm].z);
-        mlp_fwd(n, qm, E, n->cache[qm].z, n->out_tmp);
-        hipLaunchKernelGGL(k_aggregate, grid1((int64_t)N * kH), dim3(kT), 0, n->stream, N, n->in_off, n->inv_deg,
-                           n->h[l], n->out_tmp, n->cache[qu].z);
-        mlp_fwd(n, qu, N, n->cache[qu].z, n->h[l + 1]);
-        hipLaunchKernelGGL(k_axpy, grid1((int64_t)N * kH), dim3(kT), 0, n->stream, (int64_t)N * kH, n->h[l],
-                           n->h[l + 1]);
-    }
-    mlp_fwd(n, kMlps - 1, N, n->h[kLayers], n->y);
+    const int N = n->N, nt = row_tiles(N);
+    hipLaunchKernelGGL((k_node_fwd<kDin, kH, ZInput>), tile_grid(nt, kFwdBlocks), dim3(kT), 0, n->stream, N,
+                       ZInput{n->x}, n->w + mlp_off(0).W1, n->h[0], n->hb[0]);
+    for (int l = 0; l < kLayers; l++)
+        hipLaunchKernelGGL(k_layer_fwd, tile_grid(n->tiles, kFwdBlocks), dim3(kT), 0, n->stream, n->tiles, n->tile_n0,
+                           n->in_off, zmsg(n, l), n->inv_deg, n->h[l & 1], n->h[(l + 1) & 1], n->hb[l + 1],
+                           n->agg[l], n->w + mlp_off(1 + 2 * l).W1, n->w + mlp_off(2 + 2 * l).W1);
+    hipLaunchKernelGGL((k_node_fwd<kH, kDout, ZNode>), tile_grid(nt, kFwdBlocks), dim3(kT), 0, n->stream, N,
+                       ZNode{n->hb[kLayers], nullptr}, n->w + mlp_off(kMlps - 1).W1, n->y, (u16 *)nullptr);
 }
 
-int backward(plbfs_mpnn *n) {
-    const int N = n->N, E = n->E;
-    int rc;
-    // dh = d dec / d h
-    if ((rc = mlp_bwd(n, kMlps - 1, n->dy, n->dh))) return rc;
+void backward(plbfs_mpnn *n) {
+    const int N = n->N;
+    const size_t P = n->P;
+    const dim3 gn(n->parts_n), ge(n->parts_e), block(kT);
+    hipStream_t st = n->stream;
+    auto part = [&](int q) { return n->part + mlp_off(q).W1; };
+    auto w = [&](int q) { return n->w + mlp_off(q).W1; };
+    hipLaunchKernelGGL((k_node_bwd<kH, kDout, kH / 16, ZNode>), gn, block, 0, st, N, ZNode{n->hb[kLayers], nullptr},
+                       DyNode{n->dy, kDout}, w(kMlps - 1), n->dh, part(kMlps - 1), P);
     for (int l = kLayers - 1; l >= 0; l--) {
         const int qm = 1 + 2 * l, qu = 2 + 2 * l;
-        float *du = n->dbuf1;  // [N, 128]
-        if ((rc = mlp_bwd(n, qu, n->dh, du))) return rc;
-        float *dm = n->out_tmp;  // [E, 64]
-        hipLaunchKernelGGL(k_dmsg, grid1((int64_t)E * kH), dim3(kT), 0, n->stream, E, n->dst, n->inv_deg, du, dm);
-        float *dz = n->dbuf2;  // [E, 144]
-        if ((rc = mlp_bwd(n, qm, dm, dz))) return rc;
-        hipLaunchKernelGGL(k_dh_layer, grid1((int64_t)N * kH), dim3(kT), 0, n->stream, N, n->in_off, n->out_off,
-                           n->out_edge, du, dz, n->dh);
+        hipLaunchKernelGGL((k_node_bwd<kKupd, kH, kKupd / 16, ZNode>), gn, block, 0, st, N,
+                           ZNode{n->hb[l], n->agg[l]}, DyNode{n->dh, kH}, w(qu), n->du, part(qu), P);
+        hipLaunchKernelGGL(k_msg_bwd, ge, block, 0, st, n->tiles, n->tile_n0, n->in_off, zmsg(n, l),
+                           DyMsg{n->dst, n->du, n->inv_deg}, w(qm), n->dh, n->dzs, part(qm), P);
+        hipLaunchKernelGGL(k_dh_out, grid1((int64_t)N * (kH / 4)), block, 0, st, N, n->out_off, n->out_edge, n->dzs,
+                           n->dh);
     }
-    return mlp_bwd(n, 0, n->dh, nullptr);
+    hipLaunchKernelGGL((k_node_bwd<kDin, kH, 0, ZInput>), gn, block, 0, st, N, ZInput{n->x}, DyNode{n->dh, kH}, w(0),
+                       (float *)nullptr, part(0), P);
+    hipLaunchKernelGGL(k_sum_parts, dim3((unsigned)((P + 63) / 64)), block, 0, st, (int)P, n->parts_n, n->parts_e,
+                       n->part, n->g);
 }
 
 }  // namespace
@@ -486,11 +714,12 @@ extern "C" int plbfs_mpnn_create(int32_t n_nodes, int32_t n_edges, const int32_t
     });
     n->h_order = ord;
     std::vector<int32_t> s(E), d(E), in_off(N + 1, 0), out_off(N + 1, 0), out_edge(E);
-    std::vector<float> f((size_t)E * kDedge), inv_deg(N);
+    std::vector<u16> f((size_t)E * kDedge);
+    std::vector<float> inv_deg(N);
     for (int e = 0; e < E; e++) {
         s[e] = src[ord[e]];
         d[e] = dst[ord[e]];
-        std::memcpy(&f[(size_t)e * kDedge], edge_feat + (size_t)ord[e] * kDedge, kDedge * sizeof(float));
+        for (int k = 0; k < kDedge; k++) f[(size_t)e * kDedge + k] = to_bf16(edge_feat[(size_t)ord[e] * kDedge + k]);
         in_off[d[e] + 1]++;
         out_off[s[e] + 1]++;
     }
@@ -506,37 +735,45 @@ extern "C" int plbfs_mpnn_create(int32_t n_nodes, int32_t n_edges, const int32_t
     int rc;
     if ((rc = upload_t(n, &n->src, s)) || (rc = upload_t(n, &n->dst, d)) || (rc = upload_t(n, &n->in_off, in_off)) ||
         (rc = upload_t(n, &n->out_off, out_off)) || (rc = upload_t(n, &n->out_edge, out_edge)) ||
-        (rc = upload_t(n, &n->inv_deg, inv_deg)) || (rc = upload_t(n, &n->ef, f)))
+        (rc = upload_t(n, &n->inv_deg, inv_deg)) || (rc = upload_t(n, &n->fb, f)))
         return fail(rc);
+    // edge tiles: nodes while they and their in-edges fit, at least one
+    std::vector<int32_t> t0(1, 0);
+    for (int i = 0; i < N;) {
+        int k = i + 1;
+        while (k < N && k - i < kTileNodes && in_off[k + 1] - in_off[i] <= kTileRows) k++;
+        t0.push_back(k);
+        i = k;
+    }
+    n->tiles = (int)t0.size() - 1;
+    if ((rc = upload_t(n, &n->tile_n0, t0))) return fail(rc);
     n->P = n_params_total();
     const size_t P = n->P;
     std::vector<float> zero(P, 0.f);
     if ((rc = upload_t(n, &n->w, zero)) || (rc = upload_t(n, &n->g, zero)) || (rc = upload_t(n, &n->m1, zero)) ||
         (rc = upload_t(n, &n->m2, zero)))
         return fail(rc);
-    const size_t NE = (size_t)std::max(N, E);
     auto fa = [&](float **p, size_t count) { return malloc_t(n, (void **)p, count * sizeof(float)); };
+    auto ha = [&](u16 **p, size_t count) { return malloc_t(n, (void **)p, count * sizeof(u16)); };
     if ((rc = fa(&n->x, (size_t)N * kDin)) || (rc = fa(&n->y, (size_t)N * kDout)) ||
         (rc = fa(&n->tgt, (size_t)N * kDout)) || (rc = fa(&n->mask, (size_t)N * kDout)) ||
-        (rc = fa(&n->dy, (size_t)N * kDout)) || (rc = fa(&n->out_tmp, NE * kH)) ||
-        (rc = fa(&n->dbuf0, NE * kH)) || (rc = fa(&n->dbuf1, (size_t)N * kKupd)) ||
-        (rc = fa(&n->dh, (size_t)N * kH)))
+        (rc = fa(&n->dy, (size_t)N * kDout)) || (rc = fa(&n->h[0], (size_t)N * kH)) ||
+        (rc = fa(&n->h[1], (size_t)N * kH)))
         return fail(rc);
-    if (n->train && (rc = fa(&n->dbuf2, (size_t)E * kKmsg + 1))) return fail(rc);
-    for (int l = 0; l <= kLayers; l++)
-        if ((rc = fa(&n->h[l], (size_t)N * kH))) return fail(rc);
-    // activations kept for the backward pass; without training every message
-    // layer shares one buffer set and every update layer another
-    for (int q = 0; q < kMlps; q++) {
-        const MlpShape sh = mlp_shape(q);
-        const size_t rows = (q % 2 == 1 && q < kMlps - 1) ? (size_t)E : (size_t)N;
-        MlpCache &c = n->cache[q];
-        if (!n->train && q >= 3 && q < kMlps - 1) {
-            c = n->cache[q % 2 == 1 ? 1 : 2];
+    for (int l = 0; l <= kLayers; l++) {
+        if (!n->train && l >= 2) {
+            n->hb[l] = n->hb[l & 1];
             continue;
         }
-        if ((q > 0 && q < kMlps - 1 && (rc = fa(&c.z, rows * sh.k + 1))) || (rc = fa(&c.a1, rows * kH + 1)) ||
-            (rc = fa(&c.s1, rows * kH + 1)))
+        if ((rc = ha(&n->hb[l], (size_t)N * kH))) return fail(rc);
+    }
+    if (n->train) {
+        n->parts_n = std::min(row_tiles(N), kMaxParts);
+        n->parts_e = std::min(n->tiles, kMaxParts);
+        for (int l = 0; l < kLayers; l++)
+            if ((rc = ha(&n->agg[l], (size_t)N * kH))) return fail(rc);
+        if ((rc = fa(&n->dh, (size_t)N * kH)) || (rc = fa(&n->du, (size_t)N * kKupd)) ||
+            (rc = fa(&n->dzs, (size_t)E * kH)) || (rc = fa(&n->part, P * std::max(n->parts_n, n->parts_e))))
             return fail(rc);
     }
     n->mse_blocks = (int)(((int64_t)N * kDout + kT - 1) / kT);
@@ -573,7 +810,6 @@ extern "C" int plbfs_mpnn_get_params(plbfs_mpnn *n, float *params) {
 extern "C" int plbfs_mpnn_forward(plbfs_mpnn *n, const float *x, float *y) {
     if (!n || !x || !y) return plbfs_fail(PLBFS_ERR_INPUT, "null argument");
     HIP_TRY(hipMemcpyAsync(n->x, x, (size_t)n->N * kDin * sizeof(float), hipMemcpyHostToDevice, n->stream));
-    n->cache[0].z = n->x;
     forward(n);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipMemcpyAsync(y, n->y, (size_t)n->N * kDout * sizeof(float), hipMemcpyDeviceToHost, n->stream));
@@ -585,12 +821,10 @@ namespace {
 
 int loss_grad_device(plbfs_mpnn *n, double *loss) {
     const int64_t ny = (int64_t)n->N * kDout;
-    n->cache[0].z = n->x;
     forward(n);
     hipLaunchKernelGGL(k_mse, grid1(ny), dim3(kT), 0, n->stream, ny, n->mse_scale, n->y, n->tgt, n->mask, n->dy,
                        n->mse_part);
-    int rc = backward(n);
-    if (rc) return rc;
+    backward(n);
     HIP_TRY(hipGetLastError());
     if (loss) {
         std::vector<double> part(n->mse_blocks);

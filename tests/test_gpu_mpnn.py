@@ -89,3 +89,46 @@ def test_training_reduces_loss(gpu_available):
     hist = net.train(X, T, mpnn.output_mask(N), epochs=40, lr=2e-3, seed=3)
     assert np.all(np.isfinite(hist))
     assert hist[-1] < 0.2 * hist[0], hist
+
+
+@pytest.mark.parametrize("n,degrees", [
+    (1, [0]),                      # one node without edges
+    (5, [3, 0, 4, 1, 2]),
+    (16, [4]),                     # one tile exactly: 16 nodes, 64 edges
+    (17, [4]),                     # one node more
+    (33, [6]),                     # tiles end at 60 of 64 edges
+    (65, [0, 1, 2, 3]),
+    (40, [63, 64, 65, 2, 0]),      # nodes that fill a tile, overfill it, or share one
+    (12, [200, 1, 129, 64]),       # a node over several chunks of 64 edges
+])
+def test_edge_tiles_match_reference(gpu_available, n, degrees):
+    """Graphs whose in-degrees meet the edges of the kernels' tiles (16 nodes, 64
+    edges, one node of more), forward and backward, at the bars of this file."""
+    rng = np.random.default_rng(n)
+    dst = np.repeat(np.arange(n), [degrees[k % len(degrees)] for k in range(n)]).astype(np.int32)
+    src = rng.integers(0, n, size=len(dst)).astype(np.int32)
+    order = rng.permutation(len(dst))
+    src, dst = src[order], dst[order]
+    ef = rng.normal(size=(len(dst), 16)).astype(np.float32)
+    x = rng.normal(size=(n, 16)).astype(np.float32)
+    tgt = rng.normal(size=(n, 16)).astype(np.float32)
+    P, shapes, mask = M.init_params(6), M.mlp_shapes(), mpnn.output_mask(n)
+    net = mpnn.Mpnn(n, src, dst, ef, train=True)
+    net.set_params(mpnn.flatten_params(P, shapes))
+    y = net.forward(x)
+    loss, g = net.loss_grad(x, tgt, mask)
+    G = M.Graph(src, dst, n)
+    lr, _, gr = M.loss_and_grads(P, G, x.astype(np.float64), ef[G.order].astype(np.float64),
+                                 tgt.astype(np.float64), mask.astype(np.float64), bf16_mode=True)
+    yr, _ = M.forward(P, G, x.astype(np.float64), ef[G.order].astype(np.float64), bf16_mode=True)
+    assert rel(y[:, :4], yr[:, :4]) < 1e-2
+    assert abs(loss - lr) / lr < 1e-2
+    gg = mpnn.unflatten(g, shapes)
+    for name, _, _ in shapes:
+        for key in ("W1", "b1", "W2", "b2"):
+            assert np.linalg.norm(gg[name][key] - gr[name][key]) < 3e-2 * max(np.linalg.norm(gr[name][key]), 1e-6), (
+                name, key)
+    # inference buffers give the same prediction
+    infer = mpnn.Mpnn(n, src, dst, ef, train=False)
+    infer.set_params(mpnn.flatten_params(P, shapes))
+    assert np.array_equal(infer.forward(x), y)
