@@ -77,6 +77,8 @@ __device__ __forceinline__ int xcd_block(int bid, int nblk, int remap) {
     return x * q + (x < r ? x : r) + k;
 }
 
+constexpr int kNoEnt = 0xffff;  // no face (see DevMesh::g_ent)
+
 // 16 B chunks per face item (see DevMesh::it_p).
 template <typename S>
 inline constexpr int kItemChunks = std::is_same<S, float>::value ? 3 : 5;
@@ -93,6 +95,7 @@ struct DevMesh {
     int block_cells;  // cells per flux block (a multiple of 64)
     int stage;        // 1: flux blocks stage their own cells' records in LDS
     int grad_stage;   // 1: gradient blocks stage their own cells' states in LDS
+    int max_slots;    // most stencil slots of a cell
     int64_t E;
     const uint8_t *st_cnt;
     const int32_t *st_nbr;
@@ -112,7 +115,12 @@ struct DevMesh {
     const double *it_dt;
     const uint16_t *it_side;
     S b0[3];
-    const int32_t *g_off, *g_ent;
+    // a cell's faces in the reference face order, entry s of cell i at s * N + i:
+    // slot << 1 | is_owner, kNoEnt behind the last one (max_ent: most of a cell);
+    // with a border pass g_ent_split instead, as in the layout, -1 behind the last
+    const uint16_t *g_ent;
+    const int32_t *g_ent_split;
+    int max_ent;
     // [n_blocks] nonzero where a flux block holds a cell the immersed boundary
     // spreads force to; null: every block reads the body force
     const int32_t *blk_force;

@@ -64,6 +64,16 @@ __device__ __forceinline__ void block_fluxes(const DevMesh<S> &m, const DevParam
     }
 }
 
+// Gather entries face by face (see DevMesh::g_ent); conv turns the layout's entry.
+template <typename T, typename F>
+static std::vector<T> entries_by_face(const Layout &L, int max_ent, T none, F conv) {
+    const size_t N = (size_t)L.N;
+    std::vector<T> v(N * max_ent, none);
+    for (size_t i = 0; i < N; i++)
+        for (int k = L.g_off[i]; k < L.g_off[i + 1]; k++) v[(size_t)(k - L.g_off[i]) * N + i] = conv(L.g_ent[k]);
+    return v;
+}
+
 // Face items in groups of 64 (see DevMesh::it_p).
 template <typename S>
 static std::vector<float4> pack_items(const Layout &L) {
@@ -510,6 +520,7 @@ int create_ctx(const plbfs_mesh_view *mesh, const plbfs_params *params, const pl
     d.n_border = (int)L.n_border;
     d.bflux = nullptr;
     d.blk_force = nullptr;
+    d.max_slots = *std::max_element(L.st_cnt.begin(), L.st_cnt.end());
     for (int a = 0; a < 3; a++) d.b0[a] = L.b0[a];
     d.block_cells = L.block_cells;
     d.stage = stage ? 1 : 0;
@@ -532,6 +543,21 @@ int create_ctx(const plbfs_mesh_view *mesh, const plbfs_params *params, const pl
         dp[q].v = patches[q].v;
         dp[q].w = patches[q].w;
     }
+    // the entries of the border pass hold indices beyond 16 bits; without it a slot
+    // is below kMaxLds / 16
+    static_assert(kMaxLds / 16 < kNoEnt >> 1, "slots fit the 16-bit entries");
+    d.max_ent = 1;
+    for (int i = 0; i < N; i++) d.max_ent = std::max(d.max_ent, L.g_off[i + 1] - L.g_off[i]);
+    d.g_ent = nullptr;
+    d.g_ent_split = nullptr;
+    if (d.n_border > 0)
+        rc = upload(c, (int32_t **)&d.g_ent_split,
+                    entries_by_face<int32_t>(L, d.max_ent, -1, [](int32_t e) { return e; }));
+    else
+        rc = upload(c, (uint16_t **)&d.g_ent, entries_by_face<uint16_t>(L, d.max_ent, kNoEnt, [](int32_t e) {
+                        return (uint16_t)((e >> 2) << 1 | (e & 1));
+                    }));
+    if (rc) return fail(rc);
     std::vector<int32_t> bpatch = L.b_patch;
     if (bpatch.empty()) bpatch.push_back(0);
     std::vector<int32_t> bpartner = L.b_partner;
@@ -549,7 +575,6 @@ int create_ctx(const plbfs_mesh_view *mesh, const plbfs_params *params, const pl
         (rc = upload(c, (int32_t **)&d.blk_item_off, L.blk_item_off)) ||
         (rc = upload(c, (float4 **)&d.it_p, c->f32 ? pack_items<float>(L) : pack_items<double>(L))) ||
         (rc = upload(c, (uint16_t **)&d.it_side, std::vector<uint16_t>(L.it_side.begin(), L.it_side.end()))) ||
-        (rc = upload(c, (int32_t **)&d.g_off, L.g_off)) || (rc = upload(c, (int32_t **)&d.g_ent, L.g_ent)) ||
         (rc = upload(c, (int32_t **)&d.b_patch, bpatch)) || (rc = upload(c, (int32_t **)&d.b_partner, bpartner)) ||
         (rc = upload(c, (DevPatch **)&d.patches, dp)))
         return fail(rc);
@@ -570,9 +595,10 @@ int create_ctx(const plbfs_mesh_view *mesh, const plbfs_params *params, const pl
         e.block_cells = d.block_cells;
         e.stage = d.stage;
         e.grad_stage = d.grad_stage;
+        e.max_slots = d.max_slots;
         e.st_cnt = d.st_cnt; e.st_nbr = d.st_nbr; e.vol = d.vol; e.inv_vol = d.inv_vol; e.cfl_area = d.cfl_area;
-        e.blk_item_off = d.blk_item_off; e.it_p = d.it_p; e.it_side = d.it_side; e.it_dt = nullptr; e.g_off = d.g_off;
-        e.g_ent = d.g_ent; e.b_patch = d.b_patch; e.b_partner = d.b_partner;
+        e.blk_item_off = d.blk_item_off; e.it_p = d.it_p; e.it_side = d.it_side; e.it_dt = nullptr;
+        e.g_ent = d.g_ent; e.g_ent_split = d.g_ent_split; e.max_ent = d.max_ent; e.b_patch = d.b_patch; e.b_partner = d.b_partner;
         e.b_fix = (const float4 *)c->b_fix;
         auto to32 = [](const std::vector<double> &v) { return std::vector<float>(v.begin(), v.end()); };
         std::vector<DevPatch> dp32 = dp;
