@@ -19,7 +19,7 @@
 
 namespace plbfs {
 constexpr int kBlock = 256;
-// default cells per flux block (face slots of one block share its LDS)
+// cells per flux block of a large mesh (face slots of one block share its LDS)
 constexpr int kFluxBlockCells = 256;
 // Dynamic LDS per flux workgroup.  gfx950 gives a workgroup 160 KiB
 // (hipDeviceProp_t::sharedMemPerBlock), static and dynamic LDS together; the
@@ -81,6 +81,7 @@ struct plbfs_ctx {
     plbfs::Ctrl *ctrl = nullptr;
     size_t lds_bytes = 0;
     int cell_grid = 0;  // blocks of kBlock cells for the per-cell kernels
+    int bound_blocks = 0;  // flux blocks that the scratch bound of plbfs_run_noalloc counts
     int total_steps = 0;
     std::vector<double> last_hist;
     IbmState ibm;

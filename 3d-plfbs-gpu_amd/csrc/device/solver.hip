@@ -374,7 +374,11 @@ __global__ __launch_bounds__(kBlock) void k_residual_only(DevMesh<S> m, DevParam
 // kScratchBytes bounds what one call may use.  Calls that overlap on one
 // device share the array and race.
 constexpr size_t kScratchBytes = (size_t)8 << 20;
-static __device__ __align__(256) double scratch[kScratchBytes / sizeof(double)];
+// The bound counts kFluxBlockCells cells a block where the mesh size chose the block
+// size; the partials of the smaller blocks it may choose (at most 1,024 instead of
+// 256 blocks, 40 B each) fit behind it.
+constexpr size_t kScratchSpare = (size_t)32 << 10;
+static __device__ __align__(256) double scratch[(kScratchBytes + kScratchSpare) / sizeof(double)];
 
 constexpr int kMaxScratchDevices = 64;
 static std::mutex g_scratch_mu;
@@ -425,12 +429,23 @@ static bool env_flag(const char *name, bool def) {
     return v[0] != '0';
 }
 
+// Larger blocks duplicate fewer border faces; but a block takes its time whatever
+// the others do, some 10 us for 64 cells (one face item a thread), 20 for 256, so a
+// mesh of fewer 256-cell blocks than the 256 CUs is faster in smaller ones.  Step in
+// FP64, us, with 64 / 192 / 256 cells: 216 hexes 62 / 82 / 82, 16k 94 / 118 / 131, 32k
+// 101 / 116 / 120, 17k tets 73 / 80 / 88, 83k tets 171 / 163 / 175, 221k hexes 252 / 246
+// / 243, 384k tets 299 / 284 / 279.
+static int default_block_cells(int n_cells) {
+    if (n_cells < 256 * 256) return 64;
+    if (n_cells < 2 * 256 * 256) return 192;
+    return kFluxBlockCells;
+}
+
 extern "C" int plbfs_create(const plbfs_mesh_view *mesh, const plbfs_params *params, const plbfs_patch *patches,
                             int32_t n_patches, const int32_t *bface_patch, plbfs_ctx **out) {
-    // cells per flux block (a multiple of 64): larger blocks duplicate fewer
-    // border faces but need more LDS
-    int block_cells = kFluxBlockCells;
-    if (const char *bc = std::getenv("PLBFS_BLOCK_CELLS")) block_cells = std::atoi(bc);
+    // cells per flux block (a multiple of 64)
+    const char *bc = std::getenv("PLBFS_BLOCK_CELLS");
+    const int block_cells = bc ? std::atoi(bc) : default_block_cells(mesh ? mesh->n_cells : 0);
     if (block_cells < 64 || block_cells % 64 || block_cells > 4 * kBlock)
         return plbfs_fail(PLBFS_ERR_INPUT, "PLBFS_BLOCK_CELLS must be a multiple of 64 up to %d", 4 * kBlock);
     // measured on MI355X (4.09M tets): staging the flux block's own records in
@@ -444,7 +459,9 @@ extern "C" int plbfs_create(const plbfs_mesh_view *mesh, const plbfs_params *par
     // slower (FP64 0.555 -> 0.617 ms, FP32 0.331 -> 0.364 ms; its faces
     // gather both sides from global memory), so duplication is the default
     const bool split = env_flag("PLBFS_SPLIT_BORDER", false);
-    return create_ctx(mesh, params, patches, n_patches, bface_patch, block_cells, 1, flux_stage, split, out);
+    const int rc = create_ctx(mesh, params, patches, n_patches, bface_patch, block_cells, 1, flux_stage, split, out);
+    if (rc == PLBFS_OK && !bc) (*out)->bound_blocks = (mesh->n_cells + kFluxBlockCells - 1) / kFluxBlockCells;
+    return rc;
 }
 
 // Fixed ghost states to the device: (rho, u, v, w) per boundary face in the
@@ -510,6 +527,7 @@ int create_ctx(const plbfs_mesh_view *mesh, const plbfs_params *params, const pl
     if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess)
         return fail(plbfs_fail(PLBFS_ERR_HIP, "hipStreamCreate"));
     const int N = L.N;
+    c->bound_blocks = L.n_blocks;
     DevMesh<double> &d = c->dm;
     d.N = N;
     d.G = L.G;
@@ -955,9 +973,9 @@ extern "C" int plbfs_run(plbfs_ctx *c, int32_t max_steps, plbfs_result *out) {
 
 static size_t round256(size_t b) { return (b + 255) / 256 * 256; }
 
-// Bytes of scratch a run of max_steps steps needs on context c.
+// Bytes of scratch a run of max_steps steps needs on context c, as the bound counts them.
 static size_t scratch_need(const plbfs_ctx *c, int64_t max_steps) {
-    return round256(sizeof(Ctrl)) + round256((size_t)c->L.n_blocks * 5 * sizeof(double)) +
+    return round256(sizeof(Ctrl)) + round256((size_t)c->bound_blocks * 5 * sizeof(double)) +
            round256((size_t)c->cell_grid * sizeof(double)) + (size_t)max_steps * 4 * sizeof(double);
 }
 

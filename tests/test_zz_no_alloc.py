@@ -100,3 +100,31 @@ def test_noalloc_run_refuses_more_than_its_scratch(gpu_available):
     assert e.value.rc == -1 and "scratch" in str(e.value)
     for q, x in enumerate(a.state()):
         assert np.array_equal(x, before[q]), q
+
+
+@pytest.mark.parametrize("block_cells", ["", "64", "256"])
+def test_noalloc_bound_counts_256_cells_a_block(gpu_available, monkeypatch, block_cells):
+    """The longest run that fits and the next one: the bound counts the control
+    block, 40 B a flux block (of 256 cells unless the block size is given) and 8 B a
+    256 cells, each rounded up to 256 B, and 32 B a step."""
+    if block_cells:
+        monkeypatch.setenv("PLBFS_BLOCK_CELLS", block_cells)
+    pm = channel_mesh(20, 10, 10)
+    case = pc.channel_case(re=40.0, length_scale=5.0)
+    case.tolerance = 1e30  # stops after the first step
+    case.check_interval = 1
+    hm = HostMesh.from_polymesh(pm, case.visc, case.gamma, case.fneq_min)
+    a = GpuSolver(hm, case.params, case.patches_for(pm.patch_names))
+    g = hm.geometry()
+    a.set_state(*case.initial_state(g["cx"], g["cy"], g["cz"]))
+
+    def up(b):
+        return (b + 255) // 256 * 256
+
+    n = pm.n_cells
+    blocks = -(-n // int(block_cells or 256))
+    most = ((8 << 20) - 256 - up(40 * blocks) - up(8 * -(-n // 256))) // 32
+    assert a.run_noalloc(most)["steps"] == 1
+    with pytest.raises(nat.PlbfsError):
+        a.run_noalloc(most + 1)
+    a.close()
