@@ -323,9 +323,8 @@ struct plbfs_batch {
     IbmArgs ia{};
     std::vector<void *> ibm_allocs;
     uint8_t *force_rec = nullptr;  // in ibm_allocs
-    // graph of one step
-    hipGraphExec_t graph = nullptr;
-    bool graph_ok = false;
+    // graphs of one step and of kGraphSteps steps
+    hipGraphExec_t graph = nullptr, graph_many = nullptr;
 };
 
 namespace {
@@ -356,9 +355,10 @@ void free_list(std::vector<void *> &list) {
 }
 
 void drop_graph(plbfs_batch *b) {
-    if (b->graph) (void)hipGraphExecDestroy(b->graph);
-    b->graph = nullptr;
-    b->graph_ok = false;
+    for (hipGraphExec_t *g : {&b->graph, &b->graph_many}) {
+        if (*g) (void)hipGraphExecDestroy(*g);
+        *g = nullptr;
+    }
 }
 
 plbfs_mesh_view view_of(plbfs_batch *b) {
@@ -587,19 +587,23 @@ int launch_batch_step(plbfs_batch *b) {
     return PLBFS_OK;
 }
 
-int build_batch_graph(plbfs_batch *b) {
-    if (b->graph_ok) return PLBFS_OK;
-    hipStream_t s = b->base->stream;
+// Captures `steps` steps into *exec unless that is done already.
+int build_batch_graph(plbfs_batch *b, int steps, hipGraphExec_t *exec) {
+    if (*exec) return PLBFS_OK;
+    hipStream_t st = b->base->stream;
     hipGraph_t g;
-    HIP_TRY(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-    int rc = launch_batch_step(b);
-    hipError_t e = hipStreamEndCapture(s, &g);
+    HIP_TRY(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
+    int rc = PLBFS_OK;
+    for (int s = 0; s < steps && rc == PLBFS_OK; s++) rc = launch_batch_step(b);
+    hipError_t e = hipStreamEndCapture(st, &g);
     if (rc) return rc;
     if (e != hipSuccess) return plbfs_fail(PLBFS_ERR_HIP, "graph capture: %s", hipGetErrorString(e));
-    e = hipGraphInstantiate(&b->graph, g, nullptr, nullptr, 0);
+    e = hipGraphInstantiate(exec, g, nullptr, nullptr, 0);
     hipGraphDestroy(g);
-    if (e != hipSuccess) return plbfs_fail(PLBFS_ERR_HIP, "graph instantiate: %s", hipGetErrorString(e));
-    b->graph_ok = true;
+    if (e != hipSuccess) {
+        *exec = nullptr;
+        return plbfs_fail(PLBFS_ERR_HIP, "graph instantiate: %s", hipGetErrorString(e));
+    }
     return PLBFS_OK;
 }
 
@@ -633,15 +637,20 @@ int run_steps(plbfs_batch *b, int max_steps, float *ms_out) {
         hipLaunchKernelGGL(kb_init_dt<double>, rgrid, dim3(kBlock), 0, c->stream, c->dm, c->prm, args_of(b),
                            (const double4 *)b->stA, b->dtl);
     HIP_TRY(hipGetLastError());
-    if ((rc = build_batch_graph(b))) return rc;
     const int interval = std::max(1, b->params.check_interval);
     hipEvent_t e0, e1;
     HIP_TRY(hipEventCreate(&e0));
     HIP_TRY(hipEventCreate(&e1));
     HIP_TRY(hipEventRecord(e0, c->stream));
-    for (int s = 0; s < max_steps; s++) {
-        HIP_TRY(hipGraphLaunch(b->graph, c->stream));
-        if ((s + 1) % interval == 0 || s == max_steps - 1) {
+    for (int s = 0; s < max_steps;) {
+        const int left = std::min(interval - s % interval, max_steps - s);  // steps to the next check
+        const bool many = left >= kGraphSteps;
+        const int n = many ? kGraphSteps : 1;
+        hipGraphExec_t &g = many ? b->graph_many : b->graph;
+        if ((rc = build_batch_graph(b, n, &g))) return rc;
+        HIP_TRY(hipGraphLaunch(g, c->stream));
+        s += n;
+        if (n == left) {
             HIP_TRY(hipMemcpyAsync(&h, b->ctrl, sizeof(Ctrl), hipMemcpyDeviceToHost, c->stream));
             HIP_TRY(hipStreamSynchronize(c->stream));
             if (h.done) break;

@@ -19,6 +19,11 @@
 
 namespace plbfs {
 constexpr int kBlock = 256;
+// Time steps of the longer captured graph.  The first kernel of a graph starts 8.5 us
+// after the last one of the graph before, about a kernel inside one right away:
+// 216 hexes 56.7 -> 53.0 us a step with 4 steps a graph, 52.4 with 16, whose
+// capture costs a context's first run 0.3 ms instead of nothing measurable.
+constexpr int kGraphSteps = 4;
 // cells per flux block of a large mesh (face slots of one block share its LDS)
 constexpr int kFluxBlockCells = 256;
 // Dynamic LDS per flux workgroup.  gfx950 gives a workgroup 160 KiB
@@ -93,9 +98,8 @@ struct plbfs_ctx {
         hipEvent_t a, b;
     };
     std::vector<EvPair> pending;
-    // graph of one step
-    hipGraphExec_t graph_exec = nullptr;
-    bool graph_ok = false;
+    // graphs of one step and of kGraphSteps steps
+    hipGraphExec_t graph_exec = nullptr, graph_many = nullptr;
     bool use_graph = true;
     // this device's copy of the file-scope scratch array of solver.hip
     // (plbfs_run_noalloc), resolved once per device at creation
@@ -145,6 +149,9 @@ struct TimedLaunch {
         }
     }
 };
+
+// Drops the captured steps (their kernels' arguments are about to change).
+void drop_graphs(plbfs_ctx *c);
 
 // plbfs_create with an explicit flux block size (64..1024 cells, a multiple of
 // 64), LDS sized for lds_cases cases per block (the batched solver sizes its

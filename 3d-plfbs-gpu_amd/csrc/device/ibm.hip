@@ -180,11 +180,7 @@ static int set_ibm(plbfs_ctx *c, const plbfs_ibm_nodes *nodes, int rebuilds) {
     // work can read them (the captured step graph that references them is
     // dropped below)
     HIP_TRY(hipStreamSynchronize(c->stream));
-    if (c->graph_exec) {
-        (void)hipGraphExecDestroy(c->graph_exec);
-        c->graph_exec = nullptr;
-    }
-    c->graph_ok = false;
+    drop_graphs(c);
     for (void *p : c->ibm_allocs) (void)hipFree(p);
     c->ibm_allocs.clear();
     c->dm.blk_force = nullptr;
@@ -236,11 +232,7 @@ static int set_ibm(plbfs_ctx *c, const plbfs_ibm_nodes *nodes, int rebuilds) {
     HIP_TRY(hipMemset(c->fbody, 0, (size_t)3 * N * sizeof(double)));
     s.on = true;
     c->prm.use_body_force = 1;
-    if (c->graph_exec) {
-        (void)hipGraphExecDestroy(c->graph_exec);
-        c->graph_exec = nullptr;
-    }
-    c->graph_ok = false;
+    drop_graphs(c);
     return PLBFS_OK;
 }
 

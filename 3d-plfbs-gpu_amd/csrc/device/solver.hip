@@ -401,11 +401,15 @@ static int resolve_scratch(int device, char **out) {
     return PLBFS_OK;
 }
 
-static int release(plbfs_ctx *c) {
-    if (c->graph_exec) {
-        hipGraphExecDestroy(c->graph_exec);
-        c->graph_exec = nullptr;
+void drop_graphs(plbfs_ctx *c) {
+    for (hipGraphExec_t *g : {&c->graph_exec, &c->graph_many}) {
+        if (*g) (void)hipGraphExecDestroy(*g);
+        *g = nullptr;
     }
+}
+
+static int release(plbfs_ctx *c) {
+    drop_graphs(c);
     for (void *p : c->allocs) hipFree(p);
     c->allocs.clear();
     for (void *p : c->ibm_allocs) hipFree(p);
@@ -878,11 +882,7 @@ static int launch_step(plbfs_ctx *c, const RunScratch &w, bool timed, bool rebui
 
 static int ensure_hist(plbfs_ctx *c, int steps) {
     if (steps <= c->hist_cap) return PLBFS_OK;
-    if (c->graph_exec) {
-        hipGraphExecDestroy(c->graph_exec);
-        c->graph_exec = nullptr;
-        c->graph_ok = false;
-    }
+    drop_graphs(c);
     int cap = std::max(steps, 1024);
     int rc = dalloc(c, (void **)&c->hist, (size_t)cap * 4 * sizeof(double));
     if (rc) return rc;
@@ -890,18 +890,22 @@ static int ensure_hist(plbfs_ctx *c, int steps) {
     return PLBFS_OK;
 }
 
-static int build_graph(plbfs_ctx *c) {
-    if (c->graph_ok || !c->use_graph || c->timing) return PLBFS_OK;
+// Captures `steps` time steps into *exec unless that is done already.
+static int build_graph(plbfs_ctx *c, int steps, hipGraphExec_t *exec) {
+    if (*exec) return PLBFS_OK;
     hipGraph_t g;
     HIP_TRY(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-    int rc = launch_step(c, ctx_scratch(c), false, true);
+    int rc = PLBFS_OK;
+    for (int s = 0; s < steps && rc == PLBFS_OK; s++) rc = launch_step(c, ctx_scratch(c), false, true);
     hipError_t e = hipStreamEndCapture(c->stream, &g);
     if (rc) return rc;
     if (e != hipSuccess) return plbfs_fail(PLBFS_ERR_HIP, "graph capture: %s", hipGetErrorString(e));
-    e = hipGraphInstantiate(&c->graph_exec, g, nullptr, nullptr, 0);
+    e = hipGraphInstantiate(exec, g, nullptr, nullptr, 0);
     hipGraphDestroy(g);
-    if (e != hipSuccess) return plbfs_fail(PLBFS_ERR_HIP, "graph instantiate: %s", hipGetErrorString(e));
-    c->graph_ok = true;
+    if (e != hipSuccess) {
+        *exec = nullptr;
+        return plbfs_fail(PLBFS_ERR_HIP, "graph instantiate: %s", hipGetErrorString(e));
+    }
     return PLBFS_OK;
 }
 
@@ -921,35 +925,42 @@ extern "C" int plbfs_run(plbfs_ctx *c, int32_t max_steps, plbfs_result *out) {
     int rc = check_ghost_state(c);
     if (rc) return rc;
     if ((rc = ensure_hist(c, max_steps))) return rc;
-    if (rc) return rc;
     Ctrl h{};
     HIP_TRY(hipMemcpyAsync(c->ctrl, &h, sizeof(Ctrl), hipMemcpyHostToDevice, c->stream));
     const RunScratch w = ctx_scratch(c);
     if ((rc = launch_run_start(c, w))) return rc;
-    if ((rc = build_graph(c))) return rc;
     const int interval = std::max(1, c->params.check_interval);
+    const bool graph = c->use_graph && !c->timing;
     hipEvent_t ev0, ev1;
     HIP_TRY(hipEventCreate(&ev0));
     HIP_TRY(hipEventCreate(&ev1));
     HIP_TRY(hipEventRecord(ev0, c->stream));
-    for (int s = 0; s < max_steps; s++) {
-        if (c->graph_ok && !c->timing) {
+    for (int s = 0; s < max_steps;) {
+        const int left = std::min(interval - s % interval, max_steps - s);  // steps to the next check
+        int n = 1;
+        if (graph && left >= kGraphSteps) {
+            n = kGraphSteps;
+            if ((rc = build_graph(c, n, &c->graph_many))) return rc;
+            HIP_TRY(hipGraphLaunch(c->graph_many, c->stream));
+        } else if (graph) {
+            if ((rc = build_graph(c, 1, &c->graph_exec))) return rc;
             HIP_TRY(hipGraphLaunch(c->graph_exec, c->stream));
         } else if ((rc = launch_step(c, w, c->timing, true))) {
             return rc;
         }
-        if ((s + 1) % interval == 0 || s == max_steps - 1) {
+        s += n;
+        if (n == left) {
             HIP_TRY(hipMemcpyAsync(&h, c->ctrl, sizeof(Ctrl), hipMemcpyDeviceToHost, c->stream));
             HIP_TRY(hipStreamSynchronize(c->stream));
             if (h.done && h.rebuild && h.status == PLBFS_OK && !h.converged) {
                 // new candidate lists around the nodes' positions after step
                 // h.step, then on from there: the launches after the stop were
                 // no-ops, so the loop resumes at the step count
-                if ((rc = ibm_rebuild(c)) || (rc = ensure_hist(c, max_steps)) || (rc = build_graph(c))) return rc;
+                if ((rc = ibm_rebuild(c)) || (rc = ensure_hist(c, max_steps))) return rc;
                 h.done = 0;
                 h.rebuild = 0;
                 HIP_TRY(hipMemcpyAsync(c->ctrl, &h, sizeof(Ctrl), hipMemcpyHostToDevice, c->stream));
-                s = h.step - 1;
+                s = h.step;
                 continue;
             }
             if (h.done) break;

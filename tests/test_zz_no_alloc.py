@@ -128,3 +128,24 @@ def test_noalloc_bound_counts_256_cells_a_block(gpu_available, monkeypatch, bloc
     with pytest.raises(nat.PlbfsError):
         a.run_noalloc(most + 1)
     a.close()
+
+
+@pytest.mark.parametrize("steps,interval", [(1, 10), (3, 10), (4, 10), (5, 10), (7, 4), (9, 5), (12, 3), (13, 6)])
+def test_step_graphs_match_direct_launches(gpu_available, steps, interval):
+    """plbfs_run replays graphs of four steps and of one between its checks,
+    plbfs_run_noalloc launches each kernel: the same steps and bits whatever is left
+    between two checks, also when called again."""
+    pm = channel_mesh(10, 6, 6)
+    case = pc.channel_case(re=40.0, length_scale=5.0)
+    case.check_interval = interval
+    hm = HostMesh.from_polymesh(pm, case.visc, case.gamma, case.fneq_min)
+    st = perturbed_state(case, oracle_for(pm, case), amp=0.01, seed=3)
+    a, b = (GpuSolver(hm, case.params, case.patches_for(pm.patch_names)) for _ in range(2))
+    for s in (a, b):
+        s.set_state(*st)
+    for _ in range(2):
+        ra, rb = a.run(steps), b.run_noalloc(steps)
+        assert ra["steps"] == rb["steps"] == steps
+        assert np.array_equal(ra["hist"], rb["hist"])
+        for x, y in zip(a.state(), b.state()):
+            assert np.array_equal(x, y)
