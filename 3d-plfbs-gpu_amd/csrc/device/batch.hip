@@ -320,6 +320,7 @@ struct plbfs_batch {
     bool ibm_dirty = false, ibm_on = false;
     int ibm_kernel = 0;
     double ibm_h = 1, ibm_dt = 0, ibm_margin = 0;
+    bool ibm_wide = false;
     IbmArgs ia{};
     std::vector<void *> ibm_allocs;
     uint8_t *force_rec = nullptr;  // in ibm_allocs
@@ -488,19 +489,23 @@ int ibm_upload(plbfs_batch *b) {
     a.k_dA = 0;
     a.margin = b->ibm_margin;
     a.n_affected = (int)cp_cell.size();
-    std::vector<double> z((size_t)3 * n_total, 0.0), zn(n_total, 0.0);
+    std::vector<double> z((size_t)3 * n_total, 0.0);
+    std::vector<int2> pairs;
+    std::vector<double4> geo;
+    ibm_arrays(b->base->L, cp_node, cp_pair, pairs, geo, b->ibm_kernel, b->ibm_h, b->ibm_wide);
     int rc;
-    int32_t *nc = nullptr, *npo = nullptr, *npc = nullptr, *cpc = nullptr, *cpk = nullptr, *cpo = nullptr,
-            *cpn = nullptr, *cpp = nullptr;
-    double *kd = nullptr, *ccd = nullptr, *pw = nullptr;
+    int32_t *nc = nullptr, *npo = nullptr, *npc = nullptr, *cpc = nullptr, *cpk = nullptr, *cpo = nullptr;
+    int2 *cpp = nullptr;
+    double4 *gd = nullptr;
+    double *kd = nullptr, *pw = nullptr;
     double *xcd = nullptr;  // the lists were built around the positions given to set_ibm
     if ((rc = bupload(M, &a.xref, xr)) || (rc = bupload(M, &a.x, xx)) || (rc = bupload(M, &a.x0, xx)) ||
         (rc = bupload(M, &xcd, xx)) ||
-        (rc = bupload(M, &a.vel, z)) || (rc = bupload(M, &a.force, z)) || (rc = bupload(M, &a.norm, zn)) ||
+        (rc = bupload(M, &a.vel, z)) || (rc = bupload(M, &a.force, z)) ||
+        (rc = balloc(M, (void **)&a.fn, (size_t)n_total * sizeof(double4))) ||
         (rc = bupload(M, &kd, kda)) || (rc = bupload(M, &nc, ncase)) || (rc = bupload(M, &npo, np_off)) ||
         (rc = bupload(M, &npc, np_cell)) || (rc = bupload(M, &cpc, cp_cell)) || (rc = bupload(M, &cpk, cp_case)) ||
-        (rc = bupload(M, &cpo, cp_off)) || (rc = bupload(M, &cpn, cp_node)) || (rc = bupload(M, &cpp, cp_pair)) ||
-        (rc = bupload(M, &ccd, b->base->L.centroid)) ||
+        (rc = bupload(M, &cpo, cp_off)) || (rc = bupload(M, &cpp, pairs)) || (rc = bupload(M, &gd, geo)) ||
         (rc = balloc(M, (void **)&pw, np_cell.size() * sizeof(double))))
         return rc;
     a.xc = xcd;
@@ -512,11 +517,9 @@ int ibm_upload(plbfs_batch *b) {
     a.cp_cell = cpc;
     a.cp_case = cpk;
     a.cp_off = cpo;
-    a.cp_node = cpn;
     a.cp_pair = cpp;
     a.pw = pw;
-    a.cc = ccd;
-    a.vol = b->base->dm.vol;
+    a.geo = gd;
     a.case_done = b->done;
     a.case_status = b->status;
     {
@@ -526,7 +529,7 @@ int ibm_upload(plbfs_batch *b) {
         if ((rc = bupload(M, &b->force_rec, fr))) return rc;
     }
     HIP_TRY(hipMemset(b->fbody, 0, (size_t)3 * b->N * b->B * sizeof(double)));
-    hipLaunchKernelGGL(k_ibm_weights, dim3((n_total + kNodesPerBlock - 1) / kNodesPerBlock), dim3(kIbmThreads), 0,
+    hipLaunchKernelGGL(k_ibm_weights, dim3((n_total + kIbmWide - 1) / kIbmWide), dim3(kIbmThreads), 0,
                        b->base->stream, a);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(b->base->stream));
@@ -567,13 +570,8 @@ void launch_batch_stages(plbfs_batch *b, const DevMesh<S> &dm_base) {
 int launch_batch_step(plbfs_batch *b) {
     plbfs_ctx *c = b->base;
     if (b->ibm_on) {
-        const dim3 grid((b->ia.n + kNodesPerBlock - 1) / kNodesPerBlock);
-        if (b->f32)
-            hipLaunchKernelGGL(k_ibm_nodes<float4>, grid, dim3(kIbmThreads), 0, c->stream, b->ia, b->ctrl,
-                               (const float4 *)b->stA);
-        else
-            hipLaunchKernelGGL(k_ibm_nodes<double4>, grid, dim3(kIbmThreads), 0, c->stream, b->ia, b->ctrl,
-                               (const double4 *)b->stA);
+        if (b->f32) launch_ibm_nodes(b->ia, b->ibm_wide, c->stream, b->ctrl, (const float4 *)b->stA);
+        else launch_ibm_nodes(b->ia, b->ibm_wide, c->stream, b->ctrl, (const double4 *)b->stA);
         hipLaunchKernelGGL(k_ibm_spread, dim3((b->ia.n_affected + kSpreadPerBlock - 1) / kSpreadPerBlock),
                            dim3(kIbmThreads), 0, c->stream, b->ia, b->ctrl, b->fbody);
     }

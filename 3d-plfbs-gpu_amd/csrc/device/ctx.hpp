@@ -44,18 +44,20 @@ struct IbmState {
     int n = 0;
     int kernel = 0;
     double h = 1, dt = 0, stiffness = 0, node_area = 0, margin = 0;
-    double *x = nullptr, *x0 = nullptr, *xref = nullptr, *vel = nullptr, *force = nullptr, *norm = nullptr;
+    double *x = nullptr, *x0 = nullptr, *xref = nullptr, *vel = nullptr, *force = nullptr;
+    double4 *fn = nullptr;           // per node force and spreading normaliser
     double *xc = nullptr;            // [3][n] positions the candidate lists were built around
     std::vector<double> xref_host;   // [3n] interleaved anchors, kept for list rebuilds
     int rebuilds = 0;                // list rebuilds since plbfs_set_ibm
     int32_t *np_off = nullptr, *np_cell = nullptr;           // node -> candidate cells
-    int32_t *cp_cell = nullptr, *cp_off = nullptr, *cp_node = nullptr;  // affected cell -> nodes
-    int32_t *cp_pair = nullptr;  // node-major pair index of each cell-major entry
+    int32_t *cp_cell = nullptr, *cp_off = nullptr;  // affected cell -> nodes
+    int2 *cp_pair = nullptr;     // (node, node-major pair index) of each cell-major entry
     int32_t *blk_force = nullptr;  // [n_blocks] 1 where a flux block holds an affected cell
     double *pw = nullptr;        // [n_pairs] kernel weights at the current node positions
     int n_affected = 0;
     int64_t n_pairs = 0;
-    double *cell_c = nullptr;  // [3][N] centroids, Hilbert order
+    double4 *geo = nullptr;      // [N] centroid and volume, Hilbert order
+    bool wide = false;           // four wavefronts per node (ibm_wide)
 };
 
 struct plbfs_ctx {
@@ -178,3 +180,6 @@ struct IbmPairs {
     std::vector<int32_t> cp_pair;                   // ... and their node-major pair index
 };
 int build_ibm_pairs(const plbfs::Layout &L, const plbfs_ibm_nodes *nodes, IbmPairs &P);
+// The kernels' records: pairs by cell, cell centroids and volumes, wavefronts per node.
+void ibm_arrays(const plbfs::Layout &L, const std::vector<int32_t> &cp_node, const std::vector<int32_t> &cp_pair,
+                std::vector<int2> &pairs, std::vector<double4> &geo, int kernel, double h, bool &wide);

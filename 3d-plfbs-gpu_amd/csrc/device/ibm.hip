@@ -9,9 +9,9 @@
 // uses a 2-point hat; here every node has a precomputed list of candidate
 // cells (centroids within the kernel support plus a drift margin of the
 // anchor), sorted by cell, so that
-//   interpolation  = one 64-wide wavefront per node, lanes stride over the
+//   interpolation  = one or four wavefronts per node, lanes stride over the
 //                    node's pairs, shuffle butterfly reduction (fixed order);
-//   spreading      = one thread per affected cell summing over its pairs in
+//   spreading      = 16 lanes per affected cell summing over its pairs in
 //                    node order (pairs regrouped by cell on the host).
 // Weights are normalised per node, W_cn = delta V_c / sum delta V, which is
 // the reference's formula on its uniform unit grid.  No atomics.
@@ -52,17 +52,15 @@ IbmArgs make_args(plbfs_ctx *c, bool rebuild = false) {
     a.xref = s.xref;
     a.vel = s.vel;
     a.force = s.force;
-    a.norm = s.norm;
+    a.fn = s.fn;
     a.np_off = s.np_off;
     a.np_cell = s.np_cell;
     a.cp_cell = s.cp_cell;
     a.cp_off = s.cp_off;
-    a.cp_node = s.cp_node;
     a.cp_pair = s.cp_pair;
     a.pw = s.pw;
     a.n_affected = s.n_affected;
-    a.cc = s.cell_c;
-    a.vol = c->dm.vol;
+    a.geo = s.geo;
     return a;
 }
 
@@ -72,14 +70,10 @@ int ibm_launch(plbfs_ctx *c, Ctrl *ctrl, bool timed, bool rebuild) {
     if (!c->ibm.on) return PLBFS_OK;
     const IbmArgs a = make_args(c, rebuild);
     TimedLaunch t(c, PLBFS_KSTAT_IBM, timed);
-    const dim3 grid((a.n + kNodesPerBlock - 1) / kNodesPerBlock);
-    if (c->f32)
-        hipLaunchKernelGGL(k_ibm_nodes<float4>, grid, dim3(kIbmThreads), 0, c->stream, a, ctrl, (const float4 *)c->stA);
-    else
-        hipLaunchKernelGGL(k_ibm_nodes<double4>, grid, dim3(kIbmThreads), 0, c->stream, a, ctrl,
-                           (const double4 *)c->stA);
-    hipLaunchKernelGGL(k_ibm_spread, dim3((a.n_affected + kSpreadPerBlock - 1) / kSpreadPerBlock), dim3(kIbmThreads), 0, c->stream, a,
-                       ctrl, c->fbody);
+    if (c->f32) launch_ibm_nodes(a, c->ibm.wide, c->stream, ctrl, (const float4 *)c->stA);
+    else launch_ibm_nodes(a, c->ibm.wide, c->stream, ctrl, (const double4 *)c->stA);
+    hipLaunchKernelGGL(k_ibm_spread, dim3((a.n_affected + kSpreadPerBlock - 1) / kSpreadPerBlock), dim3(kIbmThreads),
+                       0, c->stream, a, ctrl, c->fbody);
     HIP_TRY(hipGetLastError());
     return PLBFS_OK;
 }
@@ -166,6 +160,20 @@ int build_ibm_pairs(const plbfs::Layout &L, const plbfs_ibm_nodes *nodes, IbmPai
     return PLBFS_OK;
 }
 
+void ibm_arrays(const plbfs::Layout &L, const std::vector<int32_t> &cp_node, const std::vector<int32_t> &cp_pair,
+                std::vector<int2> &pairs, std::vector<double4> &geo, int kernel, double h, bool &wide) {
+    pairs.resize(cp_node.size());
+    for (size_t p = 0; p < pairs.size(); p++) pairs[p] = int2{cp_node[p], cp_pair[p]};
+    const size_t N = (size_t)L.N;
+    geo.resize(N);
+    double volume = 0;
+    for (size_t i = 0; i < N; i++) {
+        geo[i] = double4{L.centroid[i], L.centroid[N + i], L.centroid[2 * N + i], L.vol[i]};
+        volume += L.vol[i];
+    }
+    wide = ibm_wide(kernel, h, L.N, volume);
+}
+
 static int set_ibm(plbfs_ctx *c, const plbfs_ibm_nodes *nodes, int rebuilds) {
     IbmPairs P;
     int rc = build_ibm_pairs(c->L, nodes, P);
@@ -174,8 +182,7 @@ static int set_ibm(plbfs_ctx *c, const plbfs_ibm_nodes *nodes, int rebuilds) {
     const int N = c->L.N;
     const double h = nodes->h;
     const double margin = P.margin;
-    const std::vector<int32_t> &np_off = P.np_off, &np_cell = P.np_cell, &cp_cell = P.cp_cell, &cp_off = P.cp_off,
-                               &cp_node = P.cp_node;
+    const std::vector<int32_t> &np_off = P.np_off, &np_cell = P.np_cell, &cp_cell = P.cp_cell, &cp_off = P.cp_off;
     // device arrays; the previous node set's arrays are freed once no queued
     // work can read them (the captured step graph that references them is
     // dropped below)
@@ -200,7 +207,10 @@ static int set_ibm(plbfs_ctx *c, const plbfs_ibm_nodes *nodes, int rebuilds) {
     s.n_pairs = (int64_t)np_cell.size();
     s.xref_host.assign(nodes->x_ref, nodes->x_ref + 3 * (size_t)n);
     s.rebuilds = rebuilds;
-    std::vector<double> xr((size_t)3 * n), xx((size_t)3 * n), z((size_t)3 * n, 0.0), zn(n, 0.0);
+    std::vector<double> xr((size_t)3 * n), xx((size_t)3 * n), z((size_t)3 * n, 0.0);
+    std::vector<int2> pairs;
+    std::vector<double4> geo;
+    ibm_arrays(c->L, P.cp_node, P.cp_pair, pairs, geo, s.kernel, h, s.wide);
     for (int k = 0; k < n; k++)
         for (int q = 0; q < 3; q++) {
             xr[(size_t)q * n + k] = nodes->x_ref[3 * k + q];
@@ -208,11 +218,11 @@ static int set_ibm(plbfs_ctx *c, const plbfs_ibm_nodes *nodes, int rebuilds) {
         }
     if ((rc = upload(M, &s.xref, xr)) || (rc = upload(M, &s.x, xx)) || (rc = upload(M, &s.x0, xx)) ||
         (rc = upload(M, &s.xc, xx)) ||
-        (rc = upload(M, &s.vel, z)) || (rc = upload(M, &s.force, z)) || (rc = upload(M, &s.norm, zn)) ||
+        (rc = upload(M, &s.vel, z)) || (rc = upload(M, &s.force, z)) || (rc = dalloc(M, (void **)&s.fn, (size_t)n * sizeof(double4))) ||
         (rc = upload(M, &s.np_off, np_off)) || (rc = upload(M, &s.np_cell, np_cell)) ||
         (rc = upload(M, &s.cp_cell, cp_cell)) || (rc = upload(M, &s.cp_off, cp_off)) ||
-        (rc = upload(M, &s.cp_node, cp_node)) || (rc = upload(M, &s.cp_pair, P.cp_pair)) ||
-        (rc = upload(M, &s.cell_c, c->L.centroid)) || (rc = dalloc(M, (void **)&s.pw, np_cell.size() * sizeof(double))))
+        (rc = upload(M, &s.cp_pair, pairs)) || (rc = upload(M, &s.geo, geo)) ||
+        (rc = dalloc(M, (void **)&s.pw, np_cell.size() * sizeof(double))))
         return rc;
     {
         // flux blocks that hold an affected cell: only these read the body force
@@ -224,8 +234,8 @@ static int set_ibm(plbfs_ctx *c, const plbfs_ibm_nodes *nodes, int rebuilds) {
     }
     {
         const IbmArgs a = make_args(c);
-        hipLaunchKernelGGL(k_ibm_weights, dim3((n + kNodesPerBlock - 1) / kNodesPerBlock), dim3(kIbmThreads), 0,
-                           c->stream, a);
+        hipLaunchKernelGGL(k_ibm_weights, dim3((n + kIbmWide - 1) / kIbmWide), dim3(kIbmThreads), 0, c->stream,
+                           a);
         HIP_TRY(hipGetLastError());
         HIP_TRY(hipStreamSynchronize(c->stream));
     }

@@ -269,3 +269,31 @@ def test_node_outside_its_support_stops_only_its_case(gpu_available):
     for q in range(4):
         assert np.array_equal(bt.state(0)[q], s0[q]), q
         assert np.array_equal(bt.state(2)[q], s2[q]), q
+
+
+@pytest.mark.parametrize("h,kernel", [(1.0, 1), (2.0, 0), (0.8, 0)])
+@pytest.mark.parametrize("precision", [0, 1])
+def test_batch_immersed_nodes_on_fine_cells_equal_single_runs(gpu_available, precision, h, kernel):
+    """Tets smaller than the kernel width: nodes of over 512 candidate cells take four
+    wavefronts each (the first two), fewer take one, and either way in a batch as
+    in its cases' single runs, bit for bit."""
+    pm = channel_mesh(10, 8, 8, tets=True)
+    cases = cases_for([30.0, 60.0], precision, fneq_min=0.55)
+    for c in cases:
+        c.lsq_exact_det = 1
+    st = perturbed_state(cases[0], oracle_for(pm, cases[0]), amp=0.01, seed=5)
+    hm, bt = make_batch(pm, cases)
+    bt.set_tiling(64, 2)
+    bt.set_state(-1, *st)
+    ibm = []
+    for b, c in enumerate(cases):
+        X, dA = objects.fibonacci_sphere(30 + 7 * b, (4.0 + 0.3 * b, 4.0, 4.0), 1.2)
+        ibm.append(dict(x_ref=X, x=X, stiffness=0.5, node_area=dA, dt=c.time_marching_step, h=h, kernel=kernel))
+        bt.set_ibm(b, **ibm[b])
+    rc, res = bt.run(10)
+    assert rc == 0, res
+    for b, c in enumerate(cases):
+        r1, s1 = single_run(pm, c, st, 10, ibm[b])
+        assert r1["rc"] == 0
+        for x, y in zip(bt.state(b), s1):
+            assert np.array_equal(x, y)
