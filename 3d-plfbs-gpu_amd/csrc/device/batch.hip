@@ -273,11 +273,19 @@ __global__ __launch_bounds__(kBlock) void kb_scatter(int N, int B, int b, double
     st[idx] = V4<S>{(S)(q.x - rho0), (S)q.y, (S)q.z, (S)q.w};
 }
 
-__global__ __launch_bounds__(kBlock) void kb_gather(int N, int B, int b, const double4 *__restrict__ src,
-                                                    double4 *__restrict__ dst) {
+// Case b's conservatives (primitives before its first step) to [4][N] primitives in
+// file order.
+__global__ __launch_bounds__(kBlock) void kb_export(int N, int B, int b, const int32_t *__restrict__ inv,
+                                                    const int32_t *__restrict__ steps,
+                                                    const double4 *__restrict__ src, double *__restrict__ out) {
     const int i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= N) return;
-    dst[i] = src[(size_t)i * B + b];
+    const double4 q = src[(size_t)inv[i] * B + b];
+    const bool divide = steps[b] > 0;
+    out[i] = q.x;
+    out[(size_t)N + i] = divide ? q.y / q.x : q.y;
+    out[2 * (size_t)N + i] = divide ? q.z / q.x : q.z;
+    out[3 * (size_t)N + i] = divide ? q.w / q.x : q.w;
 }
 
 }  // namespace
@@ -366,6 +374,9 @@ plbfs_mesh_view view_of(plbfs_batch *b) {
     return plbfs_mesh_view{b->N, b->F, b->NI, b->owner.data(), b->nbr.data(), b->cc.data(), b->vol.data(),
                            b->fc.data(), b->fn.data(), b->fa.data(), b->fdt.data()};
 }
+
+// Per-case results: residuals [B][4], status, step count and convergence flag [B].
+size_t case_bytes(int B) { return (size_t)B * (4 * sizeof(double) + 3 * sizeof(int32_t)); }
 
 size_t lds_bytes_for(const plbfs::Layout &L, int C, bool f32, bool stage) {
     const size_t b = f32 ? flux_lds_bytes<float>(L.max_items_per_block, L.block_cells, stage, C)
@@ -624,8 +635,7 @@ int run_steps(plbfs_batch *b, int max_steps, float *ms_out) {
     plbfs_ctx *c = b->base;
     int rc;
     if (b->ibm_dirty && (rc = ibm_upload(b))) return rc;
-    Ctrl h{};
-    HIP_TRY(hipMemcpyAsync(b->ctrl, &h, sizeof(Ctrl), hipMemcpyHostToDevice, c->stream));
+    HIP_TRY(hipMemsetAsync(b->ctrl, 0, sizeof(Ctrl), c->stream));
     const int64_t NR = (int64_t)b->N * b->B;
     const dim3 rgrid((unsigned)((NR + kBlock - 1) / kBlock));
     if (b->f32)
@@ -636,10 +646,7 @@ int run_steps(plbfs_batch *b, int max_steps, float *ms_out) {
                            (const double4 *)b->stA, b->dtl);
     HIP_TRY(hipGetLastError());
     const int interval = std::max(1, b->params.check_interval);
-    hipEvent_t e0, e1;
-    HIP_TRY(hipEventCreate(&e0));
-    HIP_TRY(hipEventCreate(&e1));
-    HIP_TRY(hipEventRecord(e0, c->stream));
+    HIP_TRY(hipEventRecord(c->ev0, c->stream));
     for (int s = 0; s < max_steps;) {
         const int left = std::min(interval - s % interval, max_steps - s);  // steps to the next check
         const bool many = left >= kGraphSteps;
@@ -649,17 +656,17 @@ int run_steps(plbfs_batch *b, int max_steps, float *ms_out) {
         HIP_TRY(hipGraphLaunch(g, c->stream));
         s += n;
         if (n == left) {
-            HIP_TRY(hipMemcpyAsync(&h, b->ctrl, sizeof(Ctrl), hipMemcpyDeviceToHost, c->stream));
+            HIP_TRY(hipMemcpyAsync(c->host, b->ctrl, sizeof(Ctrl), hipMemcpyDeviceToHost, c->stream));
             HIP_TRY(hipStreamSynchronize(c->stream));
+            Ctrl h;
+            std::memcpy(&h, c->host, sizeof h);
             if (h.done) break;
         }
     }
-    HIP_TRY(hipEventRecord(e1, c->stream));
-    HIP_TRY(hipEventSynchronize(e1));
+    HIP_TRY(hipEventRecord(c->ev1, c->stream));
+    HIP_TRY(hipEventSynchronize(c->ev1));
     float ms = 0;
-    (void)hipEventElapsedTime(&ms, e0, e1);
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
+    (void)hipEventElapsedTime(&ms, c->ev0, c->ev1);
     if (ms_out) *ms_out = ms;
     return PLBFS_OK;
 }
@@ -731,12 +738,12 @@ extern "C" int plbfs_batch_create(const plbfs_mesh_view *mesh, const plbfs_param
         (rc = bupload(b, &b->d_visc, b->visc)) || (rc = bupload(b, &b->d_v3g, v3g)) ||
         (rc = bupload(b, &b->d_dtcap, dtcap)) ||
         (rc = balloc(b, (void **)&b->done, n_cases * sizeof(int32_t))) ||
-        (rc = balloc(b, (void **)&b->status, n_cases * sizeof(int32_t))) ||
-        (rc = balloc(b, (void **)&b->steps, n_cases * sizeof(int32_t))) ||
-        (rc = balloc(b, (void **)&b->conv, n_cases * sizeof(int32_t))) ||
-        (rc = balloc(b, (void **)&b->res, n_cases * 4 * sizeof(double))) ||
+        (rc = balloc(b, (void **)&b->res, case_bytes(n_cases))) ||
         (rc = balloc(b, (void **)&b->ctrl, sizeof(Ctrl))))
         return fail(rc);
+    b->status = reinterpret_cast<int32_t *>(b->res + (size_t)4 * n_cases);
+    b->steps = b->status + n_cases;
+    b->conv = b->steps + n_cases;
     if (hipMemset(b->fbody, 0, NR * 3 * sizeof(double)) != hipSuccess || reset_case_ctl(b))
         return fail(plbfs_fail(PLBFS_ERR_HIP, "batch initialisation"));
     *out = b;
@@ -791,26 +798,11 @@ extern "C" int plbfs_batch_get_state(plbfs_batch *b, int32_t case_id, double *rh
     const int N = b->N;
     hipStream_t s = b->base->stream;
     // the conservative state t0 holds the solution in both precisions
-    hipLaunchKernelGGL(kb_gather, dim3((N + kBlock - 1) / kBlock), dim3(kBlock), 0, s, N, b->B, (int)case_id,
-                       (const double4 *)b->t0, (double4 *)b->scratch);
+    hipLaunchKernelGGL(kb_export, dim3((N + kBlock - 1) / kBlock), dim3(kBlock), 0, s, N, b->B, (int)case_id,
+                       b->base->inv, b->steps, (const double4 *)b->t0, b->scratch);
     HIP_TRY(hipGetLastError());
-    std::vector<double> h((size_t)4 * N);
-    HIP_TRY(hipMemcpyAsync(h.data(), b->scratch, h.size() * sizeof(double), hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
-    int32_t steps = 0;
-    HIP_TRY(hipMemcpy(&steps, b->steps + case_id, sizeof(int32_t), hipMemcpyDeviceToHost));
-    const std::vector<int32_t> &perm = b->base->L.perm;
-    for (int n = 0; n < N; n++) {
-        const double *q = &h[(size_t)4 * n];
-        const int i = perm[n];
-        // before any step t0 holds the initial primitives, afterwards conservatives
-        const double r = q[0];
-        if (rho) rho[i] = r;
-        if (u) u[i] = steps > 0 ? q[1] / r : q[1];
-        if (v) v[i] = steps > 0 ? q[2] / r : q[2];
-        if (w) w[i] = steps > 0 ? q[3] / r : q[3];
-    }
-    return PLBFS_OK;
+    double *outs[4] = {rho, u, v, w};
+    return fields_to_host(b->base, b->scratch, outs);
 }
 
 extern "C" int plbfs_batch_set_ibm(plbfs_batch *b, int32_t case_id, const plbfs_ibm_nodes *nodes) {
@@ -843,12 +835,13 @@ extern "C" int plbfs_batch_run(plbfs_batch *b, int32_t max_steps, plbfs_result *
     int rc = run_steps(b, max_steps, &ms);
     if (rc) return rc;
     const int B = b->B;
-    std::vector<int32_t> st(B), steps(B), conv(B);
-    std::vector<double> res((size_t)4 * B);
-    HIP_TRY(hipMemcpy(st.data(), b->status, B * sizeof(int32_t), hipMemcpyDeviceToHost));
-    HIP_TRY(hipMemcpy(steps.data(), b->steps, B * sizeof(int32_t), hipMemcpyDeviceToHost));
-    HIP_TRY(hipMemcpy(conv.data(), b->conv, B * sizeof(int32_t), hipMemcpyDeviceToHost));
-    HIP_TRY(hipMemcpy(res.data(), b->res, res.size() * sizeof(double), hipMemcpyDeviceToHost));
+    // residuals, status, step counts and flags lie behind each other (case_bytes)
+    std::vector<char> all(case_bytes(B));
+    char *host = all.size() <= kHostBytes ? b->base->host : all.data();
+    HIP_TRY(hipMemcpyAsync(host, b->res, all.size(), hipMemcpyDeviceToHost, b->base->stream));
+    HIP_TRY(hipStreamSynchronize(b->base->stream));
+    const double *res = reinterpret_cast<const double *>(host);
+    const int32_t *st = reinterpret_cast<const int32_t *>(res + (size_t)4 * B), *steps = st + B, *conv = steps + B;
     int worst = PLBFS_OK;
     for (int c = 0; c < B; c++) {
         if (results) {

@@ -33,6 +33,10 @@ constexpr int kFluxBlockCells = 256;
 constexpr int kMaxLds = 159 * 1024;
 }
 
+// Results up to this size come to the host through the context's pinned buffer in
+// one copy; a copy straight into pageable memory costs a call some 25 us each.
+constexpr size_t kHostBytes = (size_t)256 << 10;
+
 struct KStat {
     double ms = 0;
     int launches = 0;
@@ -86,6 +90,9 @@ struct plbfs_ctx {
     double *hist = nullptr;
     int hist_cap = 0;
     plbfs::Ctrl *ctrl = nullptr;
+    int32_t *inv = nullptr;                 // [N] file cell -> cell
+    char *host = nullptr;                   // kHostBytes of pinned host memory for small results
+    hipEvent_t ev0 = nullptr, ev1 = nullptr;  // ends of a run's time loop
     size_t lds_bytes = 0;
     int cell_grid = 0;  // blocks of kBlock cells for the per-cell kernels
     int bound_blocks = 0;  // flux blocks that the scratch bound of plbfs_run_noalloc counts
@@ -151,6 +158,10 @@ struct TimedLaunch {
         }
     }
 };
+
+// Fields on the device, [4][N] in file order, to the caller's arrays (null: skipped),
+// once the stream has written them.
+int fields_to_host(plbfs_ctx *c, const double *src, double *const out[4]);
 
 // Drops the captured steps (their kernels' arguments are about to change).
 void drop_graphs(plbfs_ctx *c);

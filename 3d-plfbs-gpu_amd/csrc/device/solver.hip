@@ -334,6 +334,19 @@ __global__ __launch_bounds__(kFinalizeThreads) void k_finalize(int nblk, double 
     }
 }
 
+// Cell records to [4][N] in file order; divide: conservatives to primitives.
+__global__ __launch_bounds__(kBlock) void k_export(int N, const int32_t *__restrict__ inv,
+                                                   const double4 *__restrict__ src, int divide,
+                                                   double *__restrict__ out) {
+    const int i = blockIdx.x * kBlock + threadIdx.x;
+    if (i >= N) return;
+    const double4 q = src[inv[i]];
+    out[i] = q.x;
+    out[(size_t)N + i] = divide ? q.y / q.x : q.y;
+    out[2 * (size_t)N + i] = divide ? q.z / q.x : q.z;
+    out[3 * (size_t)N + i] = divide ? q.w / q.x : q.w;
+}
+
 // One residual evaluation for diagnostics: flux gather only (stage-independent).
 template <typename S>
 __global__ __launch_bounds__(kBlock) void k_residual_only(DevMesh<S> m, DevParams prm,
@@ -414,6 +427,12 @@ static int release(plbfs_ctx *c) {
     c->allocs.clear();
     for (void *p : c->ibm_allocs) hipFree(p);
     c->ibm_allocs.clear();
+    for (hipEvent_t *e : {&c->ev0, &c->ev1}) {
+        if (*e) (void)hipEventDestroy(*e);
+        *e = nullptr;
+    }
+    if (c->host) (void)hipHostFree(c->host);
+    c->host = nullptr;
     if (c->stream) {
         hipStreamDestroy(c->stream);
         c->stream = nullptr;
@@ -530,6 +549,9 @@ int create_ctx(const plbfs_mesh_view *mesh, const plbfs_params *params, const pl
     if ((rc = resolve_scratch(c->device, &c->scratch))) return fail(rc);
     if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess)
         return fail(plbfs_fail(PLBFS_ERR_HIP, "hipStreamCreate"));
+    if (hipEventCreate(&c->ev0) != hipSuccess || hipEventCreate(&c->ev1) != hipSuccess ||
+        hipHostMalloc((void **)&c->host, kHostBytes, hipHostMallocDefault) != hipSuccess)
+        return fail(plbfs_fail(PLBFS_ERR_HIP, "events and host buffer"));
     const int N = L.N;
     c->bound_blocks = L.n_blocks;
     DevMesh<double> &d = c->dm;
@@ -598,7 +620,7 @@ int create_ctx(const plbfs_mesh_view *mesh, const plbfs_params *params, const pl
         (rc = upload(c, (float4 **)&d.it_p, c->f32 ? pack_items<float>(L) : pack_items<double>(L))) ||
         (rc = upload(c, (uint16_t **)&d.it_side, std::vector<uint16_t>(L.it_side.begin(), L.it_side.end()))) ||
         (rc = upload(c, (int32_t **)&d.b_patch, bpatch)) || (rc = upload(c, (int32_t **)&d.b_partner, bpartner)) ||
-        (rc = upload(c, (DevPatch **)&d.patches, dp)))
+        (rc = upload(c, (DevPatch **)&d.patches, dp)) || (rc = upload(c, &c->inv, L.inv)))
         return fail(rc);
     if (!c->f32) {
         if ((rc = upload(c, (double **)&d.st_w, L.st_w)) ||
@@ -694,6 +716,21 @@ static int to_device_state(plbfs_ctx *c, const double *rho, const double *u, con
     return PLBFS_OK;
 }
 
+int fields_to_host(plbfs_ctx *c, const double *src, double *const out[4]) {
+    const size_t N = (size_t)c->L.N, bytes = N * sizeof(double);
+    if (4 * bytes <= kHostBytes) {
+        HIP_TRY(hipMemcpyAsync(c->host, src, 4 * bytes, hipMemcpyDeviceToHost, c->stream));
+        HIP_TRY(hipStreamSynchronize(c->stream));
+        for (int q = 0; q < 4; q++)
+            if (out[q]) std::memcpy(out[q], c->host + q * bytes, bytes);
+        return PLBFS_OK;
+    }
+    for (int q = 0; q < 4; q++)
+        if (out[q]) HIP_TRY(hipMemcpyAsync(out[q], src + q * N, bytes, hipMemcpyDeviceToHost, c->stream));
+    HIP_TRY(hipStreamSynchronize(c->stream));
+    return PLBFS_OK;
+}
+
 // Copies nf interleaved values per cell back to file order (one array per value).
 static int from_device_fields(plbfs_ctx *c, const double *src, int nf, double *const *out) {
     const int N = c->L.N;
@@ -758,25 +795,14 @@ static int check_ghost_state(const plbfs_ctx *c) {
 
 extern "C" int plbfs_get_state(plbfs_ctx *c, double *rho, double *u, double *v, double *w) {
     if (!c) return plbfs_fail(PLBFS_ERR_INPUT, "null argument");
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    double *outs[4] = {rho, u, v, w};
-    if (!c->f32) return from_device_fields(c, c->stA, 4, outs);
     // FP32 storage: the FP64 conservative state t0 holds the solution (before
     // any step it still holds the initial primitives)
-    const int N = c->L.N;
-    std::vector<double> h((size_t)4 * N);
-    HIP_TRY(hipMemcpy(h.data(), c->t0, h.size() * sizeof(double), hipMemcpyDeviceToHost));
-    for (int n = 0; n < N; n++) {
-        const double *q = &h[(size_t)4 * n];
-        const int i = c->L.perm[n];
-        const double r = q[0];
-        const bool cons = c->total_steps > 0;
-        if (rho) rho[i] = r;
-        if (u) u[i] = cons ? q[1] / r : q[1];
-        if (v) v[i] = cons ? q[2] / r : q[2];
-        if (w) w[i] = cons ? q[3] / r : q[3];
-    }
-    return PLBFS_OK;
+    double *outs[4] = {rho, u, v, w};
+    double *tmp = c->stB;  // rewritten before it is read in a step
+    hipLaunchKernelGGL(k_export, dim3((c->L.N + kBlock - 1) / kBlock), dim3(kBlock), 0, c->stream, c->L.N, c->inv,
+                       (const double4 *)(c->f32 ? c->t0 : c->stA), c->f32 && c->total_steps > 0 ? 1 : 0, tmp);
+    HIP_TRY(hipGetLastError());
+    return fields_to_host(c, tmp, outs);
 }
 
 // ---- launches -------------------------------------------------------------
@@ -880,6 +906,10 @@ static int launch_step(plbfs_ctx *c, const RunScratch &w, bool timed, bool rebui
     return PLBFS_OK;
 }
 
+__global__ void k_clear_ctrl(Ctrl *ctrl) {
+    if (threadIdx.x == 0) *ctrl = Ctrl{};
+}
+
 static int ensure_hist(plbfs_ctx *c, int steps) {
     if (steps <= c->hist_cap) return PLBFS_OK;
     drop_graphs(c);
@@ -925,16 +955,19 @@ extern "C" int plbfs_run(plbfs_ctx *c, int32_t max_steps, plbfs_result *out) {
     int rc = check_ghost_state(c);
     if (rc) return rc;
     if ((rc = ensure_hist(c, max_steps))) return rc;
-    Ctrl h{};
-    HIP_TRY(hipMemcpyAsync(c->ctrl, &h, sizeof(Ctrl), hipMemcpyHostToDevice, c->stream));
     const RunScratch w = ctx_scratch(c);
+    hipLaunchKernelGGL(k_clear_ctrl, dim3(1), dim3(64), 0, c->stream, c->ctrl);
     if ((rc = launch_run_start(c, w))) return rc;
     const int interval = std::max(1, c->params.check_interval);
     const bool graph = c->use_graph && !c->timing;
-    hipEvent_t ev0, ev1;
-    HIP_TRY(hipEventCreate(&ev0));
-    HIP_TRY(hipEventCreate(&ev1));
-    HIP_TRY(hipEventRecord(ev0, c->stream));
+    // the control block comes to the pinned buffer, with the history behind it
+    // at the last check where it fits
+    Ctrl h{};
+    const size_t hist0 = 256, hist_bytes = (size_t)max_steps * 4 * sizeof(double);
+    static_assert(sizeof(Ctrl) <= 256, "the history follows the control block");
+    const bool small = hist0 + hist_bytes <= kHostBytes;
+    bool have_hist = max_steps == 0;
+    HIP_TRY(hipEventRecord(c->ev0, c->stream));
     for (int s = 0; s < max_steps;) {
         const int left = std::min(interval - s % interval, max_steps - s);  // steps to the next check
         int n = 1;
@@ -950,8 +983,13 @@ extern "C" int plbfs_run(plbfs_ctx *c, int32_t max_steps, plbfs_result *out) {
         }
         s += n;
         if (n == left) {
-            HIP_TRY(hipMemcpyAsync(&h, c->ctrl, sizeof(Ctrl), hipMemcpyDeviceToHost, c->stream));
+            have_hist = small && s == max_steps;
+            HIP_TRY(hipEventRecord(c->ev1, c->stream));
+            HIP_TRY(hipMemcpyAsync(c->host, c->ctrl, sizeof(Ctrl), hipMemcpyDeviceToHost, c->stream));
+            if (have_hist)
+                HIP_TRY(hipMemcpyAsync(c->host + hist0, c->hist, hist_bytes, hipMemcpyDeviceToHost, c->stream));
             HIP_TRY(hipStreamSynchronize(c->stream));
+            std::memcpy(&h, c->host, sizeof h);
             if (h.done && h.rebuild && h.status == PLBFS_OK && !h.converged) {
                 // new candidate lists around the nodes' positions after step
                 // h.step, then on from there: the launches after the stop were
@@ -966,18 +1004,15 @@ extern "C" int plbfs_run(plbfs_ctx *c, int32_t max_steps, plbfs_result *out) {
             if (h.done) break;
         }
     }
-    HIP_TRY(hipEventRecord(ev1, c->stream));
-    HIP_TRY(hipEventSynchronize(ev1));
+    if (max_steps == 0) HIP_TRY(hipEventRecord(c->ev1, c->stream));
+    HIP_TRY(hipEventSynchronize(c->ev1));
     resolve_timing(c);
     float ms = 0;
-    hipEventElapsedTime(&ms, ev0, ev1);
-    hipEventDestroy(ev0);
-    hipEventDestroy(ev1);
-    HIP_TRY(hipMemcpy(&h, c->ctrl, sizeof(Ctrl), hipMemcpyDeviceToHost));
+    hipEventElapsedTime(&ms, c->ev0, c->ev1);
     c->last_hist.assign((size_t)h.step * 4, 0.0);
-    if (h.step > 0)
-        HIP_TRY(hipMemcpy(c->last_hist.data(), c->hist, (size_t)std::min(h.step, c->hist_cap) * 4 * sizeof(double),
-                          hipMemcpyDeviceToHost));
+    const size_t got = (size_t)std::min(h.step, c->hist_cap) * 4 * sizeof(double);
+    if (have_hist) std::memcpy(c->last_hist.data(), c->host + hist0, got);
+    else if (h.step > 0) HIP_TRY(hipMemcpy(c->last_hist.data(), c->hist, got, hipMemcpyDeviceToHost));
     fill_result(c, h, ms, out);
     return h.status;
 }
@@ -988,10 +1023,6 @@ static size_t round256(size_t b) { return (b + 255) / 256 * 256; }
 static size_t scratch_need(const plbfs_ctx *c, int64_t max_steps) {
     return round256(sizeof(Ctrl)) + round256((size_t)c->bound_blocks * 5 * sizeof(double)) +
            round256((size_t)c->cell_grid * sizeof(double)) + (size_t)max_steps * 4 * sizeof(double);
-}
-
-__global__ void k_clear_ctrl(Ctrl *ctrl) {
-    if (threadIdx.x == 0) *ctrl = Ctrl{};
 }
 
 extern "C" int plbfs_run_noalloc(plbfs_ctx *c, int32_t max_steps, plbfs_result *out, double *hist_out) {
@@ -1022,13 +1053,13 @@ extern "C" int plbfs_run_noalloc(plbfs_ctx *c, int32_t max_steps, plbfs_result *
     for (int s = 0; s < max_steps; s++) {
         if ((rc = launch_step(c, w, false, false))) return rc;
         if ((s + 1) % interval == 0 || s == max_steps - 1) {
-            HIP_TRY(hipMemcpyAsync(&h, w.ctrl, sizeof(Ctrl), hipMemcpyDeviceToHost, c->stream));
+            HIP_TRY(hipMemcpyAsync(c->host, w.ctrl, sizeof(Ctrl), hipMemcpyDeviceToHost, c->stream));
             HIP_TRY(hipStreamSynchronize(c->stream));
+            std::memcpy(&h, c->host, sizeof h);
             if (h.done) break;
         }
     }
-    HIP_TRY(hipMemcpyAsync(&h, w.ctrl, sizeof(Ctrl), hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
+    if (max_steps == 0) HIP_TRY(hipStreamSynchronize(c->stream));
     const double ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     if (hist_out && h.step > 0)
         HIP_TRY(hipMemcpy(hist_out, w.hist, (size_t)h.step * 4 * sizeof(double), hipMemcpyDeviceToHost));

@@ -165,7 +165,7 @@ class GpuSolver:
         nat.check(nat.lib().plbfs_set_state(self.h, *(nat.dptr(x) for x in a)))
 
     def state(self):
-        a = [np.zeros(self.N) for _ in range(4)]
+        a = [np.empty(self.N) for _ in range(4)]
         nat.check(nat.lib().plbfs_get_state(self.h, *(nat.dptr(x) for x in a)))
         return a
 
@@ -288,7 +288,7 @@ class GpuBatch:
         nat.check(nat.lib().plbfs_batch_set_state(self.h, int(case), *(nat.dptr(x) for x in a)))
 
     def state(self, case):
-        a = [np.zeros(self.N) for _ in range(4)]
+        a = [np.empty(self.N) for _ in range(4)]
         nat.check(nat.lib().plbfs_batch_get_state(self.h, int(case), *(nat.dptr(x) for x in a)))
         return a
 
