@@ -167,7 +167,7 @@ int fields_to_host(plbfs_ctx *c, const double *src, double *const out[4]);
 void drop_graphs(plbfs_ctx *c);
 
 // plbfs_create with an explicit flux block size (64..1024 cells, a multiple of
-// 64), LDS sized for lds_cases cases per block (the batched solver sizes its
+// 64, or 0: chosen for the mesh), LDS sized for lds_cases cases per block (the batched solver sizes its
 // own), staging of the flux block's own records, and border faces either
 // evaluated once by a separate pass (split_border) or by both blocks.
 int create_ctx(const plbfs_mesh_view *mesh, const plbfs_params *params, const plbfs_patch *patches,

@@ -388,9 +388,10 @@ __global__ __launch_bounds__(kBlock) void k_residual_only(DevMesh<S> m, DevParam
 // device share the array and race.
 constexpr size_t kScratchBytes = (size_t)8 << 20;
 // The bound counts kFluxBlockCells cells a block where the mesh size chose the block
-// size; the partials of the smaller blocks it may choose (at most 1,024 instead of
-// 256 blocks, 40 B each) fit behind it.
-constexpr size_t kScratchSpare = (size_t)32 << 10;
+// size; the partials of the smaller blocks it may choose (up to 1,024 instead of 256,
+// or 5,958 instead of 4,096, 40 B each) fit behind it.
+constexpr size_t kScratchSpare = (size_t)128 << 10;
+static_assert(40 * ((size_t)16 * 65536 / kMinAutoBlock + 1 - 4096) + 512 <= kScratchSpare, "partials fit");
 static __device__ __align__(256) double scratch[(kScratchBytes + kScratchSpare) / sizeof(double)];
 
 constexpr int kMaxScratchDevices = 64;
@@ -452,24 +453,12 @@ static bool env_flag(const char *name, bool def) {
     return v[0] != '0';
 }
 
-// Larger blocks duplicate fewer border faces; but a block takes its time whatever
-// the others do, some 10 us for 64 cells (one face item a thread), 20 for 256, so a
-// mesh of fewer 256-cell blocks than the 256 CUs is faster in smaller ones.  Step in
-// FP64, us, with 64 / 192 / 256 cells: 216 hexes 62 / 82 / 82, 16k 94 / 118 / 131, 32k
-// 101 / 116 / 120, 17k tets 73 / 80 / 88, 83k tets 171 / 163 / 175, 221k hexes 252 / 246
-// / 243, 384k tets 299 / 284 / 279.
-static int default_block_cells(int n_cells) {
-    if (n_cells < 256 * 256) return 64;
-    if (n_cells < 2 * 256 * 256) return 192;
-    return kFluxBlockCells;
-}
-
 extern "C" int plbfs_create(const plbfs_mesh_view *mesh, const plbfs_params *params, const plbfs_patch *patches,
                             int32_t n_patches, const int32_t *bface_patch, plbfs_ctx **out) {
-    // cells per flux block (a multiple of 64)
+    // cells per flux block (a multiple of 64), by default chosen for the mesh
     const char *bc = std::getenv("PLBFS_BLOCK_CELLS");
-    const int block_cells = bc ? std::atoi(bc) : default_block_cells(mesh ? mesh->n_cells : 0);
-    if (block_cells < 64 || block_cells % 64 || block_cells > 4 * kBlock)
+    const int block_cells = bc ? std::atoi(bc) : 0;
+    if (bc && (block_cells < 64 || block_cells % 64 || block_cells > 4 * kBlock))
         return plbfs_fail(PLBFS_ERR_INPUT, "PLBFS_BLOCK_CELLS must be a multiple of 64 up to %d", 4 * kBlock);
     // measured on MI355X (4.09M tets): staging the flux block's own records in
     // LDS costs more (staging phase + barrier) than the L2 traffic it saves,
@@ -529,8 +518,8 @@ int create_ctx(const plbfs_mesh_view *mesh, const plbfs_params *params, const pl
     const size_t sbytes = c->f32 ? sizeof(float) : sizeof(double);
     const bool stage = flux_stage;
     c->lds_bytes = lds_cases == 1
-                       ? (c->f32 ? flux_lds_bytes<float>(L.max_items_per_block, block_cells, stage)
-                                 : flux_lds_bytes<double>(L.max_items_per_block, block_cells, stage))
+                       ? (c->f32 ? flux_lds_bytes<float>(L.max_items_per_block, L.block_cells, stage)
+                                 : flux_lds_bytes<double>(L.max_items_per_block, L.block_cells, stage))
                        : (size_t)L.max_items_per_block * 4 * sbytes * lds_cases;
     if (c->lds_bytes > kMaxLds) {
         // L refers into c: read what the message needs before c is freed

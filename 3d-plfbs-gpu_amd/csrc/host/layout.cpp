@@ -116,6 +116,40 @@ struct NearestCell {
     }
 };
 
+// Cells per flux block by mesh size.  Larger blocks duplicate fewer border faces, but
+// a block takes its time whatever the others do: a pass of its 256 threads over its face
+// items at a time and then its cells, some 10 us for 64 cells of one pass, 20 for 256.
+//   - fewer 256-cell blocks than the 256 CUs: 64 cells.  Step in FP64, us, with 64 / 192 /
+//     256 cells: 216 hexes 62 / 82 / 82, 16k 94 / 118 / 131, 32k 101 / 116 / 120.
+//   - up to 16 of them a CU: the size whose passes are full and that gives every CU the
+//     same number of blocks, by the estimate below.  221k hexes, 208 / 216 / 224 / 256
+//     cells (1064 / 1024 / 988 / 864 blocks of 754 / 782 / 809 / 919 items): flux 40.8 / 35.1 /
+//     38.8 / 40.3 us in FP64, 28.3 / 26.5 / 28.5 / 28.6 in FP32; 83k tets, 192 / 256 cells:
+//     20.2 / 22.5.
+//   - beyond: 256 cells (4.1M tets within 1 % up to 448).
+static int auto_block_cells(const plbfs_mesh_view &m, const std::vector<int32_t> &inv) {
+    constexpr int kCus = 256, kThreads = 256;
+    const int64_t N = m.n_cells;
+    if (N < (int64_t)kCus * 256) return 64;
+    if (N > (int64_t)16 * kCus * 256) return 256;
+    int64_t cut = 0;  // faces between two 256-cell blocks; their number goes with the blocks' surface
+    for (int f = 0; f < m.n_internal_faces; f++) cut += inv[m.owner[f]] / 256 != inv[m.neighbour[f]] / 256;
+    int best = 256;
+    double best_cost = 1e300;
+    for (int b = 256; b >= kMinAutoBlock; b -= 8) {
+        const double blocks = (double)((N + b - 1) / b);
+        const double items = (m.n_faces + cut * std::cbrt(256.0 / b)) / blocks;
+        // the mean block may exceed whole passes by a few items (half the blocks then
+        // do not); a pass over the cells takes some 1.2 of a pass over the items
+        const double cost = std::ceil(blocks / kCus) * (std::ceil(items / kThreads - 0.08) + 1.2);
+        if (cost < best_cost) {
+            best_cost = cost;
+            best = b;
+        }
+    }
+    return best;
+}
+
 int build_layout(const plbfs_mesh_view &m, const plbfs_params &p, const plbfs_patch *patches, int n_patches,
                  const int32_t *bface_patch, int block_cells, bool split_border, Layout &L) {
     const int N = m.n_cells, F = m.n_faces, NI = m.n_internal_faces, G = F - NI;
@@ -140,7 +174,7 @@ int build_layout(const plbfs_mesh_view &m, const plbfs_params &p, const plbfs_pa
         if (f >= NI && m.neighbour[f] != N + f - NI)
             return plbfs_fail(PLBFS_ERR_INPUT, "face %d: boundary neighbour must be the ghost index", f);
     }
-    if (block_cells < 64 || block_cells > 1024 || block_cells % 64)
+    if (block_cells != 0 && (block_cells < 64 || block_cells > 1024 || block_cells % 64))
         return plbfs_fail(PLBFS_ERR_INPUT, "block_cells %d", block_cells);
     L = Layout();
     L.N = N; L.F = F; L.NI = NI; L.G = G;
@@ -397,7 +431,8 @@ int build_layout(const plbfs_mesh_view &m, const plbfs_params &p, const plbfs_pa
     }
 
     // block face items and per-cell gather lists
-    const int C = block_cells;
+    if (block_cells == 0) L.block_cells = auto_block_cells(m, L.inv);
+    const int C = L.block_cells;
     L.n_blocks = (N + C - 1) / C;
     L.blk_item_off.assign(L.n_blocks + 1, 0);
     L.g_off.assign(N + 1, 0);

@@ -23,6 +23,7 @@
 namespace plbfs {
 
 constexpr int kMaxSlots = 6;  // LSQ slots per cell (the reference's RHS arrays hold 6, gradients.cpp)
+constexpr int kMinAutoBlock = 176;  // smallest flux block that build_layout picks for a mesh of 65,536 cells or more
 constexpr int kGeoPerItem = 11;  // n(3), area, dt, r_owner(3), r_neighbour(3)
 
 struct Layout {
@@ -87,7 +88,8 @@ struct Layout {
 inline bool rho_keeps_ghost(int t) { return t == 4 || t == 5 || t == 9; }
 inline bool vel_keeps_ghost(int t) { return t == 4 || t == 5 || t == 7 || t == 9; }
 
-// Builds the layout.  Returns PLBFS_OK or an error code (message via plbfs_fail).
+// Builds the layout, with flux blocks of block_cells cells (a multiple of 64) or, for 0, of a
+// size that suits the mesh.  Returns PLBFS_OK or an error code (message via plbfs_fail).
 int build_layout(const plbfs_mesh_view &m, const plbfs_params &p, const plbfs_patch *patches, int n_patches,
                  const int32_t *bface_patch, int block_cells, bool split_border, Layout &L);
 

@@ -318,3 +318,33 @@ def test_wall_forces_match_reference_sums(gpu_available):
         assert abs(dl[1] - lift) <= 1e-10 * max(1.0, abs(lift)), (name, dl, lift)
         checked += 1
     assert checked == len(pm.patch_names)
+
+
+@pytest.mark.parametrize("dims,tets,sizes", [((40, 40, 40), False, (64, 64)), ((41, 40, 40), False, (176, 256)),
+                                             ((23, 22, 22), True, (176, 256)), ((3, 3, 3), False, (64, 64))])
+@pytest.mark.parametrize("precision", [0, 1])
+def test_chosen_flux_block_size_changes_no_field(gpu_available, monkeypatch, dims, tets, sizes, precision):
+    """The block size that a mesh gets on either side of 65,536 cells, against blocks
+    of 256 cells: the same fields, bit for bit."""
+    pm = channel_mesh(*dims, tets=tets)
+    case = pc.channel_case(re=40.0, length_scale=6.0, fneq_min=0.55)
+    case.lsq_exact_det = 1 if tets else 0
+    case.precision = precision
+    hm = HostMesh.from_polymesh(pm, case.visc, case.gamma, case.fneq_min)
+    g = hm.geometry()
+    n = pm.n_cells
+    rho, u, v, w = case.initial_state(g["cx"][:n], g["cy"][:n], g["cz"][:n])
+    st = (rho + 1e-3 * np.sin(g["cx"][:n]), u * (1 + 0.02 * np.cos(g["cy"][:n])), v, w + 1e-4 * np.sin(g["cz"][:n]))
+    out = []
+    for blk in ("", "256"):
+        if blk:
+            monkeypatch.setenv("PLBFS_BLOCK_CELLS", blk)
+        s = GpuSolver(hm, case.params, case.patches_for(pm.patch_names))
+        b = s.layout_info()["block_cells"]
+        assert b == 256 if blk else sizes[0] <= b <= sizes[1]
+        s.set_state(*st)
+        assert s.run(6)["rc"] == 0
+        out.append(s.state())
+        s.close()
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
