@@ -83,7 +83,7 @@ void kb_flux_border(DevMesh<S> m, DevParams prm, BatchArgs a, const Ctrl *__rest
     if (j >= m.n_border || a.done[b]) return;
     const SideLoader<S, RecB> ld{st_in, grad, RecB{a.B, b}, nullptr, 0, 0, 1, 0};
     S F[4];
-    item_flux<S>(m, prm, m.border0 + j, ld, a.v3g[b], a.dtcap[b], F);
+    item_flux<S>(m, prm, load_item<S>(m, m.border0 + j), ld, a.v3g[b], a.dtcap[b], F);
     const size_t nbd = (size_t)m.n_border;
 #pragma unroll
     for (int q = 0; q < 4; q++) m.bflux[(q * nbd + j) * a.B + b] = F[q];
@@ -123,7 +123,7 @@ __global__ __launch_bounds__(kBlock) void kb_flux(DevMesh<S> m, DevParams prm, B
         const SideLoader<S, RecB> ld{st_in, grad, RecB{B, b}, sRec, c0, nst, C, c};
         for (int el = threadIdx.x / C; el < e1 - e0; el += kBlock / C) {
             S F[4];
-            item_flux<S>(m, prm, e0 + el, ld, v3g, dtcap, F);
+            item_flux<S>(m, prm, load_item<S>(m, e0 + el), ld, v3g, dtcap, F);
 #pragma unroll
             for (int q = 0; q < 4; q++) sF[q * stride + el * C + c] = F[q];
         }
@@ -136,14 +136,14 @@ __global__ __launch_bounds__(kBlock) void kb_flux(DevMesh<S> m, DevParams prm, B
     for (int il = threadIdx.x / C; live && il < ncell; il += kBlock / C) {
         const int i = c0 + il;
         double R[4];
-        gather_residual<S>(m, i, sF, stride, C, c, R, B, b);
+        gather_residual<S>(m, i, load_faces<S>(m, i), sF, stride, C, c, R, B, b);
         const size_t r = (size_t)i * B + b;
         if (prm.use_body_force && a.force_rec[r]) {
             R[1] += fbody[r];
             R[2] += fbody[NR + r];
             R[3] += fbody[2 * NR + r];
         }
-        const int e = rk_update<S>(m, prm, visc, sa, i, r, R, st_out, t0, t1, dtl, sq);
+        const int e = rk_update<S>(m, prm, visc, sa, i, r, load_rk<S>(m, sa, i, r, t0, t1, dtl), R, st_out, t0, t1, dtl, sq);
         if (e == 1) err = 1;
         else if (e == 2 && err == 0) err = 2;
     }

@@ -31,6 +31,7 @@ constexpr int kFluxBlockCells = 256;
 // flux kernels' static arrays take at most 160 B, and a launch whose total
 // exceeds 160 KiB is not refused by the runtime but faults, so 1 KiB stays free.
 constexpr int kMaxLds = 159 * 1024;
+constexpr size_t kMaxStageLds = 64 * 1024;  // of k_stage: two blocks a CU
 }
 
 // Results up to this size come to the host through the context's pinned buffer in
@@ -94,6 +95,7 @@ struct plbfs_ctx {
     char *host = nullptr;                   // kHostBytes of pinned host memory for small results
     hipEvent_t ev0 = nullptr, ev1 = nullptr;  // ends of a run's time loop
     size_t lds_bytes = 0;
+    size_t stage_lds = 0;  // LDS of k_stage, 0: gradients and fluxes are kernels of their own
     int cell_grid = 0;  // blocks of kBlock cells for the per-cell kernels
     int bound_blocks = 0;  // flux blocks that the scratch bound of plbfs_run_noalloc counts
     int total_steps = 0;

@@ -114,6 +114,14 @@ struct DevMesh {
     const float4 *it_p;
     const double *it_dt;
     const uint16_t *it_side;
+    // k_stage: the cells that a flux block's items read, max_local places a block, their
+    // stencil neighbours (slot by slot; kNoNbr behind the last) and weights (st_w, slot
+    // after slot in pieces of 16 B, piece k of place p at k * n_places + p) and an item's
+    // two places
+    const int32_t *loc_cell, *loc_nbr;
+    const float4 *loc_w;
+    const uint32_t *it_loc;
+    int max_local, n_places, n_patches;
     S b0[3];
     // a cell's faces in the reference face order, entry s of cell i at s * N + i:
     // slot << 1 | is_owner, kNoEnt behind the last one (max_ent: most of a cell);
@@ -149,36 +157,26 @@ struct DevParams {
 template <typename T>
 __device__ __forceinline__ void ghost_state(const DevPatch &P, const T po[4], const T pp[4], const T fx[4],
                                             T pg[4]) {
+    // selects between values at hand: a chain of branches costs each slot of a small
+    // mesh's wavefronts the latency of every branch's loads
     const int rt = P.rho_type, vt = P.vel_type;
-    if (rt == 1) pg[0] = (T)P.rho - (po[0] - (T)P.rho);
-    else if (rt == 3) pg[0] = pp[0];
-    else if (rt == 6 || rt == 7) pg[0] = (T)P.rho;
-    else if (rt == 4 || rt == 5 || rt == 9) pg[0] = fx[0];
-    else pg[0] = po[0];  // 2 (neumann, dx = 0) and 8 (symmetry)
-    if (vt == 4 || vt == 5 || vt == 7 || vt == 9) {
-        pg[1] = fx[1];
-        pg[2] = fx[2];
-        pg[3] = fx[3];
-    } else if (vt == 1) {
-        pg[1] = (T)P.u - (po[1] - (T)P.u);
-        pg[2] = (T)P.v - (po[2] - (T)P.v);
-        pg[3] = (T)P.w - (po[3] - (T)P.w);
-    } else if (vt == 6) {
-        pg[1] = (T)P.u;
-        pg[2] = (T)P.v;
-        pg[3] = (T)P.w;
-    } else if (vt == 8) {
-        pg[1] = po[1];
-        pg[2] = -po[2];
-        pg[3] = po[3];
-    } else if (vt == 3) {
-        pg[1] = pp[1];
-        pg[2] = pp[2];
-        pg[3] = pp[3];
-    } else {
-        pg[1] = po[1];
-        pg[2] = po[2];
-        pg[3] = po[3];
+    const T b[4] = {(T)P.rho, (T)P.u, (T)P.v, (T)P.w};
+    const bool rfix = rt == 4 || rt == 5 || rt == 9, vfix = vt == 4 || vt == 5 || vt == 7 || vt == 9;
+    T r = po[0];  // 2 (neumann, dx = 0) and 8 (symmetry)
+    r = rt == 3 ? pp[0] : r;
+    r = rfix ? fx[0] : r;
+    r = rt == 6 || rt == 7 ? b[0] : r;
+    r = rt == 1 ? b[0] - (po[0] - b[0]) : r;
+    pg[0] = r;
+#pragma unroll
+    for (int q = 1; q < 4; q++) {
+        T v = po[q];
+        if (q == 2) v = vt == 8 ? -po[q] : v;
+        v = vt == 3 ? pp[q] : v;
+        v = vfix ? fx[q] : v;
+        v = vt == 6 ? b[q] : v;
+        v = vt == 1 ? b[q] - (po[q] - b[q]) : v;
+        pg[q] = v;
     }
 }
 

@@ -58,7 +58,7 @@ __device__ __forceinline__ void block_fluxes(const DevMesh<S> &m, const DevParam
     }
     for (int e = e0 + threadIdx.x; e < e1; e += kBlock) {
         S F[4];
-        item_flux<S>(m, prm, e, ld, prm.visc3_invgam, INFINITY, F);
+        item_flux<S>(m, prm, load_item<S>(m, e), ld, prm.visc3_invgam, INFINITY, F);
 #pragma unroll
         for (int q = 0; q < 4; q++) sF[q * nslot + (e - e0)] = F[q];
     }
@@ -93,6 +93,21 @@ static std::vector<float4> pack_items(const Layout &L) {
         const int32_t on[2] = {L.it_own[e], L.it_nbr[e]};
         std::memcpy(reinterpret_cast<char *>(f) + 16 * K - sizeof on, on, sizeof on);
         for (size_t k = 0; k < K; k++) std::memcpy(p + 64 * k, reinterpret_cast<const char *>(f) + 16 * k, 16);
+    }
+    return v;
+}
+
+// The stencil weights of k_stage's places, in pieces of 16 B.
+template <typename S>
+static std::vector<float4> pack_weights(const Layout &L) {
+    constexpr size_t kPer = 16 / sizeof(S), kPieces = (3 * kMaxSlots + kPer - 1) / kPer;
+    const size_t P = L.loc_cell.size(), N = (size_t)L.N;
+    std::vector<float4> v(P * kPieces);
+    for (size_t p = 0; p < P; p++) {
+        if (L.loc_cell[p] < 0) continue;
+        S w[kPer * kPieces] = {};
+        for (int q = 0; q < 3 * kMaxSlots; q++) w[q] = (S)L.st_w[(size_t)q * N + L.loc_cell[p]];
+        for (size_t k = 0; k < kPieces; k++) std::memcpy(&v[k * P + p], w + k * kPer, 16);
     }
     return v;
 }
@@ -157,45 +172,52 @@ __global__ __launch_bounds__(kBlock) void k_flux_border(DevMesh<S> m, DevParams 
     if (t >= m.n_border) return;
     const SideLoader<S, Rec1> ld{st_in, grad, Rec1{}, nullptr, 0, 0, 1, 0};
     S F[4];
-    item_flux<S>(m, prm, m.border0 + t, ld, prm.visc3_invgam, INFINITY, F);
+    item_flux<S>(m, prm, load_item<S>(m, m.border0 + t), ld, prm.visc3_invgam, INFINITY, F);
     const size_t nbd = (size_t)m.n_border;
 #pragma unroll
     for (int q = 0; q < 4; q++) m.bflux[q * nbd + t] = F[q];
 }
 
-// 6 waves per SIMD in FP32 and 4 in FP64, the most that hold without spills (77
-// and 127 VGPRs).
+// What a cell's update reads from global memory.
 template <typename S>
-constexpr int kFluxMinWaves = std::is_same<S, float>::value ? 6 : 4;
+struct CellIn {
+    CellFaces<S> faces;
+    RkIn<S> rk;
+    double force[3];
+};
+
+template <typename S, bool kAhead>
+__device__ __forceinline__ void load_rk(const DevMesh<S> &m, StageArgs sa, bool force, int i, const double4 *t0,
+                                        const Acc<S> *t1, const double *dtl, const double *fbody, CellIn<S> &in) {
+    in.rk = load_rk<S, kAhead>(m, sa, i, (size_t)i, t0, t1, dtl);
+    if (force)
+        for (int q = 0; q < 3; q++) in.force[q] = fbody[(size_t)q * m.N + i];
+}
+
+// Residual and RK stage of cell i; returns its error code.
+template <typename S, bool kAhead>
+__device__ __forceinline__ int cell_update(const DevMesh<S> &m, const DevParams &prm, StageArgs sa, const S *sF,
+                                           bool force, int i, const CellIn<S> &in, V4<S> *__restrict__ st_out,
+                                           double4 *__restrict__ t0, Acc<S> *__restrict__ t1,
+                                           double *__restrict__ dtl, double sq[4]) {
+    double R[4];
+    gather_residual<S, kAhead>(m, i, in.faces, sF, m.max_items, 1, 0, R);
+    if (force) {
+        R[1] += in.force[0];
+        R[2] += in.force[1];
+        R[3] += in.force[2];
+    }
+    return rk_update<S, kAhead>(m, prm, prm.visc, sa, i, (size_t)i, in.rk, R, st_out, t0, t1, dtl, sq);
+}
 
 template <typename S>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kFluxMinWaves<S>))) void k_flux_update(
-    DevMesh<S> m, DevParams prm, StageArgs sa, const Ctrl *__restrict__ ctrl, const V4<S> *__restrict__ st_in,
-    const V4<S> *__restrict__ grad, V4<S> *__restrict__ st_out, double4 *__restrict__ t0, Acc<S> *__restrict__ t1,
-    double *__restrict__ dtl, const double *__restrict__ fbody, double *__restrict__ partials) {
-    extern __shared__ double lds[];
-    if (ctrl->done) return;
-    const int N = m.N;
-    const int blk = xcd_block(blockIdx.x, gridDim.x, m.xcd_remap);
-    const int nslot = m.max_items;
-    const S *sF = reinterpret_cast<const S *>(lds);
-    block_fluxes<S>(m, prm, st_in, grad, lds, blk);
-    __syncthreads();
-    double sq[4] = {0, 0, 0, 0};
-    int err = 0;
-    const int c_end = min(N, (blk + 1) * m.block_cells);
-    for (int i = blk * m.block_cells + threadIdx.x; i < c_end; i += kBlock) {
-        double R[4];
-        gather_residual<S>(m, i, sF, nslot, 1, 0, R);
-        if (prm.use_body_force && (!m.blk_force || m.blk_force[blk])) {
-            R[1] += fbody[i];
-            R[2] += fbody[(size_t)N + i];
-            R[3] += fbody[2 * (size_t)N + i];
-        }
-        const int e = rk_update<S>(m, prm, prm.visc, sa, i, (size_t)i, R, st_out, t0, t1, dtl, sq);
-        if (e == 1) err = 1;
-        else if (e == 2 && err == 0) err = 2;
-    }
+__device__ __forceinline__ bool block_force(const DevMesh<S> &m, const DevParams &prm, int blk) {
+    return prm.use_body_force && (!m.blk_force || m.blk_force[blk]);
+}
+
+// Block blk's residual sums (last stage).
+__device__ __forceinline__ void block_sums(StageArgs sa, int blk, const double sq[4], int err,
+                                           double *__restrict__ partials) {
     if (sa.stage == 3) {
         __shared__ double red[kBlock / 64][5];
         const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -217,6 +239,128 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kFluxMin
             for (int c = 0; c < 5; c++) partials[(size_t)blk * 5 + c] = s[c];
         }
     }
+}
+
+// 6 waves per SIMD in FP32 and 4 in FP64, the most that hold without spills (77
+// and 127 VGPRs).
+template <typename S>
+constexpr int kFluxMinWaves = std::is_same<S, float>::value ? 6 : 4;
+
+template <typename S>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kFluxMinWaves<S>))) void k_flux_update(
+    DevMesh<S> m, DevParams prm, StageArgs sa, const Ctrl *__restrict__ ctrl, const V4<S> *__restrict__ st_in,
+    const V4<S> *__restrict__ grad, V4<S> *__restrict__ st_out, double4 *__restrict__ t0, Acc<S> *__restrict__ t1,
+    double *__restrict__ dtl, const double *__restrict__ fbody, double *__restrict__ partials) {
+    extern __shared__ double lds[];
+    if (ctrl->done) return;
+    const int blk = xcd_block(blockIdx.x, gridDim.x, m.xcd_remap);
+    const S *sF = reinterpret_cast<const S *>(lds);
+    block_fluxes<S>(m, prm, st_in, grad, lds, blk);
+    __syncthreads();
+    const bool force = block_force(m, prm, blk);
+    double sq[4] = {0, 0, 0, 0};
+    int err = 0;
+    const int c_end = min(m.N, (blk + 1) * m.block_cells);
+    for (int i = blk * m.block_cells + threadIdx.x; i < c_end; i += kBlock) {
+        constexpr bool kAhead = std::is_same<S, double>::value;
+        CellIn<S> in;
+        in.faces = load_faces<S>(m, i);
+        load_rk<S, kAhead>(m, sa, force, i, t0, t1, dtl, fbody, in);
+        const int e = cell_update<S, kAhead>(m, prm, sa, sF, force, i, in, st_out, t0, t1, dtl, sq);
+        if (e == 1) err = 1;
+        else if (e == 2 && err == 0) err = 2;
+    }
+    block_sums(sa, blk, sq, err, partials);
+}
+
+// One RK stage of a mesh of up to 1024 64-cell flux blocks: k_grad and k_flux_update in
+// one kernel, with the gradients of every cell that the block's items read computed
+// here, into LDS, by each block that reads them (some 160 for 64 hexes).  Such a mesh
+// is bound by latencies and not by work: a launch and a round through memory saved are
+// worth the repeated sums.  What depends on the block's and the thread's number alone
+// (places, neighbours, weights, the first item, the cell's update) is loaded at the
+// start, so that it arrives while the control block does; patches are read from LDS.
+// Step in FP64, two kernels / one / one with these loads at the start: 216 hexes 52.4 /
+// 46.0 / 35.5 us, 32k 89 / 67 / 51.5, 64k tets 106 / 107 / 83; FP32 59k hexes 102 / 86 / 82.
+// Of a launch's 8 us at 216 cells 1.3 are the first loads, 2.2 the gradients, 2 the fluxes, 2
+// the update: chains of dependent instructions at one wavefront a SIMD.
+template <typename S>
+__global__ __launch_bounds__(kBlock) void k_stage(DevMesh<S> m, DevParams prm, StageArgs sa,
+                                                  const Ctrl *__restrict__ ctrl, const V4<S> *__restrict__ st_in,
+                                                  V4<S> *__restrict__ st_out, double4 *__restrict__ t0,
+                                                  Acc<S> *__restrict__ t1, double *__restrict__ dtl,
+                                                  const double *__restrict__ fbody, double *__restrict__ partials) {
+    extern __shared__ double lds[];
+    const int done = ctrl->done;
+    const int blk = blockIdx.x;
+    const int e0 = m.blk_item_off[blk], e1 = m.blk_item_off[blk + 1];
+    const bool force = block_force(m, prm, blk);
+    S *sF = reinterpret_cast<S *>(lds);
+    float4 *rec = reinterpret_cast<float4 *>(reinterpret_cast<char *>(lds) + staged_offset<S>(m.max_items));
+    DevPatch *sP = reinterpret_cast<DevPatch *>(rec + kLocalRec<S> * m.max_local);
+    // a place's cell, neighbours and weights
+    constexpr int kPer = 16 / sizeof(S), kPieces = (3 * kMaxSlots + kPer - 1) / kPer;
+    int i = -1, nbr[kMaxSlots];
+    float4 w[kPieces];
+    auto place = [&](int k) {
+        const int p = blk * m.max_local + k;
+        i = k < m.max_local ? m.loc_cell[p] : -1;
+        if (k < m.max_local) {
+#pragma unroll
+            for (int s = 0; s < kMaxSlots; s++) nbr[s] = s < m.max_slots ? m.loc_nbr[s * m.n_places + p] : kNoNbr;
+#pragma unroll
+            for (int q = 0; q < kPieces; q++)
+                if (q * kPer < 3 * m.max_slots) w[q] = m.loc_w[(size_t)q * m.n_places + p];
+        }
+    };
+    place(threadIdx.x);
+    for (int k = threadIdx.x; k < m.n_patches; k += kBlock) sP[k] = m.patches[k];
+    const int e = e0 + threadIdx.x;
+    Item<S> it{};
+    uint32_t places = 0;
+    if (e < e1) {
+        it = load_item<S>(m, e);
+        places = m.it_loc[e];
+    }
+    const int c = blk * m.block_cells + threadIdx.x;
+    const bool live = (int)threadIdx.x < m.block_cells && c < m.N;
+    CellIn<S> in;
+    if (live) {
+        in.faces = load_faces<S, true>(m, c);
+        load_rk<S, true>(m, sa, force, c, t0, t1, dtl, fbody, in);
+    }
+    if (done) return;
+    __syncthreads();
+    DevMesh<S> ml = m;
+    ml.patches = sP;
+    for (int k = threadIdx.x; k < m.max_local; k += kBlock) {
+        if (k != (int)threadIdx.x) place(k);
+        if (i < 0) break;
+        S g[12];
+        const auto weight = [&](int s, int c) {
+            const int q = 3 * s + c;
+            S v[kPer];
+            __builtin_memcpy(v, &w[q / kPer], 16);
+            return v[q % kPer];
+        };
+        lsq_sums<S, kMaxSlots>(ml, i, nbr, kMaxSlots, weight, GlobalStates<S, Rec1>{st_in, Rec1{}}, g);
+        LocalLoader<S>::put(rec + kLocalRec<S> * k, st_in[i], g);
+    }
+    __syncthreads();
+    for (int f = e; f < e1; f += kBlock) {
+        if (f != e) {
+            it = load_item<S>(m, f);
+            places = m.it_loc[f];
+        }
+        S F[4];
+        item_flux<S>(ml, prm, it, LocalLoader<S>{rec, places}, prm.visc3_invgam, INFINITY, F);
+#pragma unroll
+        for (int q = 0; q < 4; q++) sF[q * m.max_items + (f - e0)] = F[q];
+    }
+    __syncthreads();
+    double sq[4] = {0, 0, 0, 0};
+    const int err = live ? cell_update<S, true>(m, prm, sa, sF, force, c, in, st_out, t0, t1, dtl, sq) : 0;
+    block_sums(sa, blk, sq, err, partials);
 }
 
 // Global minimum of the local time steps for the "min" and "talts" modes
@@ -364,7 +508,7 @@ __global__ __launch_bounds__(kBlock) void k_residual_only(DevMesh<S> m, DevParam
     const int c_end = min(N, (blk + 1) * m.block_cells);
     for (int i = blk * m.block_cells + threadIdx.x; i < c_end; i += kBlock) {
         double R[4];
-        gather_residual<S>(m, i, sF, nslot, 1, 0, R);
+        gather_residual<S>(m, i, load_faces<S>(m, i), sF, nslot, 1, 0, R);
         if (prm.use_body_force) {
             R[1] += fbody[i];
             R[2] += fbody[(size_t)N + i];
@@ -543,6 +687,15 @@ int create_ctx(const plbfs_mesh_view *mesh, const plbfs_params *params, const pl
         return fail(plbfs_fail(PLBFS_ERR_HIP, "events and host buffer"));
     const int N = L.N;
     c->bound_blocks = L.n_blocks;
+    // A stage in one kernel on meshes below 65,536 cells (blocks of 64 cells; larger blocks
+    // do not fit).  The repeated gradients grow with the mesh, and the gain falls: 59k hexes in
+    // FP64 118 -> 105 us a step, 64k tets 106 -> 83.
+    if (L.one_kernel && lds_cases == 1 && !stage) {
+        const size_t b = (c->f32 ? staged_offset<float>(L.max_items_per_block)
+                                 : staged_offset<double>(L.max_items_per_block)) +
+                         (size_t)L.max_local * 16 * (c->f32 ? kLocalRec<float> : kLocalRec<double>) + (size_t)n_patches * sizeof(DevPatch);
+        if (b <= kMaxStageLds) c->stage_lds = b;
+    }
     DevMesh<double> &d = c->dm;
     d.N = N;
     d.G = L.G;
@@ -591,6 +744,18 @@ int create_ctx(const plbfs_mesh_view *mesh, const plbfs_params *params, const pl
                         return (uint16_t)((e >> 2) << 1 | (e & 1));
                     }));
     if (rc) return fail(rc);
+    d.max_local = L.max_local;
+    d.n_places = L.n_blocks * L.max_local;
+    d.n_patches = n_patches;
+    d.loc_cell = d.loc_nbr = nullptr;
+    d.it_loc = nullptr;
+    d.loc_w = nullptr;
+    if (c->stage_lds && ((rc = upload(c, (int32_t **)&d.loc_cell, L.loc_cell)) ||
+                         (rc = upload(c, (int32_t **)&d.loc_nbr, L.loc_nbr)) ||
+                         (rc = upload(c, (float4 **)&d.loc_w,
+                                      c->f32 ? pack_weights<float>(L) : pack_weights<double>(L))) ||
+                         (rc = upload(c, (uint32_t **)&d.it_loc, L.it_loc))))
+        return fail(rc);
     std::vector<int32_t> bpatch = L.b_patch;
     if (bpatch.empty()) bpatch.push_back(0);
     std::vector<int32_t> bpartner = L.b_partner;
@@ -633,6 +798,8 @@ int create_ctx(const plbfs_mesh_view *mesh, const plbfs_params *params, const pl
         e.blk_item_off = d.blk_item_off; e.it_p = d.it_p; e.it_side = d.it_side; e.it_dt = nullptr;
         e.g_ent = d.g_ent; e.g_ent_split = d.g_ent_split; e.max_ent = d.max_ent; e.b_patch = d.b_patch; e.b_partner = d.b_partner;
         e.b_fix = (const float4 *)c->b_fix;
+        e.loc_cell = d.loc_cell; e.loc_nbr = d.loc_nbr; e.loc_w = d.loc_w; e.it_loc = d.it_loc;
+        e.max_local = d.max_local; e.n_places = d.n_places; e.n_patches = d.n_patches;
         auto to32 = [](const std::vector<double> &v) { return std::vector<float>(v.begin(), v.end()); };
         std::vector<DevPatch> dp32 = dp;
         for (auto &q : dp32) q.rho -= p.ref_rho;
@@ -840,6 +1007,14 @@ static void launch_stages(plbfs_ctx *c, const DevMesh<S> &dm, const RunScratch &
     const int nb = c->L.n_blocks;
     void *in = c->stA, *outb = c->stB;
     for (int k = 0; k < 4; k++) {
+        if (c->stage_lds && !timed) {
+            const StageArgs sa{kAlpha[k], kBeta[k], k};
+            hipLaunchKernelGGL(k_stage<S>, dim3(nb), dim3(kBlock), c->stage_lds, c->stream, dm, c->prm, sa, w.ctrl,
+                               (const V4<S> *)in, (V4<S> *)outb, (double4 *)c->t0, (Acc<S> *)c->t1, c->dtl, c->fbody,
+                               w.partials);
+            std::swap(in, outb);
+            continue;
+        }
         {
             TimedLaunch t(c, PLBFS_KSTAT_GRAD, timed);
             hipLaunchKernelGGL(k_grad<S>, dim3(c->cell_grid), dim3(kBlock), 0, c->stream, dm, w.ctrl, (const V4<S> *)in,

@@ -99,15 +99,10 @@ struct StagedStates {
 // launch, whatever the number of cells; 221k hexes in FP32 15.8 -> 13.1 us).  FP64
 // takes one slot at a time: with two it holds 4 instead of 6 wavefronts per SIMD,
 // and 384k tets take 23.0 instead of 20.3 us.
-template <typename S, typename ST>
-__device__ __forceinline__ void lsq_grad(const DevMesh<S> &m, int i, const ST &state, S g[12]) {
-    constexpr int kSlots = std::is_same<S, float>::value ? 3 : 1;
-    const int N = m.N;
-    int nbr[kMaxSlots];
-#pragma unroll
-    for (int s = 0; s < kMaxSlots; s++)
-        if (s < m.max_slots) nbr[s] = m.st_nbr[(size_t)s * N + i];
-    const int cnt = m.st_cnt[i];
+template <typename S, int kSlots, typename ST, typename W>
+__device__ __forceinline__ void lsq_sums(const DevMesh<S> &m, int i, const int nbr[kMaxSlots], int cnt,
+                                         const W &weight, const ST &state, S g[12]) {
+    const auto none = [&](int s) { return kSlots == kMaxSlots && nbr[s] == kNoNbr; };
     const V4<S> q0 = state(i);
     const S p0[4] = {q0.x, q0.y, q0.z, q0.w};
 #pragma unroll
@@ -117,6 +112,7 @@ __device__ __forceinline__ void lsq_grad(const DevMesh<S> &m, int i, const ST &s
         if (s0 >= m.max_slots) break;
         V4<S> qj[kSlots];
         S w[kSlots][3];
+        int pb[kSlots];
 #pragma unroll
         for (int u = 0; u < kSlots; u++) {
             const int s = s0 + u;
@@ -124,16 +120,17 @@ __device__ __forceinline__ void lsq_grad(const DevMesh<S> &m, int i, const ST &s
             // (periodic ghosts were replaced by their partner cell in st_nbr)
             qj[u] = state(nbr[s] >= 0 ? nbr[s] : i);
 #pragma unroll
-            for (int c = 0; c < 3; c++) w[u][c] = m.st_w[((size_t)s * 3 + c) * N + i];
+            for (int c = 0; c < 3; c++) w[u][c] = weight(s, c);
+            if constexpr (kSlots == kMaxSlots) pb[u] = m.b_patch[nbr[s] < 0 && !none(s) ? -1 - nbr[s] : 0];
         }
 #pragma unroll
         for (int u = 0; u < kSlots; u++) {
             const int s = s0 + u;
             if (s >= kMaxSlots || s >= m.max_slots) continue;
             S pj[4] = {qj[u].x, qj[u].y, qj[u].z, qj[u].w};
-            if (nbr[s] < 0) {
+            if (nbr[s] < 0 && !none(s)) {
                 const int b = -1 - nbr[s];
-                const DevPatch P = m.patches[m.b_patch[b]];
+                const DevPatch P = m.patches[kSlots == kMaxSlots ? pb[u] : m.b_patch[b]];
                 S fx[4] = {0, 0, 0, 0};
                 if (P.flags & kGhostFixed) {
                     const V4<S> f = m.b_fix[b];
@@ -141,7 +138,7 @@ __device__ __forceinline__ void lsq_grad(const DevMesh<S> &m, int i, const ST &s
                 }
                 ghost_state<S>(P, p0, p0, fx, pj);
             }
-            if (s < cnt) {
+            if (s < cnt && !none(s)) {
 #pragma unroll
                 for (int q = 0; q < 4; q++) {
                     const S d = pj[q] - p0[q];
@@ -152,6 +149,16 @@ __device__ __forceinline__ void lsq_grad(const DevMesh<S> &m, int i, const ST &s
             }
         }
     }
+}
+
+template <typename S, typename ST>
+__device__ __forceinline__ void lsq_grad(const DevMesh<S> &m, int i, const ST &state, S g[12]) {
+    int nbr[kMaxSlots];
+#pragma unroll
+    for (int s = 0; s < kMaxSlots; s++)
+        if (s < m.max_slots) nbr[s] = m.st_nbr[(size_t)s * m.N + i];
+    const auto weight = [&](int s, int c) { return m.st_w[((size_t)s * 3 + c) * m.N + i]; };
+    lsq_sums<S, std::is_same<S, float>::value ? 3 : 1>(m, i, nbr, m.st_cnt[i], weight, state, g);
 }
 
 template <typename S>
@@ -193,6 +200,43 @@ struct SideLoader {
             const V4<S> *gc = grad + kGradRec<S> * (size_t)c;
             unpack_side<S>(st[c], gc[0], gc[1], gc[2], p, g);
         }
+    }
+    __device__ __forceinline__ void sides(int o, int j, S po[4], S go[12], S pn[4], S gn[12]) const {
+        side(o, po, go);
+        side(j, pn, gn);
+    }
+};
+
+// The same from LDS, where the block holds the records of every cell its items read:
+// state and gradient, kLocalRec 16-byte pieces apart.  One piece more than a record
+// has, so that the records of a wavefront's lanes start in all banks and not in two.
+template <typename S>
+constexpr int kLocalRec = sizeof(S) + 1;
+
+template <typename S>
+struct LocalLoader {
+    const float4 *rec;
+    uint32_t places;  // of the item's two cells (DevMesh::it_loc)
+    static __device__ __forceinline__ void put(float4 *q, V4<S> st, const S g[12]) {
+        S v[16] = {st.x, st.y, st.z, st.w};
+#pragma unroll
+        for (int k = 0; k < 12; k++) v[4 + k] = g[k];
+#pragma unroll
+        for (unsigned k = 0; k < sizeof(S); k++) __builtin_memcpy(q + k, reinterpret_cast<const char *>(v) + 16 * k, 16);
+    }
+    __device__ __forceinline__ void side(unsigned k, S p[4], S g[12]) const {
+        const float4 *q = rec + kLocalRec<S> * k;
+        S v[16];
+#pragma unroll
+        for (unsigned k = 0; k < sizeof(S); k++) __builtin_memcpy(reinterpret_cast<char *>(v) + 16 * k, q + k, 16);
+#pragma unroll
+        for (int k = 0; k < 4; k++) p[k] = v[k];
+#pragma unroll
+        for (int k = 0; k < 12; k++) g[k] = v[4 + k];
+    }
+    __device__ __forceinline__ void sides(int, int, S po[4], S go[12], S pn[4], S gn[12]) const {
+        side(places & 0xffff, po, go);
+        side(places >> 16, pn, gn);
     }
 };
 
@@ -236,13 +280,19 @@ inline size_t flux_lds_bytes(int max_items, int block_cells, bool stage, int C =
 // dt: a batch stores the geometric 0.5 sqrt(A) and caps it per case with
 // 3 nu / (gamma fneq_min), the min the host applies for one case
 // (src/unstructured_mesh.cpp:979-983); a single case passes infinity.
-template <typename S, typename LD>
-__device__ __forceinline__ void item_flux(const DevMesh<S> &m, const DevParams &prm, int64_t e, const LD &ld,
-                                          double v3g, double dtcap, S F[4]) {
+template <typename S>
+struct Item {
     S geo[10];  // n A, owner offset, neighbour offset or n (each x, y, z), dt
     int2 on;
+    unsigned side;
+};
+
+template <typename S>
+__device__ __forceinline__ Item<S> load_item(const DevMesh<S> &m, int64_t e) {
+    Item<S> it;
+    S *geo = it.geo;
     const float4 *ip = m.it_p + ((e >> 6) * (64 * kItemChunks<S>) + (e & 63));
-    const unsigned side = m.it_side[e];
+    it.side = m.it_side[e];
     if constexpr (std::is_same<S, double>::value) {
         double2 q[kItemChunks<S>];
 #pragma unroll
@@ -250,14 +300,21 @@ __device__ __forceinline__ void item_flux(const DevMesh<S> &m, const DevParams &
         geo[0] = q[0].x; geo[1] = q[0].y; geo[2] = q[1].x; geo[3] = q[1].y; geo[4] = q[2].x;
         geo[5] = q[2].y; geo[6] = q[3].x; geo[7] = q[3].y; geo[8] = q[4].x;
         geo[9] = m.it_dt[e];
-        on = __builtin_bit_cast(int2, q[4].y);
+        it.on = __builtin_bit_cast(int2, q[4].y);
     } else {
         const float4 q0 = ip[0], q1 = ip[64], q2 = ip[128];
         geo[0] = q0.x; geo[1] = q0.y; geo[2] = q0.z; geo[3] = q0.w; geo[4] = q1.x;
         geo[5] = q1.y; geo[6] = q1.z; geo[7] = q1.w; geo[8] = q2.x; geo[9] = q2.y;
-        on = int2{__float_as_int(q2.z), __float_as_int(q2.w)};
+        it.on = int2{__float_as_int(q2.z), __float_as_int(q2.w)};
     }
-    const int o = on.x, nb = on.y;
+    return it;
+}
+
+template <typename S, typename LD>
+__device__ __forceinline__ void item_flux(const DevMesh<S> &m, const DevParams &prm, const Item<S> &it, const LD &ld,
+                                          double v3g, double dtcap, S F[4]) {
+    const S *geo = it.geo;
+    const int o = it.on.x, nb = it.on.y;
     const S dt = fmin(geo[9], (S)dtcap);
     // the neighbour's record; for a boundary face that of its ghost's partner cell,
     // where it has one (and any record, not used, where it has none)
@@ -267,8 +324,7 @@ __device__ __forceinline__ void item_flux(const DevMesh<S> &m, const DevParams &
         if (j < 0) j = o;
     }
     S po[4], go[12], pn[4], gN[12];
-    ld.side(o, po, go);
-    ld.side(j, pn, gN);
+    ld.sides(o, j, po, go, pn, gN);
     // both sides' states at the face centre, as of an interior face
     S pI[4], pN[4];
 #pragma unroll
@@ -316,7 +372,7 @@ __device__ __forceinline__ void item_flux(const DevMesh<S> &m, const DevParams &
     }
     const S p0[4] = {(pI[0] + pN[0]) * (S)0.5, (pI[1] + pN[1]) * (S)0.5, (pI[2] + pN[2]) * (S)0.5,
                      (pI[3] + pN[3]) * (S)0.5};
-    lattice_flux<std::is_same<S, float>::value, S>(geo, dt, (S)v3g, side, p0, pI, go, pN, gN, (S)prm.invgam,
+    lattice_flux<std::is_same<S, float>::value, S>(geo, dt, (S)v3g, it.side, p0, pI, go, pN, gN, (S)prm.invgam,
                                                    (S)prm.c45, (S)prm.c15, (S)prm.rho0, F);
 }
 
@@ -327,35 +383,64 @@ __device__ __forceinline__ void item_flux(const DevMesh<S> &m, const DevParams &
 // dependent load and 16 B a tet more: 4.1M tets 488 -> 474 us in FP64, 288 -> 277 in
 // FP32.
 template <typename S>
-__device__ __forceinline__ void gather_residual(const DevMesh<S> &m, int i, const S *sF, int stride, int C, int c,
-                                                double R[4], int B = 1, int b = 0) {
+struct CellFaces {
+    int ent[kMaxSlots];  // without split borders
+    double iv;
+    float corr[3];  // FP32 with kAhead
+};
+
+template <typename S, bool kAhead = std::is_same<S, double>::value>
+__device__ __forceinline__ CellFaces<S> load_faces(const DevMesh<S> &m, int i) {
     const size_t N = (size_t)m.N;
-    const double iv = m.inv_vol[i];
+    CellFaces<S> in;
+    in.iv = m.inv_vol[i];
+    if (m.n_border == 0) {
+#pragma unroll
+        for (int s = 0; s < kMaxSlots; s++)
+            if (s < m.max_ent) in.ent[s] = m.g_ent[s * N + i];
+    }
+    if constexpr (kAhead && std::is_same<S, float>::value) {
+#pragma unroll
+        for (int q = 0; q < 3; q++) in.corr[q] = m.corr[q * N + i];
+    }
+    return in;
+}
+
+// kAhead reads every slot before the first sum and holds them all: the flux kernel's FP32
+// registers would spill (276 -> 400 us), so it is for FP64 and for k_stage.
+template <typename S, bool kAhead = std::is_same<S, double>::value>
+__device__ __forceinline__ void gather_residual(const DevMesh<S> &m, int i, const CellFaces<S> &in, const S *sF,
+                                                int stride, int C, int c, double R[4], int B = 1, int b = 0) {
+    const size_t N = (size_t)m.N;
+    const double iv = in.iv;
     R[0] = R[1] = R[2] = R[3] = 0;
     auto add = [&](const S v[4], int own) {
-        if (own) {
+        const double w = flip_sign(iv, (unsigned)own, 0);
 #pragma unroll
-            for (int q = 0; q < 4; q++) R[q] = R[q] + (-(double)v[q] * iv);
-        } else {
-#pragma unroll
-            for (int q = 0; q < 4; q++) R[q] = R[q] + ((double)v[q] * iv);
-        }
+        for (int q = 0; q < 4; q++) R[q] = fma((double)v[q], w, R[q]);
     };
     auto slot = [&](int sl, S v[4]) {
 #pragma unroll
         for (int q = 0; q < 4; q++) v[q] = sF[q * stride + sl * C + c];
     };
     if (m.n_border == 0) {
-        int ent[kMaxSlots];
+        if constexpr (kAhead) {
+            // (no face: slot 0, not added)
+            S v[kMaxSlots][4];
 #pragma unroll
-        for (int s = 0; s < kMaxSlots; s++)
-            if (s < m.max_ent) ent[s] = m.g_ent[s * N + i];
+            for (int s = 0; s < kMaxSlots; s++)
+                if (s < m.max_ent) slot(in.ent[s] != kNoEnt ? in.ent[s] >> 1 : 0, v[s]);
 #pragma unroll
-        for (int s = 0; s < kMaxSlots; s++) {
-            if (s < m.max_ent && ent[s] != kNoEnt) {
-                S v[4];
-                slot(ent[s] >> 1, v);
-                add(v, ent[s] & 1);
+            for (int s = 0; s < kMaxSlots; s++)
+                if (s < m.max_ent && in.ent[s] != kNoEnt) add(v[s], in.ent[s] & 1);
+        } else {
+#pragma unroll
+            for (int s = 0; s < kMaxSlots; s++) {
+                if (s < m.max_ent && in.ent[s] != kNoEnt) {
+                    S v[4];
+                    slot(in.ent[s] >> 1, v);
+                    add(v, in.ent[s] & 1);
+                }
             }
         }
     } else {
@@ -377,9 +462,8 @@ __device__ __forceinline__ void gather_residual(const DevMesh<S> &m, int i, cons
     }
     if constexpr (std::is_same<S, float>::value) {
         // rho0/3 sum(+-n A)/V of the cell, omitted from the single-precision face fluxes
-        R[1] += (double)m.corr[i];
-        R[2] += (double)m.corr[N + i];
-        R[3] += (double)m.corr[2 * N + i];
+#pragma unroll
+        for (int q = 0; q < 3; q++) R[1 + q] += (double)(kAhead ? in.corr[q] : m.corr[q * N + i]);
     }
 }
 
@@ -388,13 +472,35 @@ __device__ __forceinline__ void gather_residual(const DevMesh<S> &m, int i, cons
 // new primitive solution, t0 and the next local time step, adds R^2 to sq and
 // returns 1 for NaN or 2 for rho blow-up (src/Solver.cpp:448-493).
 template <typename S>
+struct RkIn {
+    double dt;
+    double4 t0;
+    Acc<S> t1;             // behind the first stage
+    double cfl_area, vol;  // last stage, with kAhead
+};
+
+template <typename S, bool kAhead = false>
+__device__ __forceinline__ RkIn<S> load_rk(const DevMesh<S> &m, StageArgs sa, int i, size_t r, const double4 *t0,
+                                           const Acc<S> *t1, const double *dtl) {
+    RkIn<S> in;
+    in.dt = dtl[r];
+    in.t0 = t0[r];
+    if (sa.stage != 0) in.t1 = t1[r];
+    if (kAhead && sa.stage == 3) {
+        in.cfl_area = m.cfl_area[i];
+        in.vol = m.vol[i];
+    }
+    return in;
+}
+
+template <typename S, bool kAhead = false>
 __device__ __forceinline__ int rk_update(const DevMesh<S> &m, const DevParams &prm, double visc, StageArgs sa,
-                                         int i, size_t r, const double R[4], V4<S> *__restrict__ st_out,
-                                         double4 *__restrict__ t0, Acc<S> *__restrict__ t1,
-                                         double *__restrict__ dtl, double sq[4]) {
+                                         int i, size_t r, const RkIn<S> &in, const double R[4],
+                                         V4<S> *__restrict__ st_out, double4 *__restrict__ t0,
+                                         Acc<S> *__restrict__ t1, double *__restrict__ dtl, double sq[4]) {
     constexpr bool F32 = std::is_same<S, float>::value;
-    const double dti = dtl[r];
-    const double4 ta = t0[r];
+    const double dti = in.dt;
+    const double4 ta = in.t0;
     const double a0 = ta.x, a1 = ta.y, a2 = ta.z, a3 = ta.w;
     // Solver.cpp:412-416
     double f1 = a0 + R[0] * dti * sa.alpha;
@@ -411,7 +517,7 @@ __device__ __forceinline__ int rk_update(const DevMesh<S> &m, const DevParams &p
         if (sa.stage == 0) {
             b0 = a0; b1 = a1; b2 = a2; b3 = a3;
         } else {
-            const Acc<S> tb = t1[r];
+            const Acc<S> tb = in.t1;
             b0 = tb.x; b1 = tb.y; b2 = tb.z; b3 = tb.w;
         }
         b0 = b0 + db * R[0];
@@ -422,7 +528,7 @@ __device__ __forceinline__ int rk_update(const DevMesh<S> &m, const DevParams &p
         // increments only; the conservative state is t0 + increments
         double d0 = 0, d1 = 0, d2 = 0, d3 = 0;
         if (sa.stage != 0) {
-            const Acc<S> tb = t1[r];
+            const Acc<S> tb = in.t1;
             d0 = tb.x; d1 = tb.y; d2 = tb.z; d3 = tb.w;
         }
         d0 += db * R[0];
@@ -447,7 +553,8 @@ __device__ __forceinline__ int rk_update(const DevMesh<S> &m, const DevParams &p
     st_out[r] = V4<S>{(S)(s0 - r0), (S)s1, (S)s2, (S)s3};
     t0[r] = double4{b0, b1, b2, b3};
     if (prm.time_stepping == PLBFS_DT_CONSTANT) dtl[r] = prm.cfl;
-    else dtl[r] = local_dt(prm, visc, s0, s1, m.cfl_area[i], m.vol[i]);
+    else dtl[r] = local_dt(prm, visc, s0, s1, kAhead ? in.cfl_area : m.cfl_area[i],
+                           kAhead ? in.vol : m.vol[i]);
     sq[0] += R[0] * R[0];
     sq[1] += R[1] * R[1];
     sq[2] += R[2] * R[2];

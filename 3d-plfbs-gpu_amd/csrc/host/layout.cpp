@@ -120,7 +120,8 @@ struct NearestCell {
 // a block takes its time whatever the others do: a pass of its 256 threads over its face
 // items at a time and then its cells, some 10 us for 64 cells of one pass, 20 for 256.
 //   - fewer 256-cell blocks than the 256 CUs: 64 cells.  Step in FP64, us, with 64 / 192 /
-//     256 cells: 216 hexes 62 / 82 / 82, 16k 94 / 118 / 131, 32k 101 / 116 / 120.
+//     256 cells and two kernels a stage: 216 hexes 62 / 82 / 82, 16k 94 / 118 / 131, 32k 101 /
+//     116 / 120.
 //   - up to 16 of them a CU: the size whose passes are full and that gives every CU the
 //     same number of blocks, by the estimate below.  221k hexes, 208 / 216 / 224 / 256
 //     cells (1064 / 1024 / 988 / 864 blocks of 754 / 782 / 809 / 919 items): flux 40.8 / 35.1 /
@@ -130,7 +131,7 @@ struct NearestCell {
 static int auto_block_cells(const plbfs_mesh_view &m, const std::vector<int32_t> &inv) {
     constexpr int kCus = 256, kThreads = 256;
     const int64_t N = m.n_cells;
-    if (N < (int64_t)kCus * 256) return 64;
+    if (N < (int64_t)kCus * 256) return kOneKernelCells;
     if (N > (int64_t)16 * kCus * 256) return 256;
     int64_t cut = 0;  // faces between two 256-cell blocks; their number goes with the blocks' surface
     for (int f = 0; f < m.n_internal_faces; f++) cut += inv[m.owner[f]] / 256 != inv[m.neighbour[f]] / 256;
@@ -511,6 +512,40 @@ int build_layout(const plbfs_mesh_view &m, const plbfs_params &p, const plbfs_pa
         g[9] = cc[3 * nb + 1] - fc[3 * f + 1];
         g[10] = cc[3 * nb + 2] - fc[3 * f + 2];
         for (int q = 0; q < kGeoPerItem; q++) L.it_geo[(size_t)q * E + e] = g[q];
+    }
+    // cells that each block reads
+    L.one_kernel = block_cells == 0 && C == kOneKernelCells && !split_border;
+    if (L.one_kernel) {
+        std::vector<std::vector<int32_t>> cells(L.n_blocks);
+        std::vector<int32_t> place(N, -1), of(N, -1);  // a cell's place in block of[cell]'s list
+        L.it_loc.resize(E);
+        for (int blk = 0; blk < L.n_blocks; blk++) {
+            auto add = [&](int cell) {
+                if (of[cell] != blk) {
+                    of[cell] = blk;
+                    place[cell] = (int)cells[blk].size();
+                    cells[blk].push_back(cell);
+                }
+                return (uint32_t)place[cell];
+            };
+            for (int i = blk * C; i < std::min(N, (blk + 1) * C); i++) add(i);
+            for (int e = L.blk_item_off[blk]; e < L.blk_item_off[blk + 1]; e++) {
+                const int nb = L.it_nbr[e], partner = nb < 0 ? L.b_partner[-1 - nb] : nb;
+                const uint32_t o = add(L.it_own[e]);
+                L.it_loc[e] = o | (partner < 0 ? o : add(partner)) << 16;
+            }
+            L.max_local = std::max(L.max_local, (int)cells[blk].size());
+        }
+        const size_t P = (size_t)L.n_blocks * L.max_local;
+        L.loc_cell.assign(P, -1);
+        L.loc_nbr.assign(P * kMaxSlots, kNoNbr);
+        for (int blk = 0; blk < L.n_blocks; blk++)
+            for (size_t k = 0; k < cells[blk].size(); k++) {
+                const size_t p = (size_t)blk * L.max_local + k;
+                L.loc_cell[p] = cells[blk][k];
+                for (int s = 0; s < L.st_cnt[cells[blk][k]]; s++)
+                    L.loc_nbr[s * P + p] = L.st_nbr[(size_t)s * N + cells[blk][k]];
+            }
     }
     return PLBFS_OK;
 }

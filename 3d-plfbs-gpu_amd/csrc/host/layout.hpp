@@ -23,6 +23,8 @@
 namespace plbfs {
 
 constexpr int kMaxSlots = 6;  // LSQ slots per cell (the reference's RHS arrays hold 6, gradients.cpp)
+constexpr int32_t kNoNbr = INT32_MIN;  // no stencil neighbour (Layout::loc_nbr)
+constexpr int kOneKernelCells = 64;  // flux block of a mesh below 65,536 cells
 constexpr int kMinAutoBlock = 176;  // smallest flux block that build_layout picks for a mesh of 65,536 cells or more
 constexpr int kGeoPerItem = 11;  // n(3), area, dt, r_owner(3), r_neighbour(3)
 
@@ -59,6 +61,14 @@ struct Layout {
     std::vector<uint32_t> it_side;
     std::vector<double> it_geo;  // [kGeoPerItem*E], component-major
     double b0[3] = {0, 0, 0};    // boundary face 0: its ghost's centroid from the face centre
+    // cells that a block's items read (one_kernel), in a list of max_local places per block: its
+    // own cells first, -1 behind the last.  loc_nbr holds the places' st_nbr, slot by slot for all
+    // lists, and it_loc the places of an item's owner and of its neighbour (a boundary face: its
+    // ghost's partner cell, or the owner) as two 16-bit values
+    bool one_kernel = false;
+    int max_local = 0;
+    std::vector<int32_t> loc_cell, loc_nbr;
+    std::vector<uint32_t> it_loc;
     // per-cell gather list in file face order, entries (index << 2) | border << 1 | is_owner:
     // index is the block-local slot, or with the border bit the border item's index
     std::vector<int32_t> g_off;  // [N+1]
@@ -89,7 +99,9 @@ inline bool rho_keeps_ghost(int t) { return t == 4 || t == 5 || t == 9; }
 inline bool vel_keeps_ghost(int t) { return t == 4 || t == 5 || t == 7 || t == 9; }
 
 // Builds the layout, with flux blocks of block_cells cells (a multiple of 64) or, for 0, of a
-// size that suits the mesh.  Returns PLBFS_OK or an error code (message via plbfs_fail).
+// size that suits the mesh; where that is kOneKernelCells cells, also the lists of the cells that
+// each block reads, for the stage kernel that computes their gradients itself.  Returns PLBFS_OK
+// or an error code (message via plbfs_fail).
 int build_layout(const plbfs_mesh_view &m, const plbfs_params &p, const plbfs_patch *patches, int n_patches,
                  const int32_t *bface_patch, int block_cells, bool split_border, Layout &L);
 

@@ -7,7 +7,8 @@ to the field's max magnitude); fields after 100 steps to 1e-10 relative
 import numpy as np
 import pytest
 
-from helpers import cavity_mesh, channel_mesh, initial_state, oracle_for, perturbed_state, rel_err
+from helpers import (cavity_mesh, channel_mesh, initial_state, oracle_for, periodic_z_case, periodic_z_mesh,
+                     perturbed_state, rel_err)
 from plbfs import _native as nat
 from plbfs import case as pc
 from plbfs.solver import GpuSolver, HostMesh
@@ -348,3 +349,44 @@ def test_chosen_flux_block_size_changes_no_field(gpu_available, monkeypatch, dim
         s.close()
     for a, b in zip(*out):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("dims,tets", [((2, 2, 2), False), ((4, 4, 4), False), ((5, 13, 2), False), ((7, 6, 5), True),
+                                       ((11, 10, 9), False)])
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("kind,stepping", [("periodic", "min"), ("channel", "local"), ("inlet", "constant")])
+def test_one_kernel_stage_equals_two_kernels(gpu_available, monkeypatch, dims, tets, precision, kind, stepping):
+    """The small meshes' stage kernel against the gradient and flux kernels on the same
+    flux blocks (asked for by size): same fields, residuals and time steps, bit for bit.
+    A few cells, one whole block, a block of two cells behind two, several blocks."""
+    if kind == "periodic":
+        if tets:
+            pytest.skip("partners are ambiguous on tets")
+        pm, case = periodic_z_mesh(*dims), periodic_z_case(float(dims[2]))
+    else:
+        pm, case = channel_mesh(*dims, tets=tets), pc.channel_case(re=40.0, length_scale=4.0, fneq_min=0.55)
+    if kind == "inlet":
+        for bc, types in zip(case.bcs.values(), (("inlet", "inlet"), ("dirichlet", "wall"), ("symmetry-x", "symmetry-x"))):
+            bc.update(vel_type=types[0], rho_type=types[1])
+    case.lsq_exact_det = 1 if tets else 0
+    case.precision = precision
+    case.time_stepping = stepping
+    if stepping == "constant":
+        case.cfl = 0.05
+    hm = HostMesh.from_polymesh(pm, case.visc, case.gamma, case.fneq_min)
+    g = hm.geometry()
+    n = pm.n_cells
+    rho, u, v, w = case.initial_state(g["cx"][:n], g["cy"][:n], g["cz"][:n])
+    st = (rho + 1e-3 * np.sin(g["cx"][:n]), u * (1 + 0.02 * np.cos(g["cy"][:n])), v, w + 1e-4 * np.sin(g["cz"][:n]))
+    out = []
+    for blk in ("", "64"):
+        if blk:
+            monkeypatch.setenv("PLBFS_BLOCK_CELLS", blk)
+        s = GpuSolver(hm, case.params, case.patches_for(pm.patch_names))
+        s.set_state(*st)
+        r = s.run(6)
+        out.append([r["rc"], r["hist"], s.dt_local()] + list(s.state()))
+        s.close()
+    assert out[0][0] == out[1][0]
+    for a, b in zip(out[0][1:], out[1][1:]):
+        assert np.array_equal(a, b, equal_nan=True)
