@@ -37,7 +37,6 @@ namespace {
 
 struct BatchArgs {
     int B, C;
-    int stage;              // 1: stage the tile's own (cell, case) records in LDS
     const double *visc;     // [B] nu
     const double *v3g;      // [B] 3 nu / gamma
     const double *dtcap;    // [B] streaming dt cap 3 nu / (gamma fneq_min), or infinity
@@ -51,20 +50,21 @@ struct CaseCtl {
     double *res;  // [B][4]
 };
 
+// Record numbers fit 32 bits: 2^32 records need more than the 288 GB of HBM.
 template <typename S>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(std::is_same<S, float>::value ? 6 : 4))) void kb_grad(
     DevMesh<S> m, BatchArgs a, const Ctrl *__restrict__ ctrl, const V4<S> *__restrict__ st,
     V4<S> *__restrict__ grad) {
     if (ctrl->done) return;
-    const int64_t idx = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    const int i = (int)(idx / a.B);
-    const int b = (int)(idx - (int64_t)i * a.B);
-    if (i >= m.N || a.done[b]) return;
+    const unsigned B = (unsigned)a.B;
+    const unsigned idx = (unsigned)xcd_block(blockIdx.x, gridDim.x, 1) * kBlock + threadIdx.x;
+    const unsigned i = idx / B, b = idx - i * B;
+    if (i >= (unsigned)m.N || a.done[b]) return;
     S g[12];
-    lsq_grad<S>(m, i, GlobalStates<S, RecB>{st, RecB{a.B, b}}, g);
+    lsq_grad<S>(m, (int)i, GlobalStates<S, RecB>{st, RecB{B, b}}, g);
     // the batch keeps the state apart from the gradients, [cell][3][B]: the
     // cases of a cell are contiguous in each store here and load in kb_flux
-    V4<S> *gi = grad + RecB{a.B, b}.grad(i);
+    V4<S> *gi = grad + RecB{B, b}.grad((int)i);
     gi[0] = V4<S>{g[0], g[1], g[2], g[3]};
     gi[a.B] = V4<S>{g[4], g[5], g[6], g[7]};
     gi[2 * a.B] = V4<S>{g[8], g[9], g[10], g[11]};
@@ -81,7 +81,7 @@ void kb_flux_border(DevMesh<S> m, DevParams prm, BatchArgs a, const Ctrl *__rest
     const int64_t k = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     const int j = (int)(k / a.B), b = (int)(k - (int64_t)j * a.B);
     if (j >= m.n_border || a.done[b]) return;
-    const SideLoader<S, RecB> ld{st_in, grad, RecB{a.B, b}, nullptr, 0, 0, 1, 0};
+    const SideLoader<S, RecB, false> ld{st_in, grad, RecB{(unsigned)a.B, (unsigned)b}, nullptr, 0, 0, 1, 0};
     S F[4];
     item_flux<S>(m, prm, load_item<S>(m, m.border0 + j), ld, a.v3g[b], a.dtcap[b], F);
     const size_t nbd = (size_t)m.n_border;
@@ -89,7 +89,7 @@ void kb_flux_border(DevMesh<S> m, DevParams prm, BatchArgs a, const Ctrl *__rest
     for (int q = 0; q < 4; q++) m.bflux[(q * nbd + j) * a.B + b] = F[q];
 }
 
-template <typename S>
+template <typename S, bool kStaged>
 __global__ __launch_bounds__(kBlock) void kb_flux(DevMesh<S> m, DevParams prm, BatchArgs a, StageArgs sa,
                                                   const Ctrl *__restrict__ ctrl, const V4<S> *__restrict__ st_in,
                                                   const V4<S> *__restrict__ grad, V4<S> *__restrict__ st_out,
@@ -99,7 +99,10 @@ __global__ __launch_bounds__(kBlock) void kb_flux(DevMesh<S> m, DevParams prm, B
     extern __shared__ double lds[];
     if (ctrl->done) return;
     const int N = m.N, B = a.B, C = a.C;
-    const int blk = blockIdx.x, b0 = blockIdx.y * C;
+    // consecutive flux blocks on one XCD, whose L2 then holds their common cells (of 128
+    // cases on 65k cells in FP32 fetched 1130 -> 950 MB a launch, kb_grad 364 -> 100 MB;
+    // step of 11 cases on 3.9k cells in FP64 142.6 -> 135.2 us, 24 on 65k 1157 -> 1131)
+    const int blk = xcd_block(blockIdx.x, gridDim.x, 1), b0 = blockIdx.y * C;
     const int e0 = m.blk_item_off[blk], e1 = m.blk_item_off[blk + 1];
     const int stride = m.max_items * C;
     S *sF = reinterpret_cast<S *>(lds);
@@ -107,7 +110,7 @@ __global__ __launch_bounds__(kBlock) void kb_flux(DevMesh<S> m, DevParams prm, B
     const int ncell = min(N, c0 + m.block_cells) - c0;
     V4<S> *sRec = nullptr;
     int nst = 0;
-    if (a.stage) {
+    if constexpr (kStaged) {
         sRec = reinterpret_cast<V4<S> *>(reinterpret_cast<char *>(lds) + staged_offset<S>(m.max_items, C));
         stage_records<S>(st_in, grad, B, b0, C, c0, ncell, sRec);
         nst = ncell;
@@ -120,7 +123,7 @@ __global__ __launch_bounds__(kBlock) void kb_flux(DevMesh<S> m, DevParams prm, B
     const bool live = b < B && !a.done[b];
     if (live) {
         const double v3g = a.v3g[b], dtcap = a.dtcap[b];
-        const SideLoader<S, RecB> ld{st_in, grad, RecB{B, b}, sRec, c0, nst, C, c};
+        const SideLoader<S, RecB, kStaged> ld{st_in, grad, RecB{(unsigned)B, (unsigned)b}, sRec, c0, nst, C, c};
         for (int el = threadIdx.x / C; el < e1 - e0; el += kBlock / C) {
             S F[4];
             item_flux<S>(m, prm, load_item<S>(m, e0 + el), ld, v3g, dtcap, F);
@@ -437,7 +440,7 @@ int retile(plbfs_batch *b, int block_cells, int C, int stage) {
 }
 
 BatchArgs args_of(plbfs_batch *b) {
-    return BatchArgs{b->B, b->C, b->stage, b->d_visc, b->d_v3g, b->d_dtcap, b->done, b->force_rec};
+    return BatchArgs{b->B, b->C, b->d_visc, b->d_v3g, b->d_dtcap, b->done, b->force_rec};
 }
 
 int ibm_upload(plbfs_batch *b) {
@@ -571,7 +574,7 @@ void launch_batch_stages(plbfs_batch *b, const DevMesh<S> &dm_base) {
         if (nbr > 0)
             hipLaunchKernelGGL(kb_flux_border<S>, dim3((unsigned)((nbr + kBlock - 1) / kBlock)), dim3(kBlock), 0,
                                c->stream, dm, prm, a, b->ctrl, (const V4<S> *)in, (const V4<S> *)b->grad);
-        hipLaunchKernelGGL(kb_flux<S>, fgrid, dim3(kBlock), c->lds_bytes, c->stream, dm, prm, a, sa, b->ctrl,
+        hipLaunchKernelGGL((b->stage ? kb_flux<S, true> : kb_flux<S, false>), fgrid, dim3(kBlock), c->lds_bytes, c->stream, dm, prm, a, sa, b->ctrl,
                            (const V4<S> *)in, (const V4<S> *)b->grad, (V4<S> *)out, (double4 *)b->t0,
                            (Acc<S> *)b->t1, b->dtl, b->fbody, b->partials);
         std::swap(in, out);

@@ -322,7 +322,7 @@ __device__ __forceinline__ void side_point(unsigned side, T dt, const T p[4], co
     h[P] = opaque(pop_eq<EX, EY, EZ, DEV, T>(p[0] + tau * d[0], p[1] + tau * d[1], p[2] + tau * d[2],
                                              p[3] + tau * d[3], s3, c45, c15, rho0));
     if constexpr (OUT) {
-        const bool both = (side >> (kPairs + P)) & 1u;
+        const bool both = (side & (1u << (kPairs + P))) != 0;
         if (__builtin_amdgcn_ballot_w64(both) != 0) {
             const T ho = pop_eq<EX, EY, EZ, DEV, T>(p[0] - tau * d[0], p[1] - tau * d[1], p[2] - tau * d[2],
                                                     p[3] - tau * d[3], -s3, c45, c15, rho0);
@@ -398,13 +398,14 @@ __device__ __forceinline__ void lattice_flux(const T nA[3], T dt, T v3g, unsigne
     const T om = (T)1 - tau;
     // sum e e^T feq(I) = rho_I (I/3 + u u^T/gamma); in DEV form rho0 I/3 is dropped
     const T iso = DEV ? s0 * (T)(1.0 / 3.0) : rI * (T)(1.0 / 3.0);
-    const T k = om * rI;
-    const T mxx = om * iso + k * (ux * ux * invgam) + tau * pxx;
-    const T myy = om * iso + k * (uy * uy * invgam) + tau * pyy;
-    const T mzz = om * iso + k * (uz * uz * invgam) + tau * pzz;
-    const T mxy = k * (ux * uy * invgam) + tau * pxy;
-    const T mxz = k * (ux * uz * invgam) + tau * pxz;
-    const T myz = k * (uy * uz * invgam) + tau * pyz;
+    const T k = om * rI * invgam, m0 = om * iso;
+    const T kx = k * ux, ky = k * uy, kz = k * uz;
+    const T mxx = m0 + tau * pxx + kx * ux;
+    const T myy = m0 + tau * pyy + ky * uy;
+    const T mzz = m0 + tau * pzz + kz * uz;
+    const T mxy = tau * pxy + kx * uy;
+    const T mxz = tau * pxz + kx * uz;
+    const T myz = tau * pyz + ky * uz;
     F[0] = sx * nA[0] + sy * nA[1] + sz * nA[2];
     F[1] = mxx * nA[0] + mxy * nA[1] + mxz * nA[2];
     F[2] = mxy * nA[0] + myy * nA[1] + myz * nA[2];

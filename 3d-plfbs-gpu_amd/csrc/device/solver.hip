@@ -43,15 +43,15 @@ constexpr int kFinalizeThreads = 256;
 // Fluxes of flux block blk's face items into their LDS slots, four arrays of
 // max_items; the caller's barrier follows.  With staging the block's own records
 // are first copied into LDS behind the slots.
-template <typename S>
+template <typename S, bool kStaged>
 __device__ __forceinline__ void block_fluxes(const DevMesh<S> &m, const DevParams &prm, const V4<S> *st,
                                              const V4<S> *grad, double *lds, int blk) {
     const int e0 = m.blk_item_off[blk], e1 = m.blk_item_off[blk + 1];
     const int nslot = m.max_items;
     S *sF = reinterpret_cast<S *>(lds);
     V4<S> *sRec = reinterpret_cast<V4<S> *>(reinterpret_cast<char *>(lds) + staged_offset<S>(m.max_items));
-    SideLoader<S, Rec1> ld{st, grad, Rec1{}, sRec, blk * m.block_cells, 0, 1, 0};
-    if (m.stage) {
+    SideLoader<S, Rec1, kStaged> ld{st, grad, Rec1{}, sRec, blk * m.block_cells, 0, 1, 0};
+    if constexpr (kStaged) {
         ld.nc = min(m.N, ld.c0 + m.block_cells) - ld.c0;
         stage_records<S>(st, grad, 0, 0, 1, ld.c0, ld.nc, sRec);
         __syncthreads();
@@ -170,7 +170,7 @@ __global__ __launch_bounds__(kBlock) void k_flux_border(DevMesh<S> m, DevParams 
     if (ctrl->done) return;
     const int t = blockIdx.x * kBlock + threadIdx.x;
     if (t >= m.n_border) return;
-    const SideLoader<S, Rec1> ld{st_in, grad, Rec1{}, nullptr, 0, 0, 1, 0};
+    const SideLoader<S, Rec1, false> ld{st_in, grad, Rec1{}, nullptr, 0, 0, 1, 0};
     S F[4];
     item_flux<S>(m, prm, load_item<S>(m, m.border0 + t), ld, prm.visc3_invgam, INFINITY, F);
     const size_t nbd = (size_t)m.n_border;
@@ -246,7 +246,7 @@ __device__ __forceinline__ void block_sums(StageArgs sa, int blk, const double s
 template <typename S>
 constexpr int kFluxMinWaves = std::is_same<S, float>::value ? 6 : 4;
 
-template <typename S>
+template <typename S, bool kStaged>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kFluxMinWaves<S>))) void k_flux_update(
     DevMesh<S> m, DevParams prm, StageArgs sa, const Ctrl *__restrict__ ctrl, const V4<S> *__restrict__ st_in,
     const V4<S> *__restrict__ grad, V4<S> *__restrict__ st_out, double4 *__restrict__ t0, Acc<S> *__restrict__ t1,
@@ -255,7 +255,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kFluxMin
     if (ctrl->done) return;
     const int blk = xcd_block(blockIdx.x, gridDim.x, m.xcd_remap);
     const S *sF = reinterpret_cast<const S *>(lds);
-    block_fluxes<S>(m, prm, st_in, grad, lds, blk);
+    block_fluxes<S, kStaged>(m, prm, st_in, grad, lds, blk);
     __syncthreads();
     const bool force = block_force(m, prm, blk);
     double sq[4] = {0, 0, 0, 0};
@@ -503,7 +503,8 @@ __global__ __launch_bounds__(kBlock) void k_residual_only(DevMesh<S> m, DevParam
     const int blk = xcd_block(blockIdx.x, gridDim.x, m.xcd_remap);
     const int nslot = m.max_items;
     const S *sF = reinterpret_cast<const S *>(lds);
-    block_fluxes<S>(m, prm, st_in, grad, lds, blk);
+    if (m.stage) block_fluxes<S, true>(m, prm, st_in, grad, lds, blk);
+    else block_fluxes<S, false>(m, prm, st_in, grad, lds, blk);
     __syncthreads();
     const int c_end = min(N, (blk + 1) * m.block_cells);
     for (int i = blk * m.block_cells + threadIdx.x; i < c_end; i += kBlock) {
@@ -1026,8 +1027,8 @@ static void launch_stages(plbfs_ctx *c, const DevMesh<S> &dm, const RunScratch &
             if (dm.n_border > 0)
                 hipLaunchKernelGGL(k_flux_border<S>, dim3((dm.n_border + kBlock - 1) / kBlock), dim3(kBlock), 0,
                                    c->stream, dm, c->prm, w.ctrl, (const V4<S> *)in, (const V4<S> *)c->grad);
-            hipLaunchKernelGGL(k_flux_update<S>, dim3(nb),
-                               dim3(kBlock), c->lds_bytes, c->stream, dm, c->prm, sa, w.ctrl, (const V4<S> *)in,
+            hipLaunchKernelGGL((dm.stage ? k_flux_update<S, true> : k_flux_update<S, false>), dim3(nb), dim3(kBlock),
+                               c->lds_bytes, c->stream, dm, c->prm, sa, w.ctrl, (const V4<S> *)in,
                                (const V4<S> *)c->grad, (V4<S> *)outb, (double4 *)c->t0, (Acc<S> *)c->t1, c->dtl,
                                c->fbody, w.partials);
         }

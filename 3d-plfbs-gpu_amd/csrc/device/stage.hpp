@@ -17,10 +17,10 @@ struct Rec1 {
     __device__ __forceinline__ size_t operator()(int c) const { return (size_t)c; }
 };
 struct RecB {
-    int B, b;
-    __device__ __forceinline__ size_t operator()(int c) const { return (size_t)c * B + b; }
+    unsigned B, b;  // unsigned: a product is one widening multiplication
+    __device__ __forceinline__ size_t operator()(int c) const { return (size_t)(unsigned)c * B + b; }
     // first of cell c's three gradient V4, B apart ([cell][3][B])
-    __device__ __forceinline__ size_t grad(int c) const { return (size_t)c * 3 * B + b; }
+    __device__ __forceinline__ size_t grad(int c) const { return (size_t)(unsigned)c * (3 * B) + b; }
 };
 
 // Per-cell RK accumulator between stages: the running sum t1 itself in FP64
@@ -172,12 +172,13 @@ __device__ __forceinline__ void unpack_side(V4<S> q, V4<S> a, V4<S> b, V4<S> d, 
     g[8] = d.x; g[9] = d.y; g[10] = d.z; g[11] = d.w;
 }
 
-// Where a face item reads a cell's state and gradient: cells of the block's own
-// range [c0, c0 + nc) from the copy the block staged in LDS (sRec: state, grad x3
-// per cell), every other cell from global memory.  With nc = 0 every read goes
-// to global memory.  The batch keeps the gradients as [cell][3][B], so that
+// Where a face item reads a cell's state and gradient: global memory, or with kStaged
+// for cells of the block's own range [c0, c0 + nc) the copy the block staged in LDS
+// (sRec: state, grad x3 per cell).  That choice is a branch a side, whose merge can
+// wait for the owner's loads before the neighbour's are issued, so kernels that do not
+// stage are built without it (flux of 4.1M tets in FP64 476 -> 439 us).  The batch keeps the gradients as [cell][3][B], so that
 // consecutive cases of a cell are contiguous in each of the four loads.
-template <typename S, typename R>
+template <typename S, typename R, bool kStaged>
 struct SideLoader {
     const V4<S> *__restrict__ st;
     const V4<S> *__restrict__ grad;
@@ -186,11 +187,15 @@ struct SideLoader {
     int c0, nc;
     int C, cl;  // cases staged per cell and this item's case lane (1, 0 for one case)
     __device__ __forceinline__ void side(int c, S p[4], S g[12]) const {
-        const unsigned rel = (unsigned)(c - c0);
-        if (rel < (unsigned)nc) {
-            const V4<S> *q = sRec + 4 * (rel * C + cl);
-            unpack_side<S>(opaque4(q[0]), opaque4(q[1]), opaque4(q[2]), opaque4(q[3]), p, g);
-        } else if constexpr (!std::is_same<R, Rec1>::value) {
+        if constexpr (kStaged) {
+            const unsigned rel = (unsigned)(c - c0);
+            if (rel < (unsigned)nc) {
+                const V4<S> *q = sRec + 4 * (rel * C + cl);
+                unpack_side<S>(opaque4(q[0]), opaque4(q[1]), opaque4(q[2]), opaque4(q[3]), p, g);
+                return;
+            }
+        }
+        if constexpr (!std::is_same<R, Rec1>::value) {
             const V4<S> *gc = grad + rec.grad(c);
             unpack_side<S>(st[rec(c)], gc[0], gc[rec.B], gc[2 * rec.B], p, g);
         } else if constexpr (kGradOff<S> == 1) {
@@ -253,7 +258,7 @@ __device__ __forceinline__ void stage_records(const V4<S> *__restrict__ st, cons
             if constexpr (kGradOff<S> == 1) sRec[k] = grad[kGradRec<S> * (size_t)(c0 + il) + q];
             else sRec[k] = q == 0 ? st[c0 + il] : grad[kGradRec<S> * (size_t)(c0 + il) + q - 1];
         } else if (b0 + cl < B) {
-            const RecB rb{B, b0 + cl};
+            const RecB rb{(unsigned)B, (unsigned)(b0 + cl)};
             sRec[k] = q == 0 ? st[rb(c0 + il)] : grad[rb.grad(c0 + il) + (size_t)(q - 1) * B];
         }
     }
@@ -288,10 +293,10 @@ struct Item {
 };
 
 template <typename S>
-__device__ __forceinline__ Item<S> load_item(const DevMesh<S> &m, int64_t e) {
+__device__ __forceinline__ Item<S> load_item(const DevMesh<S> &m, unsigned e) {
     Item<S> it;
     S *geo = it.geo;
-    const float4 *ip = m.it_p + ((e >> 6) * (64 * kItemChunks<S>) + (e & 63));
+    const float4 *ip = m.it_p + ((size_t)(e >> 6) * (64 * kItemChunks<S>) + (e & 63));
     it.side = m.it_side[e];
     if constexpr (std::is_same<S, double>::value) {
         double2 q[kItemChunks<S>];
@@ -325,12 +330,19 @@ __device__ __forceinline__ void item_flux(const DevMesh<S> &m, const DevParams &
     }
     S po[4], go[12], pn[4], gN[12];
     ld.sides(o, j, po, go, pn, gN);
-    // both sides' states at the face centre, as of an interior face
+    // both sides' states at the face centre, as of an interior face.  FP32, whose batch
+    // is bound by instructions, takes a chain of three (2% of a batch step); FP64 starts
+    // with the gradients, which arrive before the states (4.1M tets 458 -> 439 us).
     S pI[4], pN[4];
 #pragma unroll
     for (int q = 0; q < 4; q++) {
-        pI[q] = po[q] - (geo[3] * go[3 * q] + geo[4] * go[3 * q + 1] + geo[5] * go[3 * q + 2]);
-        pN[q] = pn[q] - (geo[6] * gN[3 * q] + geo[7] * gN[3 * q + 1] + geo[8] * gN[3 * q + 2]);
+        if constexpr (std::is_same<S, float>::value) {
+            pI[q] = po[q] - geo[3] * go[3 * q] - geo[4] * go[3 * q + 1] - geo[5] * go[3 * q + 2];
+            pN[q] = pn[q] - geo[6] * gN[3 * q] - geo[7] * gN[3 * q + 1] - geo[8] * gN[3 * q + 2];
+        } else {
+            pI[q] = po[q] - (geo[3] * go[3 * q] + geo[4] * go[3 * q + 1] + geo[5] * go[3 * q + 2]);
+            pN[q] = pn[q] - (geo[6] * gN[3 * q] + geo[7] * gN[3 * q + 1] + geo[8] * gN[3 * q + 2]);
+        }
     }
     if (nb < 0) {
         const int b = -1 - nb;
@@ -421,7 +433,7 @@ __device__ __forceinline__ void gather_residual(const DevMesh<S> &m, int i, cons
     };
     auto slot = [&](int sl, S v[4]) {
 #pragma unroll
-        for (int q = 0; q < 4; q++) v[q] = sF[q * stride + sl * C + c];
+        for (int q = 0; q < 4; q++) v[q] = sF[q * stride + (int)__umul24(sl, C) + c];
     };
     if (m.n_border == 0) {
         if constexpr (kAhead) {
