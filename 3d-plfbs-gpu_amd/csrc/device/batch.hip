@@ -14,8 +14,8 @@
 //             their slots in the reference face order and update.
 // After the fourth stage kb_finalize (one workgroup per case) reduces the
 // per-block partials in a fixed order into the case's residual and freezes a
-// converged or failed case; kb_alldone stops the replay once every case is
-// frozen.  One step is captured once as a hipGraph and replayed.
+// converged or failed case; its last workgroup stops the replay once every case is
+// frozen.  Steps are captured once as hipGraphs and replayed.
 //
 // Tiling (cells per flux block, cases per workgroup) is picked by
 // plbfs_batch_autotune from timed trial steps of the candidates that fit LDS.
@@ -89,8 +89,14 @@ void kb_flux_border(DevMesh<S> m, DevParams prm, BatchArgs a, const Ctrl *__rest
     for (int q = 0; q < 4; q++) m.bflux[(q * nbd + j) * a.B + b] = F[q];
 }
 
+// Threads of kb_flux: kBlock, or twice that where no CU gets two blocks; the second half
+// takes face items only, so the sums keep their order.  Step of 11 cases on 3.9k cells in
+// FP64 (183 blocks) 130 -> 105.5 us, 32 on 2.9k in FP32 (180) 137 -> 106; with several
+// blocks a CU, which fill each other's waits, it changes nothing (770 blocks: 223 and 224).
+constexpr int kMaxFluxThreads = 2 * kBlock;
+
 template <typename S, bool kStaged>
-__global__ __launch_bounds__(kBlock) void kb_flux(DevMesh<S> m, DevParams prm, BatchArgs a, StageArgs sa,
+__global__ __launch_bounds__(kMaxFluxThreads) void kb_flux(DevMesh<S> m, DevParams prm, BatchArgs a, StageArgs sa,
                                                   const Ctrl *__restrict__ ctrl, const V4<S> *__restrict__ st_in,
                                                   const V4<S> *__restrict__ grad, V4<S> *__restrict__ st_out,
                                                   double4 *__restrict__ t0, Acc<S> *__restrict__ t1,
@@ -116,15 +122,15 @@ __global__ __launch_bounds__(kBlock) void kb_flux(DevMesh<S> m, DevParams prm, B
         nst = ncell;
         __syncthreads();
     }
-    // kBlock is a multiple of C: thread t serves case lane c = t % C, items
-    // t / C, t / C + kBlock / C, ..., so its case's flags and viscosity are
+    // the block is a multiple of C: thread t serves case lane c = t % C, items
+    // t / C, t / C + blockDim / C, ..., so its case's flags and viscosity are
     // read once
     const int c = threadIdx.x % C, b = b0 + c;
     const bool live = b < B && !a.done[b];
     if (live) {
         const double v3g = a.v3g[b], dtcap = a.dtcap[b];
         const SideLoader<S, RecB, kStaged> ld{st_in, grad, RecB{(unsigned)B, (unsigned)b}, sRec, c0, nst, C, c};
-        for (int el = threadIdx.x / C; el < e1 - e0; el += kBlock / C) {
+        for (int el = threadIdx.x / C; el < e1 - e0; el += blockDim.x / C) {
             S F[4];
             item_flux<S>(m, prm, load_item<S>(m, e0 + el), ld, v3g, dtcap, F);
 #pragma unroll
@@ -136,7 +142,7 @@ __global__ __launch_bounds__(kBlock) void kb_flux(DevMesh<S> m, DevParams prm, B
     int err = 0;
     const size_t NR = (size_t)N * B;
     const double visc = live ? a.visc[b] : 0.0;
-    for (int il = threadIdx.x / C; live && il < ncell; il += kBlock / C) {
+    for (int il = threadIdx.x / C; live && threadIdx.x < kBlock && il < ncell; il += kBlock / C) {
         const int i = c0 + il;
         double R[4];
         gather_residual<S>(m, i, load_faces<S>(m, i), sF, stride, C, c, R, B, b);
@@ -153,9 +159,11 @@ __global__ __launch_bounds__(kBlock) void kb_flux(DevMesh<S> m, DevParams prm, B
     if (sa.stage == 3) {
         __syncthreads();  // the face slots are no longer read; reuse the LDS
         double *red = lds;
+        if (threadIdx.x < kBlock) {
 #pragma unroll
-        for (int q = 0; q < 4; q++) red[threadIdx.x * 5 + q] = sq[q];
-        red[threadIdx.x * 5 + 4] = (double)err;
+            for (int q = 0; q < 4; q++) red[threadIdx.x * 5 + q] = sq[q];
+            red[threadIdx.x * 5 + 4] = (double)err;
+        }
         __syncthreads();
         if ((int)threadIdx.x < C) {
             const int b = b0 + threadIdx.x;
@@ -173,14 +181,30 @@ __global__ __launch_bounds__(kBlock) void kb_flux(DevMesh<S> m, DevParams prm, B
 
 constexpr int kFinThreads = 256;
 
+// A case's block of kb_finalize at its end, with whether the case is done.  The last
+// of them counts the step and ends the run once no case is live.  The counter holds the
+// arrivals and, from bit 32, the cases that are done, so a block reads nothing that
+// another one wrote.  A kernel of its own for this took 4.5 us a step.
+__device__ __forceinline__ void case_arrived(Ctrl *ctrl, int B, bool done) {
+    const unsigned long long one = 1ull | (unsigned long long)done << 32;
+    const unsigned long long v = atomicAdd(&ctrl->arrived, one) + one;
+    if ((unsigned)v != gridDim.x) return;
+    __hip_atomic_store(&ctrl->arrived, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    ctrl->step = ctrl->step + 1;
+    if ((int)(v >> 32) == B) ctrl->done = 1;
+}
+
 // One workgroup per case: fixed-order sum of the block partials
 // (src/residuals.cpp:35-44,139-147) and the case's stop test.
 __global__ __launch_bounds__(kFinThreads) void kb_finalize(int nblk, int B, double n_cells, double ref_rho,
-                                                           double ref_mom, double tol, const Ctrl *__restrict__ ctrl,
+                                                           double ref_mom, double tol, Ctrl *__restrict__ ctrl,
                                                            CaseCtl cc, const double *__restrict__ partials) {
     if (ctrl->done) return;
     const int b = blockIdx.x;
-    if (cc.done[b]) return;
+    if (cc.done[b]) {
+        if (threadIdx.x == 0) case_arrived(ctrl, B, true);
+        return;
+    }
     __shared__ double red[kFinThreads][5];
     double s[5] = {0, 0, 0, 0, 0};
     // a thread's blocks k = tid, tid + T, ... in that order; four at a time
@@ -226,28 +250,13 @@ __global__ __launch_bounds__(kFinThreads) void kb_finalize(int nblk, int B, doub
             if (e == 1) cc.status[b] = PLBFS_ERR_NAN;
             else if (e == 2) cc.status[b] = PLBFS_ERR_RHO;
         }
-        if (cc.status[b] != PLBFS_OK) {
-            cc.done[b] = 1;
-        } else if (fmax(fmax(r[3], r[1]), r[2]) < tol) {
-            cc.converged[b] = 1;
+        const bool conv = fmax(fmax(r[3], r[1]), r[2]) < tol;
+        const bool done = cc.status[b] != PLBFS_OK || conv;
+        if (done) {
+            if (cc.status[b] == PLBFS_OK) cc.converged[b] = 1;
             cc.done[b] = 1;
         }
-    }
-}
-
-__global__ __launch_bounds__(kFinThreads) void kb_alldone(int B, Ctrl *__restrict__ ctrl,
-                                                          const int32_t *__restrict__ done) {
-    if (ctrl->done) return;
-    __shared__ int live;
-    if (threadIdx.x == 0) live = 0;
-    __syncthreads();
-    int mine = 0;
-    for (int b = threadIdx.x; b < B; b += kFinThreads) mine |= done[b] ? 0 : 1;
-    if (mine) live = 1;  // benign same-value race
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        ctrl->step = ctrl->step + 1;
-        if (!live) ctrl->done = 1;
+        case_arrived(ctrl, B, done);
     }
 }
 
@@ -562,6 +571,7 @@ void launch_batch_stages(plbfs_batch *b, const DevMesh<S> &dm_base) {
     const int64_t NR = (int64_t)b->N * b->B;
     const dim3 rgrid((unsigned)((NR + kBlock - 1) / kBlock));
     const dim3 fgrid(c->L.n_blocks, (b->B + b->C - 1) / b->C);
+    const dim3 fthreads(fgrid.x * fgrid.y <= kCus ? kMaxFluxThreads : kBlock);
     DevParams prm = c->prm;
     prm.use_body_force = b->ibm_on ? 1 : 0;
     static const double kAl[4] = {1.0, 0.5, 0.5, 1.0};
@@ -574,7 +584,7 @@ void launch_batch_stages(plbfs_batch *b, const DevMesh<S> &dm_base) {
         if (nbr > 0)
             hipLaunchKernelGGL(kb_flux_border<S>, dim3((unsigned)((nbr + kBlock - 1) / kBlock)), dim3(kBlock), 0,
                                c->stream, dm, prm, a, b->ctrl, (const V4<S> *)in, (const V4<S> *)b->grad);
-        hipLaunchKernelGGL((b->stage ? kb_flux<S, true> : kb_flux<S, false>), fgrid, dim3(kBlock), c->lds_bytes, c->stream, dm, prm, a, sa, b->ctrl,
+        hipLaunchKernelGGL((b->stage ? kb_flux<S, true> : kb_flux<S, false>), fgrid, fthreads, c->lds_bytes, c->stream, dm, prm, a, sa, b->ctrl,
                            (const V4<S> *)in, (const V4<S> *)b->grad, (V4<S> *)out, (double4 *)b->t0,
                            (Acc<S> *)b->t1, b->dtl, b->fbody, b->partials);
         std::swap(in, out);
@@ -594,7 +604,6 @@ int launch_batch_step(plbfs_batch *b) {
     CaseCtl cc{b->done, b->status, b->steps, b->conv, b->res};
     hipLaunchKernelGGL(kb_finalize, dim3(b->B), dim3(kFinThreads), 0, c->stream, c->L.n_blocks, b->B,
                        (double)b->N, c->prm.ref_rho, c->prm.ref_mom, c->prm.tol, b->ctrl, cc, b->partials);
-    hipLaunchKernelGGL(kb_alldone, dim3(1), dim3(kFinThreads), 0, c->stream, b->B, b->ctrl, b->done);
     HIP_TRY(hipGetLastError());
     return PLBFS_OK;
 }

@@ -38,6 +38,7 @@ struct Ctrl {
     int32_t step;    // steps completed in this run
     int32_t converged;
     int32_t rebuild;  // nonzero: an immersed node drifted half its list margin
+    unsigned long long arrived;  // blocks of the step's last kernel so far; 0 between kernels
     double res[4];
 };
 

@@ -297,3 +297,32 @@ def test_batch_immersed_nodes_on_fine_cells_equal_single_runs(gpu_available, pre
         assert r1["rc"] == 0
         for x, y in zip(bt.state(b), s1):
             assert np.array_equal(x, y)
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("cases_per_block", [1, 4])
+def test_flux_threads_on_few_blocks_change_nothing(gpu_available, precision, cases_per_block):
+    """256 flux blocks (twice the threads) against 320: the cases that both batches hold
+    agree in fields and residuals, bit for bit.  64 blocks of 64 hexes less one cell."""
+    pm = channel_mesh(13, 35, 9)
+    case = pc.channel_case(re=40.0, length_scale=4.0, fneq_min=0.55)
+    case.precision = precision
+    hm = HostMesh.from_polymesh(pm, 0.01, case.gamma, 0.0)
+    g = hm.geometry()
+    n = pm.n_cells
+    rho, u, v, w = case.initial_state(g["cx"][:n], g["cy"][:n], g["cz"][:n])
+    st = (rho + 1e-3 * np.sin(g["cx"][:n]), u * (1 + 0.02 * np.cos(g["cy"][:n])), v, w + 1e-4 * np.sin(g["cz"][:n]))
+    out = []
+    for cases in (4 * cases_per_block, 5 * cases_per_block):
+        b = GpuBatch(hm, case.params, case.patches_for(pm.patch_names), [0.02 + 0.003 * k for k in range(cases)])
+        b.set_tiling(64, cases_per_block, 0)
+        for k in range(cases):
+            b.set_state(k, *st)
+        rc, res = b.run(6)
+        assert rc == 0
+        out.append([(b.state(k), res[k]["residual"]) for k in range(4 * cases_per_block)])
+        b.close()
+    for (fa, ra), (fb, rb) in zip(*out):
+        assert ra == rb
+        for x, y in zip(fa, fb):
+            assert np.array_equal(x, y)
