@@ -383,16 +383,21 @@ __global__ __launch_bounds__(kBlock) void k_dt_blockmin(int N, const Ctrl *__res
     }
 }
 
+// Every block takes the minimum over all blocks' minima: by its whole width (by one
+// thread, one after the other, 6.4 us at 64 blocks; step of 16k cells 57 -> 52 us).
 __global__ __launch_bounds__(kBlock) void k_dt_apply(int N, int nblk, int mode, const Ctrl *__restrict__ ctrl,
                                                      const double *__restrict__ bmin, double *__restrict__ dtl) {
     if (ctrl->done) return;
-    __shared__ double smin;
-    if (threadIdx.x == 0) {
-        double s = 100000000000.0;
-        for (int q = 0; q < nblk; q++) s = (bmin[q] < s) ? bmin[q] : s;
-        smin = s;
-    }
+    __shared__ double red[kBlock / 64];
+    double s = 100000000000.0;
+    for (int q = threadIdx.x; q < nblk; q += kBlock) s = (bmin[q] < s) ? bmin[q] : s;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) s = fmin(s, __shfl_xor(s, off, 64));
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
     __syncthreads();
+    double smin = red[0];
+#pragma unroll
+    for (int q = 1; q < kBlock / 64; q++) smin = fmin(smin, red[q]);
     const int i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= N) return;
     const double mn = smin;

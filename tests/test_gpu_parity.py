@@ -390,3 +390,23 @@ def test_one_kernel_stage_equals_two_kernels(gpu_available, monkeypatch, dims, t
     assert out[0][0] == out[1][0]
     for a, b in zip(out[0][1:], out[1][1:]):
         assert np.array_equal(a, b, equal_nan=True)
+
+
+@pytest.mark.parametrize("dims", [(16, 16, 1), (17, 16, 1), (41, 40, 40)])
+def test_minimum_time_step_over_many_blocks(gpu_available, dims):
+    """The global minimum over 1, 2 and 257 blocks of 256 cells: every cell's step in
+    the "min" mode is the smallest of the local ones."""
+    pm, case = channel_mesh(*dims), pc.channel_case(re=40.0, length_scale=4.0)
+    hm = HostMesh.from_polymesh(pm, case.visc, case.gamma, case.fneq_min)
+    g = hm.geometry()
+    n = pm.n_cells
+    rho, u, v, w = case.initial_state(g["cx"][:n], g["cy"][:n], g["cz"][:n])
+    dt = []
+    for stepping in ("local", "min"):
+        case.time_stepping = stepping
+        s = GpuSolver(hm, case.params, case.patches_for(pm.patch_names))
+        s.set_state(rho, u * (1 + 0.5 * np.cos(g["cx"][:n])), v, w)
+        dt.append(s.dt_local())
+        s.close()
+    assert dt[0].max() > dt[0].min()
+    assert np.all(dt[1] == dt[0].min())
