@@ -60,9 +60,36 @@ __host__ __device__ __forceinline__ unsigned short to_bf16(float f) {
     return (unsigned short)(u >> 16);
 }
 
-__device__ __forceinline__ float silu(float a) { return a / (1.0f + expf(-a)); }
+// SiLU and its derivative: a sigmoid of finite values only, 1 + e^-a from the exponential
+// of the nearest power of two and the rest (its argument in two parts, log2 e = hi + lo), and
+// the quotients by reciprocal and one correction with the exact remainder, which
+// rounds them correctly.  expf and the division spend a third of their instructions on
+// ranges that do not occur here: a below -88 is taken as -88 (SiLU -5e-37 there and 0 below), NaN stays NaN.
+// Against 64 bits over [-85, 88] the errors are those of a / (1 + expf(-a)) (largest
+// 3.09, mean 0.27668, in 2^-24 of the result), and so are the network's outputs, bit
+// for bit.
+__device__ __forceinline__ float floor88(float a) { return a < -88.f ? -88.f : a; }
+__device__ __forceinline__ float one_plus_exp(float a) {
+#pragma clang fp contract(off)
+    const float x = -fminf(a, 88.f);
+    const float hi = 1.44269502f, lo = 1.92596299e-8f;
+    const float t = x * hi, n = rintf(t);
+    const float f = (t - n) + fmaf(x, lo, fmaf(x, hi, -t));
+    return 1.0f + ldexpf(__builtin_amdgcn_exp2f(f), (int)n);
+}
+__device__ __forceinline__ float quot(float a, float d, float r) {  // a / d, r = rcp(d)
+    const float q = a * r;
+    return fmaf(fmaf(-q, d, a), r, q);
+}
+__device__ __forceinline__ float silu(float a) {
+    a = floor88(a);
+    const float d = one_plus_exp(a);
+    return quot(a, d, __builtin_amdgcn_rcpf(d));
+}
 __device__ __forceinline__ float dsilu(float a) {
-    const float s = 1.0f / (1.0f + expf(-a));
+    a = floor88(a);
+    const float d = one_plus_exp(a), r = __builtin_amdgcn_rcpf(d);
+    const float s = fmaf(fmaf(-d, r, 1.0f), r, r);
     return s * (1.0f + a * (1.0f - s));
 }
 
@@ -73,8 +100,10 @@ constexpr int kTileNodes = 16;  // nodes of an edge tile
 constexpr int kPad = 8;         // bf16 elements behind every row of an LDS tile
 constexpr int kMaxParts = 512;  // blocks (weight-gradient partials) of a backward kernel: two a CU
 
+// Nearest even, two values an instruction; equal to to_bf16 for every finite value.
 __device__ __forceinline__ bf16x4 pack4(f32x4 v) {
-    return bf16x4{(short)to_bf16(v[0]), (short)to_bf16(v[1]), (short)to_bf16(v[2]), (short)to_bf16(v[3])};
+    typedef __bf16 b4 __attribute__((ext_vector_type(4)));
+    return __builtin_bit_cast(bf16x4, __builtin_convertvector(v, b4));
 }
 
 // Operand fragments of the 16x16x16 product D = A B, D(m, n): lane l holds
@@ -168,9 +197,10 @@ __device__ __forceinline__ f32x4 silu4(f32x4 a) { return f32x4{silu(a[0]), silu(
 // higher degree takes.  agg (training): the mean, rounded as the update uses it.
 // Bound by latency: a tile is a chain of dependent loads (node range, edge ends,
 // states) and short products.  A layer of the 221,184-cell hex mesh (1.3M edges)
-// takes 0.25 ms; gathering, two products, mean and update as kernels of their own
+// takes 0.227 ms (0.252 with expf, the IEEE division and integer rounding; four
+// wavefronts a SIMD, which the compiler would give up for instruction order); gathering, two products, mean and update as kernels of their own
 // took 2.1 ms, most of it on the edge rows' way through memory.
-__global__ __launch_bounds__(kT) void k_layer_fwd(int tiles, const int *__restrict__ tile_n0,
+__global__ __launch_bounds__(kT, 4) void k_layer_fwd(int tiles, const int *__restrict__ tile_n0,
                                                   const int *__restrict__ in_off, ZMsg zm,
                                                   const float *__restrict__ inv_deg, const float *__restrict__ h,
                                                   float *__restrict__ h_out, u16 *__restrict__ hb_out,
@@ -436,7 +466,7 @@ __global__ __launch_bounds__(kT, 2) void k_node_bwd(int rows, Z zs, DyNode dy, c
 // Backward of the message MLP over the tiles of k_layer_fwd: its gradient partials, the
 // source half of the input gradient per edge (dzs, summed by k_dh_out), and
 //   dh[t] += du[t, 0:64] + sum_{e in in(t)} dz[e, 0:64].
-// 383k edges: 0.176 ms with two blocks a CU (what the registers allow), 0.284 with
+// 383k edges: 0.167 ms with two blocks a CU (what the registers allow), 0.284 with
 // one.  The kernels that this one stands for took 4 ms, 3 of them in weight
 // gradients whose few blocks each walked 4096 rows.
 __global__ __launch_bounds__(kT, 2) void k_msg_bwd(int tiles, const int *__restrict__ tile_n0,

@@ -132,3 +132,30 @@ def test_edge_tiles_match_reference(gpu_available, n, degrees):
     infer = mpnn.Mpnn(n, src, dst, ef, train=False)
     infer.set_params(mpnn.flatten_params(P, shapes))
     assert np.array_equal(infer.forward(x), y)
+
+
+@pytest.mark.parametrize("scale", [1e3, 1e6, 1e30])
+def test_saturated_units_match_reference(gpu_available, scale):
+    """Inputs so large that the encoder's units lie far outside +-88 on both sides, at this
+    file's bar for outputs (1e30: finite), and one NaN: it reaches its cell's output and
+    no cell more than six edges away."""
+    N, src, dst, ef, x, _ = problem()
+    P = M.init_params(1)
+    net = mpnn.Mpnn(N, src, dst, ef, train=False)
+    net.set_params(mpnn.flatten_params(P, M.mlp_shapes()))
+    xs = (x * scale).astype(np.float32)
+    y = net.forward(xs)
+    G = M.Graph(src, dst, N)
+    with np.errstate(over="ignore"):
+        yr, _ = M.forward(P, G, xs.astype(np.float64), ef[G.order].astype(np.float64), bf16_mode=True)
+    assert np.isfinite(y).all()
+    assert rel(y[:, :4], yr[:, :4]) < 1e-2
+    x = x.copy()
+    x[0, 0] = np.nan
+    y = net.forward(x)
+    near = np.zeros(N, bool)
+    near[0] = True
+    for _ in range(6):
+        near[dst[near[src]]] = True
+    assert np.isnan(y[0, :4]).all()
+    assert np.isfinite(y[~near]).all()
