@@ -31,6 +31,7 @@ constexpr int kFluxBlockCells = 256;
 // flux kernels' static arrays take at most 160 B, and a launch whose total
 // exceeds 160 KiB is not refused by the runtime but faults, so 1 KiB stays free.
 constexpr unsigned kCus = 256;
+constexpr int kXcdCells = 12 * 65536;
 constexpr int kMaxLds = 159 * 1024;
 constexpr size_t kMaxStageLds = 64 * 1024;  // of k_stage: two blocks a CU
 }

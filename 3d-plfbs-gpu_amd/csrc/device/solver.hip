@@ -1,11 +1,12 @@
 // PLBFS solver on one MI355X (gfx950): kernels, context and the C-ABI of
 // include/plbfs_hip.h.
 //
-// Per RK stage two kernels run back to back on the context's stream:
+// Per RK stage two kernels run back to back on the context's stream, on meshes below
+// 65,536 cells one (k_stage) that does the work of both:
 //   k_grad         one thread per cell: least-squares gradients of rho,u,v,w
 //                  from the folded stencil weights (src/gradients.cpp:319-389);
 //                  ghost neighbours are evaluated from the owner and its patch.
-//   k_flux_update  one block per 256 Hilbert-consecutive cells: every face of the
+//   k_flux_update  one block per 64 to 256 Hilbert-consecutive cells: every face of the
 //                  block is evaluated once into an LDS slot (border faces by both
 //                  blocks), then each cell gathers its faces' slots in the
 //                  reference face order and applies the RK stage update
@@ -113,13 +114,13 @@ static std::vector<float4> pack_weights(const Layout &L) {
 }
 
 // Bound by HBM: a state read, the stencil (28 B a slot in FP64) and the record
-// written are 241 B a tet, 0.99 GB in 0.198 ms on 4.1M tets in FP64 (4.97 TB/s, where
+// written are 241 B a tet, 0.99 GB in 0.187 ms on 4.1M tets in FP64 (5.3 TB/s, where
 // a large copy reaches 4.75-5.1); 0.239 ms with each lane storing its own record.
 template <typename S>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) void k_grad(DevMesh<S> m, const Ctrl *__restrict__ ctrl,
                                                  const V4<S> *__restrict__ st, V4<S> *__restrict__ grad) {
     if (ctrl->done) return;
-    const int c0 = xcd_block(blockIdx.x, gridDim.x, m.xcd_remap) * kBlock;
+    const int c0 = xcd_block(blockIdx.x, gridDim.x, 1) * kBlock;
     const int i = c0 + threadIdx.x;
     S g[12];
     V4<S> si;
@@ -242,7 +243,7 @@ __device__ __forceinline__ void block_sums(StageArgs sa, int blk, const double s
 }
 
 // 6 waves per SIMD in FP32 and 4 in FP64, the most that hold without spills (77
-// and 127 VGPRs).
+// and 126 VGPRs).
 template <typename S>
 constexpr int kFluxMinWaves = std::is_same<S, float>::value ? 6 : 4;
 
@@ -292,7 +293,7 @@ __global__ __launch_bounds__(kBlock) void k_stage(DevMesh<S> m, DevParams prm, S
                                                   const double *__restrict__ fbody, double *__restrict__ partials) {
     extern __shared__ double lds[];
     const int done = ctrl->done;
-    const int blk = blockIdx.x;
+    const int blk = xcd_block(blockIdx.x, gridDim.x, 1);
     const int e0 = m.blk_item_off[blk], e1 = m.blk_item_off[blk + 1];
     const bool force = block_force(m, prm, blk);
     S *sF = reinterpret_cast<S *>(lds);
@@ -718,10 +719,16 @@ int create_ctx(const plbfs_mesh_view *mesh, const plbfs_params *params, const pl
     d.stage = stage ? 1 : 0;
     d.grad_stage = env_flag("PLBFS_GRAD_STAGE", true) ? 1 : 0;
     c->cell_grid = (N + kBlock - 1) / kBlock;
-    // measured on MI355X (4.09M tets): the XCD-contiguous remap is ~5% slower
-    // than plain dispatch order for the flux kernel, so it is opt-in
+    // Consecutive blocks on one XCD keep the cells that they share in its L2.  k_grad and
+    // k_stage always take that order (4.1M tets in FP32 125 -> 111 us a launch, 221k hexes in
+    // FP64 16.1 -> 15.4, with the records then written where flux blocks of the same XCD read
+    // them; step of 32k hexes 50.4 -> 47.4 us).  Flux blocks take it on meshes of up to
+    // kXcdCells cells: step of 221k hexes in FP64 201.9 -> 190.6 us, of 681k 565 -> 559, FP32
+    // 351.2 -> 349.4; 1.1M hexes in FP64 901 -> 925, 1.1M tets in FP32 475 -> 482 and 4.1M tets
+    // in FP64 2.54 -> 2.65 ms: what the blocks of one XCD stream through its L2 then
+    // drives the shared cells out.
     const char *nx = std::getenv("PLBFS_XCD_REMAP");
-    d.xcd_remap = (nx && nx[0] == '1') ? 1 : 0;
+    d.xcd_remap = nx && nx[0] ? nx[0] == '1' : N <= kXcdCells;
     std::vector<DevPatch> dp(n_patches);
     for (int q = 0; q < n_patches; q++) {
         dp[q].rho_type = patches[q].rho_type;

@@ -410,3 +410,25 @@ def test_minimum_time_step_over_many_blocks(gpu_available, dims):
         s.close()
     assert dt[0].max() > dt[0].min()
     assert np.all(dt[1] == dt[0].min())
+
+
+@pytest.mark.parametrize("dims", [(4, 4, 4), (8, 8, 9), (13, 12, 11), (41, 40, 41)])
+def test_block_order_over_the_xcds_changes_no_field(gpu_available, monkeypatch, dims):
+    """Contiguous ranges of blocks per XCD against dispatch order, on 1, 9, 27 and some 300
+    blocks (remainders of 8): the same fields, bit for bit."""
+    pm, case = channel_mesh(*dims), pc.channel_case(re=40.0, length_scale=4.0, fneq_min=0.55)
+    hm = HostMesh.from_polymesh(pm, case.visc, case.gamma, case.fneq_min)
+    g = hm.geometry()
+    n = pm.n_cells
+    rho, u, v, w = case.initial_state(g["cx"][:n], g["cy"][:n], g["cz"][:n])
+    out = []
+    for order in ("0", "1"):
+        monkeypatch.setenv("PLBFS_XCD_REMAP", order)
+        monkeypatch.setenv("PLBFS_BLOCK_CELLS", "64" if n < 65536 else "256")
+        s = GpuSolver(hm, case.params, case.patches_for(pm.patch_names))
+        s.set_state(rho + 1e-3 * np.sin(g["cx"][:n]), u * (1 + 0.02 * np.cos(g["cy"][:n])), v, w)
+        assert s.run(4)["rc"] == 0
+        out.append(s.state())
+        s.close()
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
