@@ -152,7 +152,8 @@ __global__ __launch_bounds__(kMaxFluxThreads) void kb_flux(DevMesh<S> m, DevPara
             R[2] += fbody[NR + r];
             R[3] += fbody[2 * NR + r];
         }
-        const int e = rk_update<S>(m, prm, visc, sa, i, r, load_rk<S>(m, sa, i, r, t0, t1, dtl), R, st_out, t0, t1, dtl, sq);
+        double dt;
+        const int e = rk_update<S>(m, prm, visc, sa, i, r, load_rk<S>(m, sa, i, r, t0, t1, dtl), R, st_out, t0, t1, dtl, sq, dt);
         if (e == 1) err = 1;
         else if (e == 2 && err == 0) err = 2;
     }

@@ -89,7 +89,7 @@ struct plbfs_ctx {
     bool ghost_state_set = true;            // false until plbfs_set_ghost_state where needed
     void *bflux = nullptr;                  // [4][n_border] border-face fluxes (storage precision)
     double *partials = nullptr;             // [n_blocks*5]
-    double *bmin = nullptr;                 // [n_blocks]
+    double *bmin = nullptr;                 // [n_min()]
     double *hist = nullptr;
     int hist_cap = 0;
     plbfs::Ctrl *ctrl = nullptr;
@@ -100,6 +100,8 @@ struct plbfs_ctx {
     size_t stage_lds = 0;  // LDS of k_stage, 0: gradients and fluxes are kernels of their own
     int cell_grid = 0;  // blocks of kBlock cells for the per-cell kernels
     int bound_blocks = 0;  // flux blocks that the scratch bound of plbfs_run_noalloc counts
+    // time-step minima: of the cell blocks, or of k_stage's flux blocks
+    int n_min() const { return stage_lds ? std::max(cell_grid, L.n_blocks) : cell_grid; }
     int total_steps = 0;
     std::vector<double> last_hist;
     IbmState ibm;

@@ -200,7 +200,7 @@ template <typename S, bool kAhead>
 __device__ __forceinline__ int cell_update(const DevMesh<S> &m, const DevParams &prm, StageArgs sa, const S *sF,
                                            bool force, int i, const CellIn<S> &in, V4<S> *__restrict__ st_out,
                                            double4 *__restrict__ t0, Acc<S> *__restrict__ t1,
-                                           double *__restrict__ dtl, double sq[4]) {
+                                           double *__restrict__ dtl, double sq[4], double &dt_next) {
     double R[4];
     gather_residual<S, kAhead>(m, i, in.faces, sF, m.max_items, 1, 0, R);
     if (force) {
@@ -208,7 +208,7 @@ __device__ __forceinline__ int cell_update(const DevMesh<S> &m, const DevParams 
         R[2] += in.force[1];
         R[3] += in.force[2];
     }
-    return rk_update<S, kAhead>(m, prm, prm.visc, sa, i, (size_t)i, in.rk, R, st_out, t0, t1, dtl, sq);
+    return rk_update<S, kAhead>(m, prm, prm.visc, sa, i, (size_t)i, in.rk, R, st_out, t0, t1, dtl, sq, dt_next);
 }
 
 template <typename S>
@@ -267,7 +267,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kFluxMin
         CellIn<S> in;
         in.faces = load_faces<S>(m, i);
         load_rk<S, kAhead>(m, sa, force, i, t0, t1, dtl, fbody, in);
-        const int e = cell_update<S, kAhead>(m, prm, sa, sF, force, i, in, st_out, t0, t1, dtl, sq);
+        double dt;
+        const int e = cell_update<S, kAhead>(m, prm, sa, sF, force, i, in, st_out, t0, t1, dtl, sq, dt);
         if (e == 1) err = 1;
         else if (e == 2 && err == 0) err = 2;
     }
@@ -290,7 +291,9 @@ __global__ __launch_bounds__(kBlock) void k_stage(DevMesh<S> m, DevParams prm, S
                                                   const Ctrl *__restrict__ ctrl, const V4<S> *__restrict__ st_in,
                                                   V4<S> *__restrict__ st_out, double4 *__restrict__ t0,
                                                   Acc<S> *__restrict__ t1, double *__restrict__ dtl,
-                                                  const double *__restrict__ fbody, double *__restrict__ partials) {
+                                                  const double *__restrict__ fbody, double *__restrict__ partials,
+                                                  double *__restrict__ bmin) {
+    static_assert(kOneKernelCells <= 64, "a wavefront has the block's cells");
     extern __shared__ double lds[];
     const int done = ctrl->done;
     const int blk = xcd_block(blockIdx.x, gridDim.x, 1);
@@ -360,13 +363,20 @@ __global__ __launch_bounds__(kBlock) void k_stage(DevMesh<S> m, DevParams prm, S
     }
     __syncthreads();
     double sq[4] = {0, 0, 0, 0};
-    const int err = live ? cell_update<S, true>(m, prm, sa, sF, force, c, in, st_out, t0, t1, dtl, sq) : 0;
+    double dt = 1e300;
+    const int err = live ? cell_update<S, true>(m, prm, sa, sF, force, c, in, st_out, t0, t1, dtl, sq, dt) : 0;
     block_sums(sa, blk, sq, err, partials);
+    // the block's cells are the first wavefront's
+    if (bmin && threadIdx.x < 64) {
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) dt = fmin(dt, __shfl_xor(dt, off, 64));
+        if (threadIdx.x == 0) bmin[blk] = dt;
+    }
 }
 
 // Global minimum of the local time steps for the "min" and "talts" modes
-// (Solver.cpp:1746-1773): every block reduces all cells (cheap; N is read once
-// per block from L2) -- done in two kernels to keep it deterministic.
+// (Solver.cpp:1746-1773): the blocks' minima, by this kernel or by k_stage, then
+// k_dt_apply.
 __global__ __launch_bounds__(kBlock) void k_dt_blockmin(int N, const Ctrl *__restrict__ ctrl,
                                                         const double *__restrict__ dtl, double *__restrict__ bmin) {
     if (ctrl->done) return;
@@ -539,10 +549,11 @@ __global__ __launch_bounds__(kBlock) void k_residual_only(DevMesh<S> m, DevParam
 // device share the array and race.
 constexpr size_t kScratchBytes = (size_t)8 << 20;
 // The bound counts kFluxBlockCells cells a block where the mesh size chose the block
-// size; the partials of the smaller blocks it may choose (up to 1,024 instead of 256,
-// or 5,958 instead of 4,096, 40 B each) fit behind it.
+// size; the partials of the smaller blocks it may choose (up to 1,024 instead of 256
+// with 8 B more for the minimum of each, or 5,958 instead of 4,096, 40 B each) fit behind it.
 constexpr size_t kScratchSpare = (size_t)128 << 10;
 static_assert(40 * ((size_t)16 * 65536 / kMinAutoBlock + 1 - 4096) + 512 <= kScratchSpare, "partials fit");
+static_assert(48 * (1024 - 256) + 512 <= kScratchSpare, "partials and minima of the smallest blocks fit");
 static __device__ __align__(256) double scratch[(kScratchBytes + kScratchSpare) / sizeof(double)];
 
 constexpr int kMaxScratchDevices = 64;
@@ -829,7 +840,7 @@ int create_ctx(const plbfs_mesh_view *mesh, const plbfs_params *params, const pl
         (rc = dalloc(c, (void **)&c->dtl, (size_t)N * sizeof(double))) ||
         (rc = dalloc(c, (void **)&c->fbody, (size_t)3 * N * sizeof(double))) ||
         (rc = dalloc(c, (void **)&c->partials, (size_t)L.n_blocks * 5 * sizeof(double))) ||
-        (rc = dalloc(c, (void **)&c->bmin, (size_t)c->cell_grid * sizeof(double))) ||
+        (rc = dalloc(c, (void **)&c->bmin, (size_t)c->n_min() * sizeof(double))) ||
         (rc = dalloc(c, (void **)&c->ctrl, sizeof(Ctrl))) ||
         (rc = dalloc(c, &c->bflux, (size_t)4 * std::max<int64_t>(L.n_border, 1) * sbytes)))
         return fail(rc);
@@ -999,19 +1010,26 @@ static const double kBeta[4] = {1.0 / 6.0, 1.0 / 3.0, 1.0 / 3.0, 1.0 / 6.0};
 struct RunScratch {
     Ctrl *ctrl;
     double *partials;  // [n_blocks * 5]
-    double *bmin;      // [cell_grid]
+    double *bmin;      // [n_min()]
     double *hist;      // [hist_cap * 4]
     int hist_cap;
 };
 
 static RunScratch ctx_scratch(plbfs_ctx *c) { return RunScratch{c->ctrl, c->partials, c->bmin, c->hist, c->hist_cap}; }
 
-static void launch_dt_modes(plbfs_ctx *c, const RunScratch &w) {
+static bool global_dt(const plbfs_ctx *c) {
+    return c->params.time_stepping == PLBFS_DT_MIN || c->params.time_stepping == PLBFS_DT_TALTS;
+}
+
+// have_min: k_stage left its blocks' minima (a launch of k_dt_blockmin less: step of 16k
+// cells 50.9 -> 49.1 us).
+static void launch_dt_modes(plbfs_ctx *c, const RunScratch &w, bool have_min) {
     const int N = c->L.N, nb = c->cell_grid;
-    if (c->params.time_stepping == PLBFS_DT_MIN || c->params.time_stepping == PLBFS_DT_TALTS) {
-        hipLaunchKernelGGL(k_dt_blockmin, dim3(nb), dim3(kBlock), 0, c->stream, N, w.ctrl, c->dtl, w.bmin);
-        hipLaunchKernelGGL(k_dt_apply, dim3(nb), dim3(kBlock), 0, c->stream, N, nb, c->params.time_stepping,
-                           w.ctrl, w.bmin, c->dtl);
+    if (global_dt(c)) {
+        if (!have_min)
+            hipLaunchKernelGGL(k_dt_blockmin, dim3(nb), dim3(kBlock), 0, c->stream, N, w.ctrl, c->dtl, w.bmin);
+        hipLaunchKernelGGL(k_dt_apply, dim3(nb), dim3(kBlock), 0, c->stream, N, have_min ? c->L.n_blocks : nb,
+                           c->params.time_stepping, w.ctrl, w.bmin, c->dtl);
     }
 }
 
@@ -1024,7 +1042,7 @@ static void launch_stages(plbfs_ctx *c, const DevMesh<S> &dm, const RunScratch &
             const StageArgs sa{kAlpha[k], kBeta[k], k};
             hipLaunchKernelGGL(k_stage<S>, dim3(nb), dim3(kBlock), c->stage_lds, c->stream, dm, c->prm, sa, w.ctrl,
                                (const V4<S> *)in, (V4<S> *)outb, (double4 *)c->t0, (Acc<S> *)c->t1, c->dtl, c->fbody,
-                               w.partials);
+                               w.partials, k == 3 && global_dt(c) ? w.bmin : nullptr);
             std::swap(in, outb);
             continue;
         }
@@ -1058,7 +1076,7 @@ static void launch_init_dt(plbfs_ctx *c, const DevMesh<S> &dm, const Ctrl *ctrl)
 static int launch_run_start(plbfs_ctx *c, const RunScratch &w) {
     if (c->f32) launch_init_dt<float>(c, c->dm32, w.ctrl);
     else launch_init_dt<double>(c, c->dm, w.ctrl);
-    launch_dt_modes(c, w);
+    launch_dt_modes(c, w, false);
     HIP_TRY(hipGetLastError());
     return PLBFS_OK;
 }
@@ -1072,7 +1090,7 @@ static int launch_step(plbfs_ctx *c, const RunScratch &w, bool timed, bool rebui
     if (rc) return rc;
     if (c->f32) launch_stages<float>(c, c->dm32, w, timed);
     else launch_stages<double>(c, c->dm, w, timed);
-    launch_dt_modes(c, w);
+    launch_dt_modes(c, w, c->stage_lds && !timed);
     {
         TimedLaunch t(c, PLBFS_KSTAT_REDUCE, timed);
         hipLaunchKernelGGL(k_finalize, dim3(1), dim3(kFinalizeThreads), 0, c->stream, nb, (double)c->L.N,
@@ -1218,7 +1236,7 @@ extern "C" int plbfs_run_noalloc(plbfs_ctx *c, int32_t max_steps, plbfs_result *
     w.partials = reinterpret_cast<double *>(p);
     p += round256((size_t)c->L.n_blocks * 5 * sizeof(double));
     w.bmin = reinterpret_cast<double *>(p);
-    p += round256((size_t)c->cell_grid * sizeof(double));
+    p += round256((size_t)c->n_min() * sizeof(double));
     w.hist = reinterpret_cast<double *>(p);
     w.hist_cap = max_steps;
     const auto t0 = std::chrono::steady_clock::now();

@@ -509,7 +509,8 @@ template <typename S, bool kAhead = false>
 __device__ __forceinline__ int rk_update(const DevMesh<S> &m, const DevParams &prm, double visc, StageArgs sa,
                                          int i, size_t r, const RkIn<S> &in, const double R[4],
                                          V4<S> *__restrict__ st_out, double4 *__restrict__ t0,
-                                         Acc<S> *__restrict__ t1, double *__restrict__ dtl, double sq[4]) {
+                                         Acc<S> *__restrict__ t1, double *__restrict__ dtl, double sq[4],
+                                         double &dt_next) {
     constexpr bool F32 = std::is_same<S, float>::value;
     const double dti = in.dt;
     const double4 ta = in.t0;
@@ -564,9 +565,10 @@ __device__ __forceinline__ int rk_update(const DevMesh<S> &m, const DevParams &p
     const double s0 = b0, s1 = b1 / b0, s2 = b2 / b0, s3 = b3 / b0;
     st_out[r] = V4<S>{(S)(s0 - r0), (S)s1, (S)s2, (S)s3};
     t0[r] = double4{b0, b1, b2, b3};
-    if (prm.time_stepping == PLBFS_DT_CONSTANT) dtl[r] = prm.cfl;
-    else dtl[r] = local_dt(prm, visc, s0, s1, kAhead ? in.cfl_area : m.cfl_area[i],
-                           kAhead ? in.vol : m.vol[i]);
+    dt_next = prm.time_stepping == PLBFS_DT_CONSTANT
+                  ? prm.cfl
+                  : local_dt(prm, visc, s0, s1, kAhead ? in.cfl_area : m.cfl_area[i], kAhead ? in.vol : m.vol[i]);
+    dtl[r] = dt_next;
     sq[0] += R[0] * R[0];
     sq[1] += R[1] * R[1];
     sq[2] += R[2] * R[2];
