@@ -552,7 +552,7 @@ int ibm_upload(plbfs_batch *b) {
         for (size_t j = 0; j < cp_cell.size(); j++) fr[(size_t)cp_cell[j] * b->B + cp_case[j]] = 1;
         if ((rc = bupload(M, &b->force_rec, fr))) return rc;
     }
-    HIP_TRY(hipMemset(b->fbody, 0, (size_t)3 * b->N * b->B * sizeof(double)));
+    HIP_TRY(hipMemsetAsync(b->fbody, 0, (size_t)3 * b->N * b->B * sizeof(double), b->base->stream));
     hipLaunchKernelGGL(k_ibm_weights, dim3((n_total + kIbmWide - 1) / kIbmWide), dim3(kIbmThreads), 0,
                        b->base->stream, a);
     HIP_TRY(hipGetLastError());
@@ -632,14 +632,17 @@ int build_batch_graph(plbfs_batch *b, int steps, hipGraphExec_t *exec) {
 // Clears step count, convergence, status and residual of case case_id (every
 // case when case_id < 0).  The other cases keep theirs: get_state reads a
 // case's step count to know whether its t0 holds primitives or conservatives.
+// On the stream that reads them: a memset of device memory need not block the host.
 int reset_case_ctl(plbfs_batch *b, int case_id = -1) {
     const size_t k0 = case_id < 0 ? 0 : (size_t)case_id;
     const size_t n = case_id < 0 ? (size_t)b->B : 1;
-    HIP_TRY(hipMemset(b->done + k0, 0, n * sizeof(int32_t)));
-    HIP_TRY(hipMemset(b->status + k0, 0, n * sizeof(int32_t)));
-    HIP_TRY(hipMemset(b->steps + k0, 0, n * sizeof(int32_t)));
-    HIP_TRY(hipMemset(b->conv + k0, 0, n * sizeof(int32_t)));
-    HIP_TRY(hipMemset(b->res + 4 * k0, 0, n * 4 * sizeof(double)));
+    hipStream_t st = b->base->stream;
+    HIP_TRY(hipMemsetAsync(b->done + k0, 0, n * sizeof(int32_t), st));
+    HIP_TRY(hipMemsetAsync(b->status + k0, 0, n * sizeof(int32_t), st));
+    HIP_TRY(hipMemsetAsync(b->steps + k0, 0, n * sizeof(int32_t), st));
+    HIP_TRY(hipMemsetAsync(b->conv + k0, 0, n * sizeof(int32_t), st));
+    HIP_TRY(hipMemsetAsync(b->res + 4 * k0, 0, n * 4 * sizeof(double), st));
+    HIP_TRY(hipStreamSynchronize(st));
     return PLBFS_OK;
 }
 
@@ -757,7 +760,7 @@ extern "C" int plbfs_batch_create(const plbfs_mesh_view *mesh, const plbfs_param
     b->status = reinterpret_cast<int32_t *>(b->res + (size_t)4 * n_cases);
     b->steps = b->status + n_cases;
     b->conv = b->steps + n_cases;
-    if (hipMemset(b->fbody, 0, NR * 3 * sizeof(double)) != hipSuccess || reset_case_ctl(b))
+    if (hipMemsetAsync(b->fbody, 0, NR * 3 * sizeof(double), b->base->stream) != hipSuccess || reset_case_ctl(b))
         return fail(plbfs_fail(PLBFS_ERR_HIP, "batch initialisation"));
     *out = b;
     return PLBFS_OK;

@@ -234,12 +234,12 @@ static int set_ibm(plbfs_ctx *c, const plbfs_ibm_nodes *nodes, int rebuilds) {
     }
     {
         const IbmArgs a = make_args(c);
+        HIP_TRY(hipMemsetAsync(c->fbody, 0, (size_t)3 * N * sizeof(double), c->stream));
         hipLaunchKernelGGL(k_ibm_weights, dim3((n + kIbmWide - 1) / kIbmWide), dim3(kIbmThreads), 0, c->stream,
                            a);
         HIP_TRY(hipGetLastError());
         HIP_TRY(hipStreamSynchronize(c->stream));
     }
-    HIP_TRY(hipMemset(c->fbody, 0, (size_t)3 * N * sizeof(double)));
     s.on = true;
     c->prm.use_body_force = 1;
     drop_graphs(c);

@@ -929,7 +929,9 @@ extern "C" int plbfs_set_state(plbfs_ctx *c, const double *rho, const double *u,
     if (rc) return rc;
     const int N = c->L.N;
     if (!c->f32) {
-        HIP_TRY(hipMemcpy(c->stA, c->t0, (size_t)4 * N * sizeof(double), hipMemcpyDeviceToDevice));
+        // on the stream that reads it: a copy inside the device need not block the host
+        HIP_TRY(hipMemcpyAsync(c->stA, c->t0, (size_t)4 * N * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
+        HIP_TRY(hipStreamSynchronize(c->stream));
     } else {
         std::vector<float> h((size_t)4 * N);
         const double *src[4] = {rho, u, v, w};

@@ -326,3 +326,21 @@ def test_flux_threads_on_few_blocks_change_nothing(gpu_available, precision, cas
         assert ra == rb
         for x, y in zip(fa, fb):
             assert np.array_equal(x, y)
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+def test_reseeded_case_reads_back_as_set(gpu_available, precision):
+    """The state of a case that has stepped, read directly behind plbfs_batch_set_state:
+    the primitives that were set, not divided by their density."""
+    pm = channel_mesh(10, 5, 5)
+    cases = cases_for(RES, precision)
+    hm, bt = make_batch(pm, cases)
+    rng = np.random.default_rng(6)
+    bt.set_state(-1, *initial_state(cases[0], oracle_for(pm, cases[0])))
+    for b in (1, 0, 2, 1):
+        assert bt.run(3)[0] == 0
+        st = [1.01 + 0.01 * rng.random(pm.n_cells)] + [0.01 * rng.random(pm.n_cells) for _ in range(3)]
+        bt.set_state(b, *st)
+        for x, y in zip(bt.state(b), st):
+            assert np.array_equal(x, y)
+    bt.close()

@@ -432,3 +432,22 @@ def test_block_order_over_the_xcds_changes_no_field(gpu_available, monkeypatch, 
         s.close()
     for a, b in zip(*out):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("dims", [(5, 4, 3), (21, 20, 20)])
+@pytest.mark.parametrize("precision", [0, 1])
+def test_state_reads_back_as_set(gpu_available, dims, precision):
+    """The state directly behind plbfs_set_state, before and after steps were taken, in
+    one copy and (above 8,192 cells) field by field: what was set, bit for bit."""
+    pm, case = channel_mesh(*dims), pc.channel_case(re=40.0, length_scale=3.0)
+    case.precision = precision
+    hm = HostMesh.from_polymesh(pm, case.visc, case.gamma, case.fneq_min)
+    s = GpuSolver(hm, case.params, case.patches_for(pm.patch_names))
+    rng = np.random.default_rng(5)
+    for _ in range(4):
+        st = [1.0 + 0.01 * rng.random(pm.n_cells)] + [0.01 * rng.random(pm.n_cells) for _ in range(3)]
+        s.set_state(*st)
+        for a, b in zip(s.state(), st):
+            assert np.array_equal(a, b)
+        assert s.run(3)["rc"] == 0
+    s.close()
