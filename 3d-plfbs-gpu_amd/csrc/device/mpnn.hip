@@ -883,7 +883,10 @@ extern "C" int plbfs_mpnn_loss_grad(plbfs_mpnn *n, const float *x, const float *
     HIP_TRY(hipMemcpyAsync(n->mask, mask, ny * sizeof(float), hipMemcpyHostToDevice, n->stream));
     int rc = loss_grad_device(n, loss);
     if (rc) return rc;
-    if (grads) HIP_TRY(hipMemcpy(grads, n->g, n->P * sizeof(float), hipMemcpyDeviceToHost));
+    // on the network's stream: without a loss to wait for, the kernels may still run
+    if (grads)
+        HIP_TRY(hipMemcpyAsync(grads, n->g, n->P * sizeof(float), hipMemcpyDeviceToHost, n->stream));
+    HIP_TRY(hipStreamSynchronize(n->stream));
     return PLBFS_OK;
 }
 

@@ -159,3 +159,18 @@ def test_saturated_units_match_reference(gpu_available, scale):
         near[dst[near[src]]] = True
     assert np.isnan(y[0, :4]).all()
     assert np.isfinite(y[~near]).all()
+
+
+def test_gradients_without_the_loss(gpu_available):
+    """plbfs_mpnn_loss_grad with loss NULL: the gradients of this call's inputs, as with
+    a loss, though nothing else is read back."""
+    N, src, dst, ef, x, tgt = problem(7)
+    net = mpnn.Mpnn(N, src, dst, ef, train=True)
+    net.set_params(mpnn.flatten_params(M.init_params(8), M.mlp_shapes()))
+    mask = mpnn.output_mask(N)
+    for scale in (1.0, 0.5, 2.0):
+        t = (tgt * scale).astype(np.float32)
+        g = np.zeros(net.P, np.float32)
+        mpnn.nat.check(mpnn.nat.lib().plbfs_mpnn_loss_grad(net.h, mpnn.fptr(x), mpnn.fptr(t), mpnn.fptr(mask), None,
+                                                           mpnn.fptr(g)))
+        assert np.array_equal(g, net.loss_grad(x, t, mask)[1])
