@@ -823,9 +823,11 @@ extern "C" int plbfs_mpnn_destroy(plbfs_mpnn *n) {
 
 extern "C" int plbfs_mpnn_set_params(plbfs_mpnn *n, const float *params) {
     if (!n || !params) return plbfs_fail(PLBFS_ERR_INPUT, "null argument");
-    HIP_TRY(hipMemcpy(n->w, params, n->P * sizeof(float), hipMemcpyHostToDevice));
-    HIP_TRY(hipMemset(n->m1, 0, n->P * sizeof(float)));
-    HIP_TRY(hipMemset(n->m2, 0, n->P * sizeof(float)));
+    // on the network's stream, behind an Adam step that may still run
+    HIP_TRY(hipMemcpyAsync(n->w, params, n->P * sizeof(float), hipMemcpyHostToDevice, n->stream));
+    HIP_TRY(hipMemsetAsync(n->m1, 0, n->P * sizeof(float), n->stream));
+    HIP_TRY(hipMemsetAsync(n->m2, 0, n->P * sizeof(float), n->stream));
+    HIP_TRY(hipStreamSynchronize(n->stream));
     n->adam_t = 0;
     return PLBFS_OK;
 }

@@ -174,3 +174,21 @@ def test_gradients_without_the_loss(gpu_available):
         mpnn.nat.check(mpnn.nat.lib().plbfs_mpnn_loss_grad(net.h, mpnn.fptr(x), mpnn.fptr(t), mpnn.fptr(mask), None,
                                                            mpnn.fptr(g)))
         assert np.array_equal(g, net.loss_grad(x, t, mask)[1])
+
+
+def test_parameters_set_behind_an_adam_step(gpu_available):
+    """plbfs_mpnn_set_params right behind an Adam step, which returns before its kernel
+    has run: the parameters that were set, and moments of zero."""
+    N, src, dst, ef, x, tgt = problem(9)
+    net = mpnn.Mpnn(N, src, dst, ef, train=True)
+    first, mask = mpnn.flatten_params(M.init_params(9), M.mlp_shapes()), mpnn.output_mask(N)
+    stepped = []
+    for _ in range(3):
+        net.set_params(first)
+        assert np.array_equal(net.params(), first)
+        net.loss_grad(x, tgt, mask)
+        net.adam_step(1e-3)
+        stepped.append(net.params())
+        net.adam_step(1e-3)
+    assert not np.array_equal(stepped[0], first)
+    assert np.array_equal(stepped[0], stepped[1]) and np.array_equal(stepped[0], stepped[2])
