@@ -30,6 +30,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cfloat>
 #include <cmath>
 #include <cstring>
 #include <numeric>
@@ -60,15 +61,18 @@ __host__ __device__ __forceinline__ unsigned short to_bf16(float f) {
     return (unsigned short)(u >> 16);
 }
 
-// SiLU and its derivative: a sigmoid of finite values only, 1 + e^-a from the exponential
-// of the nearest power of two and the rest (its argument in two parts, log2 e = hi + lo), and
-// the quotients by reciprocal and one correction with the exact remainder, which
-// rounds them correctly.  expf and the division spend a third of their instructions on
-// ranges that do not occur here: a below -88 is taken as -88 (SiLU -5e-37 there and 0 below), NaN stays NaN.
+// SiLU and its derivative: 1 + e^-a from the exponential of the nearest power of two
+// and the rest, the argument times log2 e in two parts (Cody and Waite, "Software Manual
+// for the Elementary Functions", 1980; log2 e = hi + lo), and the quotients by
+// reciprocal and one correction with the remainder that fma gives exactly (Markstein,
+// IBM J. Res. Dev. 34, 1990).  expf and the division spend a third of their
+// instructions on ranges that do not occur here: a below -88 is taken as -88 (SiLU
+// -5e-37 there and 0 below).  NaN stays NaN, and a / (1 + e^-a) at infinity is what it
+// is by division: SiLU(inf) = inf, SiLU(-inf) and both derivatives NaN.
 // Against 64 bits over [-85, 88] the errors are those of a / (1 + expf(-a)) (largest
 // 3.09, mean 0.27668, in 2^-24 of the result), and so are the network's outputs, bit
 // for bit.
-__device__ __forceinline__ float floor88(float a) { return a < -88.f ? -88.f : a; }
+__device__ __forceinline__ float floor88(float a) { return a < -88.f ? fmaf(a, 0.f, -88.f) : a; }
 __device__ __forceinline__ float one_plus_exp(float a) {
 #pragma clang fp contract(off)
     const float x = -fminf(a, 88.f);
@@ -79,7 +83,8 @@ __device__ __forceinline__ float one_plus_exp(float a) {
 }
 __device__ __forceinline__ float quot(float a, float d, float r) {  // a / d, r = rcp(d)
     const float q = a * r;
-    return fmaf(fmaf(-q, d, a), r, q);
+    // (the remainder at q = inf is NaN, which fmaxf drops; it is never below -FLT_MAX)
+    return fmaf(fmaxf(fmaf(-q, d, a), -FLT_MAX), r, q);
 }
 __device__ __forceinline__ float silu(float a) {
     a = floor88(a);

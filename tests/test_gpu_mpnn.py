@@ -192,3 +192,29 @@ def test_parameters_set_behind_an_adam_step(gpu_available):
         net.adam_step(1e-3)
     assert not np.array_equal(stepped[0], first)
     assert np.array_equal(stepped[0], stepped[1]) and np.array_equal(stepped[0], stepped[2])
+
+
+@pytest.mark.parametrize("sign", [1.0, -1.0])
+def test_overflowed_units_show(gpu_available, sign):
+    """A cell whose hidden units overflow to inf or -inf, all weights positive: SiLU is
+    a / (1 + e^-a), so its output is inf or NaN, as are those of the cells up to six
+    edges away, and no other cell's."""
+    N, src, dst, ef, x, _ = problem()
+    net = mpnn.Mpnn(N, src, dst, ef, train=False)
+    net.set_params(np.full(net.P, 0.01, np.float32))
+    x = np.abs(x).astype(np.float32)
+    x[0] = sign * 3e38  # 16 columns: beyond the largest float in the encoder's sums
+    P = mpnn.unflatten(net.params(), M.mlp_shapes())
+    P["enc"]["W1"][:] = 1.0
+    net.set_params(mpnn.flatten_params(P, M.mlp_shapes()))
+    y = net.forward(x)
+    near = np.zeros(N, bool)
+    near[0] = True
+    for _ in range(6):
+        near[dst[near[src]]] = True
+    assert 1 < near.sum() < N
+    if sign > 0:
+        assert np.all(y[near] == np.inf)
+    else:
+        assert np.isnan(y[near]).all()
+    assert np.isfinite(y[~near]).all()
