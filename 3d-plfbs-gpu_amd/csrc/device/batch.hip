@@ -662,14 +662,16 @@ int run_steps(plbfs_batch *b, int max_steps, float *ms_out) {
                            (const double4 *)b->stA, b->dtl);
     HIP_TRY(hipGetLastError());
     const int interval = std::max(1, b->params.check_interval);
+    const GraphNeeds need(max_steps, interval);
+    if ((need.many && (rc = build_batch_graph(b, kGraphSteps, &b->graph_many))) ||
+        (need.one && (rc = build_batch_graph(b, 1, &b->graph))))
+        return rc;
     HIP_TRY(hipEventRecord(c->ev0, c->stream));
     for (int s = 0; s < max_steps;) {
         const int left = std::min(interval - s % interval, max_steps - s);  // steps to the next check
         const bool many = left >= kGraphSteps;
         const int n = many ? kGraphSteps : 1;
-        hipGraphExec_t &g = many ? b->graph_many : b->graph;
-        if ((rc = build_batch_graph(b, n, &g))) return rc;
-        HIP_TRY(hipGraphLaunch(g, c->stream));
+        HIP_TRY(hipGraphLaunch(many ? b->graph_many : b->graph, c->stream));
         s += n;
         if (n == left) {
             HIP_TRY(hipMemcpyAsync(c->host, b->ctrl, sizeof(Ctrl), hipMemcpyDeviceToHost, c->stream));

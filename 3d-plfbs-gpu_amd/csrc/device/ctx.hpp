@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <vector>
 
 #include "../host/host_common.hpp"
@@ -171,6 +172,17 @@ int fields_to_host(plbfs_ctx *c, const double *src, double *const out[4]);
 
 // Drops the captured steps (their kernels' arguments are about to change).
 void drop_graphs(plbfs_ctx *c);
+
+// Whether max_steps steps with a check every `interval` replay the graph of kGraphSteps
+// steps and that of one.  A run captures them ahead of the events around its time loop.
+struct GraphNeeds {
+    bool many, one;
+    GraphNeeds(int max_steps, int interval) {
+        const int full = std::min(max_steps, interval), rest = max_steps % interval;
+        many = full >= plbfs::kGraphSteps;
+        one = full % plbfs::kGraphSteps || rest % plbfs::kGraphSteps;
+    }
+};
 
 // plbfs_create with an explicit flux block size (64..1024 cells, a multiple of
 // 64, or 0: chosen for the mesh), LDS sized for lds_cases cases per block (the batched solver sizes its

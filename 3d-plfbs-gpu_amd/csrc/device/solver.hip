@@ -1164,6 +1164,10 @@ extern "C" int plbfs_run(plbfs_ctx *c, int32_t max_steps, plbfs_result *out) {
     static_assert(sizeof(Ctrl) <= 256, "the history follows the control block");
     const bool small = hist0 + hist_bytes <= kHostBytes;
     bool have_hist = max_steps == 0;
+    const GraphNeeds need(max_steps, interval);
+    if (graph && ((need.many && (rc = build_graph(c, kGraphSteps, &c->graph_many))) ||
+                  (need.one && (rc = build_graph(c, 1, &c->graph_exec)))))
+        return rc;
     HIP_TRY(hipEventRecord(c->ev0, c->stream));
     for (int s = 0; s < max_steps;) {
         const int left = std::min(interval - s % interval, max_steps - s);  // steps to the next check

@@ -344,3 +344,20 @@ def test_reseeded_case_reads_back_as_set(gpu_available, precision):
         for x, y in zip(bt.state(b), st):
             assert np.array_equal(x, y)
     bt.close()
+
+
+def test_autotune_times_steps_alone(gpu_available):
+    """Trials of four steps, which replay one captured graph: the time a step that the
+    tuner returns is that of its tiling's later runs, within a quarter (a step of
+    this batch takes some 0.1 ms, a capture twice that).  The least of three each."""
+    pm = channel_mesh(10, 5, 5)
+    cases = cases_for(RES)
+    st = initial_state(cases[0], oracle_for(pm, cases[0]))
+    tuned, later = [], []
+    for _ in range(3):
+        hm, bt = make_batch(pm, cases)
+        bt.set_state(-1, *st)
+        tuned.append(bt.autotune(4)[3])
+        later += [bt.run(4)[1][0]["ms"] / 4 for _ in range(4)][1:]
+        bt.close()
+    assert min(tuned) < 1.25 * min(later), (tuned, later)
