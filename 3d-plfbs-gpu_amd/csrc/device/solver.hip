@@ -80,17 +80,17 @@ template <typename S>
 static std::vector<float4> pack_items(const Layout &L) {
     const size_t E = (size_t)L.n_items, K = kItemChunks<S>;
     std::vector<float4> v((E + 63) / 64 * 64 * K);
-    const double *g = L.it_geo.data();
     for (size_t e = 0; e < E; e++) {
+        const double *g = &L.it_geo[kGeoPerItem * e];
         float4 *p = &v[(e >> 6) * 64 * K + (e & 63)];
         S f[12];
         const int third = L.it_nbr[e] < 0 ? 0 : 8;  // the normal, or the neighbour's offset
         for (int a = 0; a < 3; a++) {
-            f[a] = (S)(g[a * E + e] * g[3 * E + e]);
-            f[3 + a] = (S)g[(5 + a) * E + e];
-            f[6 + a] = (S)g[(third + a) * E + e];
+            f[a] = (S)(g[a] * g[3]);
+            f[3 + a] = (S)g[5 + a];
+            f[6 + a] = (S)g[third + a];
         }
-        if (std::is_same<S, float>::value) f[9] = (S)g[4 * E + e];
+        if (std::is_same<S, float>::value) f[9] = (S)g[4];
         const int32_t on[2] = {L.it_own[e], L.it_nbr[e]};
         std::memcpy(reinterpret_cast<char *>(f) + 16 * K - sizeof on, on, sizeof on);
         for (size_t k = 0; k < K; k++) std::memcpy(p + 64 * k, reinterpret_cast<const char *>(f) + 16 * k, 16);
@@ -98,19 +98,24 @@ static std::vector<float4> pack_items(const Layout &L) {
     return v;
 }
 
-// The stencil weights of k_stage's places, in pieces of 16 B.
+// Neighbours and stencil weights of k_stage's places from their cells' (at creation: on the
+// host it took a tenth of a 32k-cell solver's creation).
 template <typename S>
-static std::vector<float4> pack_weights(const Layout &L) {
-    constexpr size_t kPer = 16 / sizeof(S), kPieces = (3 * kMaxSlots + kPer - 1) / kPer;
-    const size_t P = L.loc_cell.size(), N = (size_t)L.N;
-    std::vector<float4> v(P * kPieces);
-    for (size_t p = 0; p < P; p++) {
-        if (L.loc_cell[p] < 0) continue;
-        S w[kPer * kPieces] = {};
-        for (int q = 0; q < 3 * kMaxSlots; q++) w[q] = (S)L.st_w[(size_t)q * N + L.loc_cell[p]];
-        for (size_t k = 0; k < kPieces; k++) std::memcpy(&v[k * P + p], w + k * kPer, 16);
+__global__ __launch_bounds__(kBlock) void k_places(DevMesh<S> m, int32_t *__restrict__ nbr, float4 *__restrict__ w) {
+    constexpr int kPer = 16 / sizeof(S), kPieces = (3 * kMaxSlots + kPer - 1) / kPer;
+    const int p = blockIdx.x * kBlock + threadIdx.x;
+    if (p >= m.n_places) return;
+    const int c = m.loc_cell[p], cnt = c >= 0 ? m.st_cnt[c] : 0;
+    for (int s = 0; s < kMaxSlots; s++)
+        nbr[(size_t)s * m.n_places + p] = s < cnt ? m.st_nbr[(size_t)s * m.N + c] : kNoNbr;
+    for (int k = 0; k < kPieces; k++) {
+        S v[kPer];
+        for (int u = 0; u < kPer; u++) {
+            const int q = k * kPer + u;
+            v[u] = q < 3 * cnt ? m.st_w[(size_t)q * m.N + c] : (S)0;
+        }
+        __builtin_memcpy(&w[(size_t)k * m.n_places + p], v, 16);
     }
-    return v;
 }
 
 // Bound by HBM: a state read, the stencil (28 B a slot in FP64) and the record
@@ -774,16 +779,26 @@ int create_ctx(const plbfs_mesh_view *mesh, const plbfs_params *params, const pl
     d.loc_cell = d.loc_nbr = nullptr;
     d.it_loc = nullptr;
     d.loc_w = nullptr;
-    if (c->stage_lds && ((rc = upload(c, (int32_t **)&d.loc_cell, L.loc_cell)) ||
-                         (rc = upload(c, (int32_t **)&d.loc_nbr, L.loc_nbr)) ||
-                         (rc = upload(c, (float4 **)&d.loc_w,
-                                      c->f32 ? pack_weights<float>(L) : pack_weights<double>(L))) ||
-                         (rc = upload(c, (uint32_t **)&d.it_loc, L.it_loc))))
-        return fail(rc);
-    std::vector<int32_t> bpatch = L.b_patch;
-    if (bpatch.empty()) bpatch.push_back(0);
-    std::vector<int32_t> bpartner = L.b_partner;
-    if (bpartner.empty()) bpartner.push_back(-1);
+    int32_t *loc_nbr = nullptr;
+    float4 *loc_w = nullptr;
+    if (c->stage_lds) {
+        std::vector<int32_t> v(L.loc_cell);
+        v.insert(v.end(), L.it_loc.begin(), L.it_loc.end());
+        const size_t P = (size_t)d.n_places, per = 16 / sbytes;
+        if ((rc = upload(c, (int32_t **)&d.loc_cell, v)) ||
+            (rc = dalloc(c, (void **)&loc_nbr, P * kMaxSlots * sizeof(int32_t))) ||
+            (rc = dalloc(c, (void **)&loc_w, P * ((3 * kMaxSlots + per - 1) / per) * sizeof(float4))))
+            return fail(rc);
+        d.it_loc = reinterpret_cast<const uint32_t *>(d.loc_cell + P);
+        d.loc_nbr = loc_nbr;
+        d.loc_w = loc_w;
+    }
+    // patches of the boundary faces, then their partners; at least one of each
+    std::vector<int32_t> bface = L.b_patch;
+    if (bface.empty()) bface.push_back(0);
+    const size_t partners = bface.size();
+    bface.insert(bface.end(), L.b_partner.begin(), L.b_partner.end());
+    if (L.b_partner.empty()) bface.push_back(-1);
     std::vector<double> bdmag = L.b_dmag;
     if (bdmag.empty()) bdmag.push_back(1.0);
     c->ghost_fixed = L.b_fixed;
@@ -797,13 +812,14 @@ int create_ctx(const plbfs_mesh_view *mesh, const plbfs_params *params, const pl
         (rc = upload(c, (int32_t **)&d.blk_item_off, L.blk_item_off)) ||
         (rc = upload(c, (float4 **)&d.it_p, c->f32 ? pack_items<float>(L) : pack_items<double>(L))) ||
         (rc = upload(c, (uint16_t **)&d.it_side, std::vector<uint16_t>(L.it_side.begin(), L.it_side.end()))) ||
-        (rc = upload(c, (int32_t **)&d.b_patch, bpatch)) || (rc = upload(c, (int32_t **)&d.b_partner, bpartner)) ||
-        (rc = upload(c, (DevPatch **)&d.patches, dp)) || (rc = upload(c, &c->inv, L.inv)))
+        (rc = upload(c, (int32_t **)&d.b_patch, bface)) || (rc = upload(c, (DevPatch **)&d.patches, dp)) ||
+        (rc = upload(c, &c->inv, L.inv)))
         return fail(rc);
+    d.b_partner = d.b_patch + partners;
     if (!c->f32) {
-        if ((rc = upload(c, (double **)&d.st_w, L.st_w)) ||
-            (rc = upload(c, (double **)&d.it_dt, std::vector<double>(L.it_geo.begin() + 4 * L.n_items,
-                                                                     L.it_geo.begin() + 5 * L.n_items))) ||
+        std::vector<double> dt((size_t)L.n_items);
+        for (size_t e = 0; e < dt.size(); e++) dt[e] = L.it_geo[kGeoPerItem * e + 4];
+        if ((rc = upload(c, (double **)&d.st_w, L.st_w)) || (rc = upload(c, (double **)&d.it_dt, dt)) ||
             (rc = upload(c, (double **)&d.b_dmag, bdmag)))
             return fail(rc);
     } else {
@@ -832,6 +848,12 @@ int create_ctx(const plbfs_mesh_view *mesh, const plbfs_params *params, const pl
             (rc = upload(c, (DevPatch **)&e.patches, dp32)))
             return fail(rc);
     }
+    if (c->stage_lds) {
+        const dim3 grid((d.n_places + kBlock - 1) / kBlock);
+        if (c->f32) hipLaunchKernelGGL(k_places<float>, grid, dim3(kBlock), 0, c->stream, c->dm32, loc_nbr, loc_w);
+        else hipLaunchKernelGGL(k_places<double>, grid, dim3(kBlock), 0, c->stream, c->dm, loc_nbr, loc_w);
+        if (hipGetLastError() != hipSuccess) return fail(plbfs_fail(PLBFS_ERR_HIP, "k_places"));
+    }
     const size_t n4 = (size_t)4 * N * sbytes;
     const size_t nacc = (size_t)4 * N * (c->f32 ? sizeof(float) : sizeof(double));
     if ((rc = dalloc(c, (void **)&c->stA, n4)) || (rc = dalloc(c, (void **)&c->stB, (size_t)4 * N * sizeof(double))) ||
@@ -846,14 +868,9 @@ int create_ctx(const plbfs_mesh_view *mesh, const plbfs_params *params, const pl
         return fail(rc);
     c->dm.bflux = (double *)c->bflux;
     c->dm32.bflux = (float *)c->bflux;
-    {
-        std::vector<double> z((size_t)3 * N, 0.0);
-        if (hipMemcpy(c->fbody, z.data(), z.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess)
-            return fail(plbfs_fail(PLBFS_ERR_HIP, "upload body force"));
-        Ctrl h{};
-        if (hipMemcpy(c->ctrl, &h, sizeof(Ctrl), hipMemcpyHostToDevice) != hipSuccess)
-            return fail(plbfs_fail(PLBFS_ERR_HIP, "upload ctrl"));
-    }
+    if (hipMemsetAsync(c->fbody, 0, (size_t)3 * N * sizeof(double), c->stream) != hipSuccess ||
+        hipMemsetAsync(c->ctrl, 0, sizeof(Ctrl), c->stream) != hipSuccess)
+        return fail(plbfs_fail(PLBFS_ERR_HIP, "clear body force and control block"));
     DevParams &prm = c->prm;
     prm.visc = p.visc;
     prm.gamma = p.gamma;
@@ -1370,6 +1387,7 @@ extern "C" int plbfs_get_body_force(plbfs_ctx *c, double *f) {
     if (!c || !f) return plbfs_fail(PLBFS_ERR_INPUT, "null argument");
     const int N = c->L.N;
     std::vector<double> h((size_t)3 * N);
+    HIP_TRY(hipStreamSynchronize(c->stream));
     HIP_TRY(hipMemcpy(h.data(), c->fbody, h.size() * sizeof(double), hipMemcpyDeviceToHost));
     for (int n = 0; n < N; n++)
         for (int q = 0; q < 3; q++) f[(size_t)c->L.perm[n] * 3 + q] = h[(size_t)q * N + n];

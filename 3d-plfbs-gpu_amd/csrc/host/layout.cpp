@@ -19,7 +19,17 @@
 
 namespace plbfs {
 
-// Hilbert index via the transpose form of Skilling, "Programming the Hilbert
+// The low 21 bits of x, two places between any two of them.
+static uint64_t spread3(uint64_t x) {
+    x &= 0x1fffff;
+    x = (x | x << 32) & 0x1f00000000ffffull;
+    x = (x | x << 16) & 0x1f0000ff0000ffull;
+    x = (x | x << 8) & 0x100f00f00f00f00full;
+    x = (x | x << 4) & 0x10c30c30c30c30c3ull;
+    return (x | x << 2) & 0x1249249249249249ull;
+}
+
+// Hilbert index of up to 21 bits an axis via the transpose form of Skilling, "Programming the Hilbert
 // curve", AIP Conf. Proc. 707 (2004): axes -> transpose, then bit interleave.
 uint64_t hilbert_key3(uint32_t x, uint32_t y, uint32_t z, int bits) {
     uint32_t X[3] = {x, y, z};
@@ -27,13 +37,11 @@ uint64_t hilbert_key3(uint32_t x, uint32_t y, uint32_t z, int bits) {
     for (uint32_t Q = M; Q > 1; Q >>= 1) {
         const uint32_t P = Q - 1;
         for (int i = 0; i < 3; i++) {
-            if (X[i] & Q) {
-                X[0] ^= P;
-            } else {
-                const uint32_t t = (X[0] ^ X[i]) & P;
-                X[0] ^= t;
-                X[i] ^= t;
-            }
+            // X[0] inverted below bit Q where X[i] has it, else exchanged with X[i] (by
+            // masks: half of these branches would be mispredicted)
+            const uint32_t on = X[i] & Q ? ~0u : 0u, t = (X[0] ^ X[i]) & P & ~on;
+            X[0] ^= (P & on) | t;
+            X[i] ^= t;
         }
     }
     for (int i = 1; i < 3; i++) X[i] ^= X[i - 1];
@@ -41,10 +49,7 @@ uint64_t hilbert_key3(uint32_t x, uint32_t y, uint32_t z, int bits) {
     for (uint32_t Q = M; Q > 1; Q >>= 1)
         if (X[2] & Q) t ^= Q - 1;
     for (int i = 0; i < 3; i++) X[i] ^= t;
-    uint64_t key = 0;
-    for (int q = bits - 1; q >= 0; q--)
-        for (int i = 0; i < 3; i++) key = (key << 1) | ((X[i] >> q) & 1u);
-    return key;
+    return spread3(X[0]) << 2 | spread3(X[1]) << 1 | spread3(X[2]);
 }
 
 // the type codes of src/preprocessor.cpp:239-258
@@ -484,22 +489,18 @@ int build_layout(const plbfs_mesh_view &m, const plbfs_params &p, const plbfs_pa
     L.it_geo.resize((size_t)kGeoPerItem * E);
     if (G > 0)
         for (int a = 0; a < 3; a++) L.b0[a] = cc[3 * N + a] - fc[3 * NI + a];
-    static const int kPairs[7][3] = {{1, 0, 0}, {0, 1, 0}, {0, 0, 1}, {1, 1, 1}, {1, 1, -1}, {1, -1, 1}, {-1, 1, 1}};
     for (size_t e = 0; e < E; e++) {
         const int f = item_face[e];
         const int o = m.owner[f], nb = m.neighbour[f];
         L.it_own[e] = L.inv[o];
         L.it_nbr[e] = (f < NI) ? L.inv[nb] : -1 - (f - NI);
+        const double x = fn[3 * f], y = fn[3 * f + 1], z = fn[3 * f + 2];
+        const double en[7] = {x, y, z, x + y + z, x + y - z, x - y + z, -x + y + z};
         uint32_t side = 0;
-        for (int pr = 0; pr < 7; pr++) {
-            double c = 0.0;
-            for (int a = 0; a < 3; a++)
-                if (kPairs[pr][a]) c = c + kPairs[pr][a] * fn[3 * f + a];
-            if (c < 0.0) side |= 1u << pr;
-            else if (!(c > 0.0)) side |= 1u << (7 + pr);
-        }
+        for (int pr = 0; pr < 7; pr++)
+            side |= (uint32_t)(en[pr] < 0.0) << pr | (uint32_t)!(en[pr] < 0.0 || en[pr] > 0.0) << (7 + pr);
         L.it_side[e] = side;
-        double g[kGeoPerItem];
+        double *g = &L.it_geo[kGeoPerItem * e];
         g[0] = fn[3 * f];
         g[1] = fn[3 * f + 1];
         g[2] = fn[3 * f + 2];
@@ -511,20 +512,20 @@ int build_layout(const plbfs_mesh_view &m, const plbfs_params &p, const plbfs_pa
         g[8] = cc[3 * nb] - fc[3 * f];
         g[9] = cc[3 * nb + 1] - fc[3 * f + 1];
         g[10] = cc[3 * nb + 2] - fc[3 * f + 2];
-        for (int q = 0; q < kGeoPerItem; q++) L.it_geo[(size_t)q * E + e] = g[q];
     }
     // cells that each block reads
     L.one_kernel = block_cells == 0 && C == kOneKernelCells && !split_border;
     if (L.one_kernel) {
-        std::vector<std::vector<int32_t>> cells(L.n_blocks);
-        std::vector<int32_t> place(N, -1), of(N, -1);  // a cell's place in block of[cell]'s list
+        std::vector<int32_t> cells, first(L.n_blocks + 1, 0);  // the lists, one behind the other
+        std::vector<int32_t> place(N, -1), of(N, -1);          // a cell's place in block of[cell]'s list
+        cells.reserve((size_t)4 * N);
         L.it_loc.resize(E);
         for (int blk = 0; blk < L.n_blocks; blk++) {
             auto add = [&](int cell) {
                 if (of[cell] != blk) {
                     of[cell] = blk;
-                    place[cell] = (int)cells[blk].size();
-                    cells[blk].push_back(cell);
+                    place[cell] = (int)cells.size() - first[blk];
+                    cells.push_back(cell);
                 }
                 return (uint32_t)place[cell];
             };
@@ -534,18 +535,14 @@ int build_layout(const plbfs_mesh_view &m, const plbfs_params &p, const plbfs_pa
                 const uint32_t o = add(L.it_own[e]);
                 L.it_loc[e] = o | (partner < 0 ? o : add(partner)) << 16;
             }
-            L.max_local = std::max(L.max_local, (int)cells[blk].size());
+            first[blk + 1] = (int32_t)cells.size();
+            L.max_local = std::max(L.max_local, first[blk + 1] - first[blk]);
         }
         const size_t P = (size_t)L.n_blocks * L.max_local;
         L.loc_cell.assign(P, -1);
-        L.loc_nbr.assign(P * kMaxSlots, kNoNbr);
         for (int blk = 0; blk < L.n_blocks; blk++)
-            for (size_t k = 0; k < cells[blk].size(); k++) {
-                const size_t p = (size_t)blk * L.max_local + k;
-                L.loc_cell[p] = cells[blk][k];
-                for (int s = 0; s < L.st_cnt[cells[blk][k]]; s++)
-                    L.loc_nbr[s * P + p] = L.st_nbr[(size_t)s * N + cells[blk][k]];
-            }
+            std::copy(cells.begin() + first[blk], cells.begin() + first[blk + 1],
+                      L.loc_cell.begin() + (size_t)blk * L.max_local);
     }
     return PLBFS_OK;
 }

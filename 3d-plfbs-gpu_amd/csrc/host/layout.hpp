@@ -23,7 +23,7 @@
 namespace plbfs {
 
 constexpr int kMaxSlots = 6;  // LSQ slots per cell (the reference's RHS arrays hold 6, gradients.cpp)
-constexpr int32_t kNoNbr = INT32_MIN;  // no stencil neighbour (Layout::loc_nbr)
+constexpr int32_t kNoNbr = INT32_MIN;  // no stencil neighbour (DevMesh::loc_nbr)
 constexpr int kOneKernelCells = 64;  // flux block of a mesh below 65,536 cells
 constexpr int kMinAutoBlock = 176;  // smallest flux block that build_layout picks for a mesh of 65,536 cells or more
 constexpr int kGeoPerItem = 11;  // n(3), area, dt, r_owner(3), r_neighbour(3)
@@ -59,15 +59,14 @@ struct Layout {
     // where neither e.n < 0 nor e.n > 0 (both take the owner's); e.n summed in
     // x,y,z order in FP64 as src/Solver.cpp:958-1273
     std::vector<uint32_t> it_side;
-    std::vector<double> it_geo;  // [kGeoPerItem*E], component-major
+    std::vector<double> it_geo;  // [E][kGeoPerItem]
     double b0[3] = {0, 0, 0};    // boundary face 0: its ghost's centroid from the face centre
     // cells that a block's items read (one_kernel), in a list of max_local places per block: its
-    // own cells first, -1 behind the last.  loc_nbr holds the places' st_nbr, slot by slot for all
-    // lists, and it_loc the places of an item's owner and of its neighbour (a boundary face: its
-    // ghost's partner cell, or the owner) as two 16-bit values
+    // own cells first, -1 behind the last; it_loc holds the places of an item's owner and of its
+    // neighbour (a boundary face: its ghost's partner cell, or the owner) as two 16-bit values
     bool one_kernel = false;
     int max_local = 0;
-    std::vector<int32_t> loc_cell, loc_nbr;
+    std::vector<int32_t> loc_cell;
     std::vector<uint32_t> it_loc;
     // per-cell gather list in file face order, entries (index << 2) | border << 1 | is_owner:
     // index is the block-local slot, or with the border bit the border item's index
