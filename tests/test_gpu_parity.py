@@ -451,24 +451,3 @@ def test_state_reads_back_as_set(gpu_available, dims, precision):
             assert np.array_equal(a, b)
         assert s.run(3)["rc"] == 0
     s.close()
-
-
-def test_stage_kernel_lists_cost_little_at_creation(gpu_available, monkeypatch):
-    """A solver of 32k cells, which holds the stage kernel's lists, is created within
-    1.05 of the time of one that does not (256-cell blocks): the lists' share of the
-    host's work is some 4 %.  The least of eight creations each."""
-    import time
-    pm, case = channel_mesh(32, 32, 31), pc.channel_case(re=40.0, length_scale=4.0)
-    hm = HostMesh.from_polymesh(pm, case.visc, case.gamma, case.fneq_min)
-    ms = {"": [], "256": []}
-    for _ in range(8):
-        for blk in ms:
-            if blk:
-                monkeypatch.setenv("PLBFS_BLOCK_CELLS", blk)
-            else:
-                monkeypatch.delenv("PLBFS_BLOCK_CELLS", raising=False)
-            t0 = time.perf_counter()
-            s = GpuSolver(hm, case.params, case.patches_for(pm.patch_names))
-            ms[blk].append(1e3 * (time.perf_counter() - t0))
-            s.close()
-    assert min(ms[""]) < 1.05 * min(ms["256"]), ms
