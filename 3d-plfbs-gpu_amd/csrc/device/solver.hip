@@ -1057,8 +1057,9 @@ static void launch_stages(plbfs_ctx *c, const DevMesh<S> &dm, const RunScratch &
     const int nb = c->L.n_blocks;
     void *in = c->stA, *outb = c->stB;
     for (int k = 0; k < 4; k++) {
-        if (c->stage_lds && !timed) {
+        if (c->stage_lds) {
             const StageArgs sa{kAlpha[k], kBeta[k], k};
+            TimedLaunch t(c, PLBFS_KSTAT_FLUX, timed);
             hipLaunchKernelGGL(k_stage<S>, dim3(nb), dim3(kBlock), c->stage_lds, c->stream, dm, c->prm, sa, w.ctrl,
                                (const V4<S> *)in, (V4<S> *)outb, (double4 *)c->t0, (Acc<S> *)c->t1, c->dtl, c->fbody,
                                w.partials, k == 3 && global_dt(c) ? w.bmin : nullptr);
@@ -1109,7 +1110,7 @@ static int launch_step(plbfs_ctx *c, const RunScratch &w, bool timed, bool rebui
     if (rc) return rc;
     if (c->f32) launch_stages<float>(c, c->dm32, w, timed);
     else launch_stages<double>(c, c->dm, w, timed);
-    launch_dt_modes(c, w, c->stage_lds && !timed);
+    launch_dt_modes(c, w, c->stage_lds != 0);
     {
         TimedLaunch t(c, PLBFS_KSTAT_REDUCE, timed);
         hipLaunchKernelGGL(k_finalize, dim3(1), dim3(kFinalizeThreads), 0, c->stream, nb, (double)c->L.N,

@@ -408,8 +408,11 @@ def main():
     g_bytes, f_bytes = algorithmic_bytes(info, P=P, Gb=P)
     flux_ms = kt["flux"][0] / max(kt["flux"][1], 1)
     grad_ms = kt["grad"][0] / max(kt["grad"][1], 1)
+    one_kernel = kt["grad"][1] == 0  # below 65,536 cells, where the flux figure is the whole stage's
+    if one_kernel:
+        f_bytes, g_bytes = f_bytes + g_bytes, 0
     flux_gbs = f_bytes / (flux_ms * 1e-3) / 1e9
-    grad_gbs = g_bytes / (grad_ms * 1e-3) / 1e9
+    grad_gbs = 0.0 if one_kernel else g_bytes / (grad_ms * 1e-3) / 1e9
     ibm_ms = kt["ibm"][0] / max(args.steps, 1)
     print("kernels: flux %.3f ms (%.0f GB/s alg), grad %.3f ms (%.0f GB/s alg), ibm %.3f ms/step, reduce %.3f ms" %
           (flux_ms, flux_gbs, grad_ms, grad_gbs, ibm_ms, kt["reduce"][0] / max(kt["reduce"][1], 1)),
@@ -442,7 +445,8 @@ def main():
                    "block_cells": block_cells,
                    "lsq_determinant": "exact" if case.lsq_exact_det else "reference"},
         "roofline": {"bound": "hbm", "achieved": flux_gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                     "frac": flux_gbs / HBM_PEAK_GBS, "traffic": traffic, "kernel": "k_flux_update",
+                     "frac": flux_gbs / HBM_PEAK_GBS, "traffic": traffic,
+                     "kernel": "k_stage" if one_kernel else "k_flux_update",
                      "kernel_ms": flux_ms, "alg_bytes_per_launch": f_bytes,
                      "grad_kernel": {"achieved": grad_gbs, "kernel_ms": grad_ms, "alg_bytes_per_launch": g_bytes},
                      "step_alg_bytes_per_cell": 4 * (g_bytes + f_bytes) / pm.n_cells,

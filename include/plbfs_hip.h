@@ -205,8 +205,11 @@ int plbfs_eval_residual(plbfs_ctx *ctx, double *grads, double *R);
 /* Local time step of every interior cell for the current state [N]. */
 int plbfs_get_dt(plbfs_ctx *ctx, double *dt);
 
-/* Per-kernel device timing over the last plbfs_run (hipEvents recorded around
- * every launch when enabled).  name_out receives a NUL-separated list. */
+/* Per-kernel device timing over the plbfs_run calls since it was enabled (hipEvents
+ * recorded around every launch, which a run then makes directly instead of replaying
+ * graphs).  On a mesh whose stages run as one kernel (below 65,536 cells, without
+ * PLBFS_BLOCK_CELLS) that kernel counts under PLBFS_KSTAT_FLUX, its gradients with
+ * it, and PLBFS_KSTAT_GRAD has no launches. */
 int plbfs_enable_timing(plbfs_ctx *ctx, int32_t on);
 int plbfs_kernel_stats(plbfs_ctx *ctx, int32_t which, double *total_ms, int32_t *launches);
 

@@ -157,3 +157,25 @@ def test_staging_changes_nothing_in_the_two_kernels(gpu_available, monkeypatch, 
            for f, g in ((0, 1), (flux_stage, grad_stage))]
     assert out[0][0] == 0
     assert_equal(*out)
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("mode", ["local", "min"])
+@pytest.mark.parametrize("env", [{}, {"BLOCK_CELLS": 64}])
+def test_timed_run_launches_what_other_runs_launch(gpu_available, monkeypatch, env, mode, precision):
+    """Kernel statistics of a run: one launch a stage where the stage kernel serves the
+    mesh, counted as the flux's, a gradient and a flux launch elsewhere; same results."""
+    pm, case = channel_mesh(10, 6, 6), pc.channel_case(re=40.0, length_scale=4.0)
+    case.time_stepping = mode
+    case.precision = precision
+    st = perturbed_state(case, oracle_for(pm, case), amp=0.01, seed=3)
+    plain = results(solver(monkeypatch, pm, case, st, env), 5)
+    s = solver(monkeypatch, pm, case, st, env)
+    s.enable_timing(True)
+    r = s.run(5)
+    stats = [s.kernel_stats(k) for k in range(4)]
+    assert [n for _, n in stats] == [20 if env else 0, 20, 0, 5]
+    assert all((ms > 0) == (n > 0) for ms, n in stats)
+    timed = (r["rc"], list(s.state()) + [s.dt_local()], r["hist"])
+    s.close()
+    assert_equal(plain, timed)
