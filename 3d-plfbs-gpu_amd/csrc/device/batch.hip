@@ -572,7 +572,7 @@ void launch_batch_stages(plbfs_batch *b, const DevMesh<S> &dm_base) {
     const int64_t NR = (int64_t)b->N * b->B;
     const dim3 rgrid((unsigned)((NR + kBlock - 1) / kBlock));
     const dim3 fgrid(c->L.n_blocks, (b->B + b->C - 1) / b->C);
-    const dim3 fthreads(fgrid.x * fgrid.y <= kCus ? kMaxFluxThreads : kBlock);
+    const dim3 fthreads(fgrid.x * fgrid.y <= (unsigned)kCus ? kMaxFluxThreads : kBlock);
     DevParams prm = c->prm;
     prm.use_body_force = b->ibm_on ? 1 : 0;
     static const double kAl[4] = {1.0, 0.5, 0.5, 1.0};

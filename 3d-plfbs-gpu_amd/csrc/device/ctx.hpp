@@ -27,12 +27,12 @@ constexpr int kBlock = 256;
 constexpr int kGraphSteps = 4;
 // cells per flux block of a large mesh (face slots of one block share its LDS)
 constexpr int kFluxBlockCells = 256;
+// largest mesh whose flux blocks take contiguous ranges per XCD (create_ctx has the figures)
+constexpr int kXcdCells = 12 * 65536;
 // Dynamic LDS per flux workgroup.  gfx950 gives a workgroup 160 KiB
 // (hipDeviceProp_t::sharedMemPerBlock), static and dynamic LDS together; the
 // flux kernels' static arrays take at most 160 B, and a launch whose total
 // exceeds 160 KiB is not refused by the runtime but faults, so 1 KiB stays free.
-constexpr unsigned kCus = 256;
-constexpr int kXcdCells = 12 * 65536;
 constexpr int kMaxLds = 159 * 1024;
 constexpr size_t kMaxStageLds = 64 * 1024;  // of k_stage: two blocks a CU
 }

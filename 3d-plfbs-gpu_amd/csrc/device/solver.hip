@@ -554,11 +554,10 @@ __global__ __launch_bounds__(kBlock) void k_residual_only(DevMesh<S> m, DevParam
 // device share the array and race.
 constexpr size_t kScratchBytes = (size_t)8 << 20;
 // The bound counts kFluxBlockCells cells a block where the mesh size chose the block
-// size; the partials of the smaller blocks it may choose (up to 1,024 instead of 256
-// with 8 B more for the minimum of each, or 5,958 instead of 4,096, 40 B each) fit behind it.
-constexpr size_t kScratchSpare = (size_t)128 << 10;
-static_assert(40 * ((size_t)16 * 65536 / kMinAutoBlock + 1 - 4096) + 512 <= kScratchSpare, "partials fit");
-static_assert(48 * (1024 - 256) + 512 <= kScratchSpare, "partials and minima of the smallest blocks fit");
+// size; the partials of the smaller blocks it may choose (up to 1,024 blocks instead of 256,
+// 40 B each and 8 B for a minimum) fit behind it.
+constexpr size_t kScratchSpare = (size_t)40 << 10;
+static_assert(48 * (kResidentBlocks - 256) + 512 <= kScratchSpare, "partials and minima of the smallest blocks fit");
 static __device__ __align__(256) double scratch[(kScratchBytes + kScratchSpare) / sizeof(double)];
 
 constexpr int kMaxScratchDevices = 64;

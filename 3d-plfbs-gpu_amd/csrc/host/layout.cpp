@@ -127,22 +127,28 @@ struct NearestCell {
 //   - fewer 256-cell blocks than the 256 CUs: 64 cells.  Step in FP64, us, with 64 / 192 /
 //     256 cells and two kernels a stage: 216 hexes 62 / 82 / 82, 16k 94 / 118 / 131, 32k 101 /
 //     116 / 120.
-//   - up to 16 of them a CU: the size whose passes are full and that gives every CU the
-//     same number of blocks, by the estimate below.  221k hexes, 208 / 216 / 224 / 256
-//     cells (1064 / 1024 / 988 / 864 blocks of 754 / 782 / 809 / 919 items): flux 40.8 / 35.1 /
-//     38.8 / 40.3 us in FP64, 28.3 / 26.5 / 28.5 / 28.6 in FP32; 83k tets, 192 / 256 cells:
-//     20.2 / 22.5.
-//   - beyond: 256 cells (4.1M tets within 1 % up to 448).
+//   - up to 4 of them a CU: the size whose passes are full and that gives every CU the
+//     same number of blocks, by the estimate below, of those with at most 4 blocks a CU, which
+//     are all resident at once in both precisions.  221k hexes, 208 / 216 / 224 / 256 cells
+//     (1064 / 1024 / 988 / 864 blocks of 754 / 782 / 809 / 919 items): flux 40.8 / 35.1 /
+//     38.8 / 40.3 us in FP64, 28.3 / 26.5 / 28.5 / 28.6 in FP32; step, chosen size / 256 cells, of 85k
+//     hexes 131 / 135 in FP64 and 109 / 110 in FP32, 133k hexes 150 / 160 and 121 / 126, 94k
+//     tets 111 / 116 and 91 / 95.
+//   - beyond: 256 cells.  A block that waits for another's place evens the CUs out by
+//     itself, and the estimate's sizes only add border faces: step with 200 to 216 / 256 cells, 216k
+//     tets (1079 blocks) 169 / 163 us in FP64 and 127 / 125 in FP32, 257k tets 185 / 172 and
+//     137 / 131, 343k hexes 289 / 281 and 195 / 188, 623k tets 412 / 404 and 250 / 237, 885k
+//     hexes 709 / 723 and 436 / 450; 4.1M tets within 1 % up to 448.
 static int auto_block_cells(const plbfs_mesh_view &m, const std::vector<int32_t> &inv) {
-    constexpr int kCus = 256, kThreads = 256;
+    constexpr int kThreads = 256;
     const int64_t N = m.n_cells;
     if (N < (int64_t)kCus * 256) return kOneKernelCells;
-    if (N > (int64_t)16 * kCus * 256) return 256;
+    if (N > (int64_t)kResidentBlocks * 256) return 256;
     int64_t cut = 0;  // faces between two 256-cell blocks; their number goes with the blocks' surface
     for (int f = 0; f < m.n_internal_faces; f++) cut += inv[m.owner[f]] / 256 != inv[m.neighbour[f]] / 256;
     int best = 256;
     double best_cost = 1e300;
-    for (int b = 256; b >= kMinAutoBlock; b -= 8) {
+    for (int b = 256; b >= kMinAutoBlock && (N + b - 1) / b <= kResidentBlocks; b -= 8) {
         const double blocks = (double)((N + b - 1) / b);
         const double items = (m.n_faces + cut * std::cbrt(256.0 / b)) / blocks;
         // the mean block may exceed whole passes by a few items (half the blocks then

@@ -25,6 +25,8 @@ namespace plbfs {
 constexpr int kMaxSlots = 6;  // LSQ slots per cell (the reference's RHS arrays hold 6, gradients.cpp)
 constexpr int32_t kNoNbr = INT32_MIN;  // no stencil neighbour (DevMesh::loc_nbr)
 constexpr int kOneKernelCells = 64;  // flux block of a mesh below 65,536 cells
+constexpr int kCus = 256;  // of an MI355X
+constexpr int kResidentBlocks = 4 * kCus;  // flux blocks of 256 threads that run at once
 constexpr int kMinAutoBlock = 176;  // smallest flux block that build_layout picks for a mesh of 65,536 cells or more
 constexpr int kGeoPerItem = 11;  // n(3), area, dt, r_owner(3), r_neighbour(3)
 

@@ -179,3 +179,19 @@ def test_timed_run_launches_what_other_runs_launch(gpu_available, monkeypatch, e
     timed = (r["rc"], list(s.state()) + [s.dt_local()], r["hist"])
     s.close()
     assert_equal(plain, timed)
+
+
+@pytest.mark.parametrize("dims,tets,most", [((48, 48, 48), False, 255), ((62, 62, 62), False, 256),
+                                            ((32, 32, 32), True, 256), ((33, 33, 33), True, 256),
+                                            ((35, 35, 35), True, 256), ((66, 65, 65), False, 256)])
+def test_small_flux_blocks_all_run_at_once(gpu_available, monkeypatch, dims, tets, most):
+    """The mesh size chooses fewer than 256 cells a flux block only while all blocks find a
+    place, four a CU: 215,622 and 257,250 tets and 278,850 hexes do not."""
+    pm, case = channel_mesh(*dims, tets=tets), pc.channel_case(re=40.0, length_scale=6.0, fneq_min=0.55)
+    monkeypatch.delenv("PLBFS_BLOCK_CELLS", raising=False)
+    hm = HostMesh.from_polymesh(pm, case.visc, case.gamma, case.fneq_min)
+    s = GpuSolver(hm, case.params, case.patches_for(pm.patch_names))
+    info = s.layout_info()
+    s.close()
+    assert 176 <= info["block_cells"] <= most
+    assert info["block_cells"] == 256 or info["blocks"] <= 1024
