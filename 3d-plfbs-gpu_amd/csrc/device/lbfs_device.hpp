@@ -93,7 +93,7 @@ struct DevMesh {
     int n_border;
     S *bflux;
     int xcd_remap;
-    int block_cells;  // cells per flux block (a multiple of 64)
+    int block_cells;  // cells per flux block (a multiple of 8)
     int stage;        // 1: flux blocks stage their own cells' records in LDS
     int grad_stage;   // 1: gradient blocks stage their own cells' states in LDS
     int max_slots;    // most stencil slots of a cell

@@ -119,8 +119,9 @@ __global__ __launch_bounds__(kBlock) void k_places(DevMesh<S> m, int32_t *__rest
 }
 
 // Bound by HBM: a state read, the stencil (28 B a slot in FP64) and the record
-// written are 241 B a tet, 0.99 GB in 0.187 ms on 4.1M tets in FP64 (5.3 TB/s, where
-// a large copy reaches 4.75-5.1); 0.239 ms with each lane storing its own record.
+// written are 241 B a tet, 0.98 GB in 0.181 ms on 4.1M tets in FP64 (5.4 TB/s; 6.0 by
+// the counters' 1.08 GB, part of it from the last-level cache, where a large copy reaches
+// 4.75-5.1); 0.239 ms with each lane storing its own record.
 template <typename S>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) void k_grad(DevMesh<S> m, const Ctrl *__restrict__ ctrl,
                                                  const V4<S> *__restrict__ st, V4<S> *__restrict__ grad) {

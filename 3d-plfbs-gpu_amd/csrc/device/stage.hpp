@@ -60,8 +60,6 @@ __device__ __forceinline__ T wave_sum(T x) {
     return x;
 }
 
-// Least-squares gradient of cell i (src/gradients.cpp:319-389): folded stencil
-// weights times neighbour differences; ghost neighbours from the owner's patch.
 // Passes a value through an empty asm statement (no instruction is emitted).
 // Without it the optimiser merges "load from LDS" and "load from global" on
 // the two sides of a branch into one flat load through a selected pointer,
@@ -92,6 +90,8 @@ struct StagedStates {
     }
 };
 
+// Least-squares gradient of cell i (src/gradients.cpp:319-389): folded stencil
+// weights times neighbour differences; ghost neighbours from the owner's patch.
 //
 // The slots' indices are all loaded first, and the neighbours and weights of kSlots
 // slots before their sums: with each slot's index behind the last slot's branch

@@ -190,9 +190,11 @@ int plbfs_run(plbfs_ctx *ctx, int32_t max_steps, plbfs_result *out);
  * kernels with the same results as plbfs_run, but launches them directly (no
  * graph, no events; solve_ms is host wall time) and keeps the control block,
  * per-block residual partials, dt minima and the residual history in a
- * fixed array of 8 MiB per device, held until the process ends.  A call needs
- * about 256 B + 40 B per flux block + 8 B per 256 cells + 32 B per step of it
- * and fails with PLBFS_ERR_INPUT beyond that.  hist_out [4*max_steps] (or
+ * fixed array per device, held until the process ends.  A call may take 8 MiB
+ * of it: 256 B + 40 B per flux block + 8 B per 256 cells, each rounded up to
+ * 256 B, + 32 B per step, and fails with PLBFS_ERR_INPUT beyond that.  Where the
+ * mesh size chose the block size, blocks count as of 256 cells; what smaller
+ * blocks take beyond that lies behind the 8 MiB.  hist_out [4*max_steps] (or
  * NULL) receives the residual history; plbfs_get_residual_history keeps to
  * plbfs_run.  Calls that overlap on one device share the array and race. */
 int plbfs_run_noalloc(plbfs_ctx *ctx, int32_t max_steps, plbfs_result *out, double *hist_out);
@@ -216,7 +218,9 @@ int plbfs_kernel_stats(plbfs_ctx *ctx, int32_t which, double *total_ms, int32_t 
 /* Layout facts for roofline accounting, written to info[0..9]: cells, faces,
  * face work items per stage (faces on block borders are evaluated by both
  * blocks), stencil slots, boundary faces, flux blocks, most items in one
- * block, gather entries, cells per flux block, LDS bytes per flux block. */
+ * block, gather entries, cells per flux block, LDS bytes per block of the flux
+ * kernel (not of the one that serves meshes below 65,536 cells, which holds the
+ * gradients too). */
 int plbfs_layout_info(plbfs_ctx *ctx, int64_t *info10);
 
 /* ---- Post-processing (src/post_processing.cpp:50-173) ---------------------

@@ -25,8 +25,9 @@ typedef struct plbfs_mpnn plbfs_mpnn;
 /* Number of FP32 parameters. */
 int plbfs_mpnn_n_params(void);
 /* Graph of n_nodes nodes and n_edges directed edges src -> dst with 16 edge
- * features each ([n_edges*16]); train != 0 keeps every layer's activations for
- * the backward pass. */
+ * features each ([n_edges*16]); train != 0 also keeps every layer's node states
+ * and mean messages as bfloat16 (the backward pass computes the hidden
+ * activations again from them) and allocates its scratch. */
 int plbfs_mpnn_create(int32_t n_nodes, int32_t n_edges, const int32_t *src, const int32_t *dst,
                       const float *edge_feat, int32_t train, plbfs_mpnn **out);
 int plbfs_mpnn_destroy(plbfs_mpnn *net);
