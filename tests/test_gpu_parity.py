@@ -11,7 +11,8 @@ from helpers import (cavity_mesh, channel_mesh, initial_state, oracle_for, perio
                      perturbed_state, rel_err)
 from plbfs import _native as nat
 from plbfs import case as pc
-from plbfs.solver import GpuSolver, HostMesh
+from plbfs import meshgen
+from plbfs.solver import GpuBatch, GpuSolver, HostMesh
 
 pytestmark = pytest.mark.gpu
 
@@ -451,3 +452,36 @@ def test_state_reads_back_as_set(gpu_available, dims, precision):
             assert np.array_equal(a, b)
         assert s.run(3)["rc"] == 0
     s.close()
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("dims,lengths", [((6, 5, 4), (9.0, 6.25, 3.0)), ((17, 9, 9), (25.5, 11.25, 6.75))])
+def test_rest_stays_at_rest_bit_for_bit(gpu_available, monkeypatch, dims, lengths, precision):
+    """A box of uniform density at rest, whose cells' volume is no power of two: the
+    pressure fluxes through a cell's opposite faces are equal and cancel exactly in its
+    residual, so nothing ever moves; by the stage kernel, the two kernels and a batch."""
+    pm = meshgen.box_mesh(*dims, lengths=lengths, permute_seed=3, patch_types=pc.CAVITY_PATCHES)
+    case = pc.cavity_case(lid_u=0.0)
+    case.precision = precision
+    case.tolerance = 0.0
+    hm = HostMesh.from_polymesh(pm, case.visc, case.gamma, case.fneq_min)
+    n = pm.n_cells
+    st = [np.full(n, 1.03)] + [np.zeros(n)] * 3
+    patches = case.patches_for(pm.patch_names)
+    for blk in ("", "64"):
+        if blk:
+            monkeypatch.setenv("PLBFS_BLOCK_CELLS", blk)
+        s = GpuSolver(hm, case.params, patches)
+        s.set_state(*st)
+        assert not s.eval_residual()[0].any()
+        assert s.run(20)["steps"] == 20
+        for a, b in zip(s.state(), st):
+            assert np.array_equal(a, b)
+        s.close()
+    bt = GpuBatch(hm, case.params, patches, [case.visc] * 3)
+    bt.set_state(-1, *st)
+    assert bt.run(20)[0] == 0
+    for k in range(3):
+        for a, b in zip(bt.state(k), st):
+            assert np.array_equal(a, b)
+    bt.close()
